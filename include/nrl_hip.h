@@ -429,6 +429,10 @@ int nrl_group_baseline_std(const int64_t* prompts, int64_t batch, int64_t prompt
  * nrl_gather_logprob_*: ChunkedDistributedGatherLogprob (model_utils.py:722-836): out[r, k] = log p at
  *   indices[r, k] (int64 [rows, K], global ids; 0 outside [vocab_start, vocab_end)); backward
  *   -p_v * sum_k g_k + sum over the k with indices[r, k] == v of g_k.
+ * nrl_gather_entropy_*: both reductions of the same rows in one pass each way (h_out / h NULL: the gathered
+ *   log-probabilities alone).  indices [n_outer, >= n_inner, K]: K values per row, index_stride_outer elements between two
+ *   outer indices; grad [n_outer, n_inner, K], grad_h [n_outer, n_inner].  dlogits has d_n_inner >= n_inner rows per outer
+ *   index; rows from n_inner on, and rows whose upstream gradients are all zero, are zero-filled.
  * nrl_soft_cross_entropy_*: DistributedCrossEntropy (model_utils.py:209-264): ce_out[r] =
  *   -sum_v softmax(teacher)_v * log_softmax(student)_v; backward g * (softmax(student) - softmax(teacher)).
  *   teacher: same dtype and [n_outer, n_inner, vocab] shape as the student, with its own row strides.
@@ -440,6 +444,11 @@ int nrl_gather_logprob_fwd(const nrl_rows* rows, const int64_t* indices, int64_t
                            void* stream);
 int nrl_gather_logprob_bwd(const nrl_rows* rows, const int64_t* indices, int64_t k, const float* lse, const float* grad,
                            void* dlogits, int64_t d_stride_outer, int64_t d_stride_inner, void* stream);
+int nrl_gather_entropy_fwd(const nrl_rows* rows, const int64_t* indices, int64_t k, int64_t index_stride_outer, float* out,
+                           float* h_out, float* lse_out, void* stream);
+int nrl_gather_entropy_bwd(const nrl_rows* rows, const int64_t* indices, int64_t k, int64_t index_stride_outer,
+                           const float* lse, const float* h, const float* grad_h, const float* grad, void* dlogits,
+                           int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, void* stream);
 int nrl_soft_cross_entropy_fwd(const nrl_rows* student, const void* teacher, int64_t t_stride_outer,
                                int64_t t_stride_inner, float* ce_out, float* lse_student_out, float* lse_teacher_out,
                                void* stream);

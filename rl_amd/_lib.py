@@ -109,6 +109,8 @@ SIGNATURES = {
     "nrl_neg_entropy_bwd": (C.c_int, [C.POINTER(NrlRows), _P, _P, _P, _P, _I64, _I64, _P]),
     "nrl_gather_logprob_fwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _P, _P, _P]),
     "nrl_gather_logprob_bwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _P, _P, _P, _I64, _I64, _P]),
+    "nrl_gather_entropy_fwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _I64, _P, _P, _P, _P]),
+    "nrl_gather_entropy_bwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _I64, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P]),
     "nrl_soft_cross_entropy_fwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _I64, _P, _P, _P, _P]),
     "nrl_soft_cross_entropy_bwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _I64, _P, _P, _P, _P, _I64, _I64, _P]),
     "nrl_nonzero_indices": (C.c_int, [_P, _I64, _P, _P, _P]),
@@ -125,7 +127,7 @@ SIGNATURES = {
 _lib = None
 
 
-ABI_VERSION = 111  # nrl_version() of the library these signatures describe
+ABI_VERSION = 112  # nrl_version() of the library these signatures describe
 
 
 def load() -> C.CDLL:

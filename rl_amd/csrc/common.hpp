@@ -146,6 +146,13 @@ template <> struct Row<NRL_F16> {
     }
 };
 
+// number of leading elements before the first 16-byte boundary of a row
+template <int DT> __device__ __forceinline__ int64_t row_head(const void* row, int64_t vocab) {
+    const uintptr_t a = reinterpret_cast<uintptr_t>(row);
+    const int64_t h = static_cast<int64_t>(((16 - (a & 15)) & 15) / Row<DT>::BYTES);
+    return h < vocab ? h : vocab;
+}
+
 // temperature applied the way an in-place divide of the logits tensor rounds it
 template <int DT, int TEMP> __device__ __forceinline__ float scale_logit(float x, float tparam) {
     if constexpr (TEMP == 0) return x;

@@ -31,47 +31,6 @@ template <int DT> __device__ __forceinline__ bool vec_ok(const void* row, int64_
     return (reinterpret_cast<uintptr_t>(row) & 15) == 0 && vocab % Row<DT>::EPV == 0;
 }
 
-// fv(values of one 16-byte vector) / f1(one element) over the row, each thread taking a strided share
-template <int DT, class FV, class F1> __device__ __forceinline__ void row_for_each_vec(const void* row, int64_t vocab, FV fv, F1 f1) {
-    constexpr int EPV = Row<DT>::EPV;
-    const int tid = threadIdx.x;
-    if (!vec_ok<DT>(row, vocab)) {
-        for (int64_t i = tid; i < vocab; i += kDBlock) f1(Row<DT>::load1(row, i));
-        return;
-    }
-    const u32x4* xv = static_cast<const u32x4*>(row);
-    const int64_t nvec = vocab / EPV;
-    int64_t base = 0;
-    for (; base + kDUnroll * kDBlock <= nvec; base += kDUnroll * kDBlock) {
-        u32x4 q[kDUnroll];
-#pragma unroll
-        for (int u = 0; u < kDUnroll; ++u) q[u] = __builtin_nontemporal_load(xv + base + u * kDBlock + tid);
-#pragma unroll
-        for (int u = 0; u < kDUnroll; ++u) {
-            float t[EPV];
-            Row<DT>::decode(q[u], t);
-            fv(t);
-        }
-    }
-    for (int64_t vi = base + tid; vi < nvec; vi += kDBlock) {
-        float t[EPV];
-        Row<DT>::decode(__builtin_nontemporal_load(xv + vi), t);
-        fv(t);
-    }
-}
-
-// f(x) for every element of the row
-template <int DT, class F> __device__ __forceinline__ void row_for_each(const void* row, int64_t vocab, F f) {
-    constexpr int EPV = Row<DT>::EPV;
-    row_for_each_vec<DT>(
-        row, vocab,
-        [&](const float(&t)[EPV]) {
-#pragma unroll
-            for (int k = 0; k < EPV; ++k) f(t[k]);
-        },
-        f);
-}
-
 // out[i] = f(x[i], y[i], i) over one row; y may be NULL (then f receives 0 for it)
 template <int DT, class F>
 __device__ __forceinline__ void row_map(const void* xrow, const void* yrow, void* out, int64_t vocab, F f) {
@@ -101,130 +60,209 @@ template <int DT> __device__ __forceinline__ void row_fill_zero(void* out, int64
     row_map<DT>(out, nullptr, out, vocab, [](float, float, int64_t) { return 0.f; });
 }
 
-// online (max, sum exp, sum exp * (x - max)): enough for the log-sum-exp and for sum_v p_v x_v
-struct Ent {
-    float m, s, t;
-};
-__device__ __forceinline__ void ent_push(Ent& a, float x) {
-    if (x > a.m) {  // (a batch of 8 with one rescale and no branch measured 4 % slower here, unlike in the soft cross entropy)
-        const float d = a.m - x, e = fast_exp2(d * kLog2e);
-        a.t = e * (a.t + d * a.s);
-        a.s = e * a.s;
-        a.m = x;
+// ---------------------------------------------------------------------------------------------
+// per row: log-sum-exp, sum_v p_v log p_v (ENT) and the log-probabilities at K given indices (K may be 0)
+// ---------------------------------------------------------------------------------------------
+// Online accumulator in base-2 units: s = sum 2^(x log2e - m2), t = the same sum weighted with its exponents.  The
+// reference point m2 is a whole number, so moving it scales by an exact power of two and the exponents themselves carry
+// one rounding each; without ENT t is not kept.
+template <bool ENT> struct RowSums {
+    float m2 = -1e30f, s = 0.f, t = 0.f;
+    __device__ __forceinline__ void move_to(float m) {  // m >= m2
+        const float d = m2 - m, e = fast_exp2(d);
+        if (ENT) t = e * __builtin_fmaf(d, s, t);
+        s *= e;
+        m2 = m;
     }
-    const float d = x - a.m, p = fast_exp2(d * kLog2e);
-    a.s += p;
-    a.t += p > 0.f ? p * d : 0.f;  // a -inf logit has probability 0 and adds nothing
-}
-__device__ __forceinline__ Ent ent_merge(Ent a, Ent b) {
-    const float m = fmaxf(a.m, b.m), da = a.m - m, db = b.m - m;
-    const float ea = fast_exp2(da * kLog2e), eb = fast_exp2(db * kLog2e);
-    Ent r;
-    r.m = m;
-    r.s = a.s * ea + b.s * eb;
-    r.t = ea * (a.t + da * a.s) + eb * (b.t + db * b.s);
-    return r;
-}
-__device__ __forceinline__ Ent ent_block(Ent a, Ent* smem) {
+    template <int N> __device__ __forceinline__ void push(const float (&v)[N]) {
+        float vm = v[0];
+#pragma unroll
+        for (int k = 1; k < N; ++k) vm = fmaxf(vm, v[k]);
+        move_to(fmaxf(m2, ceilf(vm * kLog2e)));
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const float y = __builtin_fmaf(v[k], kLog2e, -m2), p = fast_exp2(y);
+            s += p;
+            if (ENT) t = __builtin_fmaf(p, fmaxf(y, -1e30f), t);  // a -inf logit has probability 0 and adds nothing
+        }
+    }
+    __device__ __forceinline__ void push1(float x) {
+        const float one[1] = {x};
+        push<1>(one);
+    }
+    __device__ __forceinline__ void merge(RowSums o) {
+        const float m = fmaxf(m2, o.m2);
+        move_to(m);
+        o.move_to(m);
+        s += o.s;
+        t += o.t;
+    }
+};
+
+template <bool ENT> __device__ __forceinline__ RowSums<ENT> sums_block(RowSums<ENT> a, float (*smem)[3]) {
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) {
-        Ent o;
-        o.m = __shfl_xor(a.m, off, kWave);
+        RowSums<ENT> o;
+        o.m2 = __shfl_xor(a.m2, off, kWave);
         o.s = __shfl_xor(a.s, off, kWave);
-        o.t = __shfl_xor(a.t, off, kWave);
-        a = ent_merge(a, o);
+        if (ENT) o.t = __shfl_xor(a.t, off, kWave);
+        a.merge(o);
     }
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    if (lane == 0) { smem[w][0] = a.m2; smem[w][1] = a.s; smem[w][2] = a.t; }
     __syncthreads();
-    if (lane == 0) smem[w] = a;
-    __syncthreads();
-    Ent tot = smem[0];
+    RowSums<ENT> tot;
+    tot.m2 = smem[0][0]; tot.s = smem[0][1]; tot.t = smem[0][2];
 #pragma unroll
-    for (int i = 1; i < kDWaves; ++i) tot = ent_merge(tot, smem[i]);
+    for (int i = 1; i < kDWaves; ++i) {
+        RowSums<ENT> o;
+        o.m2 = smem[i][0]; o.s = smem[i][1]; o.t = smem[i][2];
+        tot.merge(o);
+    }
     return tot;
 }
 
-// ---------------------------------------------------------------------------------------------
-// sum_v p_v log p_v
-// ---------------------------------------------------------------------------------------------
-template <int DT>
-__global__ __launch_bounds__(kDBlock) void neg_entropy_fwd_kernel(RowsView x, float* __restrict__ h_out, float* __restrict__ lse_out) {
-    __shared__ Ent smem[kDWaves];
-    const int64_t r = blockIdx.x;
-    const char* row = row_ptr<DT>(x, r);
-    Ent acc{-1e30f, 0.f, 0.f};
-    row_for_each<DT>(row, x.vocab, [&](float v) { ent_push(acc, v); });
-    const Ent tot = ent_block(acc, smem);
-    if (threadIdx.x == 0) {
-        const float log_s = logf(tot.s);
-        h_out[r] = tot.t / tot.s - log_s;  // sum p (x - m) - log s
-        lse_out[r] = tot.m + log_s;
-    }
-}
-
-// d / dz of sum_v p_v log p_v, times the upstream gradient: g * p_v * (log p_v - H)
-template <int DT>
-__global__ __launch_bounds__(kDBlock) void neg_entropy_bwd_kernel(RowsView x, const float* __restrict__ lse, const float* __restrict__ h,
-                                                                  const float* __restrict__ grad, RowsView d) {
-    const int64_t r = blockIdx.x;
-    void* out = const_cast<char*>(row_ptr<DT>(d, r));
-    const float g = grad[r];
-    if (g == 0.f) { row_fill_zero<DT>(out, x.vocab); return; }
-    const float l = lse[r], hh = h[r];
-    row_map<DT>(row_ptr<DT>(x, r), nullptr, out, x.vocab, [&](float v, float, int64_t) {
-        const float lp = v - l, p = fast_exp2(lp * kLog2e);
-        return p > 0.f ? g * p * (lp - hh) : 0.f;
-    });
-}
-
-// ---------------------------------------------------------------------------------------------
-// log-probabilities at K given indices per row
-// ---------------------------------------------------------------------------------------------
 struct GatherArgs {
-    const int64_t* idx;  // [rows, K]
-    int64_t k, vstart, vend;
+    const int64_t* idx;  // [n_outer, >= n_inner, K] with `outer` elements between two values of the outer index
+    int64_t k, outer, vstart, vend;
 };
+constexpr float kLn2 = 0.6931471805599453f;
+constexpr float kLn2Hi = 0.693145751953125f, kLn2Lo = 1.4286068203094173e-6f;  // a whole number times the first part is exact
 
-template <int DT>
-__global__ __launch_bounds__(kDBlock) void gather_logprob_fwd_kernel(RowsView x, GatherArgs ga, float* __restrict__ out,
-                                                                     float* __restrict__ lse_out) {
-    __shared__ Lse smem[kDWaves];
-    const int64_t r = blockIdx.x;
+// Bound by HBM: one read of the row (K1's schedule: four 16-byte loads in flight per lane, 32 elements folded under one
+// reference point, an unaligned head and a short tail taken element by element).  The entropy costs two vector
+// operations per element on top of K1's eight.  One pass for both outputs: 2048 rows of V = 151936 bf16 take 97 us,
+// 6.4 TB/s, where the two separate passes (one branch and rescale per element in the entropy's) took 123 + 107.
+template <int DT, bool ENT>
+__global__ __launch_bounds__(kDBlock) void row_sums_fwd_kernel(RowsView x, GatherArgs ga, float* __restrict__ out,
+                                                               float* __restrict__ h_out, float* __restrict__ lse_out) {
+    constexpr int EPV = Row<DT>::EPV;
+    __shared__ float smem[kDWaves][3];
+    const int tid = threadIdx.x;
+    const int64_t r = blockIdx.x, vocab = x.vocab;
     const char* row = row_ptr<DT>(x, r);
-    Lse acc{-FLT_MAX, 0.f};
-    row_for_each_vec<DT>(
-        row, x.vocab, [&](const float(&t)[Row<DT>::EPV]) { lse_push<Row<DT>::EPV>(acc, t); }, [&](float v) { lse_push1(acc, v); });
-    const Lse tot = block_lse<kDWaves>(acc, smem);
-    const float lse = tot.m + logf(tot.s);
-    if (threadIdx.x == 0 && lse_out) lse_out[r] = lse;
-    for (int64_t j = threadIdx.x; j < ga.k; j += kDBlock) {
-        const int64_t gi = ga.idx[r * ga.k + j];
-        out[r * ga.k + j] = (gi >= ga.vstart && gi < ga.vend) ? Row<DT>::load1(row, gi - ga.vstart) - lse : 0.f;
+    const int64_t head = row_head<DT>(row, vocab), nvec = (vocab - head) / EPV, tail0 = head + nvec * EPV;
+    const u32x4* xv = reinterpret_cast<const u32x4*>(row + head * Row<DT>::BYTES);
+    RowSums<ENT> acc;
+    int64_t base = 0;
+    for (; base + kDUnroll * kDBlock <= nvec; base += kDUnroll * kDBlock) {
+        u32x4 q[kDUnroll];
+#pragma unroll
+        for (int u = 0; u < kDUnroll; ++u) q[u] = __builtin_nontemporal_load(xv + base + u * kDBlock + tid);
+        float v[kDUnroll * EPV];
+#pragma unroll
+        for (int u = 0; u < kDUnroll; ++u) {
+            float t[EPV];
+            Row<DT>::decode(q[u], t);
+#pragma unroll
+            for (int k = 0; k < EPV; ++k) v[u * EPV + k] = t[k];
+        }
+        acc.template push<kDUnroll * EPV>(v);
+    }
+    for (int64_t i = base + tid; i < nvec; i += kDBlock) {
+        float t[EPV];
+        Row<DT>::decode(__builtin_nontemporal_load(xv + i), t);
+        acc.template push<EPV>(t);
+    }
+    if (tid < head) acc.push1(Row<DT>::load1(row, tid));
+    if (tail0 + tid < vocab) acc.push1(Row<DT>::load1(row, tail0 + tid));
+    const RowSums<ENT> tot = sums_block<ENT>(acc, smem);
+    const float log_s = logf(tot.s), lse = __builtin_fmaf(tot.m2, kLn2Hi, __builtin_fmaf(tot.m2, kLn2Lo, log_s));
+    if (tid == 0) {
+        if (lse_out) lse_out[r] = lse;
+        if (ENT) h_out[r] = tot.t / tot.s * kLn2 - log_s;
+    }
+    if (ga.k > 0) {
+        const int64_t o = r / x.n_inner, i = r - o * x.n_inner;
+        const int64_t* idx = ga.idx + o * ga.outer + i * ga.k;
+        for (int64_t j = tid; j < ga.k; j += kDBlock) {
+            const int64_t gi = idx[j];
+            out[r * ga.k + j] = (gi >= ga.vstart && gi < ga.vend) ? Row<DT>::load1(row, gi - ga.vstart) - lse : 0.f;
+        }
     }
 }
 
-// dz_v = -p_v * sum_k g_k + sum_{k: idx_k = v} g_k; the K touched elements are rewritten after the streaming
-// pass with their complete value (every duplicate of an index computes and writes the same number)
-template <int DT>
-__global__ __launch_bounds__(kDBlock) void gather_logprob_bwd_kernel(RowsView x, GatherArgs ga, const float* __restrict__ lse,
-                                                                     const float* __restrict__ grad, RowsView d) {
+// dz_v = p_v * (gh * (log p_v - H) - sum_k g_k) + sum over the k with idx_k = v of g_k: one read and one write of the row.
+// The K touched elements are rewritten after the streaming pass with their complete value (every duplicate of an index
+// computes and writes the same number).  Rows at and past n_inner, and rows without any upstream gradient, are
+// zero-filled without being read.  Bound by HBM's mixed read + write rate.  2048 rows of V = 151936 bf16: 237 us (5.2 TB/s);
+// as two kernels, each with a gradient of its own that autograd then added, it was 261 + 237 + 315 us.
+constexpr int kPatchLds = 512;  // entries of an index list that fit on chip; longer ones are read from memory again
+template <int DT, bool ENT>
+__global__ __launch_bounds__(kDBlock) void row_sums_bwd_kernel(RowsView x, GatherArgs ga, const float* __restrict__ lse,
+                                                               const float* __restrict__ h, const float* __restrict__ grad_h,
+                                                               const float* __restrict__ grad, RowsView d) {
+    constexpr int EPV = Row<DT>::EPV;
     __shared__ float sm[kDWaves];
-    const int64_t r = blockIdx.x;
-    const char* row = row_ptr<DT>(x, r);
-    void* out = const_cast<char*>(row_ptr<DT>(d, r));
+    __shared__ int idx_l[kPatchLds];
+    __shared__ float g_l[kPatchLds];
+    const int tid = threadIdx.x;
+    const int64_t vocab = x.vocab;
+    const int64_t o = blockIdx.x / d.n_inner, i = blockIdx.x - o * d.n_inner;
+    char* out = static_cast<char*>(const_cast<void*>(d.p)) + (o * d.stride_outer + i * d.stride_inner) * Row<DT>::BYTES;
+    if (i >= x.n_inner) { row_fill_zero<DT>(out, vocab); return; }
+    const int64_t r = o * x.n_inner + i;
+    const int64_t* idx = ga.idx + o * ga.outer + i * ga.k;
+    const float* g = grad + r * ga.k;
+    const float gh = ENT ? grad_h[r] : 0.f;
     float part = 0.f;
-    for (int64_t j = threadIdx.x; j < ga.k; j += kDBlock) part += grad[r * ga.k + j];
-    const float gsum = block_sum<float, kDWaves>(part, sm);
-    const float l = lse[r];
-    row_map<DT>(row, nullptr, out, x.vocab, [&](float v, float, int64_t) { return -fast_exp2((v - l) * kLog2e) * gsum; });
+    bool any = gh != 0.f;
+    for (int64_t j = tid; j < ga.k; j += kDBlock) {
+        const float gj = g[j];
+        const int64_t v = idx[j];
+        part += gj;
+        any |= gj != 0.f;
+        if (j < kPatchLds) {
+            idx_l[j] = (v >= ga.vstart && v < ga.vend) ? static_cast<int>(v - ga.vstart) : -1;
+            g_l[j] = gj;
+        }
+    }
+    if (!__syncthreads_or(any)) { row_fill_zero<DT>(out, vocab); return; }
+    const float gsum = ga.k > 0 ? block_sum<float, kDWaves>(part, sm) : 0.f;
+    const float l = lse[r], hh = ENT ? h[r] : 0.f;
+    auto elem = [&](float v) -> float {
+        const float lp = v - l, p = fast_exp2(lp * kLog2e);
+        if (!ENT) return -p * gsum;
+        return p * __builtin_fmaf(fmaxf(lp - hh, -1e30f), gh, -gsum);
+    };
+    const char* row = row_ptr<DT>(x, r);
+    const int64_t head = row_head<DT>(row, vocab);
+    if (row_head<DT>(out, vocab) != head) {  // input and output rows are not congruent modulo 16 bytes
+        for (int64_t v = tid; v < vocab; v += kDBlock) Row<DT>::store1(out, v, elem(Row<DT>::load1(row, v)));
+    } else {
+        const int64_t nvec = (vocab - head) / EPV, tail0 = head + nvec * EPV;
+        const u32x4* xv = reinterpret_cast<const u32x4*>(row + head * Row<DT>::BYTES);
+        u32x4* ov = reinterpret_cast<u32x4*>(out + head * Row<DT>::BYTES);
+        auto put = [&](const u32x4& q, int64_t vi) {
+            float t[EPV];
+            Row<DT>::decode(q, t);
+#pragma unroll
+            for (int k = 0; k < EPV; ++k) t[k] = elem(t[k]);
+            __builtin_nontemporal_store(Row<DT>::encode(t), ov + vi);
+        };
+        int64_t base = 0;
+        for (; base + kDUnroll * kDBlock <= nvec; base += kDUnroll * kDBlock) {
+            u32x4 q[kDUnroll];
+#pragma unroll
+            for (int u = 0; u < kDUnroll; ++u) q[u] = __builtin_nontemporal_load(xv + base + u * kDBlock + tid);
+#pragma unroll
+            for (int u = 0; u < kDUnroll; ++u) put(q[u], base + u * kDBlock + tid);
+        }
+        for (int64_t vi = base + tid; vi < nvec; vi += kDBlock) put(__builtin_nontemporal_load(xv + vi), vi);
+        if (tid < head) Row<DT>::store1(out, tid, elem(Row<DT>::load1(row, tid)));
+        if (tail0 + tid < vocab) Row<DT>::store1(out, tail0 + tid, elem(Row<DT>::load1(row, tail0 + tid)));
+    }
+    if (ga.k == 0) return;
     __syncthreads();  // the streaming stores of this workgroup are visible to it before the patches land
-    for (int64_t j = threadIdx.x; j < ga.k; j += kDBlock) {
-        const int64_t gi = ga.idx[r * ga.k + j];
-        if (gi < ga.vstart || gi >= ga.vend) continue;
+    for (int64_t j = tid; j < ga.k; j += kDBlock) {
+        const int64_t gi = idx[j] - ga.vstart;
+        if (gi < 0 || gi >= ga.vend - ga.vstart) continue;
         float add = 0.f;
-        for (int64_t q = 0; q < ga.k; ++q) add += ga.idx[r * ga.k + q] == gi ? grad[r * ga.k + q] : 0.f;
-        const float v = Row<DT>::load1(row, gi - ga.vstart);
-        Row<DT>::store1(out, gi - ga.vstart, -fast_exp2((v - l) * kLog2e) * gsum + add);
+        if (ga.k <= kPatchLds)
+            for (int q = 0; q < static_cast<int>(ga.k); ++q) add += idx_l[q] == static_cast<int>(gi) ? g_l[q] : 0.f;
+        else
+            for (int64_t q = 0; q < ga.k; ++q) add += idx[q] - ga.vstart == gi ? g[q] : 0.f;
+        Row<DT>::store1(out, gi, elem(Row<DT>::load1(row, gi)) + add);
     }
 }
 
@@ -354,9 +392,11 @@ __global__ __launch_bounds__(kDBlock) void topk_logsoftmax_fwd_kernel(RowsView x
     __shared__ Lse smem[kDWaves];
     const int64_t r = blockIdx.x;
     const char* row = row_ptr<DT>(x, r);
+    const int64_t o = r / x.n_inner;
+    const int64_t* idx = ga.idx + o * ga.outer + (r - o * x.n_inner) * ga.k;
     auto value = [&](int64_t j) -> float {
         if (!ga.idx) return Row<DT>::load1(row, j);
-        const int64_t gi = ga.idx[r * ga.k + j];
+        const int64_t gi = idx[j];
         return (gi >= ga.vstart && gi < ga.vend) ? Row<DT>::load1(row, gi - ga.vstart) : -INFINITY;
     };
     Lse a{-FLT_MAX, 0.f};
@@ -500,57 +540,85 @@ using namespace nrl;
         default: { constexpr int DT = NRL_F16; __VA_ARGS__; break; }        \
     }
 
-extern "C" int nrl_neg_entropy_fwd(const nrl_rows* rows, float* h_out, float* lse_out, void* stream) {
+// log-sum-exp, entropy (h_out) and gathered log-probabilities (k > 0) in one pass over the rows; indices of a row are
+// `idx_outer` elements apart between two outer indices
+static int row_sums_fwd(const nrl_rows* rows, const int64_t* indices, int64_t k, int64_t idx_outer, float* out, float* h_out,
+                        float* lse_out, void* stream, const char* what) {
     if (int e = check_view(rows)) return e;
     const int64_t n = rows->n_outer * rows->n_inner;
+    if (k < 0) return fail(NRL_E_INVALID, "negative K");
     if (n == 0) return NRL_OK;
-    if (!h_out || !lse_out) return fail(NRL_E_INVALID, "null output");
+    if (k > 0 && (!indices || !out)) return fail(NRL_E_INVALID, "null argument");
+    if (k > 0 && rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");
     hipStream_t s = static_cast<hipStream_t>(stream);
     const RowsView x = view_of(rows);
-    NRL_DT_DISPATCH(rows->dtype, neg_entropy_fwd_kernel<DT><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, h_out, lse_out));
-    return check_launch("neg_entropy_fwd");
+    const GatherArgs ga{indices, k, idx_outer, rows->vocab_start, rows->vocab_end};
+    if (h_out)
+        NRL_DT_DISPATCH(rows->dtype, row_sums_fwd_kernel<DT, true><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, out, h_out, lse_out))
+    else
+        NRL_DT_DISPATCH(rows->dtype, row_sums_fwd_kernel<DT, false><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, out, h_out, lse_out))
+    return check_launch(what);
+}
+
+static int row_sums_bwd(const nrl_rows* rows, const int64_t* indices, int64_t k, int64_t idx_outer, const float* lse, const float* h,
+                        const float* grad_h, const float* grad, void* dlogits, int64_t d_n_inner, int64_t d_stride_outer,
+                        int64_t d_stride_inner, void* stream, const char* what) {
+    if (int e = check_view(rows)) return e;
+    if (k < 0) return fail(NRL_E_INVALID, "negative K");
+    if (d_n_inner < rows->n_inner) return fail(NRL_E_INVALID, "d_n_inner < n_inner");
+    const int64_t n = rows->n_outer * d_n_inner;
+    if (n == 0) return NRL_OK;
+    if (n >= (1ll << 31)) return fail(NRL_E_INVALID, "more than 2^31 rows in one launch");
+    if (!dlogits || (rows->n_inner > 0 && (!lse || (k > 0 && (!indices || !grad))))) return fail(NRL_E_INVALID, "null argument");
+    if (k > 0 && rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");
+    if (rows->vocab >= (1ll << 31)) return fail(NRL_E_INVALID, "vocabulary too large");
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const RowsView x = view_of(rows);
+    const RowsView d{dlogits, d_n_inner, rows->vocab, d_stride_outer, d_stride_inner};
+    const GatherArgs ga{indices, k, idx_outer, rows->vocab_start, rows->vocab_end};
+    if (h)
+        NRL_DT_DISPATCH(rows->dtype, row_sums_bwd_kernel<DT, true><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, lse, h, grad_h, grad, d))
+    else
+        NRL_DT_DISPATCH(rows->dtype, row_sums_bwd_kernel<DT, false><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, lse, h, grad_h, grad, d))
+    return check_launch(what);
+}
+
+extern "C" int nrl_neg_entropy_fwd(const nrl_rows* rows, float* h_out, float* lse_out, void* stream) {
+    if (rows && rows->n_outer * rows->n_inner > 0 && (!h_out || !lse_out)) return fail(NRL_E_INVALID, "null output");
+    return row_sums_fwd(rows, nullptr, 0, 0, nullptr, h_out, lse_out, stream, "neg_entropy_fwd");
 }
 
 extern "C" int nrl_neg_entropy_bwd(const nrl_rows* rows, const float* lse, const float* h, const float* grad, void* dlogits,
                                    int64_t d_stride_outer, int64_t d_stride_inner, void* stream) {
-    if (int e = check_view(rows)) return e;
-    const int64_t n = rows->n_outer * rows->n_inner;
-    if (n == 0) return NRL_OK;
-    if (!lse || !h || !grad || !dlogits) return fail(NRL_E_INVALID, "null argument");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const RowsView x = view_of(rows), d = view_of(rows, dlogits, d_stride_outer, d_stride_inner);
-    NRL_DT_DISPATCH(rows->dtype, neg_entropy_bwd_kernel<DT><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, lse, h, grad, d));
-    return check_launch("neg_entropy_bwd");
+    if (rows && rows->n_outer * rows->n_inner > 0 && (!h || !grad)) return fail(NRL_E_INVALID, "null argument");
+    return row_sums_bwd(rows, nullptr, 0, 0, lse, h, grad, nullptr, dlogits, rows ? rows->n_inner : 0, d_stride_outer, d_stride_inner,
+                        stream, "neg_entropy_bwd");
 }
 
 extern "C" int nrl_gather_logprob_fwd(const nrl_rows* rows, const int64_t* indices, int64_t k, float* out, float* lse_out,
                                       void* stream) {
-    if (int e = check_view(rows)) return e;
-    const int64_t n = rows->n_outer * rows->n_inner;
-    if (k < 0) return fail(NRL_E_INVALID, "negative K");
-    if (n == 0 || k == 0) return NRL_OK;
-    if (!indices || !out) return fail(NRL_E_INVALID, "null argument");
-    if (rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const RowsView x = view_of(rows);
-    const GatherArgs ga{indices, k, rows->vocab_start, rows->vocab_end};
-    NRL_DT_DISPATCH(rows->dtype, gather_logprob_fwd_kernel<DT><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, out, lse_out));
-    return check_launch("gather_logprob_fwd");
+    if (rows && k == 0) return check_view(rows);
+    return row_sums_fwd(rows, indices, k, rows ? rows->n_inner * k : 0, out, nullptr, lse_out, stream, "gather_logprob_fwd");
 }
 
 extern "C" int nrl_gather_logprob_bwd(const nrl_rows* rows, const int64_t* indices, int64_t k, const float* lse, const float* grad,
                                       void* dlogits, int64_t d_stride_outer, int64_t d_stride_inner, void* stream) {
-    if (int e = check_view(rows)) return e;
-    const int64_t n = rows->n_outer * rows->n_inner;
-    if (k < 0) return fail(NRL_E_INVALID, "negative K");
-    if (n == 0) return NRL_OK;
-    if (!lse || !dlogits || (k > 0 && (!indices || !grad))) return fail(NRL_E_INVALID, "null argument");
-    if (rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const RowsView x = view_of(rows), d = view_of(rows, dlogits, d_stride_outer, d_stride_inner);
-    const GatherArgs ga{indices, k, rows->vocab_start, rows->vocab_end};
-    NRL_DT_DISPATCH(rows->dtype, gather_logprob_bwd_kernel<DT><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, lse, grad, d));
-    return check_launch("gather_logprob_bwd");
+    return row_sums_bwd(rows, indices, k, rows ? rows->n_inner * k : 0, lse, nullptr, nullptr, grad, dlogits, rows ? rows->n_inner : 0,
+                        d_stride_outer, d_stride_inner, stream, "gather_logprob_bwd");
+}
+
+extern "C" int nrl_gather_entropy_fwd(const nrl_rows* rows, const int64_t* indices, int64_t k, int64_t index_stride_outer, float* out,
+                                      float* h_out, float* lse_out, void* stream) {
+    if (rows && rows->n_outer * rows->n_inner > 0 && !lse_out) return fail(NRL_E_INVALID, "null output");
+    return row_sums_fwd(rows, indices, k, index_stride_outer, out, h_out, lse_out, stream, "gather_entropy_fwd");
+}
+
+extern "C" int nrl_gather_entropy_bwd(const nrl_rows* rows, const int64_t* indices, int64_t k, int64_t index_stride_outer,
+                                      const float* lse, const float* h, const float* grad_h, const float* grad, void* dlogits,
+                                      int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, void* stream) {
+    if (h && !grad_h) return fail(NRL_E_INVALID, "an entropy without its upstream gradient");
+    return row_sums_bwd(rows, indices, k, index_stride_outer, lse, h, grad_h, grad, dlogits, d_n_inner, d_stride_outer,
+                        d_stride_inner, stream, "gather_entropy_bwd");
 }
 
 extern "C" int nrl_soft_cross_entropy_fwd(const nrl_rows* student, const void* teacher, int64_t t_stride_outer,
@@ -592,7 +660,7 @@ extern "C" int nrl_topk_logsoftmax_fwd(const nrl_rows* rows, const int64_t* indi
     if (!out) return fail(NRL_E_INVALID, "null output");
     if (rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");
     const RowsView x = view_of(rows);
-    const GatherArgs ga{indices, k, rows->vocab_start, rows->vocab_end};
+    const GatherArgs ga{indices, k, rows->n_inner * k, rows->vocab_start, rows->vocab_end};
     hipStream_t s = static_cast<hipStream_t>(stream);
     NRL_DT_DISPATCH(rows->dtype, topk_logsoftmax_fwd_kernel<DT><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(x, ga, out));
     return check_launch("topk_logsoftmax_fwd");
@@ -608,7 +676,7 @@ extern "C" int nrl_topk_logsoftmax_bwd(const nrl_rows* rows, const int64_t* indi
     if (!dlogits || (k > 0 && (!indices || !logprobs || !grad))) return fail(NRL_E_INVALID, "null argument");
     if (rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");
     const RowsView d = view_of(rows, dlogits, d_stride_outer, d_stride_inner);
-    const GatherArgs ga{indices, k, rows->vocab_start, rows->vocab_end};
+    const GatherArgs ga{indices, k, rows->n_inner * k, rows->vocab_start, rows->vocab_end};
     hipStream_t s = static_cast<hipStream_t>(stream);
     NRL_DT_DISPATCH(rows->dtype, topk_logsoftmax_bwd_kernel<DT><<<dim3((unsigned)n), dim3(kDBlock), 0, s>>>(d, ga, logprobs, grad));
     return check_launch("topk_logsoftmax_bwd");

@@ -26,13 +26,6 @@ constexpr int kUnroll = 4;   // 16-byte loads in flight per lane
 template <typename P> __device__ __forceinline__ u32x4 k2_load(const P* p) { return __builtin_nontemporal_load(p); }
 template <typename P> __device__ __forceinline__ void k2_store(u32x4 v, P* p) { __builtin_nontemporal_store(v, p); }
 
-// number of leading elements before the first 16-byte boundary of a row
-template <int DT> __device__ __forceinline__ int64_t row_head(const void* row, int64_t vocab) {
-    const uintptr_t a = reinterpret_cast<uintptr_t>(row);
-    const int64_t h = static_cast<int64_t>(((16 - (a & 15)) & 15) / Row<DT>::BYTES);
-    return h < vocab ? h : vocab;
-}
-
 // Online log-sum-exp of one row; every thread returns the row's (max, sum).
 template <int DT, int TEMP>
 __device__ __forceinline__ Lse row_online_lse(const void* row, int64_t vocab, float tparam, Lse* smem) {

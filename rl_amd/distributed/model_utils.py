@@ -604,6 +604,28 @@ class DistributedCrossEntropy(torch.autograd.Function):
         return d.reshape(ctx.in_shape), None, None, None
 
 
+class _GatherEntropy(torch.autograd.Function):
+    """``log p`` at ``indices [B, S, K]`` and (optionally) ``sum_v p log p`` of the first ``n`` rows of every sequence:
+    one pass over the logits forward and one backward, where ``ChunkedDistributedGatherLogprob`` and
+    ``ChunkedDistributedEntropy`` each make their own and autograd then adds their ``[B, S, V]`` gradients."""
+
+    @staticmethod
+    def forward(ctx, logits, indices, n, entropy):
+        x = logits.detach()
+        x = x if x.stride(-1) == 1 else x.contiguous()
+        out, h, lse = torch.ops.rl_amd.gather_entropy_fwd(x, indices, n, entropy)
+        ctx.save_for_backward(x, indices, lse, h)
+        ctx.n, ctx.entropy = n, entropy
+        return (out, h) if entropy else out
+
+    @staticmethod
+    def backward(ctx, grad, grad_h=None):
+        x, indices, lse, h = ctx.saved_tensors
+        d = torch.ops.rl_amd.gather_entropy_bwd(x, indices, ctx.n, lse, h if ctx.entropy else None,
+                                                grad_h.float() if ctx.entropy else None, grad.float())
+        return d, None, None, None
+
+
 class _TopkLogSoftmax(torch.autograd.Function):
     """log_softmax over the K logits of every row at the given vocabulary indices."""
 
@@ -656,23 +678,20 @@ def get_distillation_topk_logprobs_from_logits(
     indices = teacher_topk_indices.to(student_logits.device)
     if indices.dtype != torch.int64:
         indices = indices.long()
-    vocab = student_logits.shape[-1]
     seq = student_logits.shape[1]
     H_all = None
+    rows = max(seq - 1, 0)  # the last position predicts nothing
     if zero_outside_topk:
-        student_topk_logprobs = ChunkedDistributedGatherLogprob.apply(student_logits, indices, 0, vocab, seq, None, False)
         if calculate_entropy:
-            H_all = ChunkedDistributedEntropy.apply(student_logits, seq, None, False)
+            student_topk_logprobs, H_all = _GatherEntropy.apply(student_logits, indices, rows, True)
+        else:
+            student_topk_logprobs = _GatherEntropy.apply(student_logits, indices, rows, False)
     else:
-        student_topk_logprobs = _TopkLogSoftmax.apply(student_logits, indices)
+        student_topk_logprobs = _TopkLogSoftmax.apply(student_logits, indices)[:, :-1, :]
     teacher = teacher_topk_logits.to(student_topk_logprobs.device)
     if teacher.dim() != 3:
         raise ValueError(f"teacher_topk_logits must be [B, S, K], got {tuple(teacher.shape)}")
     if teacher.stride(2) != 1 and teacher.shape[2] > 1:
         teacher = teacher.contiguous()
-    teacher_topk_logprobs = torch.ops.rl_amd.topk_logsoftmax_fwd(teacher.detach(), None)
-    teacher_topk_logprobs = teacher_topk_logprobs[:, :-1, :]
-    student_topk_logprobs = student_topk_logprobs[:, :-1, :]
-    if calculate_entropy and H_all is not None:
-        H_all = H_all[:, :-1]
+    teacher_topk_logprobs = torch.ops.rl_amd.topk_logsoftmax_fwd(teacher.detach()[:, :-1], None)
     return student_topk_logprobs, teacher_topk_logprobs, H_all

@@ -1091,6 +1091,8 @@ _LIB.define("neg_entropy_fwd(Tensor logits) -> (Tensor, Tensor)")
 _LIB.define("neg_entropy_bwd(Tensor logits, Tensor lse, Tensor h, Tensor grad) -> Tensor")
 _LIB.define("gather_logprob_fwd(Tensor logits, Tensor indices, int vocab_start, int vocab_end) -> (Tensor, Tensor)")
 _LIB.define("gather_logprob_bwd(Tensor logits, Tensor indices, int vocab_start, int vocab_end, Tensor lse, Tensor grad) -> Tensor")
+_LIB.define("gather_entropy_fwd(Tensor logits, Tensor indices, int n_inner, bool entropy) -> (Tensor, Tensor, Tensor)")
+_LIB.define("gather_entropy_bwd(Tensor logits, Tensor indices, int n_inner, Tensor lse, Tensor? h, Tensor? grad_h, Tensor grad) -> Tensor")
 _LIB.define("soft_cross_entropy_fwd(Tensor student, Tensor teacher) -> (Tensor, Tensor, Tensor)")
 _LIB.define("soft_cross_entropy_bwd(Tensor student, Tensor teacher, Tensor lse_student, Tensor lse_teacher, Tensor grad) -> Tensor")
 
@@ -1186,6 +1188,52 @@ def _gather_logprob_bwd(logits, indices, vocab_start, vocab_end, lse, grad):
     return d
 
 
+def _gather_entropy_rows(logits, indices, n_inner):
+    rows = _plain_rows(logits)
+    if not 0 <= n_inner <= logits.shape[1]:
+        raise ValueError(f"n_inner {n_inner} does not fit logits {tuple(logits.shape)}")
+    rows.n_inner = n_inner
+    return rows, _gather_indices(logits, indices)
+
+
+def _gather_entropy_fwd(logits, indices, n_inner, entropy):
+    """The first ``n_inner`` rows of every sequence: ``log p`` at ``indices [B, S, K]`` -> ``[B, n_inner, K]``,
+    ``sum_v p log p`` (empty without ``entropy``) and the log-sum-exps, from one pass over the logits."""
+    _need_gpu(logits, indices)
+    rows, indices = _gather_entropy_rows(logits, indices, n_inner)
+    b, s, k = indices.shape
+    dev = logits.device
+    with torch.cuda.device(dev):
+        out = torch.empty((b, n_inner, k), dtype=torch.float32, device=dev)
+        h = torch.empty((b, n_inner) if entropy else (0,), dtype=torch.float32, device=dev)
+        lse = torch.empty((b, n_inner), dtype=torch.float32, device=dev)
+        with _timed("gather_entropy_fwd"):
+            code = _lib.load().nrl_gather_entropy_fwd(C.byref(rows), _ptr(indices), k, s * k, _ptr(out), _ptr(h if entropy else None),
+                                                      _ptr(lse), _stream())
+    _lib.check(code, "nrl_gather_entropy_fwd")
+    return out, h, lse
+
+
+def _gather_entropy_bwd(logits, indices, n_inner, lse, h, grad_h, grad):
+    """Gradient of both outputs of ``gather_entropy_fwd`` (of the gathered values alone without ``h``) in one pass."""
+    _need_gpu(logits, indices, lse, h, grad_h, grad)
+    rows, indices = _gather_entropy_rows(logits, indices, n_inner)
+    b, s, k = indices.shape
+    lse = _row_scalar(lse, b, n_inner, "lse")
+    if h is not None:
+        h, grad_h = _row_scalar(h, b, n_inner, "h"), _row_scalar(grad_h, b, n_inner, "grad_h")
+    if grad.dtype != torch.float32 or tuple(grad.shape) != (b, n_inner, k):
+        raise ValueError(f"grad must be fp32 [{b}, {n_inner}, {k}], got {grad.dtype} {tuple(grad.shape)}")
+    grad = grad.contiguous()
+    with torch.cuda.device(logits.device):
+        d = _grad_buffer(logits.shape, logits)
+        with _timed("gather_entropy_bwd"):
+            code = _lib.load().nrl_gather_entropy_bwd(C.byref(rows), _ptr(indices), k, s * k, _ptr(lse), _ptr(h), _ptr(grad_h), _ptr(grad),
+                                                      _ptr(d), s, d.stride(0), d.stride(1), _stream())
+    _lib.check(code, "nrl_gather_entropy_bwd")
+    return d
+
+
 def _teacher_like(student, teacher):
     if teacher.shape != student.shape:
         raise ValueError(f"student_logits and target_logits must have the same shape, got {tuple(student.shape)} and {tuple(teacher.shape)}.")
@@ -1227,6 +1275,7 @@ def _soft_cross_entropy_bwd(student, teacher, lse_student, lse_teacher, grad):
 
 for _name, _fn in (("neg_entropy_fwd", _neg_entropy_fwd), ("neg_entropy_bwd", _neg_entropy_bwd),
                    ("gather_logprob_fwd", _gather_logprob_fwd), ("gather_logprob_bwd", _gather_logprob_bwd),
+                   ("gather_entropy_fwd", _gather_entropy_fwd), ("gather_entropy_bwd", _gather_entropy_bwd),
                    ("soft_cross_entropy_fwd", _soft_cross_entropy_fwd), ("soft_cross_entropy_bwd", _soft_cross_entropy_bwd)):
     _LIB.impl(_name, _fn, "CUDA")
     _LIB.impl(_name, _fn, "CPU")
