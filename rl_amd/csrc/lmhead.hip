@@ -535,26 +535,39 @@ __device__ __forceinline__ float acc_read(float a) {
 
 __device__ __forceinline__ float round_bf16(float v) { return bf16_bits_to_f32(f32_to_bf16_bits(v)); }
 
-// Tile coordinates of workgroup w of a 1-D launch over an nbx x nby tile grid.  Workgroups go to the
-// 8 XCDs (each with its own L2) round-robin by index, so index w runs on XCD w % 8 as that XCD's
-// (w / 8)-th workgroup; an XCD's 32 compute units hold one PX x PY patch of tiles at a time (4 x 8 unless said
-// otherwise), which share PX A panels and PY B panels through that L2.  Patches past the grid yield false.
-template <int PX = 4>
-__device__ __forceinline__ bool patch_tile(uint32_t w, int64_t nbx, int64_t nby, int64_t& bx, int64_t& by) {
-    constexpr uint32_t PY = 32 / PX;
-    static_assert(PX * PY == 32, "a patch is what one XCD holds");
+// How a launch covers its tile grid.  Workgroups go to the 8 XCDs (each with its own L2) round-robin by index, so index
+// w runs on XCD w % 8 as that XCD's (w / 8)-th workgroup; an XCD's 32 compute units hold one patch of px x py tiles at a
+// time (px * py <= 32), which share px A panels and py B panels through that L2.  A launch may carry several k ranges
+// (splits) of the same tile grid: their patches follow each other.
+struct Patches {
+    uint32_t px = 4, py = 8;
+    int splits = 1;
+    __host__ __device__ int64_t along_x(int64_t nbx) const { return (nbx + px - 1) / px; }
+    __host__ __device__ int64_t along_y(int64_t nby) const { return (nby + py - 1) / py; }
+    int64_t grid(int64_t nbx, int64_t nby) const { return (along_x(nbx) * along_y(nby) * splits + 7) / 8 * 8 * 32; }
+    // How many times the busiest XCD fills its 32 compute units.  Patches at the edge of the grid are counted by the tiles
+    // they really hold, on average: a compute unit takes the next workgroup when it is free, whatever its patch.
+    double rounds(int64_t nbx, int64_t nby) const {
+        const int64_t patches = along_x(nbx) * along_y(nby) * splits, per_xcd = (patches + 7) / 8;
+        const double held = static_cast<double>(nbx) * nby * splits / patches;
+        return static_cast<double>(static_cast<int64_t>(per_xcd * held / 32.0 + 0.999));
+    }
+};
+
+// Tile coordinates (and k range) of workgroup w; slots and patches past the grid yield false.
+__device__ __forceinline__ bool patch_tile(const Patches& p, uint32_t w, int64_t nbx, int64_t nby, int64_t& bx, int64_t& by, int& split) {
     const uint32_t xcd = w & 7, s = w >> 3;
-    const uint32_t patch = (s >> 5) * 8 + xcd, t = s & 31;
-    const uint32_t ppy = static_cast<uint32_t>((nby + PY - 1) / PY);  // patches along y
-    const uint32_t px = patch / ppy, py = patch - px * ppy;
-    // the division runs on the vector unit; hand the (uniform) results back to scalar registers
-    bx = __builtin_amdgcn_readfirstlane(static_cast<int>(px * PX + t / PY));
-    by = __builtin_amdgcn_readfirstlane(static_cast<int>(py * PY + t % PY));
-    return bx < nbx && by < nby;
-}
-static int64_t patch_grid(int64_t nbx, int64_t nby, int64_t px = 4) {
-    const int64_t py = 32 / px, patches = ((nbx + px - 1) / px) * ((nby + py - 1) / py);
-    return (patches + 7) / 8 * 8 * 32;
+    const uint32_t t = s & 31;
+    uint32_t patch = (s >> 5) * 8 + xcd;
+    const uint32_t npx = static_cast<uint32_t>(p.along_x(nbx)), npy = static_cast<uint32_t>(p.along_y(nby));
+    const uint32_t sp = patch / (npx * npy);
+    patch -= sp * npx * npy;
+    const uint32_t ix = patch / npy, iy = patch - ix * npy, tx = t / p.py;
+    // the divisions run on the vector unit; hand the (uniform) results back to scalar registers
+    bx = __builtin_amdgcn_readfirstlane(static_cast<int>(ix * p.px + tx));
+    by = __builtin_amdgcn_readfirstlane(static_cast<int>(iy * p.py + (t - tx * p.py)));
+    split = __builtin_amdgcn_readfirstlane(static_cast<int>(sp));
+    return tx < p.px && split < p.splits && bx < nbx && by < nby;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -582,6 +595,7 @@ struct LmFwdArgs {
     const int64_t* targets;    // [N]
     int64_t vocab_start;       // target ids are global; rows of W are local
     int n_splits;
+    Patches patches;
     float* part_m;             // [n_splits, N]
     float* part_s;             // [n_splits, N]
     float* xt;                 // [N] target logit (written by the tile that holds it)
@@ -618,11 +632,6 @@ __device__ __forceinline__ void patch_cross(unsigned int* ctr, unsigned target, 
     __syncthreads();
 }
 
-// Token tiles per XCD patch of the forward (the other side of the patch counts vocabulary splits).  Without the
-// logits 8 token tiles x 4 splits measured 4 % faster than 4 x 8 (58.9 against 61.3 ms at 65536 tokens, V 151936);
-// with the logits written it measured 1 % slower, and 16 x 2 and 32 x 1 slower either way.
-constexpr int fwd_patch_tokens(bool save) { return save ? 4 : 8; }
-
 template <class Core, bool SAVE>
 __global__ __launch_bounds__(GB_THREADS) void lmhead_fwd_kernel(LmFwdArgs a) {
     constexpr int NI = Core::NI, NJ = Core::NJ, BV = Core::BM, BT = Core::BN;  // vocabulary rows x token columns
@@ -631,7 +640,8 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_fwd_kernel(LmFwdArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     int64_t bx, by;
-    if (!patch_tile<fwd_patch_tokens(SAVE)>(blockIdx.x, (a.op.n + BT - 1) / BT, a.n_splits, bx, by)) return;
+    int one;
+    if (!patch_tile(a.patches, blockIdx.x, (a.op.n + BT - 1) / BT, a.n_splits, bx, by, one)) return;
     const int64_t tok0 = bx * BT;
     const int split = static_cast<int>(by);
     const int64_t n_tiles = (a.op.m + BV - 1) / BV;
@@ -656,7 +666,7 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_fwd_kernel(LmFwdArgs a) {
     unsigned members = 0, common = 0, epoch = 0;
     unsigned int* arrive = nullptr;
     if (a.arrive) {
-        constexpr int PX = fwd_patch_tokens(SAVE), PY = 32 / PX;
+        const int64_t PX = a.patches.px, PY = a.patches.py;
         const int64_t nbx = (a.op.n + BT - 1) / BT, nby = a.n_splits;
         const int64_t px0 = bx / PX * PX, py0 = by / PY * PY;
         const int64_t cx = nbx - px0 < PX ? nbx - px0 : PX, cy = nby - py0 < PY ? nby - py0 : PY;
@@ -776,18 +786,28 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_fwd_kernel(LmFwdArgs a) {
     }
 }
 
-__global__ void lmhead_fwd_finish_kernel(int64_t n, int n_splits, const float* part_m, const float* part_s, const float* xt,
-                                         const int64_t* targets, int64_t vocab_start, int64_t vocab_end, float* logprob,
-                                         float* lse_out) {
-    const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (r >= n) return;
-    float m = part_m[r], s = part_s[r];
-    for (int k = 1; k < n_splits; ++k) {
-        const float om = part_m[k * n + r], os = part_s[k * n + r];
+// The partials of a token merged over the splits, 16 threads to a token (a short batch has up to 256 splits: one thread
+// walking 64 of them took 21 us for 512 tokens, this takes 6 for 128).  The merge order is fixed.
+constexpr int kFinishTokens = 16, kFinishLanes = 16;
+__global__ __launch_bounds__(kFinishTokens * kFinishLanes) void lmhead_fwd_finish_kernel(
+    int64_t n, int n_splits, const float* part_m, const float* part_s, const float* xt, const int64_t* targets, int64_t vocab_start,
+    int64_t vocab_end, float* logprob, float* lse_out) {
+    __shared__ float lm[kFinishLanes][kFinishTokens], ls[kFinishLanes][kFinishTokens];
+    const int tok = threadIdx.x % kFinishTokens, part = threadIdx.x / kFinishTokens;
+    const int64_t r = static_cast<int64_t>(blockIdx.x) * kFinishTokens + tok;
+    float m = -1e30f, s = 0.f;
+    auto merge = [&](float om, float os) {
         const float mn = fmaxf(m, om);
         s = s * fast_exp2((m - mn) * kLog2e) + os * fast_exp2((om - mn) * kLog2e);
         m = mn;
-    }
+    };
+    if (r < n)
+        for (int k = part; k < n_splits; k += kFinishLanes) merge(part_m[static_cast<int64_t>(k) * n + r], part_s[static_cast<int64_t>(k) * n + r]);
+    lm[part][tok] = m;
+    ls[part][tok] = s;
+    __syncthreads();
+    if (part != 0 || r >= n) return;
+    for (int k = 1; k < kFinishLanes; ++k) merge(lm[k][tok], ls[k][tok]);
     const float log_s = logf(s);
     const int64_t t = targets[r];
     logprob[r] = (t >= vocab_start && t < vocab_end) ? (xt[r] - m) - log_s : 0.f;
@@ -809,8 +829,8 @@ struct LmGradArgs {
     int64_t ldgt;
 };
 
-// token tiles per XCD patch of the recomputing gradient kernel (x 4 vocabulary tiles): 1.7 % faster than 4 x 8
-constexpr int kGradPatchTokens = 8;
+// XCD patch of the recomputing gradient kernel, 8 token tiles x 4 vocabulary tiles: 1.7 % faster than 4 x 8
+constexpr Patches kGradPatches{8, 4, 1};
 
 template <class Core>
 __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
@@ -822,7 +842,8 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
     const int wm = wave >> 1, wn = wave & 1;
     if (!resolve_live(a.op)) return;
     int64_t bx, by;
-    if (!patch_tile<kGradPatchTokens>(blockIdx.x, (a.op.m + BM - 1) / BM, (a.op.n + BN - 1) / BN, bx, by)) return;
+    int one;
+    if (!patch_tile(kGradPatches, blockIdx.x, (a.op.m + BM - 1) / BM, (a.op.n + BN - 1) / BN, bx, by, one)) return;
     const int64_t row0 = bx * BM, col0 = by * BN;
     {
         const int64_t grow = row0 + tid;
@@ -1122,24 +1143,37 @@ __global__ __launch_bounds__(256) void lmhead_grad_kept_kernel(LmGradKeptArgs a)
 // combined: with the prior values in flight next to the narrowing stores the compiler spills accumulators inside the
 // K loop.  A product whose k extent turns out empty on the device still delivers zeros without ACCUM; with ACCUM there
 // is nothing to do.
+// Splits: with patches.splits > 1 workgroup and split compute a k range of their own and store the partial product at
+// c + split * split_stride (MODE 0); the reduction kernels below add the partials in order.  A split whose range turns
+// out empty stores zeros.
 // ---------------------------------------------------------------------------------------------
 constexpr int GEMM_ACCUM = 1, GEMM_NARROW = 2;
 template <class Core, int MODE>
-__global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, float* c, int64_t ldc, const int32_t* row_map,
-                                                              uint16_t* cb) {
+__global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, Patches patches, float* c, int64_t ldc,
+                                                              const int32_t* row_map, uint16_t* cb, int64_t split_stride) {
     constexpr bool ACCUM = (MODE & GEMM_ACCUM) != 0, NARROW = (MODE & GEMM_NARROW) != 0;
     static_assert(!(ACCUM && NARROW), "accumulate in fp32, narrow in a pass of its own");
     constexpr int NI = Core::NI, NJ = Core::NJ, BM = Core::BM, BN = Core::BN;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[Core::LDS_BYTES];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave / Core::WAVES_N, wn = wave % Core::WAVES_N;
-    const bool runs = resolve_live(op);
+    bool runs = resolve_live(op);
     if (!runs) {
         // only an empty k extent leaves anything to write, and only where the output is not simply kept as it is
         if (op.m <= 0 || op.n <= 0 || row_map || ACCUM) return;
     }
     int64_t bx, by;
-    if (!patch_tile(blockIdx.x, (op.m + BM - 1) / BM, (op.n + BN - 1) / BN, bx, by)) return;
+    int split;
+    // (the accumulating product is never split and always takes 4 x 8 patches: with more live across its K loop it spills)
+    if (!patch_tile(ACCUM ? Patches{} : patches, blockIdx.x, (op.m + BM - 1) / BM, (op.n + BN - 1) / BN, bx, by, split)) return;
+    if (!ACCUM && patches.splits > 1) {
+        const int64_t per = ((op.k + patches.splits - 1) / patches.splits + 63) / 64 * 64, k0 = per * split;
+        op.a += k0;
+        op.b += k0 / 16 * 512;  // operand B is fragment-major: 16 k of a 32-row group are one block of 512 elements
+        op.k = op.k - k0 < per ? op.k - k0 : per;
+        runs = runs && op.k > 0;
+        c += split * split_stride;
+    }
     const int64_t row0 = bx * BM, col0 = by * BN;
     f32x16 acc[NI][NJ];
     zero_acc<Core>(acc);
@@ -1215,18 +1249,55 @@ __global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, f
     else write_back(std::false_type{});
 }
 
-// dH[n, :] += g_n * W[target_n, :] in fp32: the one-hot term of dH = G W, kept out of the bf16 product.
-// One workgroup per token; tokens without a gradient or with a target outside the shard add nothing.
-__global__ __launch_bounds__(256) void lmhead_onehot_dh_kernel(float* dh, int64_t ld_dh, const float* grad, const int64_t* targets,
-                                                              int64_t vocab_start, int64_t vocab, const uint16_t* w, int64_t ldw,
-                                                              int64_t h) {
-    const int64_t n = blockIdx.x;
-    const float g = grad[n];
-    const int64_t t = targets[n] - vocab_start;
-    if (g == 0.f || t < 0 || t >= vocab) return;
-    const uint16_t* wr = w + t * ldw;
-    float* out = dh + n * ld_dh;
-    for (int64_t c = threadIdx.x; c < h; c += 256) out[c] += g * bf16_bits_to_f32(wr[c]);
+// dH of a chunk's live tokens: the partial products of its k splits added in order (SUM; otherwise the product is
+// already in place), plus the one-hot term g_r * W[target_r, :] in fp32, which is kept out of the bf16 product.  Row r is
+// token row_map[r]; a target outside the shard adds nothing.  One workgroup per row.
+template <bool SUM>
+__global__ __launch_bounds__(256) void lmhead_finish_dh_kernel(float* dh, int64_t ld_dh, const float* parts, int n_splits,
+                                                              int64_t split_stride, const int32_t* row_map, const int32_t* live,
+                                                              int64_t live_from, const float* grad, const int64_t* targets,
+                                                              int64_t vocab_start, int64_t vocab, const uint16_t* w, int64_t ldw, int64_t h) {
+    const int64_t r = blockIdx.x;
+    if (r >= static_cast<int64_t>(live[0]) - live_from) return;
+    const float g = grad[r];
+    const int64_t t = targets[r] - vocab_start;
+    const bool hot = g != 0.f && t >= 0 && t < vocab;
+    if (!SUM && !hot) return;
+    const uint16_t* wr = w + (hot ? t : 0) * ldw;
+    float* out = dh + static_cast<int64_t>(row_map[r]) * ld_dh;
+    for (int64_t c = threadIdx.x * 4; c < h; c += 256 * 4) {  // h is a multiple of 8, the partials are 16-byte aligned
+        float v[4];
+        if (SUM) {
+            const float4 p0 = *reinterpret_cast<const float4*>(parts + r * h + c);
+            v[0] = p0.x; v[1] = p0.y; v[2] = p0.z; v[3] = p0.w;
+            for (int k = 1; k < n_splits; ++k) {
+                const float4 q = *reinterpret_cast<const float4*>(parts + k * split_stride + r * h + c);
+                v[0] += q.x; v[1] += q.y; v[2] += q.z; v[3] += q.w;
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = out[c + u];
+        }
+        if (hot) {
+            const uint2 q = *reinterpret_cast<const uint2*>(wr + c);
+            v[0] += g * bf16_bits_to_f32(q.x & 0xffffu); v[1] += g * bf16_bits_to_f32(q.x >> 16);
+            v[2] += g * bf16_bits_to_f32(q.y & 0xffffu); v[3] += g * bf16_bits_to_f32(q.y >> 16);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) out[c + u] = v[u];
+    }
+}
+
+// dW (bf16) = the partial products of its k splits added in order; n is a multiple of 8
+__global__ __launch_bounds__(256) void lmhead_sum_dw_kernel(uint16_t* dw, const float* parts, int n_splits, int64_t split_stride, int64_t n) {
+    for (int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4; i < n; i += static_cast<int64_t>(gridDim.x) * 256 * 4) {
+        float4 v = *reinterpret_cast<const float4*>(parts + i);
+        for (int k = 1; k < n_splits; ++k) {
+            const float4 q = *reinterpret_cast<const float4*>(parts + k * split_stride + i);
+            v.x += q.x; v.y += q.y; v.z += q.z; v.w += q.w;
+        }
+        *reinterpret_cast<uint2*>(dw + i) = uint2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
+    }
 }
 
 // Order-preserving list of the tokens whose upstream gradient is not zero (one workgroup walks the vector 1024
@@ -1354,28 +1425,74 @@ static int check_lmhead(const void* hidden, int64_t n, int64_t h, int64_t ldh, c
 
 using namespace nrl;
 
-// Vocabulary splits of the forward: enough workgroups for every compute unit, in multiples of the
-// 8-wide patch side, never more than there are vocabulary tiles.
-template <class Core> static int fwd_splits(int64_t n, int64_t v) {
-    const int64_t row_blocks = (n + Core::BN - 1) / Core::BN, tiles = (v + Core::BM - 1) / Core::BM;  // token blocks, vocabulary tiles
-    int64_t s = (256 + row_blocks - 1) / row_blocks;
-    s = (s + 7) / 8 * 8;
-    if (s > 64) s = 64;
-    if (s > tiles) s = tiles;
-    return static_cast<int>(s < 1 ? 1 : s);
+// How the forward covers tokens x vocabulary: a workgroup owns a block of tokens and one of `splits` shares of the
+// vocabulary tiles, and takes a compute unit whole, so what counts is how many times the busiest XCD's 32 units are
+// filled and how many tiles a workgroup walks each time.  The patch sides and the number of shares are the ones with the
+// fewest tiles one after another; 4 token blocks x 8 shares (8 x 4 without the logits, measured 4 % faster there and 1 %
+// slower with them, at 65536 tokens) where that costs no more than 2 %.  A fixed multiple of 8 shares on 4 x 8 patches left
+// half the chip idle on 512 tokens (950 us at H 4096, V 151936; now 610) and ran 10240 tokens in two rounds of which the
+// second was a quarter full.
+struct FwdPlan {
+    Patches patches;
+    int splits;
+};
+template <class Core> static FwdPlan fwd_plan(int64_t n, int64_t v, bool save) {
+    const int64_t blocks = (n + Core::BN - 1) / Core::BN, tiles = (v + Core::BM - 1) / Core::BM;  // token blocks, vocabulary tiles
+    const uint32_t want_px = save ? 4u : 8u;
+    FwdPlan best{Patches{want_px, 32u / want_px, 1}, 1};
+    double best_cost = 1e300;
+    for (uint32_t px = 1; px <= 8; ++px) {
+        if (px > 1 && static_cast<int64_t>(px) >= 2 * blocks) break;
+        const uint32_t py = 32 / px;
+        const int64_t nx = (blocks + px - 1) / px;
+        for (int64_t ny = 1; ny <= 64; ++ny) {
+            const int64_t splits = ny * py < tiles ? ny * py : tiles;
+            const Patches p{px, py, 1};
+            // (+ 1: what a workgroup spends before its first tile and after its last one, about half a tile each)
+            double cost = p.rounds(blocks, splits) * static_cast<double>((tiles + splits - 1) / splits + 1);
+            cost *= 1.0 + 0.002 * (32.0 * (px + py) / (px * py) - 12.0);  // operand panels an XCD reads per tile, against 4 x 8
+            if (px == want_px) cost *= 0.98;
+            if (cost < best_cost) { best_cost = cost; best = FwdPlan{p, static_cast<int>(splits)}; }
+            if (splits == tiles || nx * ny > 64) break;  // finer shares only add starts
+        }
+    }
+    return best;
+}
+
+// How a product covers its tile grid: a single pass over k when its tiles fill the chip, otherwise several k ranges
+// whose partial products are added afterwards.  Costs in microseconds: a 256 x 256 x 64 slab takes 1.4, a tile about 5
+// more for its start and write-back, and the partials are written and read at about 4 TB/s.  dH of 512 tokens (32 tiles,
+// V 151936 along k): 2519 us unsplit, 470 in 8 ranges.  `room`: floats available for partial products.
+static Patches gemm_plan(int64_t m, int64_t n, int64_t k, int64_t room) {
+    const int64_t nbx = (m + CoreC::BM - 1) / CoreC::BM, nby = (n + CoreC::BN - 1) / CoreC::BN, slabs = (k + 63) / 64;
+    Patches best;
+    double best_cost = 1e300;
+    for (int splits = 1; splits <= 16 && (splits == 1 || (splits * m * n <= room && slabs >= 8 * splits)); ++splits)
+        for (uint32_t px = 1; px <= 8; px *= 2) {
+            const Patches p{px, 32 / px, splits};
+            double cost = p.rounds(nbx, nby) * (1.4 * static_cast<double>((slabs + splits - 1) / splits) + 5.0);
+            cost *= 1.0 + 0.002 * (px + 32.0 / px - 12.0);
+            if (splits > 1) cost += 8.0 + static_cast<double>(splits) * m * n * 8 / 4e6;
+            if (cost < best_cost) { best_cost = cost; best = p; }
+        }
+    return best;
 }
 
 // arrival counters of the forward's XCD patches (one per 32 workgroups), behind the partials in the workspace
-static int64_t fwd_patches(int64_t n_tokens, int splits) {
-    const int64_t a = patch_grid((n_tokens + 255) / 256, splits, 4), b = patch_grid((n_tokens + 255) / 256, splits, 8);
-    return (a > b ? a : b) / 32;
+template <class Core> static int64_t fwd_workspace_floats(int64_t n, int64_t v, bool save) {
+    const FwdPlan p = fwd_plan<Core>(n, v, save);
+    return (2 * p.splits + 1) * n + p.patches.grid((n + Core::BN - 1) / Core::BN, p.splits) / 32;
 }
 
 extern "C" int64_t nrl_lmhead_fwd_workspace_bytes(int64_t n_tokens, int64_t vocab) {
     const int64_t n = n_tokens < 1 ? 1 : n_tokens;
-    const int sa = fwd_splits<CoreA>(n, vocab), sb = fwd_splits<CoreB>(n, vocab);
-    const int sm = sa > sb ? sa : sb;
-    return ((2 * sm + 1) * n + fwd_patches(n, sm)) * static_cast<int64_t>(sizeof(float));
+    int64_t most = 0;
+    for (int save = 0; save < 2; ++save) {
+        const int64_t a = fwd_workspace_floats<CoreA>(n, vocab, save), b = fwd_workspace_floats<CoreB>(n, vocab, save);
+        most = a > most ? a : most;
+        most = b > most ? b : most;
+    }
+    return most * static_cast<int64_t>(sizeof(float));
 }
 
 // How often a patch of the forward re-aligns (see patch_cross): once, before its first tile, unless the environment
@@ -1412,9 +1529,11 @@ static bool fwd_align_enabled() {
 
 template <class Core> static void launch_fwd(LmFwdArgs& a, float* ws, hipStream_t s) {
     const int64_t n = a.op.n;
-    a.n_splits = fwd_splits<Core>(n, a.op.m);
+    const FwdPlan plan = fwd_plan<Core>(n, a.op.m, a.logits != nullptr);
+    a.n_splits = plan.splits;
+    a.patches = plan.patches;
     a.part_m = ws; a.part_s = ws + static_cast<int64_t>(a.n_splits) * n; a.xt = ws + 2 * static_cast<int64_t>(a.n_splits) * n;
-    const dim3 grid((unsigned)patch_grid((n + Core::BN - 1) / Core::BN, a.n_splits, fwd_patch_tokens(a.logits != nullptr)));
+    const dim3 grid((unsigned)plan.patches.grid((n + Core::BN - 1) / Core::BN, a.n_splits));
     // xt and, right behind it, the patches' arrival counters are cleared together
     a.arrive = fwd_align_enabled() ? reinterpret_cast<unsigned int*>(a.xt + n) : nullptr;
     a.align_every = fwd_align_every();
@@ -1425,15 +1544,15 @@ template <class Core> static void launch_fwd(LmFwdArgs& a, float* ws, hipStream_
 }
 
 template <class Core> static void launch_grad(const LmGradArgs& a, hipStream_t s) {
-    lmhead_grad_kernel<Core><<<dim3((unsigned)patch_grid((a.op.m + Core::BM - 1) / Core::BM, (a.op.n + Core::BN - 1) / Core::BN, kGradPatchTokens)),
+    lmhead_grad_kernel<Core><<<dim3((unsigned)kGradPatches.grid((a.op.m + Core::BM - 1) / Core::BM, (a.op.n + Core::BN - 1) / Core::BN)),
                                dim3(GB_THREADS), 0, s>>>(a);
 }
 
 // C = or += A B^T with B in core C's fragment-major layout (op.ldb: its k extent); op.k a multiple of 64
-template <int MODE> static void launch_gemm(const GemmOperands& op, float* c, int64_t ldc, hipStream_t s, const int32_t* row_map = nullptr,
-                                            uint16_t* cb = nullptr) {
-    gemm_f32_kernel<CoreC, MODE><<<dim3((unsigned)patch_grid((op.m + CoreC::BM - 1) / CoreC::BM, (op.n + CoreC::BN - 1) / CoreC::BN)),
-                                   dim3(GB_THREADS), 0, s>>>(op, c, ldc, row_map, cb);
+template <int MODE> static void launch_gemm(const GemmOperands& op, const Patches& p, float* c, int64_t ldc, hipStream_t s,
+                                            const int32_t* row_map = nullptr, uint16_t* cb = nullptr) {
+    gemm_f32_kernel<CoreC, MODE><<<dim3((unsigned)p.grid((op.m + CoreC::BM - 1) / CoreC::BM, (op.n + CoreC::BN - 1) / CoreC::BN)),
+                                   dim3(GB_THREADS), 0, s>>>(op, p, c, ldc, row_map, cb, op.m * ldc);
 }
 
 extern "C" int64_t nrl_lmhead_kept_logits_bytes(int64_t n_tokens, int64_t vocab) {
@@ -1463,7 +1582,7 @@ extern "C" int nrl_lmhead_logprob_fwd(const void* hidden, int64_t n_tokens, int6
     if (hidden_size % CoreB::BK == 0) launch_fwd<CoreB>(a, ws, s);
     else launch_fwd<CoreA>(a, ws, s);
     const int splits = a.n_splits;
-    lmhead_fwd_finish_kernel<<<dim3((unsigned)((n_tokens + 255) / 256)), dim3(256), 0, s>>>(
+    lmhead_fwd_finish_kernel<<<dim3((unsigned)((n_tokens + kFinishTokens - 1) / kFinishTokens)), dim3(kFinishTokens * kFinishLanes), 0, s>>>(
         n_tokens, splits, a.part_m, a.part_s, a.xt, targets, vocab_start, vocab_end, logprob_out, lse_out);
     return check_launch("lmhead_logprob_fwd");
 }
@@ -1475,6 +1594,14 @@ static int64_t bwd_chunk(int64_t n) { return n < kBwdChunk ? round_up(n < 1 ? 1 
 // more than the chunk, because rows a power of two apart (16384 tokens = 32 KiB) fall on the same memory channels
 // (measured on the dW product: 1.6 % faster than unpadded; two lines more is 5 % slower, three as good as one).
 static int64_t bwd_ld_t(int64_t chunk) { return chunk + 64; }
+// dH of a chunk of `rows` tokens, with room for partial products of up to 32768 rows in all (0.5 GB at H 4096)
+static Patches dh_plan(int64_t rows, int64_t h, int64_t vp) { return gemm_plan(rows, h, vp, 32768 * h); }
+// dW of a batch that is one chunk, with room for partial products of up to 1 GiB
+static Patches dw_plan(int64_t vocab, int64_t h, int64_t rows) { return gemm_plan(vocab, h, rows, (1ll << 30) / 4); }
+static int64_t dh_parts_bytes(int64_t rows, int64_t h, int64_t vp) {
+    const int splits = rows > 0 ? dh_plan(rows, h, vp).splits : 1;
+    return splits > 1 ? splits * rows * h * 4 : 0;
+}
 
 extern "C" int64_t nrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t hidden_size, int64_t vocab) {
     const int64_t n = n_tokens < 1 ? 1 : n_tokens;
@@ -1484,10 +1611,14 @@ extern "C" int64_t nrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t hidd
     b += chunk * vp * 2;              // G
     b += vocab * bwd_ld_t(chunk) * 2;        // G^T
     b += round_up(hidden_size, 256) * bwd_ld_t(chunk) * 2;  // hidden chunk^T, fragment-major
-    b += vocab * hidden_size * 4;     // dW accumulator (fp32)
+    // dW: the fp32 accumulator of the chunks, or the partial products of a single chunk
+    b += vocab * hidden_size * 4 * (n <= chunk ? dw_plan(vocab, hidden_size, round_up(n, 64)).splits : 1);
+    // partial products of dH, of a whole chunk or of the last, shorter one
+    const int64_t whole = n >= chunk ? dh_parts_bytes(chunk, hidden_size, vp) : 0, rest = dh_parts_bytes(n % chunk, hidden_size, vp);
+    b += whole > rest ? whole : rest;
     b += n_pad * hidden_size * 2;     // hidden rows of the tokens that carry a gradient
     b += n_pad * (8 + 4 + 4 + 4);     // their targets, log-sum-exps, gradients and token indices
-    return b + 2048;
+    return b + 4096;
 }
 
 extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int64_t hidden_size, int64_t ldh,
@@ -1517,7 +1648,15 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     const int64_t ld_t = bwd_ld_t(chunk);
     uint16_t* gt = reinterpret_cast<uint16_t*>(take(vocab * ld_t * 2));
     uint16_t* ht = reinterpret_cast<uint16_t*>(take(h_pad * ld_t * 2));
-    float* dw = reinterpret_cast<float*>(take(vocab * h * 4));
+    const bool one_chunk = n_tokens <= chunk;
+    const Patches dw_patches = dw_plan(vocab, h, round_up(n_tokens < 1 ? 1 : n_tokens, 64));
+    float* dw = reinterpret_cast<float*>(take(vocab * h * 4 * (one_chunk ? dw_patches.splits : 1)));
+    float* dh_parts;
+    {
+        const int64_t n = n_tokens < 1 ? 1 : n_tokens;
+        const int64_t whole = n >= chunk ? dh_parts_bytes(chunk, h, vp) : 0, rest = dh_parts_bytes(n % chunk, h, vp);
+        dh_parts = reinterpret_cast<float*>(take(whole > rest ? whole : rest));
+    }
     uint16_t* hid_c = reinterpret_cast<uint16_t*>(take(n_pad * h * 2));
     int64_t* tgt_c = reinterpret_cast<int64_t*>(take(n_pad * 8));
     float* lse_c = reinterpret_cast<float*>(take(n_pad * 4));
@@ -1549,7 +1688,7 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     // dW is summed over the chunks in an fp32 buffer and narrowed once at the end.  The first chunk's product starts
     // the buffer (no zero fill, no read; zeros if the chunk turns out to hold no live token); when there is only one
     // chunk its product is written as bf16 straight to the output.
-    const bool single = n_tokens <= chunk && ld_dw == h;
+    const bool single = one_chunk && ld_dw == h;
     for (int64_t t0 = 0; t0 < n_tokens; t0 += chunk) {
         const int64_t rows = n_tokens - t0 < chunk ? n_tokens - t0 : chunk;   // upper bound: the live rows of this chunk
         const int64_t rows_pad = round_up(rows, 64);
@@ -1571,7 +1710,16 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
         GemmOperands dh;
         dh.a = g; dh.lda = vp; dh.b = wt; dh.ldb = vp; dh.m = rows; dh.n = h; dh.k = vp;
         dh.live = count; dh.live_from = t0; dh.live_dim = 1;
-        launch_gemm<0>(dh, dhidden_out, ld_dh, s, idx + t0);
+        const Patches dh_patches = dh_plan(rows, h, vp);
+        if (dh_patches.splits > 1) {
+            launch_gemm<0>(dh, dh_patches, dh_parts, h, s);
+            lmhead_finish_dh_kernel<true><<<dim3((unsigned)rows), dim3(256), 0, s>>>(
+                dhidden_out, ld_dh, dh_parts, dh_patches.splits, rows * h, idx + t0, count, t0, ga.grad, ga.targets, vocab_start, vocab, w, ldw, h);
+        } else {
+            launch_gemm<0>(dh, dh_patches, dhidden_out, ld_dh, s, idx + t0);
+            lmhead_finish_dh_kernel<false><<<dim3((unsigned)rows), dim3(256), 0, s>>>(
+                dhidden_out, ld_dh, nullptr, 1, 0, idx + t0, count, t0, ga.grad, ga.targets, vocab_start, vocab, w, ldw, h);
+        }
         // dW += G^T [V, rows] * (hidden^T [H, rows])^T
         transpose_to_frag_kernel<<<dim3((unsigned)(h_pad / 256), (unsigned)(rows_pad / 64)), dim3(256), 0, s>>>(
             hid_c + t0 * h, rows, h, h, ht, ld_t, rows_pad);
@@ -1579,9 +1727,12 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
         dwo.a = gt; dwo.lda = ld_t; dwo.b = ht; dwo.ldb = ld_t; dwo.m = vocab; dwo.n = h; dwo.k = rows_pad;
         dwo.live = count; dwo.live_from = t0; dwo.live_dim = 2;
         // (the narrowing epilogue writes with the accumulator's row stride)
-        if (single) launch_gemm<GEMM_NARROW>(dwo, dw, h, s, nullptr, static_cast<uint16_t*>(dweight_out));
-        else if (t0 == 0) launch_gemm<0>(dwo, dw, h, s);
-        else launch_gemm<GEMM_ACCUM>(dwo, dw, h, s);
+        if (single && dw_patches.splits > 1) {
+            launch_gemm<0>(dwo, dw_patches, dw, h, s);
+            lmhead_sum_dw_kernel<<<dim3(2048), dim3(256), 0, s>>>(static_cast<uint16_t*>(dweight_out), dw, dw_patches.splits, vocab * h, vocab * h);
+        } else if (single) launch_gemm<GEMM_NARROW>(dwo, dw_patches, dw, h, s, nullptr, static_cast<uint16_t*>(dweight_out));
+        else if (t0 == 0) launch_gemm<0>(dwo, Patches{}, dw, h, s);
+        else launch_gemm<GEMM_ACCUM>(dwo, Patches{}, dw, h, s);
     }
     if (n_tokens > 0 && !single) {
         uint16_t* out = static_cast<uint16_t*>(dweight_out);
@@ -1591,9 +1742,5 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
             for (int64_t r = 0; r < vocab; ++r) f32_to_bf16_kernel<<<dim3(4), dim3(256), 0, s>>>(dw + r * h, out + r * ld_dw, h);
         }
     }
-    if (n_tokens > 0)  // the one-hot term of dH in fp32, on the tokens' own rows
-        for (int64_t r = 0; r < n_tokens; r += 65535)
-            lmhead_onehot_dh_kernel<<<dim3((unsigned)(n_tokens - r < 65535 ? n_tokens - r : 65535)), dim3(256), 0, s>>>(
-                dhidden_out + r * ld_dh, ld_dh, grad + r, targets + r, vocab_start, vocab, w, ldw, h);
     return check_launch("lmhead_logprob_bwd");
 }

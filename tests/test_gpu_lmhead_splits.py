@@ -1,0 +1,50 @@
+"""The fused lm_head where its products are cut into k ranges and its forward into many vocabulary shares: few tiles and a
+long k, tile and slab remainders, a chunk whose tokens are all dead.  Bounds: see ``test_gpu_lmhead.narrowing_bounds``."""
+
+import pytest
+import torch
+
+from test_gpu_lmhead import narrowing_bounds
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _ops():
+    from rl_amd import ops  # noqa: F401
+
+    return torch.ops.rl_amd
+
+
+# (tokens, hidden, vocab): dH in many ranges of a ragged k; dH of one token; three token blocks; dW in ranges (few
+# vocabulary tiles, thousands of tokens); both products cut, a hidden size off the 64-wide slab
+@pytest.mark.parametrize("n,h,v", [(512, 256, 40009), (1, 64, 20000), (700, 128, 9000), (4100, 128, 700), (2050, 72, 4099)])
+@pytest.mark.parametrize("keep", [False, True])
+def test_split_products_match_oracle(n, h, v, keep):
+    g = torch.Generator().manual_seed(n + v)
+    hid = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    w = (torch.randn(v, h, generator=g) * 0.05).to(torch.bfloat16)
+    tgt = torch.randint(0, v, (n,), generator=g)
+    up = torch.randn(n, generator=g) * 1e-3
+    up[::5] = 0 if n > 1 else 1e-3
+    lp, lse, kept = _ops().lmhead_logprob_fwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), 0, v, keep)
+    logits = (hid.float() @ w.float().T)
+    want = torch.log_softmax(logits, -1).gather(-1, tgt.unsqueeze(-1)).squeeze(-1)
+    # one bf16 rounding of every logit (2^-9 of its size), of the target's and averaged in the log-sum-exp
+    assert (lp.cpu() - want).abs().max().item() <= 2.0 ** -7 * logits.abs().max().item() + 2e-3
+    dh, dw = _ops().lmhead_logprob_bwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), lse, up.to(DEV), 0, v, kept if keep else None)
+    o_dh, o_dw, b_dh, b_dw = narrowing_bounds(hid, w, tgt, up)
+    assert bool(((dh.cpu() - o_dh).abs() <= b_dh).all())
+    assert bool(((dw.float().cpu() - o_dw).abs() <= b_dw).all())
+    again = _ops().lmhead_logprob_bwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), lse, up.to(DEV), 0, v, kept if keep else None)
+    assert torch.equal(again[0], dh) and torch.equal(again[1], dw)  # partial products are added in a fixed order
+
+
+@pytest.mark.parametrize("n,h,v", [(300, 128, 20000), (4096, 64, 600)])
+def test_no_live_token_gives_zero_gradients(n, h, v):
+    hid = torch.randn(n, h, device=DEV).to(torch.bfloat16)
+    w = torch.randn(v, h, device=DEV).to(torch.bfloat16)
+    tgt = torch.zeros(n, dtype=torch.int64, device=DEV)
+    _, lse, _ = _ops().lmhead_logprob_fwd(hid, w, tgt, 0, v)
+    dh, dw = _ops().lmhead_logprob_bwd(hid, w, tgt, lse, torch.zeros(n, device=DEV), 0, v)
+    assert bool((dh == 0).all()) and bool((dw == 0).all())
