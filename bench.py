@@ -194,13 +194,13 @@ def timed(torch, ops, args, step):
         step()
     torch.cuda.synchronize()
     timer = EventTimer(torch)
-    ops.KERNEL_TIMER = timer
+    ops.set_kernel_timer(timer)
     t0 = time.perf_counter()
     for _ in range(args.steps):
         step()
     torch.cuda.synchronize()
     dt = time.perf_counter() - t0
-    ops.KERNEL_TIMER = None
+    ops.set_kernel_timer(None)
     return dt, timer.summary()
 
 

@@ -234,7 +234,12 @@ enum nrl_grpo_metric {
     NRL_M_POSITIVE_NLL_LOSS, NRL_M_ACTOR_LOSS, NRL_M_N_MASKED_TOKENS, NRL_GRPO_N_METRICS = 24
 };
 
-/* Every [B, Sm1] input is fp32 with unit column stride and its own row stride (so the
+/* element type of a token mask: as the data pipeline made it, no fp32 copy is needed */
+#define NRL_MASK_F32 0
+#define NRL_MASK_I64 1
+#define NRL_MASK_U8 2
+
+/* Every [B, Sm1] input is fp32 (the token mask excepted) with unit column stride and its own row stride (so the
  * reference's data[...][:, 1:] slices are passed as pointer + 1 with row stride S). */
 typedef struct nrl_grpo_inputs {
     int64_t batch, sm1;
@@ -244,10 +249,12 @@ typedef struct nrl_grpo_inputs {
     const float* gen; int64_t gen_stride;
     const float* ref; int64_t ref_stride;  /* NULL allowed when !has_kl                      */
     const float* adv; int64_t adv_stride;
-    const float* token_mask; int64_t token_mask_stride;
+    const void* token_mask; int64_t token_mask_stride;  /* fp32, or token_mask_type's elements */
     const float* sample_mask;   /* [B] */
     const float* correct_mask;  /* [B] (rewards > 0), NULL unless has_nll */
     const float* global_valid;  /* device [2]: {global_valid_seqs, global_valid_toks} */
+    const float* global_valid_toks;  /* device [1], or NULL: global_valid[1] */
+    int32_t token_mask_type;    /* NRL_MASK_* of the token_mask elements */
 } nrl_grpo_inputs;
 
 int64_t nrl_grpo_loss_workspace_bytes(int64_t batch);

@@ -59,6 +59,7 @@ class NrlGrpoInputs(C.Structure):
         ("adv", C.c_void_p), ("adv_stride", C.c_int64),
         ("token_mask", C.c_void_p), ("token_mask_stride", C.c_int64),
         ("sample_mask", C.c_void_p), ("correct_mask", C.c_void_p), ("global_valid", C.c_void_p),
+        ("global_valid_toks", C.c_void_p), ("token_mask_type", C.c_int32),
     ]
 
 
@@ -127,7 +128,7 @@ SIGNATURES = {
 _lib = None
 
 
-ABI_VERSION = 112  # nrl_version() of the library these signatures describe
+ABI_VERSION = 113  # nrl_version() of the library these signatures describe
 
 
 def load() -> C.CDLL:
@@ -152,6 +153,28 @@ def load() -> C.CDLL:
         )
     _lib = lib
     return lib
+
+
+HOST_PATH = os.path.join(_HERE, "lib", "_host.so")
+_host = None
+
+
+def host():
+    """The extension module of the calls' host side (``csrc/host_path.cpp``), loaded once with the HIP library it calls."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m rl_amd.build`. rl_amd has no other compute path.")
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries are what the extension links against)
+
+        spec = importlib.util.spec_from_file_location("rl_amd.lib._host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 class NrlError(RuntimeError):

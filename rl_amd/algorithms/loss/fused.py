@@ -17,9 +17,8 @@ import torch
 from ... import ops as _ops  # noqa: F401
 from ..._deferred import pending_temperature
 from ..._lib import NRL_TEMP_RCP
-from .loss_functions import ClippedPGLossFn, _f32, _global_valid, metrics_record_to_dict
-
-_OPS = torch.ops.rl_amd
+from ..._lib import host as _host
+from .loss_functions import ClippedPGLossFn, _scalar, metrics_record_to_dict
 
 
 def why_not_fusable(loss_fn, logits, data, sampling_params=None) -> Optional[str]:
@@ -55,50 +54,6 @@ def why_not_fusable(loss_fn, logits, data, sampling_params=None) -> Optional[str
     return None
 
 
-def _rescale(dlogits, grad_loss, loss_scale):
-    """The stored gradient was computed for an upstream factor of ``loss_scale``.  Whatever factor autograd
-    actually delivers is applied in place by one kernel that reads it from the device: the host never waits
-    for its value, no second ``[B, S, V]`` tensor exists, and when the two agree (the normal case) the kernel
-    touches no memory."""
-    if not isinstance(grad_loss, torch.Tensor) or not grad_loss.is_cuda:
-        grad_loss = torch.as_tensor(grad_loss, dtype=torch.float32, device=dlogits.device)
-    view = dlogits if dlogits.dim() == 3 else dlogits.unsqueeze(0)
-    _OPS.scale_rows_(view, grad_loss, float(loss_scale))
-    return dlogits
-
-
-def _hand_over(ctx, grad_loss):
-    dlogits, ctx.dlogits = ctx.dlogits, None
-    if dlogits is None:
-        raise RuntimeError("the single-pass loss hands its gradient buffer to autograd once; a second backward "
-                           "through the same loss needs a new forward")
-    return _rescale(dlogits, grad_loss, ctx.loss_scale)
-
-
-class _FusedLogitsLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits, targets, n_inner, prev, gen, ref, adv, token_mask, sample_mask, global_valid, iflags, fparams,
-                loss_scale, in_place, temperature):
-        x = logits.detach()
-        if in_place:
-            loss, lp, metrics = _OPS.fused_logits_grpo_loss_(
-                x, targets, n_inner, prev, gen, ref, adv, token_mask, sample_mask, global_valid, iflags, fparams, loss_scale,
-                temperature, NRL_TEMP_RCP)
-            dlogits = x  # the caller declared the logits dead; their storage now holds the gradient
-        else:
-            loss, dlogits, lp, metrics = _OPS.fused_logits_grpo_loss(
-                x, targets, n_inner, prev, gen, ref, adv, token_mask, sample_mask, global_valid, iflags, fparams, loss_scale,
-                temperature, NRL_TEMP_RCP)
-        ctx.dlogits = dlogits  # an intermediate, neither input nor output: held directly so it can be rescaled in place
-        ctx.loss_scale = loss_scale
-        ctx.mark_non_differentiable(lp, metrics)
-        return loss, lp, metrics
-
-    @staticmethod
-    def backward(ctx, grad_loss, _g_lp, _g_metrics):
-        return (_hand_over(ctx, grad_loss),) + (None,) * 14
-
-
 def fused_logits_clipped_pg_loss(
     logits: torch.Tensor,
     data: Any,
@@ -121,39 +76,18 @@ def fused_logits_clipped_pg_loss(
     if reason is not None:
         raise NotImplementedError(f"fused logits->loss path: {reason}")
     dev = logits.device
-    ids = data["input_ids"].to(dev)
-    if ids.dtype != torch.int64:
-        ids = ids.long()
-    n_inner = ids.shape[1] - 1
-    beta = loss_fn.reference_policy_kl_penalty
+    ids = data["input_ids"]
     sample_mask_in = data["sample_mask"]
-    prev = None if loss_fn.force_on_policy_ratio else _f32(data["prev_logprobs"][:, 1:], dev)
-    ref = _f32(data["reference_policy_logprobs"][:, 1:], dev) if beta != 0 else None
     iflags, fparams = loss_fn._kernel_config(False)
-    loss, _lp, metrics = _FusedLogitsLoss.apply(
-        logits, ids[:, 1:], n_inner, prev, _f32(data["generation_logprobs"][:, 1:], dev), ref,
-        _f32(data["advantages"][:, 1:], dev), _f32(data["token_mask"][:, 1:], dev), _f32(sample_mask_in, dev),
-        _global_valid(global_valid_seqs, global_valid_toks, dev), iflags, fparams, float(loss_scale), bool(in_place),
-        pending_temperature(logits),  # a divide apply_temperature_scaling left to this kernel
+    # (row (b, i) reads input_ids[b, i + 1] and column i + 1 of the loss inputs: offsets, not slices)
+    loss, metrics = _host().fused_clipped_pg(
+        logits, ids, 1, ids.shape[1] - 1, None, None if loss_fn.force_on_policy_ratio else data["prev_logprobs"],
+        data["generation_logprobs"], data["reference_policy_logprobs"] if loss_fn.reference_policy_kl_penalty != 0 else None,
+        data["advantages"], data["token_mask"], sample_mask_in, _scalar(global_valid_seqs, dev), _scalar(global_valid_toks, dev), iflags,
+        fparams, float(loss_scale), pending_temperature(logits),  # a divide apply_temperature_scaling left to this kernel
+        NRL_TEMP_RCP, bool(in_place),
     )
     return loss, metrics_record_to_dict(metrics, loss_fn, sample_mask_in)
-
-
-class _FusedPackedLogitsLoss(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits2d, targets, cu, unpacked_seqlen, prev, gen, ref, adv, token_mask, sample_mask, global_valid, iflags,
-                fparams, loss_scale, temperature):
-        loss, dlogits, lp, metrics = _OPS.fused_packed_logits_grpo_loss(
-            logits2d.detach(), targets, True, cu, unpacked_seqlen, prev, gen, ref, adv, token_mask, sample_mask, global_valid,
-            iflags, fparams, loss_scale, temperature, NRL_TEMP_RCP)
-        ctx.dlogits = dlogits  # an intermediate, neither input nor output: held directly so it can be rescaled in place
-        ctx.loss_scale = loss_scale
-        ctx.mark_non_differentiable(lp, metrics)
-        return loss, lp, metrics
-
-    @staticmethod
-    def backward(ctx, grad_loss, _g_lp, _g_metrics):
-        return (_hand_over(ctx, grad_loss),) + (None,) * 14
 
 
 def why_not_fusable_packed(loss_fn, logits, data, sampling_params=None) -> Optional[str]:
@@ -181,16 +115,12 @@ def fused_packed_logits_clipped_pg_loss(logits, data, loss_fn, cu_seqlens_q, cu_
     x = logits.squeeze(0)
     targets = _packed_targets(input_ids, cu_seqlens_q, cu_seqlens_q_padded, x.shape[0], dev).reshape(-1)
     cu = _checked_cu_seqlens(cu_seqlens_q_padded, x.shape[0], targets.shape[0], dev)
-    beta = loss_fn.reference_policy_kl_penalty
     sample_mask_in = data["sample_mask"]
-    prev = None if loss_fn.force_on_policy_ratio else _f32(data["prev_logprobs"][:, 1:], dev)
-    ref = _f32(data["reference_policy_logprobs"][:, 1:], dev) if beta != 0 else None
     iflags, fparams = loss_fn._kernel_config(False)
-    loss, _lp, metrics = _FusedPackedLogitsLoss.apply(
-        x, targets, cu, input_ids.shape[1], prev,
-        _f32(data["generation_logprobs"][:, 1:], dev), ref, _f32(data["advantages"][:, 1:], dev),
-        _f32(data["token_mask"][:, 1:], dev), _f32(sample_mask_in, dev),
-        _global_valid(global_valid_seqs, global_valid_toks, dev), iflags, fparams, float(loss_scale),
-        pending_temperature(logits),
+    loss, metrics = _host().fused_clipped_pg(
+        x, targets, 0, input_ids.shape[1] - 1, cu, None if loss_fn.force_on_policy_ratio else data["prev_logprobs"],
+        data["generation_logprobs"], data["reference_policy_logprobs"] if loss_fn.reference_policy_kl_penalty != 0 else None,
+        data["advantages"], data["token_mask"], sample_mask_in, _scalar(global_valid_seqs, dev), _scalar(global_valid_toks, dev), iflags,
+        fparams, float(loss_scale), pending_temperature(logits), NRL_TEMP_RCP, False,
     )
     return loss, metrics_record_to_dict(metrics, loss_fn, sample_mask_in)

@@ -16,6 +16,7 @@ from pydantic import BaseModel
 
 from ... import ops as _ops  # noqa: F401
 from ..._lib import METRIC_SLOTS, NRL_TIS
+from ..._lib import host as _host
 from .interfaces import LossFunction, LossInputType, LossType, MetricNormalizer
 
 _OPS = torch.ops.rl_amd
@@ -56,6 +57,11 @@ def _gpu_for(t: torch.Tensor) -> torch.device:
 
 def _f32(t, dev):
     return t.to(device=dev, dtype=torch.float32)
+
+
+def _scalar(value, dev) -> torch.Tensor:
+    """A count as a one-element tensor (which the host path moves to the loss's device if it is elsewhere)."""
+    return value if isinstance(value, torch.Tensor) else torch.tensor(float(value), dtype=torch.float32, device=dev)
 
 
 def _global_valid(seqs, toks, dev) -> torch.Tensor:
@@ -202,18 +208,7 @@ def fetch_later(record: torch.Tensor):
         fetch = lambda: values()  # noqa: E731
         fetch.ready = lambda: True
         return fetch
-    host = torch.empty(record.shape, dtype=record.dtype, pin_memory=True)
-    host.copy_(record, non_blocking=True)
-    done = torch.cuda.Event()
-    done.record()
-
-    def fetch():
-        if not done.query():
-            done.synchronize()
-        return host.tolist()
-
-    fetch.ready = done.query
-    return fetch
+    return _host().Fetch(record)
 
 
 def metrics_record_to_dict(metrics: torch.Tensor, loss_fn, sample_mask_in: torch.Tensor) -> dict:
@@ -242,29 +237,6 @@ def metrics_record_to_dict(metrics: torch.Tensor, loss_fn, sample_mask_in: torch
 
     build.ready = values.ready
     return StepMetrics(keys, build) if getattr(loss_fn, "lazy_metrics", True) else build()
-
-
-class _FusedLoss(torch.autograd.Function):
-    """loss, metrics = kernel(lp, lpu, ...); the kernel also returns d loss / d lp (and / d lpu), so the
-    backward is a scalar multiply."""
-
-    @staticmethod
-    def forward(ctx, lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct, global_valid, iflags, fparams):
-        loss, dlp, dlpu, metrics = _OPS.grpo_loss(
-            lp.detach(), None if lpu is None else lpu.detach(), prev, gen, ref, adv, token_mask, sample_mask, correct,
-            global_valid, iflags, fparams,
-        )
-        ctx.save_for_backward(dlp, dlpu)
-        ctx.has_lpu = lpu is not None and dlpu.numel() > 0
-        ctx.mark_non_differentiable(metrics)
-        return loss, metrics
-
-    @staticmethod
-    def backward(ctx, grad_loss, _grad_metrics):
-        dlp, dlpu = ctx.saved_tensors
-        g_lp = dlp * grad_loss if ctx.needs_input_grad[0] else None
-        g_lpu = dlpu * grad_loss if (ctx.has_lpu and ctx.needs_input_grad[1]) else None
-        return (g_lp, g_lpu) + (None,) * 10
 
 
 class ClippedPGLossFn(LossFunction):
@@ -402,15 +374,9 @@ class ClippedPGLossFn(LossFunction):
         beta = self.reference_policy_kl_penalty
 
         sample_mask_in = data["sample_mask"]
-        lp = _f32(lp_in, dev)
-        token_mask = _f32(data["token_mask"][:, 1:], dev)
-        sample_mask = _f32(sample_mask_in, dev)
-        adv = _f32(data["advantages"][:, 1:], dev)
-        prev = None if self.force_on_policy_ratio else _f32(data["prev_logprobs"][:, 1:], dev)
-        gen = _f32(data["generation_logprobs"][:, 1:], dev)
         ref = lpu = None
         if beta != 0:
-            ref = _f32(data["reference_policy_logprobs"][:, 1:], dev)
+            ref = data["reference_policy_logprobs"]
             unfiltered = data.get("curr_logprobs_unfiltered", None)
             if unfiltered is not None and unfiltered is not lp_in:
                 lpu = _f32(unfiltered, dev)
@@ -419,10 +385,12 @@ class ClippedPGLossFn(LossFunction):
         if has_nll:
             correct = (data["rewards"] > 0).to(device=dev, dtype=torch.float32)
         iflags, fparams = self._kernel_config(has_nll)
-
-        loss, metrics = _FusedLoss.apply(
-            lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct,
-            _global_valid(global_valid_seqs, global_valid_toks, dev), iflags, fparams,
+        # the [B, S] tensors go in as they are: the host path reads them from column 1 on and the kernels take the mask in
+        # the type the data pipeline made it
+        loss, metrics = _host().clipped_pg(
+            _f32(lp_in, dev), lpu, None if self.force_on_policy_ratio else data["prev_logprobs"], data["generation_logprobs"], ref,
+            data["advantages"], data["token_mask"], sample_mask_in, correct, _scalar(global_valid_seqs, dev),
+            _scalar(global_valid_toks, dev), iflags, fparams,
         )
         if home != dev:
             loss = loss.to(home)

@@ -70,16 +70,15 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
     const float* gen_row = in.gen + b * in.gen_stride;
     const float* ref_row = c.has_kl ? in.ref + b * in.ref_stride : nullptr;
     const float* adv_row = in.adv + b * in.adv_stride;
-    const float* tm_row = in.token_mask + b * in.token_mask_stride;
     const float smv = in.sample_mask[b];
     const float correct = c.has_nll ? in.correct_mask[b] : 0.f;
-    const float den_s = in.global_valid[0] + 1e-8f;
-    const float den_t = in.global_valid[1] + 1e-8f;
+    const float den_s = valid_seqs(in) + 1e-8f;
+    const float den_t = valid_toks(in) + 1e-8f;
 
     // ---- row statistics ----
     double s_tm = 0, s_lr = 0, s_is = 0, s_geo = 0;
     for (int64_t t = tid; t < n; t += kLossBlock) {
-        const float tm = tm_row[t];
+        const float tm = mask_at(in, b, t);
         const float prev = prev_row[t], gen = gen_row[t];
         s_tm += tm;
         s_lr += (lp_row[t] - prev) * tm;
@@ -107,7 +106,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
     for (int64_t t = tid; t < n; t += kLossBlock) {
         TokenIn ti;
         ti.lp = lp_row[t]; ti.lpu = lpu_row[t]; ti.prev = prev_row[t]; ti.gen = gen_row[t];
-        ti.ref = c.has_kl ? ref_row[t] : 0.f; ti.adv = adv_row[t]; ti.tm = tm_row[t]; ti.smv = smv; ti.correct = correct;
+        ti.ref = c.has_kl ? ref_row[t] : 0.f; ti.adv = adv_row[t]; ti.tm = mask_at(in, b, t); ti.smv = smv; ti.correct = correct;
         ti.den_t = den_t; ti.den_s = den_s;
         const TokenOut o = token_eval<GSPO>(c, st, ti);
 #pragma unroll
@@ -133,7 +132,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
         // d ratio_b / d lp[b, s] = ratio_b * tm[b, s] / (n_tm + 1e-8)
         const float k_tot = static_cast<float>(block_sum<double, kLossWaves>(gspo_k, sm_d));
         for (int64_t t = tid; t < n; t += kLossBlock) {
-            const float share = k_tot * seq_ratio * (tm_row[t] / seq_den);
+            const float share = k_tot * seq_ratio * (mask_at(in, b, t) / seq_den);
             if (a.dlpu) a.dlp[b * n + t] = share;
             else a.dlp[b * n + t] += share;
         }
@@ -166,7 +165,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_finish_kernel(GrpoArgs a, flo
     rc_min = block_min<kLossWaves>(rc_min, sm_f); rc_max = block_max<kLossWaves>(rc_max, sm_f);
     if (tid != 0) return;
 
-    const double den_s = a.in.global_valid[0] + 1e-8f, den_t = a.in.global_valid[1] + 1e-8f;
+    const double den_s = valid_seqs(a.in) + 1e-8f, den_t = valid_toks(a.in) + 1e-8f;
     const double den_loss = c.token_level_loss ? den_t : den_s;
     const float actor = static_cast<float>(tot[P_ACTOR] / den_loss);
     const float kl = c.has_kl ? static_cast<float>(tot[P_KL] / den_loss) : 0.f;
@@ -210,7 +209,7 @@ __global__ void grpo_nll_grad_kernel(GrpoArgs a) {
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < total;
          i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const int64_t b = i / n, t = i - b * n;
-        const float cm = a.in.token_mask[b * a.in.token_mask_stride + t] * a.in.sample_mask[b] * a.in.correct_mask[b];
+        const float cm = mask_at(a.in, b, t) * a.in.sample_mask[b] * a.in.correct_mask[b];
         a.dlp[i] += a.cfg.nll_weight * (-(cm / den));
     }
 }
@@ -220,10 +219,10 @@ __global__ __launch_bounds__(kLossBlock) void nll_rows_kernel(nrl_grpo_inputs in
     __shared__ double sm_d[kLossWaves];
     const int64_t b = blockIdx.x, n = in.sm1;
     const float smv = in.sample_mask[b];
-    const float den_t = in.global_valid[1] + 1e-8f;
+    const float den_t = valid_toks(in) + 1e-8f;
     double s = 0, cnt = 0;
     for (int64_t t = threadIdx.x; t < n; t += kLossBlock) {
-        const float mask = in.token_mask[b * in.token_mask_stride + t] * smv;
+        const float mask = mask_at(in, b, t) * smv;
         s += in.lp[b * in.lp_stride + t] * mask;
         cnt += mask;
         dlp[b * n + t] = -(mask / den_t);
@@ -242,7 +241,7 @@ __global__ __launch_bounds__(kLossBlock) void nll_finish_kernel(nrl_grpo_inputs 
     cnt = block_sum<double, kLossWaves>(cnt, sm_d);
     smv = block_sum<double, kLossWaves>(smv, sm_d);
     if (threadIdx.x == 0) {
-        const double den_t = in.global_valid[1] + 1e-8f;
+        const double den_t = valid_toks(in) + 1e-8f;
         const float loss = -static_cast<float>(s / den_t);
         loss_out[0] = loss;
         metrics[0] = loss; metrics[1] = static_cast<float>(cnt); metrics[2] = static_cast<float>(smv);
@@ -348,7 +347,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_seq_stats_kernel(FusedArgs a)
     double s_tm = 0, s_is = 0, s_geo = 0;
     const bool need_prev = c.sequence_level_importance_ratios || c.tis_type == NRL_TIS_SEQ_MASK;
     for (int64_t t = threadIdx.x; t < n; t += kLossBlock) {
-        const float tm = in.token_mask[b * in.token_mask_stride + t];
+        const float tm = mask_at(in, b, t);
         s_tm += tm;
         if (need_prev) {
             const float d = in.prev[b * in.prev_stride + t] - in.gen[b * in.gen_stride + t];
@@ -427,7 +426,7 @@ __global__ __launch_bounds__(kFusedBlock) void fused_logits_loss_kernel(FusedArg
             const FusedPos q = fused_where<PACKED>(a, r);
             const int64_t o = q.o, i = q.i;
             float w = 0.f;
-            if (i < a.n_inner) w = in.token_mask[o * in.token_mask_stride + i] * in.sample_mask[o];
+            if (i < a.n_inner) w = mask_at(in, o, i) * in.sample_mask[o];
             if (w != 0.f) break;
             u32x4* ov = reinterpret_cast<u32x4*>(out_row(r));
             for (int v = tid; v < nvec; v += kFusedBlock) ov[v] = zero;
@@ -498,11 +497,11 @@ __global__ __launch_bounds__(kFusedBlock) void fused_logits_loss_kernel(FusedArg
             ti.gen = in.gen[o * in.gen_stride + i];
             ti.ref = c.has_kl ? in.ref[o * in.ref_stride + i] : 0.f;
             ti.adv = in.adv[o * in.adv_stride + i];
-            ti.tm = in.token_mask[o * in.token_mask_stride + i];
+            ti.tm = mask_at(in, o, i);
             ti.smv = in.sample_mask[o];
             ti.correct = 0.f;
-            ti.den_s = in.global_valid[0] + 1e-8f;
-            ti.den_t = in.global_valid[1] + 1e-8f;
+            ti.den_s = valid_seqs(in) + 1e-8f;
+            ti.den_t = valid_toks(in) + 1e-8f;
             const TokenOut out = token_eval<false>(c, st, ti);
             float* rec = a.terms + tok * T_COUNT;
 #pragma unroll
@@ -602,6 +601,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_terms_reduce_kernel(FusedArgs
 
 static int check_inputs(const nrl_grpo_inputs* in, bool need_prev, bool need_ref, bool need_adv) {
     if (!in) return fail(NRL_E_INVALID, "inputs is NULL");
+    if (in->token_mask_type < NRL_MASK_F32 || in->token_mask_type > NRL_MASK_U8) return fail(NRL_E_INVALID, "unknown token mask type");
     if (in->batch < 0 || in->sm1 < 0) return fail(NRL_E_INVALID, "bad shape [%lld, %lld]", (long long)in->batch, (long long)in->sm1);
     if (in->batch >= (1ll << 31)) return fail(NRL_E_INVALID, "batch too large");
     if (in->batch * in->sm1 == 0) return NRL_OK;
@@ -892,6 +892,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     if (!rows || !cfg || !in) return fail(NRL_E_INVALID, "null argument");
     if (rows->dtype != NRL_F32 && rows->dtype != NRL_BF16 && rows->dtype != NRL_F16) return fail(NRL_E_INVALID, "unknown logits dtype");
     if (rows->n_outer < 0 || rows->n_inner < 0 || rows->vocab <= 0 || d_n_inner < rows->n_inner) return fail(NRL_E_INVALID, "bad shape");
+    if (in->token_mask_type < NRL_MASK_F32 || in->token_mask_type > NRL_MASK_U8) return fail(NRL_E_INVALID, "unknown token mask type");
     if (!cu && (in->batch != rows->n_outer || in->sm1 != rows->n_inner)) return fail(NRL_E_INVALID, "loss inputs and logits rows disagree");
     if (cu && (in->batch != n_seq || rows->n_outer != 1 || n_seq < 0)) return fail(NRL_E_INVALID, "packed loss inputs and cu_seqlens disagree");
     if (rows->vocab_end - rows->vocab_start != rows->vocab) return fail(NRL_E_INVALID, "vocab range does not span the columns");

@@ -24,6 +24,18 @@ struct GrpoArgs {
     double* parts;  // [B, P_COUNT]
 };
 
+// token t of sequence b in the mask's own element type (the branch is uniform over the launch)
+__device__ __forceinline__ float mask_at(const nrl_grpo_inputs& in, int64_t b, int64_t t) {
+    const int64_t i = b * in.token_mask_stride + t;
+    if (in.token_mask_type == NRL_MASK_F32) return static_cast<const float*>(in.token_mask)[i];
+    if (in.token_mask_type == NRL_MASK_I64) return static_cast<float>(static_cast<const int64_t*>(in.token_mask)[i]);
+    return static_cast<float>(static_cast<const uint8_t*>(in.token_mask)[i]);
+}
+__device__ __forceinline__ float valid_seqs(const nrl_grpo_inputs& in) { return in.global_valid[0]; }
+__device__ __forceinline__ float valid_toks(const nrl_grpo_inputs& in) {
+    return in.global_valid_toks ? in.global_valid_toks[0] : in.global_valid[1];
+}
+
 // per-sequence quantities the token terms depend on
 struct SeqStats {
     float seq_den;    // sum(token_mask) + 1e-8

@@ -1,0 +1,716 @@
+// The host side of the calls a training step makes, in C++: argument checks, outputs and workspaces, the launch through
+// the C ABI of nrl_hip.h, and the autograd nodes.  A microbatch of a few hundred rows takes the device less than 100
+// microseconds; the same path in Python (custom-op dispatch, ctypes structures, tensor slicing, conversion kernels for
+// the masks, backward nodes that need the interpreter lock on the autograd thread) took the host 240 - 460.  Everything
+// here is host code; PyTorch supplies memory, streams and the graph, the kernels are in librl_amd_hip.so.
+//
+// Tensors named `rows` are [B, S, V] logits; loss inputs are the [B, S] tensors as the data pipeline made them, whose
+// column t + 1 belongs to row t: they are read at an offset of one element instead of being sliced.
+
+#include <hip/hip_runtime.h>
+#include <torch/extension.h>
+
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <algorithm>
+#include <cstdlib>
+#include <memory>
+#include <optional>
+#include <string>
+#include <vector>
+
+#include "../../include/nrl_hip.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+// ---------------------------------------------------------------------------------------------
+// launch-time helpers
+// ---------------------------------------------------------------------------------------------
+// Optional per-launch timing: a Python object with start(name) / stop(name), None in normal use.
+py::object* g_timer = nullptr;
+struct Timed {
+    const char* name;
+    explicit Timed(const char* n) : name(g_timer ? n : nullptr) {
+        if (name) { py::gil_scoped_acquire gil; g_timer->attr("start")(name); }
+    }
+    ~Timed() {
+        if (name && g_timer) { py::gil_scoped_acquire gil; g_timer->attr("stop")(name); }
+    }
+};
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+void check(int code, const char* what) {
+    if (code == NRL_OK) return;
+    const std::string text = std::string(what) + " failed (" + std::to_string(code) + "): " + nrl_last_error();
+    TORCH_CHECK_VALUE(code != NRL_E_INVALID && code != NRL_E_WORKSPACE, text);
+    TORCH_CHECK_NOT_IMPLEMENTED(code != NRL_E_UNSUPPORTED, text);
+    TORCH_CHECK(false, text);
+}
+
+void need_gpu(const Tensor& t) {
+    TORCH_CHECK(!t.defined() || t.is_cuda(), "rl_amd ops run on the GPU only (got a CPU tensor); there is no CPU fallback");
+}
+template <typename... T> void need_gpu(const Tensor& t, const T&... more) { need_gpu(t); need_gpu(more...); }
+
+Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+template <typename T = float> T* ptr(const Tensor& t) { return t.defined() && t.numel() > 0 ? static_cast<T*>(t.data_ptr()) : nullptr; }
+
+int dtype_code(const Tensor& t) {
+    switch (t.scalar_type()) {
+        case at::kFloat: return NRL_F32;
+        case at::kBFloat16: return NRL_BF16;
+        case at::kHalf: return NRL_F16;
+        default: TORCH_CHECK_VALUE(false, "unsupported logits dtype ", t.scalar_type()); return -1;
+    }
+}
+
+Tensor f32(at::IntArrayRef shape, const Tensor& like) { return at::empty(shape, like.options().dtype(at::kFloat)); }
+Tensor workspace(int64_t bytes, const Tensor& like) { return at::empty({(bytes + 7) / 8}, like.options().dtype(at::kDouble)); }
+Tensor to_f32(const Tensor& t, const Tensor& like) {
+    if (!t.defined() || (t.device() == like.device() && t.scalar_type() == at::kFloat)) return t;
+    return t.to(like.device(), at::kFloat);
+}
+
+// An uninitialised tensor of `shape` in `like`'s dtype for a kernel that streams `like` in and the new tensor out at the
+// same time.  The kernels read and write rows at a fixed distance from each other, and how fast HBM serves the two
+// streams together depends on that distance modulo the address interleave: with both buffers on 2 MiB boundaries a 256
+// KiB row (V = 131072 bf16) loses 5 - 17 %, and distances of 64 - 256 KiB lose 8 % at V = 151936.  Starting the output
+// 1.69 MiB into the period (NRL_GRAD_PHASE overrides, for tuning) was at or near the best measured for both, so large
+// outputs are placed there inside a slightly larger allocation.
+Tensor grad_buffer(at::IntArrayRef shape, const Tensor& like) {
+    constexpr int64_t kPeriod = 1 << 21, kFrom = 64 << 20;
+    static const int64_t phase = [] {
+        const char* v = getenv("NRL_GRAD_PHASE");
+        return (v ? strtoll(v, nullptr, 0) : 0x1B0000ll) % kPeriod;
+    }();
+    int64_t n = 1;
+    for (int64_t d : shape) n *= d;
+    const int64_t size = static_cast<int64_t>(like.element_size()), bytes = n * size;
+    if (bytes < kFrom) return at::empty(shape, like.options());
+    const Tensor flat = at::empty({bytes + kPeriod}, like.options().dtype(at::kByte));
+    int64_t off = (reinterpret_cast<int64_t>(like.data_ptr()) + phase - reinterpret_cast<int64_t>(flat.data_ptr())) % kPeriod;
+    if (off < 0) off += kPeriod;
+    off -= off % 256;  // keeps every row start as aligned as in a fresh allocation
+    return flat.narrow(0, off, bytes).view(like.scalar_type()).view(shape);
+}
+
+nrl_rows make_rows(const Tensor& logits, const Tensor& targets, int64_t n_inner, int64_t v0, int64_t v1, double temperature, int64_t mode) {
+    TORCH_CHECK_VALUE(logits.dim() == 3 && (!targets.defined() || targets.dim() == 2), "expected logits [B,S,V] and targets [B,S'], got ",
+                      logits.sizes());
+    const int64_t b = logits.size(0), s = logits.size(1), v = logits.size(2);
+    TORCH_CHECK_VALUE(logits.stride(2) == 1 || v <= 1, "the vocabulary axis of the logits must be contiguous");
+    nrl_rows r{};
+    r.logits = logits.data_ptr();
+    r.dtype = dtype_code(logits);
+    r.n_outer = b; r.n_inner = n_inner; r.vocab = v;
+    r.stride_outer = logits.stride(0); r.stride_inner = logits.stride(1);
+    if (targets.defined()) {
+        TORCH_CHECK_VALUE(targets.scalar_type() == at::kLong, "targets must be int64, got ", targets.scalar_type());
+        TORCH_CHECK_VALUE(targets.size(0) == b && n_inner <= s && n_inner <= targets.size(1) && n_inner >= 0, "rows [", b, ", ", n_inner,
+                          "] do not fit logits ", logits.sizes(), " / targets ", targets.sizes());
+        r.targets = targets.data_ptr<int64_t>();
+        r.tgt_stride_outer = targets.stride(0); r.tgt_stride_inner = targets.stride(1);
+    } else {
+        TORCH_CHECK_VALUE(n_inner <= s && n_inner >= 0, "n_inner ", n_inner, " does not fit logits ", logits.sizes());
+    }
+    r.vocab_start = v0; r.vocab_end = v1;
+    r.temperature = static_cast<float>(temperature);
+    r.temp_mode = static_cast<int32_t>(mode);
+    return r;
+}
+
+// fp32 rows of [b, n] inside a tensor of [b, n + shift] read from column `shift`, unit column stride
+struct RowMat {
+    Tensor keep;
+    const float* p = nullptr;
+    int64_t stride = 0;
+};
+RowMat row_mat(const Tensor& t_in, const Tensor& like, int64_t b, int64_t n, int64_t shift, const char* name) {
+    RowMat m;
+    if (!t_in.defined()) return m;
+    Tensor t = to_f32(t_in, like);
+    // (an empty row has nothing in front of its first column either)
+    TORCH_CHECK_VALUE(t.dim() == 2 && t.size(0) == b && std::max<int64_t>(t.size(1) - shift, 0) == n, name, " must be [", b, ", ", n + shift, "], got ", t.sizes());
+    if (t.size(1) > 1 && t.stride(1) != 1) t = t.contiguous();
+    m.keep = t;
+    m.p = n > 0 ? t.data_ptr<float>() + shift : nullptr;
+    m.stride = b > 1 ? t.stride(0) : n + shift;
+    return m;
+}
+
+struct LossInputs {
+    nrl_grpo_inputs in{};
+    std::vector<Tensor> keep;
+    void rows(const Tensor& t, const Tensor& like, int64_t shift, const char* name, const float** p, int64_t* stride) {
+        RowMat m = row_mat(t, like, in.batch, in.sm1, shift, name);
+        *p = m.p;
+        *stride = m.stride;
+        if (m.keep.defined()) keep.push_back(std::move(m.keep));
+    }
+    const float* vec(const Tensor& t_in, const Tensor& like, const char* name) {
+        if (!t_in.defined()) return nullptr;
+        Tensor t = to_f32(t_in, like);
+        TORCH_CHECK_VALUE(t.dim() == 1 && t.size(0) == in.batch, name, " must be [", in.batch, "], got ", t.sizes());
+        keep.push_back(t.contiguous());
+        return keep.back().data_ptr<float>();
+    }
+    // one value on the device, from a tensor or a number
+    const float* scalar(const Tensor& t_in, const Tensor& like, const char* name) {
+        TORCH_CHECK_VALUE(t_in.numel() == 1, name, " must hold one value");
+        keep.push_back(to_f32(t_in.detach(), like));
+        return keep.back().data_ptr<float>();
+    }
+    void mask(const Tensor& t_in, const Tensor& like, int64_t shift) {
+        Tensor t = t_in.device() == like.device() ? t_in : t_in.to(like.device());
+        const auto type = t.scalar_type();
+        if (type == at::kLong) in.token_mask_type = NRL_MASK_I64;
+        else if (type == at::kByte || type == at::kBool) in.token_mask_type = NRL_MASK_U8;
+        else { in.token_mask_type = NRL_MASK_F32; t = to_f32(t, like); }
+        TORCH_CHECK_VALUE(t.dim() == 2 && t.size(0) == in.batch && std::max<int64_t>(t.size(1) - shift, 0) == in.sm1, "token_mask must be [", in.batch, ", ",
+                          in.sm1 + shift, "], got ", t.sizes());
+        if (t.size(1) > 1 && t.stride(1) != 1) t = t.contiguous();
+        in.token_mask = in.sm1 > 0 ? static_cast<const char*>(t.data_ptr()) + shift * static_cast<int64_t>(t.element_size()) : nullptr;
+        in.token_mask_stride = in.batch > 1 ? t.stride(0) : in.sm1 + shift;
+        keep.push_back(std::move(t));
+    }
+};
+
+// the [B, S] tensors of a loss call
+struct LossData {
+    Tensor prev, gen, ref, adv, token_mask, sample_mask, correct, seqs, toks;
+    int64_t shift = 1;  // columns in front of the first one that is read
+};
+
+LossInputs loss_inputs(const LossData& d, const Tensor& like, int64_t b, int64_t n) {
+    LossInputs l;
+    l.keep.reserve(12);
+    l.in.batch = b; l.in.sm1 = n;
+    l.rows(d.prev, like, d.shift, "prev", &l.in.prev, &l.in.prev_stride);
+    l.rows(d.gen, like, d.shift, "gen", &l.in.gen, &l.in.gen_stride);
+    l.rows(d.ref, like, d.shift, "ref", &l.in.ref, &l.in.ref_stride);
+    l.rows(d.adv, like, d.shift, "adv", &l.in.adv, &l.in.adv_stride);
+    l.mask(d.token_mask, like, d.shift);
+    l.in.sample_mask = l.vec(d.sample_mask, like, "sample_mask");
+    l.in.correct_mask = l.vec(d.correct, like, "correct_mask");
+    l.in.global_valid = l.scalar(d.seqs, like, "global_valid_seqs");
+    l.in.global_valid_toks = l.scalar(d.toks, like, "global_valid_toks");
+    return l;
+}
+
+nrl_grpo_cfg make_cfg(const std::vector<int64_t>& i, const std::vector<double>& f) {
+    TORCH_CHECK_VALUE(i.size() == 14 && f.size() == 9, "malformed loss configuration");
+    nrl_grpo_cfg c{};
+    int32_t* ci = &c.token_level_loss;  // the 14 switches, then the 9 numbers, in declaration order
+    float* cf = &c.ratio_clip_min;
+    for (size_t k = 0; k < i.size(); ++k) ci[k] = static_cast<int32_t>(i[k]);
+    for (size_t k = 0; k < f.size(); ++k) cf[k] = static_cast<float>(f[k]);
+    return c;
+}
+static_assert(offsetof(nrl_grpo_cfg, ratio_clip_min) == 14 * sizeof(int32_t) && sizeof(nrl_grpo_cfg) == 23 * 4, "field order of nrl_grpo_cfg");
+
+// ---------------------------------------------------------------------------------------------
+// the launches
+// ---------------------------------------------------------------------------------------------
+std::tuple<Tensor, Tensor> logprob_fwd(const Tensor& logits, const Tensor& targets, int64_t n_inner, int64_t v0, int64_t v1,
+                                       double temperature, int64_t mode, bool save_lse) {
+    need_gpu(logits, targets);
+    const nrl_rows rows = make_rows(logits, targets, n_inner, v0, v1, temperature, mode);
+    const c10::OptionalDeviceGuard guard(logits.device());
+    Tensor out = f32({logits.size(0), n_inner}, logits);
+    Tensor lse = save_lse ? f32({logits.size(0), n_inner}, logits) : f32({0}, logits);
+    Timed timed("logprob_fwd");
+    check(nrl_logprob_fwd(&rows, ptr(out), ptr(lse), stream_of(logits)), "nrl_logprob_fwd");
+    return {out, lse};
+}
+
+Tensor logprob_bwd(const Tensor& logits, const Tensor& targets, const Tensor& lse, const Tensor& grad, int64_t n_inner, int64_t v0,
+                   int64_t v1, double temperature, int64_t mode, bool in_place) {
+    need_gpu(logits, targets, lse, grad);
+    const nrl_rows rows = make_rows(logits, targets, n_inner, v0, v1, temperature, mode);
+    const int64_t b = logits.size(0), s = logits.size(1);
+    TORCH_CHECK_VALUE(lse.sizes() == at::IntArrayRef({b, n_inner}) && lse.is_contiguous() && lse.scalar_type() == at::kFloat,
+                      "lse must be a contiguous fp32 [B, n_inner] tensor");
+    TORCH_CHECK_VALUE(grad.sizes() == at::IntArrayRef({b, n_inner}) && grad.scalar_type() == at::kFloat, "grad must be fp32 [B, n_inner], got ",
+                      grad.scalar_type(), " ", grad.sizes());
+    const c10::OptionalDeviceGuard guard(logits.device());
+    Tensor d = in_place ? logits : grad_buffer(logits.sizes(), logits);
+    Timed timed("logprob_bwd");
+    check(nrl_logprob_bwd(&rows, ptr(lse), ptr(grad), grad.stride(0), grad.stride(1), ptr<void>(d), s, d.stride(0), d.stride(1),
+                          stream_of(logits)), "nrl_logprob_bwd");
+    return d;
+}
+
+Tensor scale_rows(const Tensor& x, const Tensor& factor, double divisor, bool in_place) {
+    need_gpu(x, factor);
+    TORCH_CHECK_VALUE(x.dim() == 3 && (x.stride(2) == 1 || x.size(2) <= 1), "expected [B, S, V] with a contiguous last axis, got ", x.sizes(),
+                      " strides ", x.strides());
+    TORCH_CHECK_VALUE(factor.numel() == 1, "factor must hold one element");
+    const Tensor f = to_f32(factor.detach(), x);
+    const c10::OptionalDeviceGuard guard(x.device());
+    Tensor out = in_place ? x : at::empty(x.sizes(), x.options());
+    Timed timed("scale_rows");
+    check(nrl_scale_rows(ptr<void>(x), ptr<void>(out), dtype_code(x), x.size(0), x.size(1), x.size(2), x.stride(0), x.stride(1), out.stride(0),
+                         out.stride(1), ptr(f), static_cast<float>(divisor), stream_of(x)), "nrl_scale_rows");
+    return out;
+}
+
+struct GrpoOut {
+    Tensor loss, dlp, dlpu, metrics;
+};
+GrpoOut grpo_loss(const Tensor& lp_in, const Tensor& lpu_in, const LossData& d, const nrl_grpo_cfg& cfg) {
+    need_gpu(lp_in, lpu_in);
+    TORCH_CHECK_VALUE(lp_in.dim() == 2, "logprobs must be [B, S-1], got ", lp_in.sizes());
+    const int64_t b = lp_in.size(0), n = lp_in.size(1);
+    const c10::OptionalDeviceGuard guard(lp_in.device());
+    LossInputs l = loss_inputs(d, lp_in, b, n);
+    l.rows(lp_in, lp_in, 0, "lp", &l.in.lp, &l.in.lp_stride);
+    l.rows(lpu_in, lp_in, 0, "lpu", &l.in.lpu, &l.in.lpu_stride);
+    const bool split = lpu_in.defined() && cfg.has_kl;
+    GrpoOut o{f32({}, lp_in), f32({b, n}, lp_in), split ? f32({b, n}, lp_in) : f32({0}, lp_in), f32({NRL_GRPO_N_METRICS}, lp_in)};
+    const int64_t bytes = nrl_grpo_loss_workspace_bytes(b);
+    const Tensor ws = workspace(bytes, lp_in);
+    Timed timed("grpo_loss");
+    check(nrl_grpo_loss_fwd_bwd(&cfg, &l.in, ptr(o.loss), ptr(o.dlp), split ? ptr(o.dlpu) : nullptr, ptr(o.metrics), ws.data_ptr(), bytes,
+                                stream_of(lp_in)), "nrl_grpo_loss_fwd_bwd");
+    return o;
+}
+
+struct FusedOut {
+    Tensor loss, dlogits, lp, metrics;
+};
+// cu not defined: logits [B, S, V], targets [B, >= n_inner]; otherwise packed logits [T, V] and targets [>= T]
+FusedOut fused_loss(const Tensor& logits, const Tensor& targets, int64_t n_inner, const Tensor& cu, bool pre_rolled, const LossData& d,
+                    const nrl_grpo_cfg& cfg, double loss_scale, double temperature, int64_t mode, bool in_place) {
+    need_gpu(logits, targets, cu);
+    const bool packed = cu.defined();
+    nrl_rows rows;
+    int64_t b;
+    if (packed) {
+        TORCH_CHECK_VALUE(logits.dim() == 2 && (logits.stride(1) == 1 || logits.size(1) <= 1), "packed logits must be [T, V] with a contiguous vocabulary axis");
+        TORCH_CHECK_VALUE(targets.scalar_type() == at::kLong && targets.dim() == 1 && targets.is_contiguous(), "packed targets must be a contiguous int64 [T] tensor");
+        TORCH_CHECK_VALUE(targets.size(0) >= logits.size(0), targets.size(0), " targets for ", logits.size(0), " packed positions");
+        TORCH_CHECK_VALUE(cu.scalar_type() == at::kInt && cu.dim() == 1 && cu.is_contiguous() && cu.size(0) >= 1, "cu_seqlens must be a contiguous int32 [n_seq+1] tensor");
+        TORCH_CHECK_VALUE(n_inner >= 0, "unpacked_seqlen must be at least 1");
+        const Tensor l3 = logits.unsqueeze(0), t2 = targets.unsqueeze(0);
+        rows = make_rows(l3, t2, logits.size(0), 0, logits.size(1), temperature, mode);
+        rows.stride_outer = 0;
+        rows.tgt_stride_outer = 0;
+        b = cu.size(0) - 1;
+    } else {
+        rows = make_rows(logits, targets, n_inner, 0, logits.size(2), temperature, mode);
+        b = logits.size(0);
+    }
+    const c10::OptionalDeviceGuard guard(logits.device());
+    const LossInputs l = loss_inputs(d, logits, b, n_inner);
+    FusedOut o{f32({}, logits), in_place ? logits : grad_buffer(logits.sizes(), logits), f32({b, n_inner}, logits), f32({NRL_GRPO_N_METRICS}, logits)};
+    const int64_t bytes = packed ? nrl_fused_packed_workspace_bytes(b, n_inner, logits.size(0)) : nrl_fused_workspace_bytes(b, n_inner);
+    const Tensor ws = workspace(bytes, logits);
+    const float scale = static_cast<float>(loss_scale);
+    Timed timed(packed ? "fused_packed_logits_loss" : "fused_logits_loss");
+    if (packed)
+        check(nrl_fused_packed_logits_grpo_loss(&rows, pre_rolled, ptr<int32_t>(cu), b, &cfg, &l.in, scale, ptr<void>(o.dlogits), o.dlogits.stride(0),
+                                                ptr(o.lp), ptr(o.loss), ptr(o.metrics), ws.data_ptr(), ws.numel() * 8, stream_of(logits)),
+              "nrl_fused_packed_logits_grpo_loss");
+    else
+        check(nrl_fused_logits_grpo_loss(&rows, &cfg, &l.in, scale, ptr<void>(o.dlogits), logits.size(1), o.dlogits.stride(0), o.dlogits.stride(1),
+                                         ptr(o.lp), ptr(o.loss), ptr(o.metrics), ws.data_ptr(), ws.numel() * 8, stream_of(logits)),
+              "nrl_fused_logits_grpo_loss");
+    return o;
+}
+
+struct Kept {  // what a filtered forward leaves for its backward, with the record of the kept sets if there is one
+    Tensor lp, thr, tie, lse, lpu, n, idx, x;
+};
+Kept topk_topp_fwd(const Tensor& logits, const Tensor& targets, int64_t n_inner, int64_t top_k, double top_p, double temperature, int64_t mode,
+                   bool want_unfiltered, int64_t capacity) {
+    need_gpu(logits, targets);
+    const nrl_rows rows = make_rows(logits, targets, n_inner, 0, logits.size(2), temperature, mode);
+    const int64_t b = logits.size(0);
+    const c10::OptionalDeviceGuard guard(logits.device());
+    const auto i32 = logits.options().dtype(at::kInt);
+    Kept k;
+    k.lp = targets.defined() ? f32({b, n_inner}, logits) : f32({0}, logits);
+    k.thr = f32({b, n_inner}, logits);
+    k.tie = at::empty({b, n_inner}, i32);
+    k.lse = f32({b, n_inner}, logits);
+    k.lpu = want_unfiltered ? f32({b, n_inner}, logits) : f32({0}, logits);
+    if (capacity > 0) {
+        k.n = at::empty({b, n_inner}, i32);
+        k.idx = at::empty({b, n_inner, capacity}, i32);
+        k.x = f32({b, n_inner, capacity}, logits);
+    }
+    Timed timed("topk_topp_fwd");
+    check(nrl_topk_topp_logprob_fwd(&rows, top_k, static_cast<float>(top_p), ptr(k.lp), ptr(k.thr), ptr<int32_t>(k.tie), ptr(k.lse), ptr(k.lpu), nullptr,
+                                    ptr<int32_t>(k.n), ptr<int32_t>(k.idx), ptr(k.x), capacity, stream_of(logits)), "nrl_topk_topp_logprob_fwd");
+    return k;
+}
+
+Tensor topk_topp_bwd(const Tensor& logits, const Tensor& targets, const Kept& k, const Tensor& grad, int64_t n_inner, double temperature, int64_t mode) {
+    need_gpu(logits, targets, k.thr, k.tie, k.lse, grad, k.n, k.idx, k.x);
+    const nrl_rows rows = make_rows(logits, targets, n_inner, 0, logits.size(2), temperature, mode);
+    const int64_t b = logits.size(0);
+    for (const Tensor* t : {&k.thr, &k.tie, &k.lse})
+        TORCH_CHECK_VALUE(t->sizes() == at::IntArrayRef({b, n_inner}) && t->is_contiguous(), "thr, tie and lse_kept must be contiguous [B, n_inner] tensors");
+    TORCH_CHECK_VALUE(k.thr.scalar_type() == at::kFloat && k.lse.scalar_type() == at::kFloat && k.tie.scalar_type() == at::kInt,
+                      "thr / lse_kept must be fp32 and tie int32");
+    TORCH_CHECK_VALUE(grad.sizes() == at::IntArrayRef({b, n_inner}) && grad.scalar_type() == at::kFloat, "grad must be fp32 [B, n_inner]");
+    int64_t capacity = 0;
+    if (k.n.defined()) {
+        TORCH_CHECK_VALUE(k.idx.defined() && k.x.defined(), "the kept-set record is (count, indices, values): all three or none");
+        capacity = k.idx.size(-1);
+        TORCH_CHECK_VALUE(k.n.scalar_type() == at::kInt && k.idx.scalar_type() == at::kInt && k.x.scalar_type() == at::kFloat &&
+                              k.n.sizes() == at::IntArrayRef({b, n_inner}) && k.idx.sizes() == at::IntArrayRef({b, n_inner, capacity}) &&
+                              k.x.sizes() == k.idx.sizes() && k.n.is_contiguous() && k.idx.is_contiguous() && k.x.is_contiguous() && capacity >= 1,
+                          "kept-set record: int32 [B, n], int32 [B, n, capacity], fp32 [B, n, capacity], contiguous");
+    }
+    const c10::OptionalDeviceGuard guard(logits.device());
+    Tensor d = grad_buffer(logits.sizes(), logits);
+    Timed timed("topk_topp_bwd");
+    check(nrl_topk_topp_logprob_bwd(&rows, ptr(k.thr), ptr<int32_t>(k.tie), ptr(k.lse), ptr(grad), grad.stride(0), grad.stride(1), ptr<int32_t>(k.n),
+                                    ptr<int32_t>(k.idx), ptr(k.x), capacity, ptr<void>(d), logits.size(1), d.stride(0), d.stride(1), stream_of(logits)),
+          "nrl_topk_topp_logprob_bwd");
+    return d;
+}
+
+Tensor gather_indices(const Tensor& logits, const Tensor& indices) {
+    TORCH_CHECK_VALUE(indices.scalar_type() == at::kLong && indices.dim() == 3 && indices.size(0) == logits.size(0) && indices.size(1) == logits.size(1),
+                      "indices must be int64 [", logits.size(0), ", ", logits.size(1), ", K], got ", indices.scalar_type(), " ", indices.sizes());
+    return indices.contiguous();
+}
+
+// The first n_inner rows of every sequence: log p at indices [B, S, K] -> [B, n_inner, K], sum_v p log p (empty without
+// `entropy`) and the log-sum-exps, from one pass over the logits.
+std::tuple<Tensor, Tensor, Tensor> gather_entropy_fwd(const Tensor& logits, const Tensor& indices, int64_t n_inner, bool entropy) {
+    need_gpu(logits, indices);
+    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, logits.size(2), 1.0, NRL_TEMP_RCP);
+    const Tensor idx = gather_indices(logits, indices);
+    const int64_t b = logits.size(0), s = logits.size(1), k = idx.size(2);
+    const c10::OptionalDeviceGuard guard(logits.device());
+    Tensor out = f32({b, n_inner, k}, logits), h = entropy ? f32({b, n_inner}, logits) : f32({0}, logits), lse = f32({b, n_inner}, logits);
+    Timed timed("gather_entropy_fwd");
+    check(nrl_gather_entropy_fwd(&rows, ptr<int64_t>(idx), k, s * k, ptr(out), ptr(h), ptr(lse), stream_of(logits)), "nrl_gather_entropy_fwd");
+    return {out, h, lse};
+}
+
+// gradient of both outputs of gather_entropy_fwd (of the gathered values alone without h) in one pass
+Tensor gather_entropy_bwd(const Tensor& logits, const Tensor& indices, int64_t n_inner, const Tensor& lse, const OptTensor& h_in,
+                          const OptTensor& grad_h_in, const Tensor& grad_in) {
+    Tensor h = opt(h_in), grad_h = opt(grad_h_in);
+    need_gpu(logits, indices, lse, h, grad_h, grad_in);
+    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, logits.size(2), 1.0, NRL_TEMP_RCP);
+    const Tensor idx = gather_indices(logits, indices);
+    const int64_t b = logits.size(0), s = logits.size(1), k = idx.size(2);
+    auto scalar = [&](const Tensor& t, const char* name) {
+        TORCH_CHECK_VALUE(t.scalar_type() == at::kFloat && t.sizes() == at::IntArrayRef({b, n_inner}), name, " must be fp32 [", b, ", ", n_inner, "], got ", t.sizes());
+        return t.contiguous();
+    };
+    const Tensor l = scalar(lse, "lse");
+    if (h.defined()) {
+        TORCH_CHECK_VALUE(grad_h.defined(), "an entropy without its upstream gradient");
+        h = scalar(h, "h");
+        grad_h = scalar(grad_h, "grad_h");
+    }
+    TORCH_CHECK_VALUE(grad_in.scalar_type() == at::kFloat && grad_in.sizes() == at::IntArrayRef({b, n_inner, k}), "grad must be fp32 [", b, ", ", n_inner, ", ", k,
+                      "], got ", grad_in.scalar_type(), " ", grad_in.sizes());
+    const Tensor grad = grad_in.contiguous();
+    const c10::OptionalDeviceGuard guard(logits.device());
+    Tensor d = grad_buffer(logits.sizes(), logits);
+    Timed timed("gather_entropy_bwd");
+    check(nrl_gather_entropy_bwd(&rows, ptr<int64_t>(idx), k, s * k, ptr(l), ptr(h), ptr(grad_h), ptr(grad), ptr<void>(d), s, d.stride(0), d.stride(1),
+                                 stream_of(logits)), "nrl_gather_entropy_bwd");
+    return d;
+}
+
+// -> (baseline [B], std [B], advantages [B], group index of every row [B])
+std::tuple<Tensor, Tensor, Tensor, Tensor> group_baseline_std(const Tensor& prompts_in, const Tensor& rewards_in, const Tensor& valid_in,
+                                                              const OptTensor& std_rewards_in, bool leave_one_out, bool normalize) {
+    Tensor prompts = prompts_in, std_rewards = opt(std_rewards_in);
+    need_gpu(prompts, rewards_in, valid_in, std_rewards);
+    if (prompts.dim() == 1) prompts = prompts.unsqueeze(-1);
+    TORCH_CHECK_VALUE(prompts.dim() == 2 && prompts.scalar_type() == at::kLong, "prompts must be int64 [B, Sp], got ", prompts.scalar_type(), " ", prompts.sizes());
+    const int64_t b = prompts.size(0), sp = prompts.size(1);
+    if (sp > 1 && prompts.stride(1) != 1) prompts = prompts.contiguous();
+    auto vec = [&](const Tensor& t, const char* name) {
+        if (!t.defined()) return t;
+        TORCH_CHECK_VALUE(t.scalar_type() == at::kFloat && t.dim() == 1 && t.size(0) == b, name, " must be fp32 [", b, "], got ", t.scalar_type(), " ", t.sizes());
+        return t.contiguous();
+    };
+    const Tensor rewards = vec(rewards_in, "rewards"), valid = vec(valid_in, "valid_mask");
+    std_rewards = vec(std_rewards, "std_rewards");
+    const c10::OptionalDeviceGuard guard(rewards.device());
+    Tensor baseline = f32({b}, rewards), std = f32({b}, rewards), adv = f32({b}, rewards), group = at::empty({b}, rewards.options().dtype(at::kInt));
+    const Tensor ws = workspace(nrl_group_workspace_bytes(b), rewards);
+    check(nrl_group_baseline_std(ptr<int64_t>(prompts), b, sp, b > 1 ? prompts.stride(0) : sp, ptr(rewards), ptr(valid), ptr(std_rewards), leave_one_out,
+                                 normalize, ptr(baseline), ptr(std), ptr(adv), ptr<int32_t>(group), ws.data_ptr(), ws.numel() * 8, stream_of(rewards)),
+          "nrl_group_baseline_std");
+    return {baseline, std, adv, group};
+}
+
+// ---------------------------------------------------------------------------------------------
+// autograd nodes
+// ---------------------------------------------------------------------------------------------
+// logits [B, S, V], targets [B, >= n_inner] (already aligned to the rows) -> fp32 [B, n_inner].  Saved for the backward:
+// the logits (no copy), the targets and one fp32 log-sum-exp per row; the softmax is never materialised.
+struct RowsLogprob : torch::autograd::Function<RowsLogprob> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& targets, int64_t n_inner, int64_t v0, int64_t v1, bool inference_only,
+                          double temperature, int64_t mode) {
+        Tensor logits = logits_in.detach();
+        if (logits.dim() == 3 && logits.stride(2) != 1) logits = logits.contiguous();
+        const bool save = !inference_only && logits_in.requires_grad();
+        auto [out, lse] = logprob_fwd(logits, targets, n_inner, v0, v1, temperature, mode, save);
+        if (save) ctx->save_for_backward({logits, targets, lse});
+        ctx->saved_data["args"] = std::vector<int64_t>{n_inner, v0, v1, mode, save};
+        ctx->saved_data["temperature"] = temperature;
+        return out;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const std::vector<int64_t> a = ctx->saved_data["args"].toIntVector();
+        TORCH_CHECK(a[4], "backward through a logprob computed with inference_only=True");
+        const auto saved = ctx->get_saved_variables();
+        Tensor d = logprob_bwd(saved[0], saved[1], saved[2], to_f32(grads[0], saved[0]), a[0], a[1], a[2], ctx->saved_data["temperature"].toDouble(), a[3], false);
+        variable_list out(8);
+        out[0] = d;
+        return out;
+    }
+};
+
+// loss and metrics of given logprobs; the kernel also returns d loss / d lp (and / d lpu), so the backward is a scalar multiply
+struct ClippedPg : torch::autograd::Function<ClippedPg> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& lp, const OptTensor& lpu, const LossData& d, const nrl_grpo_cfg& cfg) {
+        ctx->set_materialize_grads(false);
+        GrpoOut o = grpo_loss(lp.detach(), lpu.has_value() ? lpu->detach() : Tensor(), d, cfg);
+        ctx->save_for_backward({o.dlp, o.dlpu});
+        ctx->mark_non_differentiable({o.metrics});
+        return {o.loss, o.metrics};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        variable_list out(4);
+        if (!grads[0].defined()) return out;
+        const auto saved = ctx->get_saved_variables();
+        if (ctx->needs_input_grad(0)) out[0] = saved[0] * grads[0];
+        if (saved[1].numel() > 0 && ctx->needs_input_grad(1)) out[1] = saved[1] * grads[0];
+        return out;
+    }
+};
+
+// The single pass: the gradient of the logits exists as soon as the forward returns, computed for an upstream factor of
+// loss_scale.  Whatever factor autograd delivers is applied in place by one kernel that reads it from the device: the
+// host never waits for its value, no second [B, S, V] tensor exists, and when the two agree (the normal case) the kernel
+// touches no memory.
+struct FusedArgs {
+    Tensor targets, cu;
+    int64_t n_inner;
+    LossData data;
+    nrl_grpo_cfg cfg;
+    double loss_scale, temperature;
+    int64_t mode;
+    bool in_place;
+};
+struct FusedLoss : torch::autograd::Function<FusedLoss> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits, const FusedArgs& a) {
+        ctx->set_materialize_grads(false);
+        FusedOut o = fused_loss(logits.detach(), a.targets, a.n_inner, a.cu, true, a.data, a.cfg, a.loss_scale, a.temperature, a.mode, a.in_place);
+        // (an intermediate, neither input nor output: held directly so that it can be rescaled in place)
+        ctx->saved_data["dlogits"] = o.dlogits;
+        ctx->saved_data["loss_scale"] = a.loss_scale;
+        ctx->mark_non_differentiable({o.metrics});
+        return {o.loss, o.metrics};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        variable_list out(2);
+        if (!grads[0].defined()) return out;
+        const auto it = ctx->saved_data.find("dlogits");
+        TORCH_CHECK(it != ctx->saved_data.end(), "the single-pass loss hands its gradient buffer to autograd once; a second backward "
+                    "through the same loss needs a new forward");
+        Tensor d = it->second.toTensor();
+        ctx->saved_data.erase(it);
+        scale_rows(d.dim() == 3 ? d : d.unsqueeze(0), grads[0].is_cuda() ? grads[0] : grads[0].to(d.device()), ctx->saved_data["loss_scale"].toDouble(), true);
+        out[0] = d;
+        return out;
+    }
+};
+
+// filtered logprobs (and, when asked for, the unfiltered ones the KL term needs, without a gradient)
+struct RowsLogprobSampled : torch::autograd::Function<RowsLogprobSampled> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& targets, int64_t n_inner, int64_t top_k, double top_p, bool inference_only,
+                          double temperature, int64_t mode, int64_t capacity) {
+        Tensor logits = logits_in.detach();
+        if (logits.dim() == 3 && logits.stride(2) != 1) logits = logits.contiguous();
+        const bool save = !inference_only && logits_in.requires_grad();
+        Kept k = topk_topp_fwd(logits, targets, n_inner, top_k, top_p, temperature, mode, false, save ? capacity : 0);
+        if (save) ctx->save_for_backward({logits, targets, k.thr, k.tie, k.lse, k.n, k.idx, k.x});
+        ctx->saved_data["args"] = std::vector<int64_t>{n_inner, mode, save};
+        ctx->saved_data["temperature"] = temperature;
+        return k.lp;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const std::vector<int64_t> a = ctx->saved_data["args"].toIntVector();
+        TORCH_CHECK(a[2], "backward through a logprob computed with inference_only=True");
+        const auto s = ctx->get_saved_variables();
+        Kept k;
+        k.thr = s[2]; k.tie = s[3]; k.lse = s[4]; k.n = s[5]; k.idx = s[6]; k.x = s[7];
+        variable_list out(9);
+        out[0] = topk_topp_bwd(s[0], s[1], k, to_f32(grads[0], s[0]), a[0], ctx->saved_data["temperature"].toDouble(), a[1]);
+        return out;
+    }
+};
+
+// log p at indices [B, S, K] and (optionally) sum_v p log p of the first n rows of every sequence
+struct GatherEntropy : torch::autograd::Function<GatherEntropy> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& indices, int64_t n, bool entropy) {
+        Tensor x = logits_in.detach();
+        if (x.dim() == 3 && x.stride(2) != 1) x = x.contiguous();
+        auto [out, h, lse] = gather_entropy_fwd(x, indices, n, entropy);
+        ctx->save_for_backward({x, indices, lse, h});
+        ctx->saved_data["n"] = n;
+        ctx->saved_data["entropy"] = entropy;
+        if (!entropy) ctx->mark_non_differentiable({h});
+        return {out, h};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const bool entropy = ctx->saved_data["entropy"].toBool();
+        variable_list out(4);
+        out[0] = gather_entropy_bwd(s[0], s[1], ctx->saved_data["n"].toInt(), s[2], entropy ? OptTensor(s[3]) : OptTensor(),
+                                    entropy ? OptTensor(to_f32(grads[1], s[0])) : OptTensor(), to_f32(grads[0], s[0]));
+        return out;
+    }
+};
+
+// ---------------------------------------------------------------------------------------------
+// a small device record on its way to the host
+// ---------------------------------------------------------------------------------------------
+class Fetch {
+  public:
+    explicit Fetch(const Tensor& record) : host_(at::empty(record.sizes(), record.options().device(at::kCPU).pinned_memory(true))) {
+        const c10::OptionalDeviceGuard guard(record.device());
+        host_.copy_(record, /*non_blocking=*/true);
+        TORCH_CHECK(hipEventCreateWithFlags(&done_, hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
+        if (hipEventRecord(done_, static_cast<hipStream_t>(stream_of(record))) != hipSuccess) {
+            (void)hipEventDestroy(done_);
+            TORCH_CHECK(false, "hipEventRecord failed");
+        }
+    }
+    Fetch(const Fetch&) = delete;
+    Fetch& operator=(const Fetch&) = delete;
+    ~Fetch() { (void)hipEventDestroy(done_); }
+    bool ready() const { return hipEventQuery(done_) == hipSuccess; }
+    // waits for this copy alone, not for work enqueued afterwards
+    std::vector<double> values() const {
+        {
+            py::gil_scoped_release release;
+            TORCH_CHECK(hipEventSynchronize(done_) == hipSuccess, "waiting for a metrics record failed");
+        }
+        const Tensor d = host_.to(at::kDouble).reshape(-1);
+        return std::vector<double>(d.data_ptr<double>(), d.data_ptr<double>() + d.numel());
+    }
+
+  private:
+    Tensor host_;
+    hipEvent_t done_ = nullptr;
+};
+
+// ---------------------------------------------------------------------------------------------
+// entry points
+// ---------------------------------------------------------------------------------------------
+LossData loss_data(const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
+                   const OptTensor& correct, const Tensor& seqs, const Tensor& toks, int64_t shift) {
+    LossData d;
+    d.prev = opt(prev); d.gen = gen; d.ref = opt(ref); d.adv = adv; d.token_mask = token_mask; d.sample_mask = sample_mask; d.correct = opt(correct);
+    d.seqs = seqs; d.toks = toks; d.shift = shift;
+    return d;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    m.doc() = "host path of the rl_amd training calls";
+    m.def("set_kernel_timer", [](py::object t) {
+        delete g_timer;
+        g_timer = t.is_none() ? nullptr : new py::object(t);
+    });
+    py::class_<Fetch, std::shared_ptr<Fetch>>(m, "Fetch").def(py::init<const Tensor&>()).def("ready", &Fetch::ready).def("__call__", &Fetch::values);
+
+    m.def("grad_buffer", [](const std::vector<int64_t>& shape, const Tensor& like) { return grad_buffer(shape, like); });
+    m.def("logprob_fwd", &logprob_fwd);
+    m.def("logprob_bwd", &logprob_bwd);
+    m.def("scale_rows", &scale_rows);
+    m.def("gather_entropy_fwd", &gather_entropy_fwd);
+    m.def("gather_entropy_bwd", &gather_entropy_bwd);
+    m.def("group_baseline_std", &group_baseline_std);
+    m.def("grpo_loss", [](const Tensor& lp, const OptTensor& lpu, const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv,
+                          const Tensor& token_mask, const Tensor& sample_mask, const OptTensor& correct, const Tensor& global_valid,
+                          const std::vector<int64_t>& iflags, const std::vector<double>& fparams) {
+        TORCH_CHECK_VALUE(global_valid.scalar_type() == at::kFloat && global_valid.dim() == 1 && global_valid.size(0) == 2,
+                          "global_valid must be fp32 [2] = (valid_seqs, valid_toks)");
+        const GrpoOut o = grpo_loss(lp, opt(lpu), loss_data(prev, gen, ref, adv, token_mask, sample_mask, correct, global_valid[0], global_valid[1], 0),
+                                    make_cfg(iflags, fparams));
+        return std::make_tuple(o.loss, o.dlp, o.dlpu, o.metrics);
+    });
+    m.def("fused_loss", [](const Tensor& logits, const Tensor& targets, int64_t n_inner, const OptTensor& cu, bool pre_rolled, const OptTensor& prev,
+                           const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
+                           const Tensor& global_valid, const std::vector<int64_t>& iflags, const std::vector<double>& fparams, double loss_scale,
+                           double temperature, int64_t mode, bool in_place) {
+        TORCH_CHECK_VALUE(global_valid.scalar_type() == at::kFloat && global_valid.dim() == 1 && global_valid.size(0) == 2,
+                          "global_valid must be fp32 [2] = (valid_seqs, valid_toks)");
+        const FusedOut o = fused_loss(logits, targets, n_inner, opt(cu), pre_rolled,
+                                      loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, global_valid[0], global_valid[1], 0),
+                                      make_cfg(iflags, fparams), loss_scale, temperature, mode, in_place);
+        return std::make_tuple(o.loss, o.dlogits, o.lp, o.metrics);
+    });
+    m.def("topk_topp_fwd", [](const Tensor& logits, const OptTensor& targets, int64_t n_inner, int64_t top_k, double top_p, double temperature, int64_t mode,
+                              bool want_unfiltered, int64_t capacity) {
+        Kept k = topk_topp_fwd(logits, opt(targets), n_inner, top_k, top_p, temperature, mode, want_unfiltered, capacity);
+        std::vector<Tensor> out{k.lp, k.thr, k.tie, k.lse, k.lpu};
+        if (capacity > 0) out.insert(out.end(), {k.n, k.idx, k.x});
+        return out;
+    });
+    m.def("topk_topp_bwd", [](const Tensor& logits, const Tensor& targets, const Tensor& thr, const Tensor& tie, const Tensor& lse, const Tensor& grad,
+                              int64_t n_inner, double temperature, int64_t mode, const OptTensor& kept_n, const OptTensor& kept_idx, const OptTensor& kept_x) {
+        Kept k;
+        k.thr = thr; k.tie = tie; k.lse = lse; k.n = opt(kept_n); k.idx = opt(kept_idx); k.x = opt(kept_x);
+        return topk_topp_bwd(logits, targets, k, grad, n_inner, temperature, mode);
+    });
+
+    // differentiable calls
+    m.def("rows_logprob", [](const Tensor& logits, const Tensor& targets, int64_t shift, int64_t n_inner, int64_t v0, int64_t v1, bool inference_only,
+                             double temperature, int64_t mode) {
+        Tensor t = targets.device() == logits.device() && targets.scalar_type() == at::kLong ? targets : targets.to(logits.device(), at::kLong);
+        if (shift) t = t.narrow(1, shift, t.size(1) - shift);
+        return RowsLogprob::apply(logits, t, n_inner, v0, v1, inference_only, temperature, mode);
+    });
+    m.def("rows_logprob_sampled", [](const Tensor& logits, const Tensor& targets, int64_t shift, int64_t n_inner, int64_t top_k, double top_p,
+                                     bool inference_only, double temperature, int64_t mode, int64_t capacity) {
+        Tensor t = targets.device() == logits.device() && targets.scalar_type() == at::kLong ? targets : targets.to(logits.device(), at::kLong);
+        if (shift) t = t.narrow(1, shift, t.size(1) - shift);
+        return RowsLogprobSampled::apply(logits, t, n_inner, top_k, top_p, inference_only, temperature, mode, capacity);
+    });
+    m.def("clipped_pg", [](const Tensor& lp, const OptTensor& lpu, const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv,
+                           const Tensor& token_mask, const Tensor& sample_mask, const OptTensor& correct, const Tensor& seqs, const Tensor& toks,
+                           const std::vector<int64_t>& iflags, const std::vector<double>& fparams) {
+        const variable_list o = ClippedPg::apply(lp, lpu, loss_data(prev, gen, ref, adv, token_mask, sample_mask, correct, seqs, toks, 1), make_cfg(iflags, fparams));
+        return std::make_tuple(o[0], o[1]);
+    });
+    m.def("fused_clipped_pg", [](const Tensor& logits, const Tensor& targets, int64_t shift, int64_t n_inner, const OptTensor& cu, const OptTensor& prev,
+                                 const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
+                                 const Tensor& seqs, const Tensor& toks, const std::vector<int64_t>& iflags, const std::vector<double>& fparams,
+                                 double loss_scale, double temperature, int64_t mode, bool in_place) {
+        Tensor t = targets.device() == logits.device() && targets.scalar_type() == at::kLong ? targets : targets.to(logits.device(), at::kLong);
+        if (shift) t = t.narrow(1, shift, t.size(1) - shift);
+        const FusedArgs a{t, opt(cu), n_inner, loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, seqs, toks, 1), make_cfg(iflags, fparams),
+                          loss_scale, temperature, mode, in_place};
+        const variable_list o = FusedLoss::apply(logits, a);
+        return std::make_tuple(o[0], o[1]);
+    });
+    m.def("gather_entropy", [](const Tensor& logits, const Tensor& indices, int64_t n, bool entropy) {
+        const variable_list o = GatherEntropy::apply(logits, indices, n, entropy);
+        return std::make_tuple(o[0], o[1]);
+    });
+}

@@ -18,6 +18,7 @@ import torch
 from .. import ops as _ops  # noqa: F401  (registers torch.ops.rl_amd.*)
 from .._deferred import pending_temperature, refuse_pending
 from .._lib import NRL_TEMP_RCP
+from .._lib import host as _host
 from ..algorithms.logits_sampling_utils import (
     TrainingSamplingParams,
     need_top_k_or_top_p_filtering,
@@ -80,20 +81,10 @@ def _bwd_rows(ctx, grad_out):
     return _OPS.logprob_bwd(logits, targets, lse, grad, n_inner, vocab_start, vocab_end, temperature, NRL_TEMP_RCP)
 
 
-class _RowsLogprob(torch.autograd.Function):
-    """logits [B,S,V], targets [B,>=n_inner] (already aligned to the rows) -> fp32 [B,n_inner]."""
-
-    @staticmethod
-    def forward(ctx, logits, targets, n_inner, vocab_start, vocab_end, inference_only, temperature):
-        return _fwd_rows(ctx, logits, targets, n_inner, vocab_start, vocab_end, inference_only, temperature)
-
-    @staticmethod
-    def backward(ctx, grad_out):
-        return _bwd_rows(ctx, grad_out), None, None, None, None, None, None
-
-
-def _rows_logprob(logits, targets, n_inner, vocab_start, vocab_end, inference_only, temperature=1.0):
-    return _RowsLogprob.apply(logits, targets, n_inner, vocab_start, vocab_end, inference_only, float(temperature))
+def _rows_logprob(logits, target, n_inner, vocab_start, vocab_end, inference_only):
+    """logits [B,S,V], unshifted target [B, n_inner + 1] (row ``(b, i)`` reads ``target[b, i + 1]``) -> fp32 [B,n_inner]."""
+    temperature = pending_temperature(logits)  # a divide apply_temperature_scaling left to this kernel
+    return _host().rows_logprob(logits, target, 1, n_inner, vocab_start, vocab_end, inference_only, temperature, NRL_TEMP_RCP)
 
 
 class _LogSoftmaxRows(torch.autograd.Function):
@@ -237,11 +228,9 @@ def from_parallel_logits_to_logprobs(
         from .sampling_logprob import rows_logprob_sampled
 
         return rows_logprob_sampled(
-            vocab_parallel_logits, target[:, 1:], s - 1, sampling_params.top_k, sampling_params.top_p, inference_only
+            vocab_parallel_logits, target, s - 1, sampling_params.top_k, sampling_params.top_p, inference_only, shift=1
         )
-    return _rows_logprob(
-        vocab_parallel_logits, target[:, 1:], s - 1, vocab_start_index, vocab_end_index, inference_only
-    )
+    return _rows_logprob(vocab_parallel_logits, target, s - 1, vocab_start_index, vocab_end_index, inference_only)
 
 
 def get_next_token_logprobs_from_logits(
@@ -271,7 +260,7 @@ def get_next_token_logprobs_from_logits(
     vocab = next_token_logits.shape[-1]
     rank = vocab_parallel_rank or 0
     inference_only = not (torch.is_grad_enabled() and next_token_logits.requires_grad)
-    return from_parallel_logits_to_logprobs(
+    logprobs = from_parallel_logits_to_logprobs(
         next_token_logits,
         input_ids,
         vocab_start_index=rank * vocab,
@@ -281,7 +270,9 @@ def get_next_token_logprobs_from_logits(
         cp_group=context_parallel_group,
         chunk_size=None,
         sampling_params=sampling_params,
-    )[:, : input_ids.shape[1] - 1]
+    )
+    n = input_ids.shape[1] - 1
+    return logprobs if logprobs.shape[1] == n else logprobs[:, :n]
 
 
 def _mesh_dim_size(mesh, name: str) -> int:
@@ -604,28 +595,6 @@ class DistributedCrossEntropy(torch.autograd.Function):
         return d.reshape(ctx.in_shape), None, None, None
 
 
-class _GatherEntropy(torch.autograd.Function):
-    """``log p`` at ``indices [B, S, K]`` and (optionally) ``sum_v p log p`` of the first ``n`` rows of every sequence:
-    one pass over the logits forward and one backward, where ``ChunkedDistributedGatherLogprob`` and
-    ``ChunkedDistributedEntropy`` each make their own and autograd then adds their ``[B, S, V]`` gradients."""
-
-    @staticmethod
-    def forward(ctx, logits, indices, n, entropy):
-        x = logits.detach()
-        x = x if x.stride(-1) == 1 else x.contiguous()
-        out, h, lse = torch.ops.rl_amd.gather_entropy_fwd(x, indices, n, entropy)
-        ctx.save_for_backward(x, indices, lse, h)
-        ctx.n, ctx.entropy = n, entropy
-        return (out, h) if entropy else out
-
-    @staticmethod
-    def backward(ctx, grad, grad_h=None):
-        x, indices, lse, h = ctx.saved_tensors
-        d = torch.ops.rl_amd.gather_entropy_bwd(x, indices, ctx.n, lse, h if ctx.entropy else None,
-                                                grad_h.float() if ctx.entropy else None, grad.float())
-        return d, None, None, None
-
-
 class _TopkLogSoftmax(torch.autograd.Function):
     """log_softmax over the K logits of every row at the given vocabulary indices."""
 
@@ -682,10 +651,13 @@ def get_distillation_topk_logprobs_from_logits(
     H_all = None
     rows = max(seq - 1, 0)  # the last position predicts nothing
     if zero_outside_topk:
-        if calculate_entropy:
-            student_topk_logprobs, H_all = _GatherEntropy.apply(student_logits, indices, rows, True)
-        else:
-            student_topk_logprobs = _GatherEntropy.apply(student_logits, indices, rows, False)
+        # log p at the teacher's ids and sum_v p log p from one pass over the logits each way, where
+        # ChunkedDistributedGatherLogprob and ChunkedDistributedEntropy each make their own and autograd then adds their
+        # [B, S, V] gradients
+        refuse_pending(student_logits, "get_distillation_topk_logprobs_from_logits")
+        student_topk_logprobs, H_all = _host().gather_entropy(student_logits, indices, rows, bool(calculate_entropy))
+        if not calculate_entropy:
+            H_all = None
     else:
         student_topk_logprobs = _TopkLogSoftmax.apply(student_logits, indices)[:, :-1, :]
     teacher = teacher_topk_logits.to(student_topk_logprobs.device)

@@ -10,6 +10,7 @@ import torch
 from .. import ops as _ops  # noqa: F401
 from .._deferred import pending_temperature, refuse_pending
 from .._lib import NRL_TEMP_RCP
+from .._lib import host as _host
 
 _OPS = torch.ops.rl_amd
 
@@ -73,20 +74,14 @@ def _sampled_bwd(ctx, grad_lp):
     )
 
 
-class _RowsLogprobSampled(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, logits, targets, n_inner, top_k, top_p, inference_only, temperature):
-        return _sampled_fwd(ctx, logits, targets, n_inner, top_k, top_p, inference_only, temperature=temperature)
-
-    @staticmethod
-    def backward(ctx, grad_lp):
-        return _sampled_bwd(ctx, grad_lp), None, None, None, None, None, None
-
-
-def rows_logprob_sampled(logits, targets, n_inner, top_k, top_p, inference_only=False, temperature=1.0):
-    """logits [B,S,V], targets [B,>=n_inner] aligned with the rows -> fp32 [B,n_inner]; a target outside
-    the kept set gives ``-inf`` (``model_utils.py:445-452``)."""
-    return _RowsLogprobSampled.apply(logits, targets, n_inner, top_k, top_p, inference_only, float(temperature))
+def rows_logprob_sampled(logits, targets, n_inner, top_k, top_p, inference_only=False, temperature=1.0, shift=0):
+    """logits [B,S,V], targets [B,>=n_inner + shift] whose column ``shift`` belongs to row 0 -> fp32 [B,n_inner]; a target
+    outside the kept set gives ``-inf`` (``model_utils.py:445-452``)."""
+    if temperature == 1.0:
+        temperature = pending_temperature(logits)  # a divide apply_temperature_scaling left to this kernel
+    k = _norm_k(top_k)
+    return _host().rows_logprob_sampled(logits, targets, shift, n_inner, k, _norm_p(top_p), inference_only, float(temperature), NRL_TEMP_RCP,
+                                        _record_capacity(k))
 
 
 def packed_logprob_sampled(logits2d, targets1d, pre_rolled, cu_dev, unpacked_seqlen, top_k, top_p, inference_only,

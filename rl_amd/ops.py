@@ -3,17 +3,18 @@
 PyTorch supplies device memory and the current stream; every computation is a kernel in
 ``librl_amd_hip.so``.  Each op validates shapes on the host before a launch and raises on
 anything the kernels do not assume (CPU tensors, non-contiguous vocabulary axis, wrong dtype).
+The ops of a training step do that in C++ (``csrc/host_path.cpp``, ``_host()`` below), the others here.
 """
 
 from __future__ import annotations
 
 import ctypes as C
-import os
 
 import torch
 
 from . import _lib
 from ._deferred import refuse_pending
+from ._lib import host as _host
 
 _DTYPES = {torch.float32: _lib.NRL_F32, torch.bfloat16: _lib.NRL_BF16, torch.float16: _lib.NRL_F16}
 
@@ -22,6 +23,13 @@ _LIB = torch.library.Library("rl_amd", "DEF")
 # Optional per-launch timing: an object with ``start(name)`` / ``stop(name)`` that records events on
 # the current stream around a kernel launch (used by the benchmark harness); None in normal use.
 KERNEL_TIMER = None
+
+
+def set_kernel_timer(timer) -> None:
+    """Installs (or with ``None`` removes) the per-launch timer, here and in the C++ host path."""
+    global KERNEL_TIMER
+    KERNEL_TIMER = timer
+    _host().set_kernel_timer(timer)
 
 
 class _timed:
@@ -52,30 +60,10 @@ def _need_gpu(*tensors) -> None:
             raise RuntimeError("rl_amd ops run on the GPU only (got a CPU tensor); there is no CPU fallback")
 
 
-_PHASE = 1 << 21          # large device allocations start on 2 MiB boundaries
-# where in that period the gradient buffer starts, relative to the logits (NRL_GRAD_PHASE overrides, for tuning)
-_GRAD_PHASE = int(os.environ.get("NRL_GRAD_PHASE", "0x1B0000"), 0) % _PHASE
-_PHASED_MIN_BYTES = 64 << 20
-
-
 def _grad_buffer(shape, like: torch.Tensor) -> torch.Tensor:
-    """An uninitialised tensor of ``shape`` in ``like``'s dtype for a kernel that streams ``like`` in and the
-    new tensor out at the same time.  The kernels read and write rows at a fixed distance from each other, and
-    how fast HBM serves the two streams together depends on that distance modulo the address interleave: with
-    both buffers on 2 MiB boundaries a 256 KiB row (V = 131072 bf16) loses 5 - 17 %, and distances of 64 - 256
-    KiB lose 8 % at V = 151936.  Starting the output 1.69 MiB into the period was at or near the best measured
-    for both, so large outputs are placed there inside a slightly larger allocation."""
-    n = 1
-    for d in shape:
-        n *= int(d)
-    nbytes = n * like.element_size()
-    if nbytes < _PHASED_MIN_BYTES:
-        return torch.empty(tuple(shape), dtype=like.dtype, device=like.device)
-    flat = torch.empty((nbytes + _PHASE,), dtype=torch.uint8, device=like.device)
-    off = (like.data_ptr() + _GRAD_PHASE - flat.data_ptr()) % _PHASE
-    off -= off % 256  # keeps every row start as aligned as in a fresh allocation
-    return flat[off:off + nbytes].view(like.dtype).view(tuple(shape))
-
+    """An uninitialised tensor of ``shape`` in ``like``'s dtype, placed where HBM serves a kernel that streams ``like`` in
+    and the new tensor out best."""
+    return _host().grad_buffer([int(d) for d in shape], like)
 
 
 def _dtype_code(t: torch.Tensor) -> int:
@@ -128,35 +116,11 @@ _LIB.define(
 
 
 def _logprob_fwd(logits, targets, n_inner, vocab_start, vocab_end, temperature, temp_mode, save_lse):
-    _need_gpu(logits, targets)
-    rows = _rows(logits, targets, n_inner, vocab_start, vocab_end, temperature, temp_mode)
-    b = logits.shape[0]
-    with torch.cuda.device(logits.device):
-        out = torch.empty((b, n_inner), dtype=torch.float32, device=logits.device)
-        lse = torch.empty((b, n_inner) if save_lse else (0,), dtype=torch.float32, device=logits.device)
-        with _timed("logprob_fwd"):
-            code = _lib.load().nrl_logprob_fwd(C.byref(rows), _ptr(out), _ptr(lse if save_lse else None), _stream())
-    _lib.check(code, "nrl_logprob_fwd")
-    return out, lse
+    return _host().logprob_fwd(logits, targets, n_inner, vocab_start, vocab_end, temperature, temp_mode, save_lse)
 
 
 def _logprob_bwd(logits, targets, lse, grad, n_inner, vocab_start, vocab_end, temperature, temp_mode, in_place=False):
-    _need_gpu(logits, targets, lse, grad)
-    rows = _rows(logits, targets, n_inner, vocab_start, vocab_end, temperature, temp_mode)
-    b, s, v = logits.shape
-    if tuple(lse.shape) != (b, n_inner) or not lse.is_contiguous() or lse.dtype != torch.float32:
-        raise ValueError("lse must be a contiguous fp32 [B, n_inner] tensor")
-    if tuple(grad.shape) != (b, n_inner) or grad.dtype != torch.float32:
-        raise ValueError(f"grad must be fp32 [B, n_inner], got {grad.dtype} {tuple(grad.shape)}")
-    with torch.cuda.device(logits.device):
-        d = logits if in_place else _grad_buffer((b, s, v), logits)
-        with _timed("logprob_bwd"):
-            code = _lib.load().nrl_logprob_bwd(
-                C.byref(rows), _ptr(lse), _ptr(grad), grad.stride(0), grad.stride(1),
-                _ptr(d), s, d.stride(0), d.stride(1), _stream(),
-            )
-    _lib.check(code, "nrl_logprob_bwd")
-    return d
+    return _host().logprob_bwd(logits, targets, lse, grad, n_inner, vocab_start, vocab_end, temperature, temp_mode, in_place)
 
 
 def _logprob_bwd_inplace(logits, targets, lse, grad, n_inner, vocab_start, vocab_end, temperature, temp_mode):
@@ -192,20 +156,7 @@ _LIB.define("scale_rows(Tensor x, Tensor factor, float divisor) -> Tensor")
 def _scale_rows(x, factor, divisor, in_place=False):
     """``x * (factor / divisor)`` for a ``[B, S, V]`` tensor and a device scalar ``factor``, in ``x``'s dtype.  The
     host does not wait for the factor's value; in place, a factor equal to the divisor touches no memory."""
-    _need_gpu(x, factor)
-    if x.dim() != 3 or (x.stride(2) != 1 and x.shape[2] > 1):
-        raise ValueError(f"expected [B, S, V] with a contiguous last axis, got {tuple(x.shape)} strides {x.stride()}")
-    if factor.numel() != 1:
-        raise ValueError("factor must hold one element")
-    f = factor.detach().reshape(1).to(torch.float32)
-    b, s, v = x.shape
-    with torch.cuda.device(x.device):
-        out = x if in_place else torch.empty((b, s, v), dtype=x.dtype, device=x.device)
-        with _timed("scale_rows"):
-            code = _lib.load().nrl_scale_rows(_ptr(x), _ptr(out), _dtype_code(x), b, s, v, x.stride(0), x.stride(1),
-                                              out.stride(0), out.stride(1), _ptr(f), float(divisor), _stream())
-    _lib.check(code, "nrl_scale_rows")
-    return out
+    return _host().scale_rows(x, factor, float(divisor), in_place)
 
 
 def _scale_rows_inplace(x, factor, divisor):
@@ -385,35 +336,7 @@ def _topk_topp_logprob_fwd(logits, targets, n_inner, top_k, top_p, temperature, 
     """-> (logprob [B,n] (empty without targets), thr, tie, lse_kept, unfiltered logprob (or empty)) and, with a
     capacity, the record of the kept sets (count [B,n], indices and scaled logits [B,n,capacity]) that lets the
     backward write a gradient row without reading the logits."""
-    _need_gpu(logits, targets)
-    b, s, v = logits.shape
-    dummy = targets if targets is not None else torch.zeros((b, max(n_inner, 1)), dtype=torch.int64, device=logits.device)
-    rows = _rows(logits, dummy, n_inner, 0, v, temperature, temp_mode)
-    if targets is None:
-        rows.targets = 0
-    dev = logits.device
-    with torch.cuda.device(dev):
-        f32 = dict(dtype=torch.float32, device=dev)
-        lp = torch.empty((b, n_inner) if targets is not None else (0,), **f32)
-        thr = torch.empty((b, n_inner), **f32)
-        tie = torch.empty((b, n_inner), dtype=torch.int32, device=dev)
-        lse = torch.empty((b, n_inner), **f32)
-        lpu = torch.empty((b, n_inner) if want_unfiltered else (0,), **f32)
-        rec = None
-        if capacity > 0:
-            rec = (torch.empty((b, n_inner), dtype=torch.int32, device=dev),
-                   torch.empty((b, n_inner, capacity), dtype=torch.int32, device=dev),
-                   torch.empty((b, n_inner, capacity), **f32))
-        with _timed("topk_topp_fwd"):
-            code = _lib.load().nrl_topk_topp_logprob_fwd(
-                C.byref(rows), int(top_k), float(top_p), _ptr(lp if targets is not None else None), _ptr(thr), _ptr(tie),
-                _ptr(lse), _ptr(lpu if want_unfiltered else None), None, _ptr(rec[0] if rec else None),
-                _ptr(rec[1] if rec else None), _ptr(rec[2] if rec else None), int(capacity), _stream(),
-            )
-    _lib.check(code, "nrl_topk_topp_logprob_fwd")
-    if capacity > 0:
-        return (lp, thr, tie, lse, lpu) + rec
-    return lp, thr, tie, lse, lpu
+    return tuple(_host().topk_topp_fwd(logits, targets, n_inner, int(top_k), float(top_p), temperature, temp_mode, want_unfiltered, int(capacity)))
 
 
 def _topk_topp_logprob_fwd_rec(logits, targets, n_inner, top_k, top_p, temperature, temp_mode, want_unfiltered, capacity):
@@ -424,36 +347,7 @@ def _topk_topp_logprob_fwd_rec(logits, targets, n_inner, top_k, top_p, temperatu
 
 def _topk_topp_logprob_bwd(logits, targets, thr, tie, lse_kept, grad, n_inner, temperature, temp_mode, kept_n=None,
                            kept_idx=None, kept_x=None):
-    _need_gpu(logits, targets, thr, tie, lse_kept, grad, kept_n, kept_idx, kept_x)
-    b, s, v = logits.shape
-    rows = _rows(logits, targets, n_inner, 0, v, temperature, temp_mode)
-    for t, name in ((thr, "thr"), (tie, "tie"), (lse_kept, "lse_kept")):
-        if tuple(t.shape) != (b, n_inner) or not t.is_contiguous():
-            raise ValueError(f"{name} must be a contiguous [B, n_inner] tensor")
-    if thr.dtype != torch.float32 or lse_kept.dtype != torch.float32 or tie.dtype != torch.int32:
-        raise ValueError("thr / lse_kept must be fp32 and tie int32")
-    if tuple(grad.shape) != (b, n_inner) or grad.dtype != torch.float32:
-        raise ValueError("grad must be fp32 [B, n_inner]")
-    capacity = 0
-    if kept_n is not None:
-        if kept_idx is None or kept_x is None:
-            raise ValueError("the kept-set record is (count, indices, values): all three or none")
-        capacity = kept_idx.shape[-1]
-        ok = (kept_n.dtype == torch.int32 and kept_idx.dtype == torch.int32 and kept_x.dtype == torch.float32
-              and tuple(kept_n.shape) == (b, n_inner) and tuple(kept_idx.shape) == (b, n_inner, capacity)
-              and tuple(kept_x.shape) == (b, n_inner, capacity)
-              and kept_n.is_contiguous() and kept_idx.is_contiguous() and kept_x.is_contiguous() and capacity >= 1)
-        if not ok:
-            raise ValueError("kept-set record: int32 [B, n], int32 [B, n, capacity], fp32 [B, n, capacity], contiguous")
-    with torch.cuda.device(logits.device):
-        d = _grad_buffer((b, s, v), logits)
-        with _timed("topk_topp_bwd"):
-            code = _lib.load().nrl_topk_topp_logprob_bwd(
-                C.byref(rows), _ptr(thr), _ptr(tie), _ptr(lse_kept), _ptr(grad), grad.stride(0), grad.stride(1),
-                _ptr(kept_n), _ptr(kept_idx), _ptr(kept_x), capacity, _ptr(d), s, d.stride(0), d.stride(1), _stream(),
-            )
-    _lib.check(code, "nrl_topk_topp_logprob_bwd")
-    return d
+    return _host().topk_topp_bwd(logits, targets, thr, tie, lse_kept, grad, n_inner, temperature, temp_mode, kept_n, kept_idx, kept_x)
 
 
 def _topk_topp_filter(logits, thr, tie, temperature, temp_mode):
@@ -492,9 +386,6 @@ _LIB.define(
 _LIB.define(
     "nll_loss(Tensor lp, Tensor token_mask, Tensor sample_mask, Tensor global_valid) -> (Tensor, Tensor, Tensor)"
 )
-
-_CFG_INT = [n for n, _ in _lib.NrlGrpoCfg._fields_[:14]]
-_CFG_FLT = [n for n, _ in _lib.NrlGrpoCfg._fields_[14:]]
 
 
 def _rowmat(t, b, n, name):
@@ -542,32 +433,7 @@ def _grpo_inputs(lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct_
 
 
 def _grpo_loss(lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct_mask, global_valid, iflags, fparams):
-    if len(iflags) != len(_CFG_INT) or len(fparams) != len(_CFG_FLT):
-        raise ValueError("malformed loss configuration")
-    inp, keep, b, n = _grpo_inputs(lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct_mask, global_valid)
-    cfg = _lib.NrlGrpoCfg()
-    for name, v in zip(_CFG_INT, iflags):
-        setattr(cfg, name, int(v))
-    for name, v in zip(_CFG_FLT, fparams):
-        setattr(cfg, name, float(v))
-    lib = _lib.load()
-    dev = lp.device
-    split = lpu is not None and cfg.has_kl
-    with torch.cuda.device(dev):
-        loss = torch.empty((), dtype=torch.float32, device=dev)
-        dlp = torch.empty((b, n), dtype=torch.float32, device=dev)
-        dlpu = torch.empty((b, n) if split else (0,), dtype=torch.float32, device=dev)
-        metrics = torch.empty((_lib.NRL_GRPO_N_METRICS,), dtype=torch.float32, device=dev)
-        ws_bytes = lib.nrl_grpo_loss_workspace_bytes(b)
-        ws = torch.empty((ws_bytes // 8,), dtype=torch.float64, device=dev)
-        with _timed("grpo_loss"):
-            code = lib.nrl_grpo_loss_fwd_bwd(
-                C.byref(cfg), C.byref(inp), _ptr(loss), _ptr(dlp), _ptr(dlpu if split else None), _ptr(metrics),
-                _ptr(ws), ws_bytes, _stream(),
-            )
-    _lib.check(code, "nrl_grpo_loss_fwd_bwd")
-    del keep
-    return loss, dlp, dlpu, metrics
+    return _host().grpo_loss(lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct_mask, global_valid, iflags, fparams)
 
 
 _LIB.define(
@@ -586,36 +452,8 @@ def _fused_logits_grpo_loss(logits, targets, n_inner, prev, gen, ref, adv, token
                             fparams, loss_scale, temperature, temp_mode, in_place=False):
     """-> (loss, dlogits, logprobs [B, n_inner], metrics).  ``temperature`` != 1 divides the logits inside the
     pass the way an in-place ``div_`` of the tensor would have rounded them (``temp_mode``: on the GPU or the CPU)."""
-    if len(iflags) != len(_CFG_INT) or len(fparams) != len(_CFG_FLT):
-        raise ValueError("malformed loss configuration")
-    _need_gpu(logits, targets)
-    b, s, v = logits.shape
-    rows = _rows(logits, targets, n_inner, 0, v, float(temperature), int(temp_mode))
-    dev = logits.device
-    lp_shape = torch.empty((b, n_inner), dtype=torch.float32, device=dev)
-    inp, keep, _, _ = _grpo_inputs(lp_shape, None, prev, gen, ref, adv, token_mask, sample_mask, None, global_valid)
-    cfg = _lib.NrlGrpoCfg()
-    for name, val in zip(_CFG_INT, iflags):
-        setattr(cfg, name, int(val))
-    for name, val in zip(_CFG_FLT, fparams):
-        setattr(cfg, name, float(val))
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        loss = torch.empty((), dtype=torch.float32, device=dev)
-        metrics = torch.empty((_lib.NRL_GRPO_N_METRICS,), dtype=torch.float32, device=dev)
-        d = logits if in_place else _grad_buffer((b, s, v), logits)
-        ws_bytes = lib.nrl_fused_workspace_bytes(b, n_inner)
-        ws = torch.empty(((ws_bytes + 7) // 8,), dtype=torch.float64, device=dev)
-        with _timed("fused_logits_loss"):
-            code = lib.nrl_fused_logits_grpo_loss(
-                C.byref(rows), C.byref(cfg), C.byref(inp), float(loss_scale), _ptr(d), s, d.stride(0), d.stride(1),
-                _ptr(lp_shape), _ptr(loss), _ptr(metrics), _ptr(ws), ws.numel() * 8, _stream(),
-            )
-    if code == -2:
-        raise NotImplementedError(lib.nrl_last_error().decode(errors="replace"))
-    _lib.check(code, "nrl_fused_logits_grpo_loss")
-    del keep
-    return loss, d, lp_shape, metrics
+    return _host().fused_loss(logits, targets, n_inner, None, False, prev, gen, ref, adv, token_mask, sample_mask, global_valid, iflags,
+                              fparams, float(loss_scale), float(temperature), int(temp_mode), in_place)
 
 
 def _fused_logits_grpo_loss_inplace(logits, targets, n_inner, prev, gen, ref, adv, token_mask, sample_mask, global_valid,
@@ -641,45 +479,8 @@ _LIB.define(
 def _fused_packed_logits_grpo_loss(logits, targets, pre_rolled, cu_seqlens, unpacked_seqlen, prev, gen, ref, adv, token_mask,
                                    sample_mask, global_valid, iflags, fparams, loss_scale, temperature, temp_mode):
     """Packed [T, V] logits -> (loss, dlogits [T, V], logprobs [n_seq, unpacked_seqlen - 1], metrics)."""
-    if len(iflags) != len(_CFG_INT) or len(fparams) != len(_CFG_FLT):
-        raise ValueError("malformed loss configuration")
-    _check_packed(logits, targets, cu_seqlens, unpacked_seqlen)
-    t, v = logits.shape
-    n_seq, n_inner = cu_seqlens.shape[0] - 1, unpacked_seqlen - 1
-    rows = _lib.NrlRows()
-    rows.logits = logits.data_ptr()
-    rows.dtype = _dtype_code(logits)
-    rows.n_outer, rows.n_inner, rows.vocab = 1, t, v
-    rows.stride_outer, rows.stride_inner = 0, logits.stride(0)
-    rows.targets = targets.data_ptr()
-    rows.tgt_stride_outer, rows.tgt_stride_inner = 0, 1
-    rows.vocab_start, rows.vocab_end = 0, v
-    rows.temperature, rows.temp_mode = float(temperature), int(temp_mode)
-    dev = logits.device
-    lp = torch.empty((n_seq, n_inner), dtype=torch.float32, device=dev)
-    inp, keep, _, _ = _grpo_inputs(lp, None, prev, gen, ref, adv, token_mask, sample_mask, None, global_valid)
-    cfg = _lib.NrlGrpoCfg()
-    for name, val in zip(_CFG_INT, iflags):
-        setattr(cfg, name, int(val))
-    for name, val in zip(_CFG_FLT, fparams):
-        setattr(cfg, name, float(val))
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        loss = torch.empty((), dtype=torch.float32, device=dev)
-        metrics = torch.empty((_lib.NRL_GRPO_N_METRICS,), dtype=torch.float32, device=dev)
-        d = _grad_buffer((t, v), logits)
-        ws_bytes = lib.nrl_fused_packed_workspace_bytes(n_seq, n_inner, t)
-        ws = torch.empty(((ws_bytes + 7) // 8,), dtype=torch.float64, device=dev)
-        with _timed("fused_packed_logits_loss"):
-            code = lib.nrl_fused_packed_logits_grpo_loss(
-                C.byref(rows), int(pre_rolled), _ptr(cu_seqlens), n_seq, C.byref(cfg), C.byref(inp), float(loss_scale),
-                _ptr(d), d.stride(0), _ptr(lp), _ptr(loss), _ptr(metrics), _ptr(ws), ws.numel() * 8, _stream(),
-            )
-    if code == -2:
-        raise NotImplementedError(lib.nrl_last_error().decode(errors="replace"))
-    _lib.check(code, "nrl_fused_packed_logits_grpo_loss")
-    del keep
-    return loss, d, lp, metrics
+    return _host().fused_loss(logits, targets, unpacked_seqlen - 1, cu_seqlens, pre_rolled, prev, gen, ref, adv, token_mask, sample_mask,
+                              global_valid, iflags, fparams, float(loss_scale), float(temperature), int(temp_mode), False)
 
 
 _LIB.impl("fused_packed_logits_grpo_loss", _fused_packed_logits_grpo_loss, "CUDA")
@@ -1011,31 +812,7 @@ _LIB.define(
 
 
 def _group_baseline_std(prompts, rewards, valid, std_rewards, leave_one_out, normalize):
-    _need_gpu(prompts, rewards, valid, std_rewards)
-    if prompts.dim() == 1:
-        prompts = prompts.unsqueeze(-1)
-    if prompts.dim() != 2 or prompts.dtype != torch.int64:
-        raise ValueError(f"prompts must be int64 [B, Sp], got {prompts.dtype} {tuple(prompts.shape)}")
-    b, sp = prompts.shape
-    if sp > 1 and prompts.stride(1) != 1:
-        prompts = prompts.contiguous()
-    rewards, valid, std_rewards = _vec(rewards, b, "rewards"), _vec(valid, b, "valid_mask"), _vec(std_rewards, b, "std_rewards")
-    lib = _lib.load()
-    dev = rewards.device
-    with torch.cuda.device(dev):
-        baseline = torch.empty((b,), dtype=torch.float32, device=dev)
-        std = torch.empty((b,), dtype=torch.float32, device=dev)
-        adv = torch.empty((b,), dtype=torch.float32, device=dev)
-        group = torch.empty((b,), dtype=torch.int32, device=dev)
-        ws_bytes = lib.nrl_group_workspace_bytes(b)
-        ws = torch.empty(((ws_bytes + 7) // 8,), dtype=torch.float64, device=dev)
-        code = lib.nrl_group_baseline_std(
-            _ptr(prompts), b, sp, prompts.stride(0) if b > 1 else sp, _ptr(rewards), _ptr(valid), _ptr(std_rewards),
-            int(leave_one_out), int(normalize), _ptr(baseline), _ptr(std), _ptr(adv), _ptr(group), _ptr(ws),
-            ws.numel() * 8, _stream(),
-        )
-    _lib.check(code, "nrl_group_baseline_std")
-    return baseline, std, adv, group
+    return _host().group_baseline_std(prompts, rewards, valid, std_rewards, leave_one_out, normalize)
 
 
 _LIB.impl("group_baseline_std", _group_baseline_std, "CUDA")
@@ -1188,50 +965,16 @@ def _gather_logprob_bwd(logits, indices, vocab_start, vocab_end, lse, grad):
     return d
 
 
-def _gather_entropy_rows(logits, indices, n_inner):
-    rows = _plain_rows(logits)
-    if not 0 <= n_inner <= logits.shape[1]:
-        raise ValueError(f"n_inner {n_inner} does not fit logits {tuple(logits.shape)}")
-    rows.n_inner = n_inner
-    return rows, _gather_indices(logits, indices)
-
-
 def _gather_entropy_fwd(logits, indices, n_inner, entropy):
     """The first ``n_inner`` rows of every sequence: ``log p`` at ``indices [B, S, K]`` -> ``[B, n_inner, K]``,
     ``sum_v p log p`` (empty without ``entropy``) and the log-sum-exps, from one pass over the logits."""
-    _need_gpu(logits, indices)
-    rows, indices = _gather_entropy_rows(logits, indices, n_inner)
-    b, s, k = indices.shape
-    dev = logits.device
-    with torch.cuda.device(dev):
-        out = torch.empty((b, n_inner, k), dtype=torch.float32, device=dev)
-        h = torch.empty((b, n_inner) if entropy else (0,), dtype=torch.float32, device=dev)
-        lse = torch.empty((b, n_inner), dtype=torch.float32, device=dev)
-        with _timed("gather_entropy_fwd"):
-            code = _lib.load().nrl_gather_entropy_fwd(C.byref(rows), _ptr(indices), k, s * k, _ptr(out), _ptr(h if entropy else None),
-                                                      _ptr(lse), _stream())
-    _lib.check(code, "nrl_gather_entropy_fwd")
-    return out, h, lse
+    refuse_pending(logits, "gather_entropy_fwd")
+    return _host().gather_entropy_fwd(logits, indices, n_inner, entropy)
 
 
 def _gather_entropy_bwd(logits, indices, n_inner, lse, h, grad_h, grad):
     """Gradient of both outputs of ``gather_entropy_fwd`` (of the gathered values alone without ``h``) in one pass."""
-    _need_gpu(logits, indices, lse, h, grad_h, grad)
-    rows, indices = _gather_entropy_rows(logits, indices, n_inner)
-    b, s, k = indices.shape
-    lse = _row_scalar(lse, b, n_inner, "lse")
-    if h is not None:
-        h, grad_h = _row_scalar(h, b, n_inner, "h"), _row_scalar(grad_h, b, n_inner, "grad_h")
-    if grad.dtype != torch.float32 or tuple(grad.shape) != (b, n_inner, k):
-        raise ValueError(f"grad must be fp32 [{b}, {n_inner}, {k}], got {grad.dtype} {tuple(grad.shape)}")
-    grad = grad.contiguous()
-    with torch.cuda.device(logits.device):
-        d = _grad_buffer(logits.shape, logits)
-        with _timed("gather_entropy_bwd"):
-            code = _lib.load().nrl_gather_entropy_bwd(C.byref(rows), _ptr(indices), k, s * k, _ptr(lse), _ptr(h), _ptr(grad_h), _ptr(grad),
-                                                      _ptr(d), s, d.stride(0), d.stride(1), _stream())
-    _lib.check(code, "nrl_gather_entropy_bwd")
-    return d
+    return _host().gather_entropy_bwd(logits, indices, n_inner, lse, h, grad_h, grad)
 
 
 def _teacher_like(student, teacher):
