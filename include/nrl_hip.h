@@ -342,6 +342,15 @@ int nrl_masked_mean(const float* values, const float* mask, int64_t n_rows, int6
 int nrl_masked_mean_bwd(const float* grad_out, const float* mask, const float* denom, int64_t n_rows, int64_t n_cols,
                         float* dvalues_out, void* stream);
 
+/* Positions that are masked out or whose logprob is infinite become 0.  logprobs: fp32 [batch, n] with row stride lp_stride;
+ * mask: [batch, n] of NRL_MASK_* elements with row stride mask_stride, multiplied by sample_mask [batch] where that is not
+ * NULL.  out: fp32 [batch, n]; keep_out: uint8 [batch, n], what the backward needs; counts_out: double [batch, 2], per row the
+ * number of infinite logprobs under the mask and the sum of the mask. */
+int nrl_mask_neg_inf(const float* logprobs, int64_t lp_stride, const void* mask, int32_t mask_type, int64_t mask_stride,
+                     const float* sample_mask, int64_t batch, int64_t n, float* out, uint8_t* keep_out, double* counts_out, void* stream);
+/* grad_in[i] = keep[i] ? grad_out[i] : 0, n elements */
+int nrl_mask_neg_inf_bwd(const float* grad_out, const uint8_t* keep, int64_t n, float* grad_in, void* stream);
+
 /* log_softmax over the K logits of a row at the given vocabulary indices (the teacher's top-k), the
  * zero_outside_topk = False branch of get_distillation_topk_logprobs_from_logits
  * (nemo_rl/distributed/model_utils.py:1981-2005): out[r, j] = x[r, idx[r, j]] - logsumexp_j x[r, idx[r, j]].

@@ -95,6 +95,8 @@ SIGNATURES = {
     "nrl_calculate_kl_bwd": (C.c_int, [_P, _P, _P, _P, _I64, _I32, _I32, _F, _I32, _F, _P, _P, _P, _P]),
     "nrl_masked_mean": (C.c_int, [_P, _P, _I64, _I64, _P, _F, _I32, _P, _P, _P]),
     "nrl_masked_mean_bwd": (C.c_int, [_P, _P, _P, _I64, _I64, _P, _P]),
+    "nrl_mask_neg_inf": (C.c_int, [_P, _I64, _P, _I32, _I64, _P, _I64, _I64, _P, _P, _P, _P]),
+    "nrl_mask_neg_inf_bwd": (C.c_int, [_P, _P, _I64, _P, _P]),
     "nrl_topk_logsoftmax_fwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _P, _P]),
     "nrl_topk_logsoftmax_bwd": (C.c_int, [C.POINTER(NrlRows), _P, _I64, _P, _P, _P, _I64, _I64, _P]),
     "nrl_distill_topk_loss_workspace_bytes": (_I64, [_I64, _I64]),
@@ -128,7 +130,7 @@ SIGNATURES = {
 _lib = None
 
 
-ABI_VERSION = 113  # nrl_version() of the library these signatures describe
+ABI_VERSION = 114  # nrl_version() of the library these signatures describe
 
 
 def load() -> C.CDLL:

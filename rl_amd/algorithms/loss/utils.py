@@ -12,7 +12,7 @@ from ...distributed.model_utils import (
     get_next_token_logprobs_from_logits,
 )
 from ..logits_sampling_utils import TrainingSamplingParams, need_top_k_or_top_p_filtering
-from ..utils import mask_out_neg_inf_logprobs
+from ..utils import _mask_out_neg_inf, mask_out_neg_inf_logprobs  # noqa: F401
 from .interfaces import LossFunction, LossInputType
 
 
@@ -77,8 +77,8 @@ def prepare_loss_input(
         logprobs = logprobs_with(sampling_params, chunk_size)  # loss/utils.py:85-94: the main call chunks
 
     if need_top_k_or_top_p_filtering(sampling_params):
-        mask = data["token_mask"] * data["sample_mask"].unsqueeze(-1)
-        logprobs = mask_out_neg_inf_logprobs(logprobs, mask[:, 1:].to(logprobs.device), "curr_logprobs")
+        dev = logprobs.device
+        logprobs = _mask_out_neg_inf(logprobs, data["token_mask"][:, 1:].to(dev), data["sample_mask"].to(dev), "curr_logprobs")
         if _wants_unfiltered_kl(loss_fn):
             data["curr_logprobs_unfiltered"] = logprobs_with(None, None)  # :108-118: the unfiltered pass does not
     return {"next_token_logprobs": logprobs}, data
@@ -171,8 +171,8 @@ def prepare_packed_loss_input(
 
     logprobs = logprobs_with(sampling_params)
     if need_top_k_or_top_p_filtering(sampling_params):
-        mask = data["token_mask"] * data["sample_mask"].unsqueeze(-1)
-        logprobs = mask_out_neg_inf_logprobs(logprobs, mask[:, 1:].to(logprobs.device), "curr_logprobs")
+        dev = logprobs.device
+        logprobs = _mask_out_neg_inf(logprobs, data["token_mask"][:, 1:].to(dev), data["sample_mask"].to(dev), "curr_logprobs")
         if _wants_unfiltered_kl(loss_fn):
             data["curr_logprobs_unfiltered"] = logprobs_with(None)
     return {"next_token_logprobs": logprobs}, data

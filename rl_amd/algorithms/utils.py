@@ -2,17 +2,19 @@
 
 ``calculate_baseline_and_std_per_prompt`` runs the HIP grouping / statistics kernels, ``calculate_kl`` and
 ``masked_mean`` their own small kernels (inside ``ClippedPGLossFn`` the same arithmetic is part of the fused loss
-kernel instead).  ``mask_out_neg_inf_logprobs`` is [B, S]-sized tensor plumbing around the reference's warning.
+kernel instead), ``mask_out_neg_inf_logprobs`` one kernel that also counts for the reference's warning.
 """
 
 from __future__ import annotations
 
 import atexit
+import math
 from typing import Optional
 
 import torch
 
 from .. import ops as _ops  # noqa: F401
+from .._lib import host as _host
 
 _OPS = torch.ops.rl_amd
 
@@ -166,7 +168,7 @@ def masked_mean(
 # have arrived -- at a later call, at ``flush_neg_inf_warnings()`` or when the interpreter exits -- so the caller keeps
 # queueing work (the backward, the next microbatch).  ``DEFER_NEG_INF_WARNING = False`` prints before returning.
 DEFER_NEG_INF_WARNING = True
-_pending_warnings: list = []  # (event, pinned int64[2], name)
+_pending_warnings: list = []  # (counts on their way to the host, name)
 
 
 def _warn_neg_inf(hit: int, valid: int, logprobs_name: str) -> None:
@@ -177,15 +179,27 @@ def _warn_neg_inf(hit: int, valid: int, logprobs_name: str) -> None:
         )
 
 
+def _counts_of(values: list) -> tuple[int, int]:
+    """(infinite, valid) from the pairs of one or several sequences."""
+    valid = sum(values[1::2])
+    return int(sum(values[0::2])), int(valid) if math.isfinite(valid) else 0
+
+
+def _plain(*tensors) -> bool:
+    """Ordinary tensors outside function transforms and forward-mode differentiation, which a kernel cannot follow."""
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and not torch._C._are_functorch_transforms_active() and torch.autograd.forward_ad._current_level < 0)
+
+
 def flush_neg_inf_warnings(wait: bool = True) -> None:
     """Prints the deferred warnings whose counts have arrived, oldest first; with ``wait`` all of them."""
     while _pending_warnings:
-        event, counts, name = _pending_warnings[0]
-        if not wait and not event.query():
+        counts, name = _pending_warnings[0]
+        if not wait and not counts.ready():
             return
-        event.synchronize()
+        values = counts()
         _pending_warnings.pop(0)
-        _warn_neg_inf(int(counts[0]), int(counts[1]), name)
+        _warn_neg_inf(*_counts_of(values), name)
 
 
 atexit.register(flush_neg_inf_warnings)
@@ -194,16 +208,34 @@ atexit.register(flush_neg_inf_warnings)
 def mask_out_neg_inf_logprobs(logprobs: torch.Tensor, mask: torch.Tensor, logprobs_name: str) -> torch.Tensor:
     """``utils.py:227-257``: positions that are masked out or infinite become 0 (with the reference's
     warning when valid tokens are affected)."""
+    return _mask_out_neg_inf(logprobs, mask, None, logprobs_name)
+
+
+def _mask_out_neg_inf(logprobs: torch.Tensor, mask: torch.Tensor, sample_mask: Optional[torch.Tensor], logprobs_name: str) -> torch.Tensor:
+    """``mask_out_neg_inf_logprobs`` under ``mask * sample_mask.unsqueeze(-1)`` (``mask`` alone without a sample mask).  One
+    kernel for fp32 ``[B, n]`` logprobs on the GPU and masks in the types a data pipeline makes; tensor operations
+    otherwise."""
+    if (
+        logprobs.is_cuda and logprobs.dim() == 2 and logprobs.dtype == torch.float32 and _plain(logprobs, mask)
+        and mask.shape == logprobs.shape and mask.device == logprobs.device
+        and mask.dtype in (torch.float32, torch.int64, torch.uint8, torch.bool) and not mask.requires_grad
+        and (sample_mask is None or (sample_mask.dtype == torch.float32 and sample_mask.shape == mask.shape[:1]
+                                     and sample_mask.device == mask.device and not sample_mask.requires_grad))
+    ):
+        out, rows = _host().mask_neg_inf(logprobs, mask, sample_mask)
+        if not DEFER_NEG_INF_WARNING:
+            _warn_neg_inf(*_counts_of(rows.reshape(-1).tolist()), logprobs_name)
+        elif rows.numel() > 0:
+            flush_neg_inf_warnings(wait=False)
+            _pending_warnings.append((_host().Fetch(rows), logprobs_name))
+        return out
+    if sample_mask is not None:
+        mask = mask * sample_mask.unsqueeze(-1)
     is_inf = torch.isinf(logprobs)
-    # both counts in one transfer: the warning is the only reason this function waits for the device at all
     counts = torch.stack([(is_inf & mask.bool()).sum(), mask.sum().to(torch.int64)])
     if DEFER_NEG_INF_WARNING and counts.is_cuda:
         flush_neg_inf_warnings(wait=False)
-        host = torch.empty(2, dtype=torch.int64, pin_memory=True)
-        host.copy_(counts, non_blocking=True)
-        event = torch.cuda.Event()
-        event.record()
-        _pending_warnings.append((event, host, logprobs_name))
+        _pending_warnings.append((_host().Fetch(counts), logprobs_name))
     else:
         hit, valid = counts.tolist()
         _warn_neg_inf(hit, valid, logprobs_name)

@@ -562,6 +562,44 @@ struct RowsLogprobSampled : torch::autograd::Function<RowsLogprobSampled> {
     }
 };
 
+// logprobs [B, n] whose masked-out or infinite positions become 0, and per sequence the two counts of the warning
+struct MaskNegInf : torch::autograd::Function<MaskNegInf> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& lp_in, const Tensor& mask_in, const OptTensor& sample_in) {
+        ctx->set_materialize_grads(false);
+        const Tensor sample = opt(sample_in);
+        Tensor lp = lp_in.detach();
+        need_gpu(lp, mask_in, sample);
+        TORCH_CHECK_VALUE(lp.dim() == 2 && lp.scalar_type() == at::kFloat, "logprobs must be fp32 [B, n], got ", lp.scalar_type(), " ", lp.sizes());
+        const int64_t b = lp.size(0), n = lp.size(1);
+        const c10::OptionalDeviceGuard guard(lp.device());
+        if (n > 1 && lp.stride(1) != 1) lp = lp.contiguous();
+        LossInputs l;
+        l.in.batch = b; l.in.sm1 = n;
+        l.mask(mask_in, lp, 0);
+        const float* sm = l.vec(sample, lp, "sample_mask");
+        Tensor out = f32({b, n}, lp), keep = at::empty({b, n}, lp.options().dtype(at::kByte)), counts = at::empty({b, 2}, lp.options().dtype(at::kDouble));
+        check(nrl_mask_neg_inf(ptr(lp), lp.stride(0), l.in.token_mask, l.in.token_mask_type, l.in.token_mask_stride, sm, b, n, ptr(out), ptr<uint8_t>(keep),
+                               ptr<double>(counts), stream_of(lp)), "nrl_mask_neg_inf");
+        ctx->save_for_backward({keep});
+        ctx->mark_non_differentiable({counts});
+        return {out, counts};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        variable_list out(3);
+        if (!grads[0].defined()) return out;
+        const auto saved = ctx->get_saved_variables();
+        if (at::GradMode::is_enabled()) {  // a gradient of the gradient is wanted
+            out[0] = at::where(saved[0].to(at::kBool), grads[0], at::zeros({}, grads[0].options()));
+            return out;
+        }
+        const Tensor g = to_f32(grads[0], saved[0]).contiguous();
+        const c10::OptionalDeviceGuard guard(g.device());
+        out[0] = at::empty(g.sizes(), g.options());
+        check(nrl_mask_neg_inf_bwd(ptr(g), ptr<uint8_t>(saved[0]), g.numel(), ptr(out[0]), stream_of(g)), "nrl_mask_neg_inf_bwd");
+        return out;
+    }
+};
+
 // log p at indices [B, S, K] and (optionally) sum_v p log p of the first n rows of every sequence
 struct GatherEntropy : torch::autograd::Function<GatherEntropy> {
     static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& indices, int64_t n, bool entropy) {
@@ -691,6 +729,10 @@ PYBIND11_MODULE(_host, m) {
         Tensor t = targets.device() == logits.device() && targets.scalar_type() == at::kLong ? targets : targets.to(logits.device(), at::kLong);
         if (shift) t = t.narrow(1, shift, t.size(1) - shift);
         return RowsLogprobSampled::apply(logits, t, n_inner, top_k, top_p, inference_only, temperature, mode, capacity);
+    });
+    m.def("mask_neg_inf", [](const Tensor& lp, const Tensor& mask, const OptTensor& sample_mask) {
+        const variable_list o = MaskNegInf::apply(lp, mask, sample_mask);
+        return std::make_tuple(o[0], o[1]);
     });
     m.def("clipped_pg", [](const Tensor& lp, const OptTensor& lpu, const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv,
                            const Tensor& token_mask, const Tensor& sample_mask, const OptTensor& correct, const Tensor& seqs, const Tensor& toks,

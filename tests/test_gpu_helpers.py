@@ -150,3 +150,31 @@ def test_neg_inf_warning_immediate_and_deferred(capsys):
     assert out.count("[WARNING]") == 1 and "2/5 valid tokens have -inf in prev_logprobs" in out
     U.flush_neg_inf_warnings()  # nothing left
     assert capsys.readouterr().out == ""
+
+
+@pytest.mark.parametrize("batch,n", [(1, 1), (3, 1023), (2, 1025), (70, 33)])
+@pytest.mark.parametrize("mask_dtype", [torch.float32, torch.int64, torch.bool])
+def test_neg_inf_masking_kernel_against_tensor_operations(batch, n, mask_dtype, capsys):
+    """Values, gradient and both counts are exact: nothing is rounded.  The logprobs and the mask are column slices."""
+    g = torch.Generator().manual_seed(batch * 1000 + n)
+    lp = -torch.rand(batch, n + 1, generator=g)
+    lp[torch.rand(batch, n + 1, generator=g) < 0.2] = float("-inf")
+    lp[0, 0] = float("inf")
+    tm = (torch.rand(batch, n + 2, generator=g) < 0.7).to(mask_dtype)
+    sm = (torch.rand(batch, generator=g) < 0.8).float()
+    mask = (tm * sm.unsqueeze(-1))[:, 1 : n + 1]
+    bad = torch.isinf(lp[:, :n])
+    keep = (mask != 0) & ~bad
+    x = lp.to(DEV).requires_grad_(True)
+    U.flush_neg_inf_warnings()
+    capsys.readouterr()
+    got = U._mask_out_neg_inf(x[:, :n], tm.to(DEV)[:, 1 : n + 1], sm.to(DEV), "curr_logprobs")
+    assert torch.equal(got.detach().cpu(), torch.where(keep, lp[:, :n], 0.0))
+    up = torch.randn(batch, n, generator=g)
+    got.backward(up.to(DEV))
+    assert torch.equal(x.grad.cpu()[:, :n], torch.where(keep, up, 0.0)) and torch.all(x.grad[:, n] == 0)
+    U.flush_neg_inf_warnings()
+    hit, valid = int((bad & (mask != 0)).sum()), int(mask.sum())
+    assert (f"{hit}/{valid} valid" in capsys.readouterr().out) == (hit > 0)
+    assert torch.equal(U.mask_out_neg_inf_logprobs(x[:, :n], mask.to(DEV), "curr_logprobs"), got)
+    U.flush_neg_inf_warnings()
