@@ -179,6 +179,27 @@ __device__ __forceinline__ float wave_min(float v) {
     return v;
 }
 
+// The same for a double, by lane moves inside the rows of 16 lanes and scalar reads across them: no LDS round trips, of which
+// __shfl_xor of a double makes twelve.
+template <int CTRL> __device__ __forceinline__ double moved_double(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int lo = static_cast<int>(u), hi = static_cast<int>(u >> 32);
+    const uint32_t l = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false), h = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, (static_cast<uint64_t>(h) << 32) | l);
+}
+__device__ __forceinline__ double lane_double(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t l = __builtin_amdgcn_readlane(static_cast<int>(u), lane), h = __builtin_amdgcn_readlane(static_cast<int>(u >> 32), lane);
+    return __builtin_bit_cast(double, (static_cast<uint64_t>(h) << 32) | l);
+}
+__device__ __forceinline__ double wave_sum_double(double v) {
+    v += moved_double<0xB1>(v);   // quad_perm [1,0,3,2]
+    v += moved_double<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += moved_double<0x141>(v);  // row_half_mirror
+    v += moved_double<0x140>(v);  // row_mirror
+    return (lane_double(v, 0) + lane_double(v, 16)) + (lane_double(v, 32) + lane_double(v, 48));
+}
+
 // Sum over a workgroup of NW waves; every thread receives the total.  `smem` holds NW entries.
 // Lanes are combined in a fixed butterfly order and waves in ascending order, so the result
 // depends only on the values and the workgroup shape.

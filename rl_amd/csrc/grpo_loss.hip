@@ -24,40 +24,72 @@ namespace nrl {
 
 constexpr int kLossBlock = 256;
 constexpr int kLossWaves = kLossBlock / kWave;
+// The kernels with one workgroup per sequence have as many workgroups as a microbatch has sequences, 1 - 16: what they cost is
+// the number of dependent steps of one workgroup, so a sequence gets the largest there is.  2 sequences of
+// 2048 tokens: rows kernel 26.8 -> 16.7 us, 3 of 701: 16.0 -> 11.4 us (256 against 1024 threads).
+constexpr int kSeqBlock = 1024;
+constexpr int kSeqWaves = kSeqBlock / kWave;
 
-// Workgroup-wide reduction of one sequence's accumulators into its row of partials.
-__device__ __forceinline__ void store_row_parts(const nrl_grpo_cfg& c, double* out, double (&acc)[P_R_MIN], float r_min,
-                                                float r_max, float rc_min, float rc_max, const SeqStats& st, float smv,
-                                                double* sm_d, float* sm_f) {
-    const int tid = threadIdx.x;
-    const float tis_floor = c.tis_min;
+// Sums of N values over a workgroup with two barriers in all; thread k < N returns sum k, waves added in ascending order.
+template <int N, int NW> __device__ __forceinline__ double block_sums(const double (&v)[N], double* smem /* [NW * N] */) {
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
+    __syncthreads();
 #pragma unroll
-    for (int k = 0; k < P_R_MIN; ++k) {
-        const double tot = block_sum<double, kLossWaves>(acc[k], sm_d);
-        if (tid == 0) out[k] = tot;
+    for (int k = 0; k < N; ++k) {
+        const double s = wave_sum_double(v[k]);
+        if (lane == 0) smem[w * N + k] = s;
     }
-    const float mn = block_min<kLossWaves>(r_min, sm_f), mx = block_max<kLossWaves>(r_max, sm_f);
-    const float cmn = block_min<kLossWaves>(rc_min, sm_f), cmx = block_max<kLossWaves>(rc_max, sm_f);
-    if (tid == 0) {
-        const float seq_w = st.seq_w, seq_keep = st.seq_keep;
-        if (!c.token_level_loss) {  // sequence-level: masked mean over tokens, then weight by sample_mask
-            out[P_ACTOR] = static_cast<double>(static_cast<float>(out[P_ACTOR]) / st.seq_den) * smv;
-            out[P_KL] = static_cast<double>(static_cast<float>(out[P_KL]) / st.seq_den) * smv;
-        }
-        out[P_SAMPLE_MASK] = smv;
-        out[P_SEQ_W] = c.tis_type == NRL_TIS_SEQ_MASK ? seq_w * seq_keep : seq_w;
-        if (c.sequence_level_importance_ratios && c.tis_type == NRL_TIS_TIS) out[P_SEQ_W] = clampf(seq_w, tis_floor, c.tis_max);
-        if (c.sequence_level_importance_ratios && c.tis_type == NRL_TIS_ICEPOP)
-            out[P_SEQ_W] = (seq_w >= c.tis_min && seq_w <= c.tis_max) ? seq_w : 0.f;
-        if (c.tis_type == NRL_TIS_SEQ_MASK) out[P_OOB] = (1.f - seq_keep) * smv;
-        out[P_R_MIN] = mn; out[P_R_MAX] = mx; out[P_RC_MIN] = cmn; out[P_RC_MAX] = cmx;
+    __syncthreads();
+    double t = 0;
+    if (tid < N)
+        for (int i = 0; i < NW; ++i) t += smem[i * N + tid];
+    return t;
+}
+// one value, returned by every thread
+__device__ __forceinline__ double seq_block_sum(double v, double* smem) {
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    v = wave_sum_double(v);
+    __syncthreads();
+    if (lane == 0) smem[w] = v;
+    __syncthreads();
+    double t = 0;
+#pragma unroll
+    for (int i = 0; i < kSeqWaves; ++i) t += smem[i];
+    return t;
+}
+constexpr int kSeqSmem = kSeqWaves * P_R_MIN;
+
+// slot k of a sequence's row of partials, from the sum of its tokens' terms
+__device__ __forceinline__ double row_part(const nrl_grpo_cfg& c, int k, double sum, const SeqStats& st, float smv) {
+    if (!c.token_level_loss && (k == P_ACTOR || k == P_KL))  // sequence-level: masked mean over tokens, then weight by sample_mask
+        return static_cast<double>(static_cast<float>(sum) / st.seq_den) * smv;
+    if (k == P_SAMPLE_MASK) return smv;
+    if (k == P_SEQ_W) {
+        double v = c.tis_type == NRL_TIS_SEQ_MASK ? st.seq_w * st.seq_keep : st.seq_w;
+        if (c.sequence_level_importance_ratios && c.tis_type == NRL_TIS_TIS) v = clampf(st.seq_w, c.tis_min, c.tis_max);
+        if (c.sequence_level_importance_ratios && c.tis_type == NRL_TIS_ICEPOP) v = (st.seq_w >= c.tis_min && st.seq_w <= c.tis_max) ? st.seq_w : 0.f;
+        return v;
     }
+    if (k == P_OOB && c.tis_type == NRL_TIS_SEQ_MASK) return (1.f - st.seq_keep) * smv;
+    return sum;
+}
+
+// Workgroup-wide reduction of one sequence's accumulators (or of a share of them) into a row of partials.
+template <int NW>
+__device__ __forceinline__ void store_parts(double* out, const double (&acc)[P_R_MIN], float r_min, float r_max, float rc_min,
+                                            float rc_max, double* sm_d, float* sm_f) {
+    const int tid = threadIdx.x;
+    const double tot = block_sums<P_R_MIN, NW>(acc, sm_d);
+    const float mn = block_min<NW>(r_min, sm_f), mx = block_max<NW>(r_max, sm_f);
+    const float cmn = block_min<NW>(rc_min, sm_f), cmx = block_max<NW>(rc_max, sm_f);
+    if (tid < P_R_MIN) out[tid] = tot;
+    if (tid == 0) { out[P_R_MIN] = mn; out[P_R_MAX] = mx; out[P_RC_MIN] = cmn; out[P_RC_MAX] = cmx; }
 }
 
 template <bool GSPO>
-__global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
-    __shared__ double sm_d[kLossWaves];
-    __shared__ float sm_f[kLossWaves];
+__global__ __launch_bounds__(kSeqBlock) void grpo_rows_kernel(GrpoArgs a) {
+    __shared__ double sm_d[kSeqSmem];
+    __shared__ float sm_f[kSeqWaves];
     const nrl_grpo_cfg& c = a.cfg;
     const nrl_grpo_inputs& in = a.in;
     const int64_t b = blockIdx.x;
@@ -77,7 +109,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
 
     // ---- row statistics ----
     double s_tm = 0, s_lr = 0, s_is = 0, s_geo = 0;
-    for (int64_t t = tid; t < n; t += kLossBlock) {
+    for (int64_t t = tid; t < n; t += kSeqBlock) {
         const float tm = mask_at(in, b, t);
         const float prev = prev_row[t], gen = gen_row[t];
         s_tm += tm;
@@ -85,14 +117,14 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
         s_is += (prev - gen) * (tm * smv);
         s_geo += finite_or_zero(prev - gen) * tm;
     }
-    const float n_tm = static_cast<float>(block_sum<double, kLossWaves>(s_tm, sm_d));
+    const float n_tm = static_cast<float>(seq_block_sum(s_tm, sm_d));
     const float seq_den = n_tm + 1e-8f;
     float seq_ratio = 1.f, seq_w = 1.f, seq_keep = 1.f;
-    if (GSPO) seq_ratio = expf(static_cast<float>(block_sum<double, kLossWaves>(s_lr, sm_d)) / seq_den);
+    if (GSPO) seq_ratio = expf(static_cast<float>(seq_block_sum(s_lr, sm_d)) / seq_den);
     if (c.sequence_level_importance_ratios)
-        seq_w = finite_or_zero(expf(static_cast<float>(block_sum<double, kLossWaves>(s_is, sm_d))));
+        seq_w = finite_or_zero(expf(static_cast<float>(seq_block_sum(s_is, sm_d))));
     if (c.tis_type == NRL_TIS_SEQ_MASK) {
-        const float geo = expf(static_cast<float>(block_sum<double, kLossWaves>(s_geo, sm_d)) / seq_den);
+        const float geo = expf(static_cast<float>(seq_block_sum(s_geo, sm_d)) / seq_den);
         seq_keep = (geo >= c.tis_min && geo <= c.tis_max) ? 1.f : 0.f;
     }
     double acc[P_R_MIN];
@@ -103,7 +135,7 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
 
     SeqStats st;
     st.seq_den = seq_den; st.seq_ratio = seq_ratio; st.seq_w = seq_w; st.seq_keep = seq_keep;
-    for (int64_t t = tid; t < n; t += kLossBlock) {
+    for (int64_t t = tid; t < n; t += kSeqBlock) {
         TokenIn ti;
         ti.lp = lp_row[t]; ti.lpu = lpu_row[t]; ti.prev = prev_row[t]; ti.gen = gen_row[t];
         ti.ref = c.has_kl ? ref_row[t] : 0.f; ti.adv = adv_row[t]; ti.tm = mask_at(in, b, t); ti.smv = smv; ti.correct = correct;
@@ -130,40 +162,66 @@ __global__ __launch_bounds__(kLossBlock) void grpo_rows_kernel(GrpoArgs a) {
 
     if (GSPO) {
         // d ratio_b / d lp[b, s] = ratio_b * tm[b, s] / (n_tm + 1e-8)
-        const float k_tot = static_cast<float>(block_sum<double, kLossWaves>(gspo_k, sm_d));
-        for (int64_t t = tid; t < n; t += kLossBlock) {
+        const float k_tot = static_cast<float>(seq_block_sum(gspo_k, sm_d));
+        for (int64_t t = tid; t < n; t += kSeqBlock) {
             const float share = k_tot * seq_ratio * (mask_at(in, b, t) / seq_den);
             if (a.dlpu) a.dlp[b * n + t] = share;
             else a.dlp[b * n + t] += share;
         }
     }
 
-    store_row_parts(c, a.parts + b * P_COUNT, acc, r_min, r_max, rc_min, rc_max, st, smv, sm_d, sm_f);
+    double* out = a.parts + b * P_COUNT;
+    store_parts<kSeqWaves>(out, acc, r_min, r_max, rc_min, rc_max, sm_d, sm_f);
+    if (tid < P_R_MIN) out[tid] = row_part(c, tid, out[tid], st, smv);  // each thread what it has just stored
 }
 
-// Fixed-order reduction of the row partials and normalisation into the metrics record.
-__global__ __launch_bounds__(kLossBlock) void grpo_finish_kernel(GrpoArgs a, float* loss_out, float* metrics) {
-    __shared__ double sm_d[kLossWaves];
-    __shared__ float sm_f[kLossWaves];
+// Fixed-order reduction of the row partials and normalisation into the metrics record, by one workgroup of kSeqBlock threads.
+// A wave takes one quantity at a time and sums it over the rows, so the quantities are reduced side by side (one after the
+// other by the whole workgroup took 7 - 10 us, this takes 4 - 7).
+__device__ __forceinline__ void finish_metrics(const GrpoArgs& a, float* loss_out, float* metrics, double* tot /* shared [P_COUNT] */) {
     const nrl_grpo_cfg& c = a.cfg;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int64_t nb = a.in.batch;
-    double tot[P_R_MIN];
-#pragma unroll
-    for (int k = 0; k < P_R_MIN; ++k) tot[k] = 0;
-    float r_min = INFINITY, r_max = -INFINITY, rc_min = INFINITY, rc_max = -INFINITY;
-    for (int64_t b = tid; b < nb; b += kLossBlock) {
-        const double* p = a.parts + b * P_COUNT;
-#pragma unroll
-        for (int k = 0; k < P_R_MIN; ++k) tot[k] += p[k];
-        r_min = fminf(r_min, (float)p[P_R_MIN]); r_max = fmaxf(r_max, (float)p[P_R_MAX]);
-        rc_min = fminf(rc_min, (float)p[P_RC_MIN]); rc_max = fmaxf(rc_max, (float)p[P_RC_MAX]);
+    const int64_t chunks = a.seq_stats ? a.chunks : 1;
+    auto final_part = [&](int k, int64_t b, double sum) {
+        if (!a.seq_stats) return sum;
+        SeqStats st;
+        st.seq_den = a.seq_stats[b * 3]; st.seq_ratio = 1.f; st.seq_w = a.seq_stats[b * 3 + 1]; st.seq_keep = a.seq_stats[b * 3 + 2];
+        return row_part(c, k, sum, st, a.in.sample_mask[b]);
+    };
+    for (int k = tid / kWave; k < P_COUNT; k += kSeqWaves) {
+        if (k < P_R_MIN) {
+            double v = 0;
+            if (chunks <= 8) {  // a lane per sequence
+                for (int64_t b = lane; b < nb; b += kWave) {
+                    double sum = 0;
+                    for (int64_t q = 0; q < chunks; ++q) sum += a.parts[(b * chunks + q) * P_COUNT + k];
+                    v += final_part(k, b, sum);
+                }
+                v = wave_sum_double(v);
+            } else {  // long sequences, so a microbatch holds few of them: the wave over the shares of one after the other
+                for (int64_t b = 0; b < nb; ++b) {
+                    double sum = 0;
+                    for (int64_t q = lane; q < chunks; q += kWave) sum += a.parts[(b * chunks + q) * P_COUNT + k];
+                    v += final_part(k, b, wave_sum_double(sum));
+                }
+            }
+            if (lane == 0) tot[k] = v;
+        } else {
+            const bool low = k == P_R_MIN || k == P_RC_MIN;
+            float v = low ? INFINITY : -INFINITY;
+            for (int64_t b = lane; b < nb * chunks; b += kWave) {
+                const float p = static_cast<float>(a.parts[b * P_COUNT + k]);
+                v = low ? fminf(v, p) : fmaxf(v, p);
+            }
+            v = low ? wave_min(v) : wave_max(v);
+            if (lane == 0) tot[k] = v;
+        }
     }
-#pragma unroll
-    for (int k = 0; k < P_R_MIN; ++k) tot[k] = block_sum<double, kLossWaves>(tot[k], sm_d);
-    r_min = block_min<kLossWaves>(r_min, sm_f); r_max = block_max<kLossWaves>(r_max, sm_f);
-    rc_min = block_min<kLossWaves>(rc_min, sm_f); rc_max = block_max<kLossWaves>(rc_max, sm_f);
+    __syncthreads();
     if (tid != 0) return;
+    const float r_min = static_cast<float>(tot[P_R_MIN]), r_max = static_cast<float>(tot[P_R_MAX]);
+    const float rc_min = static_cast<float>(tot[P_RC_MIN]), rc_max = static_cast<float>(tot[P_RC_MAX]);
 
     const double den_s = valid_seqs(a.in) + 1e-8f, den_t = valid_toks(a.in) + 1e-8f;
     const double den_loss = c.token_level_loss ? den_t : den_s;
@@ -197,6 +255,11 @@ __global__ __launch_bounds__(kLossBlock) void grpo_finish_kernel(GrpoArgs a, flo
     metrics[NRL_M_IS_OOB_RATIO] = static_cast<float>(tot[P_OOB] / (c.tis_type == NRL_TIS_SEQ_MASK ? den_s : den_t));
     metrics[NRL_M_POSITIVE_NLL_LOSS] = nll;
     metrics[NRL_M_N_MASKED_TOKENS] = static_cast<float>(tot[P_N_SELECTED]);
+}
+
+__global__ __launch_bounds__(kSeqBlock) void grpo_finish_kernel(GrpoArgs a, float* loss_out, float* metrics) {
+    __shared__ double tot[P_COUNT];
+    finish_metrics(a, loss_out, metrics, tot);
 }
 
 // positive-example NLL: d loss / d lp += -weight * mask * correct / (n_correct + 1e-8)
@@ -279,7 +342,7 @@ struct FusedArgs {
     float* lp_out;     // [B, n_inner]
     float* seq_stats;  // [B, 3]: seq_den, seq_w, seq_keep
     float* terms;      // [B * n_inner, T_COUNT]
-    double* parts;     // [B, P_COUNT]
+    double* parts;     // [B, chunks, P_COUNT]
     // packed mode (cu != NULL): the logits are one row of `total` positions, sequence s occupies
     // [cu[s], cu[s+1]); the loss inputs stay [n_seq, n_inner]
     const int32_t* cu;
@@ -308,14 +371,6 @@ __device__ __forceinline__ FusedPos fused_where_packed(const FusedArgs& a, int64
     }
     return q;
 }
-// The search through the boundaries is a chain of dependent loads; done once per row ahead of the pass,
-// the persistent kernel finds a row's place with a single load.
-__global__ __launch_bounds__(256) void fused_row_pos_kernel(FusedArgs a, int64_t total) {
-    const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (r >= total) return;
-    const FusedPos q = fused_where_packed(a, r, total);
-    a.row_pos[r] = make_int4(static_cast<int>(q.o), static_cast<int>(q.i), static_cast<int>(q.tgt), 0);
-}
 template <bool PACKED>
 __device__ __forceinline__ FusedPos fused_where(const FusedArgs& a, int64_t r) {
     FusedPos q;
@@ -338,15 +393,30 @@ __device__ __forceinline__ int64_t fused_row_offset(const FusedArgs& a, int64_t 
     return o * so + (r - o * a.d_n_inner) * si;
 }
 
-__global__ __launch_bounds__(kLossBlock) void grpo_seq_stats_kernel(FusedArgs a) {
-    __shared__ double sm_d[kLossWaves];
+// Everything the pass needs beforehand, in one launch.  The first `batch` workgroups compute the per-sequence statistics.
+// Packed mode has more of them, which zero the records and logprobs (positions past a sequence's end have no packed row) and
+// find every row's place: the search through the boundaries is a chain of dependent loads, done once per row here so that the
+// persistent kernel finds it with one load.  (7 packed sequences, 16384 tokens: 8 us, four launches of 33 us before.)
+__global__ __launch_bounds__(kSeqBlock) void fused_prep_kernel(FusedArgs a, int64_t total) {
+    __shared__ double sm_d[kSeqWaves];
     const nrl_grpo_cfg& c = a.cfg;
     const nrl_grpo_inputs& in = a.in;
     const int64_t b = blockIdx.x, n = in.sm1;
+    if (b >= in.batch) {
+        const int64_t first = (b - in.batch) * kSeqBlock + threadIdx.x, step = (gridDim.x - in.batch) * kSeqBlock;
+        for (int64_t i = first; i < in.batch * n; i += step) a.lp_out[i] = 0.f;
+        float2* rec = reinterpret_cast<float2*>(a.terms);  // 8-byte aligned, an even number of floats
+        for (int64_t i = first; i < in.batch * n * (T_COUNT / 2); i += step) rec[i] = make_float2(0.f, 0.f);
+        for (int64_t r = first; r < total; r += step) {
+            const FusedPos q = fused_where_packed(a, r, total);
+            a.row_pos[r] = make_int4(static_cast<int>(q.o), static_cast<int>(q.i), static_cast<int>(q.tgt), 0);
+        }
+        return;
+    }
     const float smv = in.sample_mask[b];
     double s_tm = 0, s_is = 0, s_geo = 0;
     const bool need_prev = c.sequence_level_importance_ratios || c.tis_type == NRL_TIS_SEQ_MASK;
-    for (int64_t t = threadIdx.x; t < n; t += kLossBlock) {
+    for (int64_t t = threadIdx.x; t < n; t += kSeqBlock) {
         const float tm = mask_at(in, b, t);
         s_tm += tm;
         if (need_prev) {
@@ -355,11 +425,11 @@ __global__ __launch_bounds__(kLossBlock) void grpo_seq_stats_kernel(FusedArgs a)
             s_geo += finite_or_zero(d) * tm;
         }
     }
-    const float seq_den = static_cast<float>(block_sum<double, kLossWaves>(s_tm, sm_d)) + 1e-8f;
+    const float seq_den = static_cast<float>(seq_block_sum(s_tm, sm_d)) + 1e-8f;
     float seq_w = 1.f, seq_keep = 1.f;
-    if (c.sequence_level_importance_ratios) seq_w = finite_or_zero(expf(static_cast<float>(block_sum<double, kLossWaves>(s_is, sm_d))));
+    if (c.sequence_level_importance_ratios) seq_w = finite_or_zero(expf(static_cast<float>(seq_block_sum(s_is, sm_d))));
     if (c.tis_type == NRL_TIS_SEQ_MASK) {
-        const float geo = expf(static_cast<float>(block_sum<double, kLossWaves>(s_geo, sm_d)) / seq_den);
+        const float geo = expf(static_cast<float>(seq_block_sum(s_geo, sm_d)) / seq_den);
         seq_keep = (geo >= c.tis_min && geo <= c.tis_max) ? 1.f : 0.f;
     }
     if (threadIdx.x == 0) {
@@ -378,11 +448,6 @@ __global__ __launch_bounds__(kLossBlock) void grpo_seq_stats_kernel(FusedArgs a)
 // register slots (vector q - kFusedLdsVec).
 // NREG is the number of register slots the instantiation carries (the row must fit NREG + kFusedLdsVec
 // slots); shorter rows take a smaller instantiation instead of idling through unused slots.
-__global__ void fused_fill_zero_kernel(float* p, int64_t n) {
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-        p[i] = 0.f;
-}
-
 template <int DT, int TEMP, int NREG, bool PACKED>
 __global__ __launch_bounds__(kFusedBlock) void fused_logits_loss_kernel(FusedArgs a, int64_t n_rows) {
     constexpr int EPV = Row<DT>::EPV;
@@ -556,47 +621,32 @@ __global__ __launch_bounds__(kFusedBlock) void fused_logits_loss_kernel(FusedArg
     }
 }
 
-// one workgroup per sequence: token term records -> the sequence's row of partials.  Thread t sums the records of
-// tokens t, t + 256, ... in that order (the assignment of the three-pass kernel, so both give the same sums); a
-// record is read as ten 8-byte pairs, four records in flight per thread (eight measured slower).
-__global__ __launch_bounds__(kLossBlock) void grpo_terms_reduce_kernel(FusedArgs a) {
-    __shared__ double sm_d[kLossWaves];
-    __shared__ float sm_f[kLossWaves];
+// Token term records -> sums over shares of kTermsBlock tokens, one workgroup each: a record per thread, read as ten 8-byte
+// pairs.  A sequence in one workgroup reads its records at what one compute unit gets, 23 us for 7 packed sequences (16384
+// tokens); spread out 6 us, 4 sequences of 1024 tokens 9.6 -> 5.7 us.  The shares are added up, in order, by the
+// launch that finishes the metrics: done here by the workgroup that arrives last, the device-scope fence in front of its
+// arrival waits for the L2 to write back what the pass left there, 13 - 25 us.
+constexpr int kTermsBlock = 256, kTermsWaves = kTermsBlock / kWave;
+__global__ __launch_bounds__(kTermsBlock) void grpo_terms_reduce_kernel(FusedArgs a, int64_t chunks) {
+    __shared__ double sm_d[kTermsWaves * P_R_MIN];
+    __shared__ float sm_f[kTermsWaves];
     static_assert(T_COUNT % 2 == 0, "records are read as 8-byte pairs");
-    constexpr int kPairs = T_COUNT / 2, kAhead = 4;
-    const int64_t b = blockIdx.x, n = a.n_inner;
+    constexpr int kPairs = T_COUNT / 2;
+    const int64_t b = blockIdx.x / chunks, q = blockIdx.x - b * chunks, t = q * kTermsBlock + threadIdx.x;
     double acc[P_R_MIN];
 #pragma unroll
     for (int k = 0; k < P_R_MIN; ++k) acc[k] = 0;
     float r_min = INFINITY, r_max = -INFINITY, rc_min = INFINITY, rc_max = -INFINITY;
-    for (int64_t t0 = threadIdx.x; t0 < n; t0 += kAhead * kLossBlock) {
-        float2 v[kAhead][kPairs];
+    if (t < a.n_inner) {
+        float rec[T_COUNT];
+        const float2* p = reinterpret_cast<const float2*>(a.terms + (b * a.n_inner + t) * T_COUNT);  // 8-byte aligned: T_COUNT is even
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const int64_t t = t0 + u * kLossBlock;
-            if (t < n) {
-                const float2* rec = reinterpret_cast<const float2*>(a.terms + (b * n + t) * T_COUNT);  // 8-byte aligned: T_COUNT is even
+        for (int k = 0; k < kPairs; ++k) { const float2 v = p[k]; rec[2 * k] = v.x; rec[2 * k + 1] = v.y; }
 #pragma unroll
-                for (int k = 0; k < kPairs; ++k) v[u][k] = rec[k];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            if (t0 + u * kLossBlock >= n) break;
-            float rec[T_COUNT];
-#pragma unroll
-            for (int k = 0; k < kPairs; ++k) { rec[2 * k] = v[u][k].x; rec[2 * k + 1] = v[u][k].y; }
-#pragma unroll
-            for (int k = 0; k < P_SAMPLE_MASK; ++k) acc[k] += rec[k];
-            if (rec[T_SELECTED] != 0.f) {
-                r_min = fminf(r_min, rec[T_RATIO]); r_max = fmaxf(r_max, rec[T_RATIO]);
-                rc_min = fminf(rc_min, rec[T_RATIO_CL]); rc_max = fmaxf(rc_max, rec[T_RATIO_CL]);
-            }
-        }
+        for (int k = 0; k < P_SAMPLE_MASK; ++k) acc[k] = rec[k];
+        if (rec[T_SELECTED] != 0.f) { r_min = r_max = rec[T_RATIO]; rc_min = rc_max = rec[T_RATIO_CL]; }
     }
-    SeqStats st;
-    st.seq_den = a.seq_stats[b * 3]; st.seq_ratio = 1.f; st.seq_w = a.seq_stats[b * 3 + 1]; st.seq_keep = a.seq_stats[b * 3 + 2];
-    store_row_parts(a.cfg, a.parts + b * P_COUNT, acc, r_min, r_max, rc_min, rc_max, st, a.in.sample_mask[b], sm_d, sm_f);
+    store_parts<kTermsWaves>(a.parts + blockIdx.x * static_cast<int64_t>(P_COUNT), acc, r_min, r_max, rc_min, rc_max, sm_d, sm_f);
 }
 
 static int check_inputs(const nrl_grpo_inputs* in, bool need_prev, bool need_ref, bool need_adv) {
@@ -630,13 +680,14 @@ static int grpo_loss_impl(const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, fl
     a.dlp = dlp_out;
     a.dlpu = split ? dlpu_out : nullptr;
     a.parts = parts;
+    a.seq_stats = nullptr; a.chunks = 1;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (in->batch > 0) {
         const bool gspo = cfg->sequence_level_importance_ratios && !cfg->disable_ppo_ratio && !cfg->force_on_policy_ratio;
-        if (gspo) grpo_rows_kernel<true><<<dim3((unsigned)in->batch), dim3(kLossBlock), 0, s>>>(a);
-        else grpo_rows_kernel<false><<<dim3((unsigned)in->batch), dim3(kLossBlock), 0, s>>>(a);
+        if (gspo) grpo_rows_kernel<true><<<dim3((unsigned)in->batch), dim3(kSeqBlock), 0, s>>>(a);
+        else grpo_rows_kernel<false><<<dim3((unsigned)in->batch), dim3(kSeqBlock), 0, s>>>(a);
     }
-    grpo_finish_kernel<<<dim3(1), dim3(kLossBlock), 0, s>>>(a, loss_out, metrics_out);
+    grpo_finish_kernel<<<dim3(1), dim3(kSeqBlock), 0, s>>>(a, loss_out, metrics_out);
     if (cfg->has_nll && in->batch * in->sm1 > 0) {
         const int64_t total = in->batch * in->sm1;
         const unsigned blocks = (unsigned)((total + 255) / 256 > 1024 ? 1024 : (total + 255) / 256);
@@ -941,9 +992,11 @@ extern "C" int nrl_mask_neg_inf_bwd(const float* grad_out, const uint8_t* keep, 
 
 static int64_t align8(int64_t v) { return (v + 7) / 8 * 8; }
 
+static int64_t terms_chunks(int64_t n) { return n < 1 ? 1 : (n + kTermsBlock - 1) / kTermsBlock; }
+
 extern "C" int64_t nrl_fused_workspace_bytes(int64_t batch, int64_t n_inner) {
     const int64_t b = batch < 1 ? 1 : batch, n = n_inner < 1 ? 1 : n_inner;
-    return align8(b * 3 * 4) + align8(b * n * T_COUNT * 4) + b * P_COUNT * 8;
+    return align8(b * 3 * 4) + align8(b * n * T_COUNT * 4) + b * terms_chunks(n) * P_COUNT * 8;
 }
 
 extern "C" int64_t nrl_fused_packed_workspace_bytes(int64_t n_seq, int64_t n_inner, int64_t total) {
@@ -983,6 +1036,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
         return fail(NRL_E_UNSUPPORTED, "rows must be 16-byte aligned");
     const int64_t n_rows = rows->n_outer * d_n_inner;
     if (n_rows >= (1ll << 31)) return fail(NRL_E_INVALID, "more than 2^31 rows in one launch");
+    if (in->batch * terms_chunks(in->sm1) >= (1ll << 31)) return fail(NRL_E_INVALID, "more than 2^31 shares of sequences");
     if (!loss_out || !metrics_out || !workspace) return fail(NRL_E_INVALID, "null output or workspace");
     const int64_t need = cu ? nrl_fused_packed_workspace_bytes(in->batch, in->sm1, n_rows) : nrl_fused_workspace_bytes(in->batch, in->sm1);
     if (workspace_bytes < need) return fail(NRL_E_WORKSPACE, "workspace too small");
@@ -1008,7 +1062,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     char* ws = static_cast<char*>(workspace);
     a.seq_stats = reinterpret_cast<float*>(ws); ws += align8(in->batch * 3 * 4);
     a.terms = reinterpret_cast<float*>(ws); ws += align8(in->batch * (in->sm1 < 1 ? 1 : in->sm1) * T_COUNT * 4);
-    a.parts = reinterpret_cast<double*>(ws); ws += in->batch * P_COUNT * 8;
+    a.parts = reinterpret_cast<double*>(ws); ws += in->batch * terms_chunks(in->sm1) * P_COUNT * 8;
     a.row_pos = cu ? reinterpret_cast<int4*>(ws + ((16 - (reinterpret_cast<uintptr_t>(ws) & 15)) & 15)) : nullptr;
     int tc = 0;
     a.tparam = 1.f;
@@ -1018,13 +1072,9 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     const unsigned nb = static_cast<unsigned>(in->batch);
-    if (nb > 0) grpo_seq_stats_kernel<<<dim3(nb), dim3(kLossBlock), 0, s>>>(a);
-    if (cu && in->batch * in->sm1 > 0) {
-        // positions past a sequence's end have no packed row: their records and logprobs start at zero
-        fused_fill_zero_kernel<<<dim3(1024), dim3(256), 0, s>>>(a.terms, in->batch * in->sm1 * T_COUNT);
-        fused_fill_zero_kernel<<<dim3(256), dim3(256), 0, s>>>(a.lp_out, in->batch * in->sm1);
-    }
-    if (cu && n_rows > 0) fused_row_pos_kernel<<<dim3((unsigned)((n_rows + 255) / 256)), dim3(256), 0, s>>>(a, n_rows);
+    const int64_t fill = cu ? (n_rows > in->batch * in->sm1 * 4 ? n_rows : in->batch * in->sm1 * 4) : 0;
+    const unsigned more = static_cast<unsigned>(fill + kSeqBlock - 1 < 256ll * kSeqBlock ? (fill + kSeqBlock - 1) / kSeqBlock : 256);
+    if (nb + more > 0) fused_prep_kernel<<<dim3(nb + more), dim3(kSeqBlock), 0, s>>>(a, n_rows);
     if (n_rows > 0) {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
@@ -1052,13 +1102,14 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
 #undef NRL_FUSED_CASE
 #undef NRL_FUSED_LAUNCH
     }
-    if (nb > 0) grpo_terms_reduce_kernel<<<dim3(nb), dim3(kLossBlock), 0, s>>>(a);
     GrpoArgs fa;
     fa.cfg = *cfg;
     fa.in = *in;
     fa.dlp = nullptr; fa.dlpu = nullptr;
     fa.parts = a.parts;
-    grpo_finish_kernel<<<dim3(1), dim3(kLossBlock), 0, s>>>(fa, loss_out, metrics_out);
+    fa.seq_stats = a.seq_stats; fa.chunks = terms_chunks(in->sm1);
+    if (nb > 0) grpo_terms_reduce_kernel<<<dim3((unsigned)(nb * fa.chunks)), dim3(kTermsBlock), 0, s>>>(a, fa.chunks);
+    grpo_finish_kernel<<<dim3(1), dim3(kSeqBlock), 0, s>>>(fa, loss_out, metrics_out);
     return check_launch("fused_logits_grpo_loss");
 }
 

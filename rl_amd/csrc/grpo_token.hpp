@@ -21,7 +21,9 @@ struct GrpoArgs {
     nrl_grpo_inputs in;
     float* dlp;
     float* dlpu;
-    double* parts;  // [B, P_COUNT]
+    double* parts;  // [B, P_COUNT], or [B, chunks, P_COUNT] of sums over shares of a sequence with seq_stats
+    const float* seq_stats;  // [B, 3] (seq_den, seq_w, seq_keep) or NULL: the rows of parts are final
+    int64_t chunks;
 };
 
 // token t of sequence b in the mask's own element type (the branch is uniform over the launch)

@@ -426,3 +426,28 @@ def test_the_worker_loop_does_not_wait_for_the_device_between_loss_and_backward(
                 continue
             want = eager[k] if ("_min" in k or "_max" in k) else eager[k] / num_global_batches
             assert type(v) in (float, int) and v == want, (k, v, want)
+
+
+@pytest.mark.parametrize("cfg", [FUSABLE[0], FUSABLE[3], FUSABLE[9], FUSABLE[10]], ids=["token", "sequence", "seq-mask", "seq-weights"])
+@pytest.mark.parametrize("b,s", [(1, 2), (3, 256), (2, 257), (70, 258), (2, 2049), (3, 2050), (1, 20001)])
+def test_metrics_over_shares_of_a_sequence(cfg, b, s):
+    """Sequences are summed in shares of 256 tokens, up to 8 of them by a lane each, more by a wave: edges of both, against the
+    three-pass path (all sums are in double there and here; logprobs differ by the order of fp32 sums: 1e-4 as above)."""
+    g = torch.Generator(device=DEV).manual_seed(s)
+    logits = torch.randn(b, s, 64, generator=g, device=DEV)
+    ids = torch.randint(0, 64, (b, s), generator=g, device=DEV)
+    tm = (torch.rand(b, s, generator=g, device=DEV) < 0.8).float()
+    tm[:, -1] = 1
+    data = {"input_ids": ids, "token_mask": tm, "sample_mask": torch.ones(b, device=DEV),
+            "advantages": torch.randn(b, 1, generator=g, device=DEV).expand(b, s).contiguous()}
+    cur = torch.log_softmax(logits, -1)[:, :-1].gather(-1, ids[:, 1:, None]).squeeze(-1)
+    for k in ("prev_logprobs", "generation_logprobs", "reference_policy_logprobs"):
+        data[k] = torch.cat([torch.zeros(b, 1, device=DEV), cur + 0.02 * torch.randn(b, s - 1, generator=g, device=DEV)], 1)
+    gs, gt = data["sample_mask"].sum(), tm[:, 1:].sum()
+    fn = ClippedPGLossFn(ClippedPGLossConfig(**cfg))
+    got, gm = fused_logits_clipped_pg_loss(logits.clone().requires_grad_(True), data, fn, gs, gt)
+    loss_input, d2 = prepare_loss_input(logits.clone().requires_grad_(True), dict(data), fn)
+    want, wm = fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)
+    assert _close(got.item(), want.item(), rel=1e-4, abs_=1e-6)
+    for k in wm:
+        assert _close(float(gm[k]), float(wm[k])), (k, gm[k], wm[k])
