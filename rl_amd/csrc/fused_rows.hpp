@@ -1,0 +1,259 @@
+// The single pass over logits rows: log-sum-exp -> token logprob -> d loss / d logprob -> dlogits, with the row held on chip
+// (registers plus an LDS slice) between the reduction and the gradient, so the logits are read once and the gradient written
+// once (2 * V * sizeof(logit) per token instead of 3).  Valid when d loss / d logprob of a token depends only on that token
+// and on per-sequence quantities that do not involve the current logprobs: everything except sequence-level probability
+// ratios (GSPO) and the positive-example NLL term.  Tokens whose mask is zero are not evaluated: their gradient row is
+// zero-filled without reading the logits and their logprob is reported as 0.
+#pragma once
+
+#include <float.h>
+
+#include "grpo_token.hpp"
+
+namespace nrl {
+
+constexpr int kFusedMaxRegVec = 16;  // at most 16 16-byte vectors per lane held in registers ...
+constexpr int kFusedLdsVec = 4;      // ... and 4 in LDS
+constexpr int kFusedMaxVec = kFusedMaxRegVec + kFusedLdsVec;
+
+// What the pass needs to know about a row, 64 bytes written by fused_prep_kernel: a wave reads it with one load, a word per
+// lane, a row ahead of its use.
+enum { R_LIVE = 0, R_PREV, R_GEN, R_REF, R_ADV, R_TM, R_SMV, R_XT, R_TLOC, R_SEQ, R_POS, R_WORDS = 16 };
+
+struct FusedArgs {
+    nrl_grpo_cfg cfg;
+    nrl_grpo_inputs in;  // lp / lpu unused
+    const void* logits;
+    int64_t n_inner, d_n_inner, vocab, stride_outer, stride_inner;
+    const int64_t* targets;
+    int64_t ts_outer, ts_inner, vstart, vend;
+    float tparam, loss_scale;
+    void* dlogits;
+    int64_t ds_outer, ds_inner;
+    float* lp_out;     // [B, n_inner]
+    float* seq_stats;  // [B, 3]: seq_den, seq_w, seq_keep
+    uint32_t* rec;     // [B * n_inner, R_WORDS]; packed: [rows, R_WORDS]
+    double* parts;     // [B, chunks, P_COUNT]
+    // packed mode (cu != NULL): the logits are one row of `total` positions, sequence s occupies
+    // [cu[s], cu[s+1]); the loss inputs stay [n_seq, n_inner]
+    const int32_t* cu;
+    int64_t n_seq;
+    int pre_rolled;
+};
+
+struct FusedLaunch {
+    FusedArgs a;
+    int temp;  // 0, 1 (divide), 2 (multiply)
+    bool packed;
+    int64_t n_rows;
+    int compute_units;
+    hipStream_t stream;
+};
+void launch_fused_f32(const FusedLaunch& l);
+void launch_fused_bf16(const FusedLaunch& l);
+void launch_fused_f16(const FusedLaunch& l);
+
+template <bool PACKED>
+__device__ __forceinline__ int64_t fused_row_offset(const FusedArgs& a, int64_t r, int64_t so, int64_t si) {
+    if (PACKED) return r * si;
+    const int64_t o = r / a.d_n_inner;
+    return o * so + (r - o * a.d_n_inner) * si;
+}
+
+// 16 bytes per lane from base + offset (uniform base, `bytes` behind it) to consecutive LDS addresses from dst (uniform) on
+__device__ __forceinline__ void load_to_lds(const char* base, int bytes, int offset, u32x4* dst) {
+#ifdef __HIP_DEVICE_COMPILE__  // the resource type does not exist for the host pass
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)dst, 16, offset, 0, 0, 0);
+#endif
+}
+
+// Persistent workgroups: workgroup w walks rows w, w + gridDim.x, ...  A row's gradient goes out as one burst of stores, and
+// behind it the loads of the next row this workgroup evaluates (registers by ordinary loads, the LDS slice by direct
+// global-to-LDS loads), whose online (max, sum) is advanced as they arrive.  The pass is bound by HBM, and HBM serves long
+// runs of reads and of writes better than the two mixed: with every slot refilled right behind its store, 8 x 4096 rows
+// of V = 151936 bf16 took 3.65 ms, in runs 3.49 ms (18.4 GB, 5.26 TB/s), although the former overlaps more.
+// What lies between two rows is kept short: the row's inputs come in one load a row ahead, every wave evaluates the token
+// by itself (no broadcast, no second barrier), and only what the gradient needs is evaluated; the terms of the metrics
+// follow in the reduction behind the pass (4 x 1024 rows: 538 -> 520 us for the whole call).
+// Slot order q = 0 .. kVec-1: the LDS slots come first (vector NREG + q), then the register slots (vector q - kFusedLdsVec).
+// NREG is the number of register slots the instantiation carries (the row must fit NREG + kFusedLdsVec
+// slots); shorter rows take a smaller instantiation instead of idling through unused slots, and smaller workgroups of which
+// several share a compute unit, so that one's stretch between rows is covered by the others' memory operations.
+template <int DT, int TEMP, int BLOCK, int NREG, bool PACKED>
+__global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a, int64_t n_rows) {
+    constexpr int EPV = Row<DT>::EPV;
+    constexpr int NLDS = kFusedLdsVec, kVec = NREG + NLDS;
+    constexpr int kWavesPerBlock = BLOCK / kWave;
+    __shared__ u32x4 stash[NLDS * BLOCK];
+    __shared__ Lse sm_l[kWavesPerBlock];
+    const nrl_grpo_cfg& c = a.cfg;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int nvec = static_cast<int>(a.vocab / EPV);
+    const int64_t step = gridDim.x;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+
+    auto out_row = [&](int64_t r) -> char* {
+        return static_cast<char*>(a.dlogits) + fused_row_offset<PACKED>(a, r, a.ds_outer, a.ds_inner) * Row<DT>::BYTES;
+    };
+    auto in_row = [&](int64_t r) -> const char* {
+        return static_cast<const char*>(a.logits) + fused_row_offset<PACKED>(a, r, a.stride_outer, a.stride_inner) * Row<DT>::BYTES;
+    };
+    // Slot q holds vector slot_vec(q) of the row.  Lanes past the end of the row are pointed at the
+    // row's last vector instead: they load, compute and store exactly what that vector's own lane does
+    // (harmless duplicates), so there is no divergent branch around the memory operations and they stay in flight
+    // together.
+    auto slot_vec = [&](int q) -> int { return tid + (q < NLDS ? NREG + q : q - NLDS) * BLOCK; };
+    // (recomputed at every use from an opaque copy of the lane index: twenty precomputed offsets would
+    // not fit in the register file next to the row)
+    auto slot_cl = [&](int q) -> int {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        return min(t + (q < NLDS ? NREG + q : q - NLDS) * BLOCK, nvec - 1);
+    };
+    auto vec_at = [&](const char* base, int vc) -> const u32x4* {  // uniform base + 32-bit lane offset
+        return reinterpret_cast<const u32x4*>(base + static_cast<uint32_t>(vc) * 16u);
+    };
+    auto load_rec = [&](int64_t r) -> uint32_t {
+        if (r >= n_rows) return 0u;
+        if (!PACKED) {  // a record per token: rows behind a sequence's last token have none
+            const int64_t o = r / a.d_n_inner, i = r - o * a.d_n_inner;
+            if (i >= a.n_inner) return 0u;
+            r = o * a.n_inner + i;
+        }
+        return a.rec[r * R_WORDS + (lane & (R_WORDS - 1))];
+    };
+    auto word = [&](uint32_t rec, int k) -> uint32_t { return __builtin_amdgcn_readlane(static_cast<int>(rec), k); };
+    // First row at or after r (in this workgroup's walk) whose token takes part in the loss, with its record; rec is row
+    // r's on entry.  Rows passed over are dropped positions or masked tokens: zero gradient, nothing read.
+    auto advance = [&](int64_t r, uint32_t& rec) -> int64_t {
+        while (r < n_rows && word(rec, R_LIVE) == 0u) {
+            u32x4* ov = reinterpret_cast<u32x4*>(out_row(r));
+            rec = load_rec(r + step);
+            for (int v = tid; v < nvec; v += BLOCK) ov[v] = zero;
+            r += step;
+        }
+        return r;
+    };
+    auto load_stats = [&](uint32_t rec) -> float { return a.seq_stats[static_cast<int64_t>(word(rec, R_SEQ)) * 3 + (lane < 3 ? lane : 0)]; };
+    u32x4 regs[NREG];
+    Lse acc;
+    // LDS slot q of the incoming row: global memory -> LDS without passing through registers; each wave
+    // fills the 1 KiB of the slot that its own lanes read back.  (Buffer loads: the compiler counts them like any other
+    // memory operation.  global_load_lds it takes for an access that may complete out of order, after which the wait for the
+    // first register load is a wait for everything in flight.)
+    auto lds_fill = [&](const char* base, int q) {
+        u32x4* dst = stash + q * BLOCK + (tid & ~(kWave - 1));
+        load_to_lds(base, nvec * 16, slot_cl(q) * 16, dst);
+    };
+    auto fold = [&](int q) {  // slot q of the incoming row -> running sum; lanes past the row add nothing
+        u32x4 raw = q < NLDS ? stash[(q < NLDS ? q : 0) * BLOCK + tid] : regs[q < NLDS ? 0 : q - NLDS];
+        if (slot_vec(q) >= nvec) raw = u32x4{Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD};
+        float t[EPV];
+        Row<DT>::decode(raw, t);
+#pragma unroll
+        for (int k = 0; k < EPV; ++k) t[k] = scale_logit<DT, TEMP>(t[k], a.tparam);
+        lse_push<EPV>(acc, t);
+    };
+    // the direct-to-LDS loads are not tracked against later LDS reads by the compiler: wait for them
+    // (and everything older) by hand before the first read of a refilled LDS slot
+    auto wait_lds_fill = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+
+    auto load_row = [&](const char* base) {  // the row onto the chip, and its (max, sum)
+#pragma unroll
+        for (int q = 0; q < NLDS; ++q) lds_fill(base, q);
+#pragma unroll
+        for (int q = NLDS; q < kVec; ++q) regs[q - NLDS] = __builtin_nontemporal_load(vec_at(base, slot_cl(q)));
+        __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first is waited for
+        acc.m = -FLT_MAX;
+        acc.s = 0.f;
+#pragma unroll
+        for (int q = NLDS; q < kVec; ++q) fold(q);
+        wait_lds_fill();
+#pragma unroll
+        for (int q = 0; q < NLDS; ++q) fold(q);
+    };
+
+    uint32_t rec = load_rec(blockIdx.x);
+    int64_t r = advance(blockIdx.x, rec);
+    float stats = 0.f;
+    uint32_t ahead = 0u;  // record of row r + step
+    if (r < n_rows) {
+        stats = load_stats(rec);
+        ahead = load_rec(r + step);
+        load_row(in_row(r));
+    }
+    while (r < n_rows) {
+        char* ov = out_row(r);
+        const Lse tot = block_lse<kWavesPerBlock>(acc, sm_l);
+        const int tloc = static_cast<int>(word(rec, R_TLOC));
+        const float log_s = logf(tot.s), lse = tot.m + log_s;
+        float g;
+        {
+            auto in = [&](int k) { return __uint_as_float(word(rec, k)); };
+            auto stat = [&](int k) { return __uint_as_float(word(__float_as_uint(stats), k)); };
+            const float lp = tloc >= 0 ? (in(R_XT) - tot.m) - log_s : 0.f;
+            SeqStats st;
+            st.seq_den = stat(0); st.seq_ratio = 1.f; st.seq_w = stat(1); st.seq_keep = stat(2);
+            TokenIn ti;
+            ti.lp = lp; ti.lpu = lp;
+            ti.prev = c.force_on_policy_ratio ? lp : in(R_PREV);
+            ti.gen = in(R_GEN); ti.ref = in(R_REF); ti.adv = in(R_ADV); ti.tm = in(R_TM); ti.smv = in(R_SMV);
+            ti.correct = 0.f;
+            ti.den_s = valid_seqs(a.in) + 1e-8f;
+            ti.den_t = valid_toks(a.in) + 1e-8f;
+            const TokenOut out = token_eval<false>(c, st, ti);
+            g = (out.d_actor + out.d_lpu) * a.loss_scale;
+            if (tid == 0) a.lp_out[static_cast<int64_t>(word(rec, R_SEQ)) * a.n_inner + word(rec, R_POS)] = lp;
+        }
+        uint32_t rec_n = ahead;
+        const int64_t rn = advance(r + step, rec_n);
+        const float stats_n = load_stats(rn < n_rows ? rec_n : rec);
+        ahead = load_rec(rn + step);
+        const int tvec = tloc >= 0 ? tloc / EPV : -1;
+        const int tsub = tloc >= 0 ? tloc % EPV : -1;
+        const RowGrad rg(lse, g, a.tparam);
+#pragma unroll
+        for (int q = 0; q < kVec; ++q) {
+            const int vc = slot_cl(q);
+            const u32x4 raw = q < NLDS ? stash[(q < NLDS ? q : 0) * BLOCK + tid] : regs[q < NLDS ? 0 : q - NLDS];
+            const u32x4 d = grad_vec<DT, TEMP>(raw, vc == tvec ? tsub : -1, rg);
+            __builtin_nontemporal_store(d, const_cast<u32x4*>(vec_at(ov, vc)));
+        }
+        __builtin_amdgcn_sched_barrier(0);  // the stores stay together, and ahead of the loads
+        if (rn < n_rows) load_row(in_row(rn));
+        // sm_l is rewritten only behind the first barrier of the next block_lse, which every thread passes after reading it
+        r = rn;
+        rec = rec_n;
+        stats = stats_n;
+    }
+}
+
+template <int DT, int TEMP, int BLOCK, int NREG> void fused_launch(const FusedLaunch& l) {
+    // as many workgroups as are resident together: 1024 threads per compute unit at 128 registers, 64 KiB of LDS
+    const int64_t resident = static_cast<int64_t>(l.compute_units) * (1024 / BLOCK);
+    const dim3 grid(static_cast<unsigned>(l.n_rows < resident ? l.n_rows : resident)), block(BLOCK);
+    if (l.packed) fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, true><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
+    else fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, false><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
+}
+template <int DT, int TEMP, int BLOCK> void fused_launch(const FusedLaunch& l, int64_t slots) {
+    if (slots <= 12) fused_launch<DT, TEMP, BLOCK, 8>(l);
+    else if (slots <= 16) fused_launch<DT, TEMP, BLOCK, 12>(l);
+    else fused_launch<DT, TEMP, BLOCK, 16>(l);
+}
+template <int DT, int TEMP> void fused_launch(const FusedLaunch& l) {
+    const int64_t nvec = l.a.vocab / Row<DT>::EPV;
+    auto slots = [&](int block) { return (nvec + block - 1) / block; };
+    // the smallest workgroup that holds the row
+    if (slots(256) <= 8) fused_launch<DT, TEMP, 256, 4>(l);
+    else if (slots(256) <= kFusedMaxVec) fused_launch<DT, TEMP, 256>(l, slots(256));
+    else if (slots(512) <= kFusedMaxVec) fused_launch<DT, TEMP, 512>(l, slots(512));
+    else fused_launch<DT, TEMP, 1024>(l, slots(1024));
+}
+template <int DT> void fused_launch(const FusedLaunch& l) {
+    if (l.temp == 0) fused_launch<DT, 0>(l);
+    else if (l.temp == 1) fused_launch<DT, 1>(l);
+    else fused_launch<DT, 2>(l);
+}
+
+}  // namespace nrl

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "common.hpp"
+#include "fused_rows.hpp"
 #include "grpo_token.hpp"
 
 namespace nrl {
@@ -312,45 +313,8 @@ __global__ __launch_bounds__(kLossBlock) void nll_finish_kernel(nrl_grpo_inputs 
 }
 
 // ---------------------------------------------------------------------------------------------
-// Fused pass: logits row -> log-sum-exp -> token logprob -> loss terms and d loss / d logprob ->
-// dlogits, with the row held on chip (registers plus an LDS slice) between the reduction and the
-// gradient, so the logits are read once and the gradient written once (2 * V * sizeof(logit) per
-// token instead of 3).  Valid when d loss / d logprob of a token depends only on that token and on
-// per-sequence quantities that do not involve the current logprobs: everything except sequence-level
-// probability ratios (GSPO) and the positive-example NLL term.  Tokens whose mask is zero are not
-// evaluated: their gradient row is zero-filled without reading the logits and their logprob is
-// reported as 0.
+// The single pass (fused_rows.hpp): what runs ahead of it and behind it.
 // ---------------------------------------------------------------------------------------------
-constexpr int kFusedBlock = 1024;
-constexpr int kFusedWaves = kFusedBlock / kWave;
-constexpr int kFusedMaxRegVec = 16;  // at most 16 16-byte vectors per lane held in registers ...
-constexpr int kFusedLdsVec = 4;      // ... and 4 in LDS (64 KiB per workgroup)
-constexpr int kFusedMaxVec = kFusedMaxRegVec + kFusedLdsVec;
-constexpr int T_RATIO = P_SAMPLE_MASK, T_RATIO_CL = P_SAMPLE_MASK + 1, T_SELECTED = P_SAMPLE_MASK + 2, T_COUNT = 20;
-static_assert(P_SAMPLE_MASK + 3 <= T_COUNT, "token term record too small");
-
-struct FusedArgs {
-    nrl_grpo_cfg cfg;
-    nrl_grpo_inputs in;  // lp / lpu unused
-    const void* logits;
-    int64_t n_inner, d_n_inner, vocab, stride_outer, stride_inner;
-    const int64_t* targets;
-    int64_t ts_outer, ts_inner, vstart, vend;
-    float tparam, loss_scale;
-    void* dlogits;
-    int64_t ds_outer, ds_inner;
-    float* lp_out;     // [B, n_inner]
-    float* seq_stats;  // [B, 3]: seq_den, seq_w, seq_keep
-    float* terms;      // [B * n_inner, T_COUNT]
-    double* parts;     // [B, chunks, P_COUNT]
-    // packed mode (cu != NULL): the logits are one row of `total` positions, sequence s occupies
-    // [cu[s], cu[s+1]); the loss inputs stay [n_seq, n_inner]
-    const int32_t* cu;
-    int64_t n_seq;
-    int pre_rolled;
-    int4* row_pos;     // packed mode: [total] (sequence, position or -1, target index, 0), filled before the pass
-};
-
 // where a logits row sits in the loss inputs: sequence o, position i (i >= n_inner: the row feeds no token),
 // and the index of its target id
 struct FusedPos {
@@ -371,33 +335,16 @@ __device__ __forceinline__ FusedPos fused_where_packed(const FusedArgs& a, int64
     }
     return q;
 }
-template <bool PACKED>
-__device__ __forceinline__ FusedPos fused_where(const FusedArgs& a, int64_t r) {
-    FusedPos q;
-    if (!PACKED) {
-        q.o = r / a.d_n_inner;
-        q.i = r - q.o * a.d_n_inner;
-        q.tgt = q.o * a.ts_outer + q.i * a.ts_inner;
-        return q;
-    }
-    const int4 p = a.row_pos[r];
-    q.o = p.x;
-    q.i = p.y < 0 ? a.n_inner : p.y;
-    q.tgt = p.z;
-    return q;
-}
-template <bool PACKED>
-__device__ __forceinline__ int64_t fused_row_offset(const FusedArgs& a, int64_t r, int64_t so, int64_t si) {
-    if (PACKED) return r * si;
-    const int64_t o = r / a.d_n_inner;
-    return o * so + (r - o * a.d_n_inner) * si;
+template <int DT> __device__ __forceinline__ float fused_target_logit(const FusedArgs& a, const char* row, int64_t i, int temp) {
+    const float x = Row<DT>::load1(row, i);
+    return temp == 0 ? x : temp == 1 ? scale_logit<DT, 1>(x, a.tparam) : scale_logit<DT, 2>(x, a.tparam);
 }
 
-// Everything the pass needs beforehand, in one launch.  The first `batch` workgroups compute the per-sequence statistics.
-// Packed mode has more of them, which zero the records and logprobs (positions past a sequence's end have no packed row) and
-// find every row's place: the search through the boundaries is a chain of dependent loads, done once per row here so that the
-// persistent kernel finds it with one load.  (7 packed sequences, 16384 tokens: 8 us, four launches of 33 us before.)
-__global__ __launch_bounds__(kSeqBlock) void fused_prep_kernel(FusedArgs a, int64_t total) {
+// Everything the pass needs beforehand, in one launch.  The first `batch` workgroups compute the per-sequence statistics, the
+// others zero the logprobs (masked tokens and positions without a row keep that) and gather a record per row: where the row
+// sits in the loss inputs (in packed mode a search through the boundaries, a chain of dependent loads), the inputs, and its
+// target's logit.
+__global__ __launch_bounds__(kSeqBlock) void fused_prep_kernel(FusedArgs a, int64_t n_rows, int dtype, int temp) {
     __shared__ double sm_d[kSeqWaves];
     const nrl_grpo_cfg& c = a.cfg;
     const nrl_grpo_inputs& in = a.in;
@@ -405,11 +352,48 @@ __global__ __launch_bounds__(kSeqBlock) void fused_prep_kernel(FusedArgs a, int6
     if (b >= in.batch) {
         const int64_t first = (b - in.batch) * kSeqBlock + threadIdx.x, step = (gridDim.x - in.batch) * kSeqBlock;
         for (int64_t i = first; i < in.batch * n; i += step) a.lp_out[i] = 0.f;
-        float2* rec = reinterpret_cast<float2*>(a.terms);  // 8-byte aligned, an even number of floats
-        for (int64_t i = first; i < in.batch * n * (T_COUNT / 2); i += step) rec[i] = make_float2(0.f, 0.f);
-        for (int64_t r = first; r < total; r += step) {
-            const FusedPos q = fused_where_packed(a, r, total);
-            a.row_pos[r] = make_int4(static_cast<int>(q.o), static_cast<int>(q.i), static_cast<int>(q.tgt), 0);
+        for (int64_t r = first; r < n_rows; r += step) {
+            FusedPos q;
+            int64_t off;
+            if (a.cu) {
+                q = fused_where_packed(a, r, n_rows);
+                off = r * a.stride_inner;
+            } else {
+                q.o = r / a.d_n_inner;
+                q.i = r - q.o * a.d_n_inner;
+                off = q.o * a.stride_outer + q.i * a.stride_inner;
+                if (q.i >= n) continue;  // feeds no token: no record
+                q.tgt = q.o * a.ts_outer + q.i * a.ts_inner;
+            }
+            uint32_t w[R_WORDS];
+#pragma unroll
+            for (int k = 0; k < R_WORDS; ++k) w[k] = 0u;
+            const int64_t o = q.o, i = q.i;
+            const float tm = i >= 0 ? mask_at(in, o, i) : 0.f, smv = i >= 0 ? in.sample_mask[o] : 0.f;
+            if (tm * smv != 0.f) {
+                w[R_LIVE] = 1u;
+                if (!c.force_on_policy_ratio) w[R_PREV] = __float_as_uint(in.prev[o * in.prev_stride + i]);
+                w[R_GEN] = __float_as_uint(in.gen[o * in.gen_stride + i]);
+                if (c.has_kl) w[R_REF] = __float_as_uint(in.ref[o * in.ref_stride + i]);
+                w[R_ADV] = __float_as_uint(in.adv[o * in.adv_stride + i]);
+                w[R_TM] = __float_as_uint(tm);
+                w[R_SMV] = __float_as_uint(smv);
+                const int64_t tg = a.targets[q.tgt];
+                const bool local = tg >= a.vstart && tg < a.vend;
+                w[R_TLOC] = local ? static_cast<uint32_t>(tg - a.vstart) : 0xffffffffu;
+                if (local) {
+                    const char* row = static_cast<const char*>(a.logits) + off * (dtype == NRL_F32 ? 4 : 2);
+                    const float x = dtype == NRL_F32 ? fused_target_logit<NRL_F32>(a, row, tg - a.vstart, temp)
+                                    : dtype == NRL_BF16 ? fused_target_logit<NRL_BF16>(a, row, tg - a.vstart, temp)
+                                                        : fused_target_logit<NRL_F16>(a, row, tg - a.vstart, temp);
+                    w[R_XT] = __float_as_uint(x);
+                }
+                w[R_SEQ] = static_cast<uint32_t>(o);
+                w[R_POS] = static_cast<uint32_t>(i);
+            }
+            u32x4* out = reinterpret_cast<u32x4*>(a.rec + (a.cu ? r : o * n + i) * R_WORDS);
+#pragma unroll
+            for (int k = 0; k < R_WORDS / 4; ++k) out[k] = u32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
         }
         return;
     }
@@ -439,212 +423,45 @@ __global__ __launch_bounds__(kSeqBlock) void fused_prep_kernel(FusedArgs a, int6
     }
 }
 
-// Persistent workgroups: workgroup w walks rows w, w + gridDim.x, ...  While the gradient of one row
-// is being stored, the same slots (registers, and the LDS slice through direct global-to-LDS loads) are
-// refilled with the next row this workgroup evaluates, and the online (max, sum) of that row is advanced a few
-// vectors behind the loads, so reads, writes and the exponentials all overlap and only the
-// cross-wave merge and the one-thread loss evaluation sit between two rows.
-// Slot order q = 0 .. kFusedVec-1: the LDS slots come first (vector kFusedRegVec + q), then the
-// register slots (vector q - kFusedLdsVec).
-// NREG is the number of register slots the instantiation carries (the row must fit NREG + kFusedLdsVec
-// slots); shorter rows take a smaller instantiation instead of idling through unused slots.
-template <int DT, int TEMP, int NREG, bool PACKED>
-__global__ __launch_bounds__(kFusedBlock) void fused_logits_loss_kernel(FusedArgs a, int64_t n_rows) {
-    constexpr int EPV = Row<DT>::EPV;
-    constexpr int kFusedRegVec = NREG, kFusedVec = NREG + kFusedLdsVec;
-    constexpr int kFusedLag = NREG / 2 < 6 ? NREG / 2 : 6;  // slots between issuing a load and folding it into the running sum
-    __shared__ u32x4 stash[kFusedLdsVec * kFusedBlock];
-    __shared__ Lse sm_l[kFusedWaves];
-    __shared__ float sh_g, sh_lse;
-    const nrl_grpo_cfg& c = a.cfg;
-    const nrl_grpo_inputs& in = a.in;
-    const int tid = threadIdx.x;
-    const int nvec = static_cast<int>(a.vocab / EPV);
-    const int64_t step = gridDim.x;
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-
-    auto out_row = [&](int64_t r) -> char* {
-        return static_cast<char*>(a.dlogits) + fused_row_offset<PACKED>(a, r, a.ds_outer, a.ds_inner) * Row<DT>::BYTES;
-    };
-    auto in_row = [&](int64_t r) -> const char* {
-        return static_cast<const char*>(a.logits) + fused_row_offset<PACKED>(a, r, a.stride_outer, a.stride_inner) * Row<DT>::BYTES;
-    };
-    // Slot q holds vector slot_vec(q) of the row.  Lanes past the end of the row are pointed at the
-    // row's last vector instead: they load, compute and store exactly what that vector's own lane does
-    // (harmless duplicates), so the slot loop has no divergent branch around its memory operations and
-    // the loads of the next row stay in flight behind the stores.
-    auto slot_vec = [&](int q) -> int { return tid + (q < kFusedLdsVec ? kFusedRegVec + q : q - kFusedLdsVec) * kFusedBlock; };
-    // (recomputed at every use from an opaque copy of the lane index: twenty precomputed offsets would
-    // not fit in the register file next to the row)
-    auto slot_cl = [&](int q) -> int {
-        int t = tid;
-        asm volatile("" : "+v"(t));
-        return min(t + (q < kFusedLdsVec ? kFusedRegVec + q : q - kFusedLdsVec) * kFusedBlock, nvec - 1);
-    };
-    auto vec_at = [&](const char* base, int vc) -> const u32x4* {  // uniform base + 32-bit lane offset
-        return reinterpret_cast<const u32x4*>(base + static_cast<uint32_t>(vc) * 16u);
-    };
-    // First row at or after r (in this workgroup's walk) whose token takes part in the loss.  Rows passed
-    // over are dropped positions or masked tokens: zero gradient, logprob reported as 0, nothing read.
-    auto advance = [&](int64_t r) -> int64_t {
-        for (; r < n_rows; r += step) {
-            const FusedPos q = fused_where<PACKED>(a, r);
-            const int64_t o = q.o, i = q.i;
-            float w = 0.f;
-            if (i < a.n_inner) w = mask_at(in, o, i) * in.sample_mask[o];
-            if (w != 0.f) break;
-            u32x4* ov = reinterpret_cast<u32x4*>(out_row(r));
-            for (int v = tid; v < nvec; v += kFusedBlock) ov[v] = zero;
-            if (i < a.n_inner) {
-                const int64_t tok = o * a.n_inner + i;
-                if (tid < T_COUNT) a.terms[tok * T_COUNT + tid] = 0.f;
-                if (tid == 0) a.lp_out[tok] = 0.f;
-            }
-        }
-        return r;
-    };
-    u32x4 regs[kFusedRegVec];
-    Lse acc;
-    // LDS slot q of the incoming row: global memory -> LDS without passing through registers; each wave
-    // fills the 1 KiB of the slot that its own lanes read back
-    auto lds_fill = [&](const char* base, int q) {
-        u32x4* dst = stash + q * kFusedBlock + (tid & ~(kWave - 1));
-        __builtin_amdgcn_global_load_lds(reinterpret_cast<const __attribute__((address_space(1))) void*>(
-                                             reinterpret_cast<uintptr_t>(vec_at(base, slot_cl(q)))),
-                                         (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-    };
-    auto fold = [&](int q) {  // slot q of the incoming row -> running sum; lanes past the row add nothing
-        u32x4 raw = q < kFusedLdsVec ? stash[(q < kFusedLdsVec ? q : 0) * kFusedBlock + tid] : regs[q < kFusedLdsVec ? 0 : q - kFusedLdsVec];
-        if (slot_vec(q) >= nvec) raw = u32x4{Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD};
-        float t[EPV];
-        Row<DT>::decode(raw, t);
-#pragma unroll
-        for (int k = 0; k < EPV; ++k) t[k] = scale_logit<DT, TEMP>(t[k], a.tparam);
-        lse_push<EPV>(acc, t);
-    };
-    // the direct-to-LDS loads are not tracked against later LDS reads by the compiler: wait for them
-    // (and everything older) by hand before the first read of a refilled LDS slot
-    auto wait_lds_fill = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
-
-    int64_t r = advance(blockIdx.x);
-    if (r < n_rows) {
-        const char* xv = in_row(r);
-#pragma unroll
-        for (int q = 0; q < kFusedLdsVec; ++q) lds_fill(xv, q);
-#pragma unroll
-        for (int q = kFusedLdsVec; q < kFusedVec; ++q) regs[q - kFusedLdsVec] = __builtin_nontemporal_load(vec_at(xv, slot_cl(q)));
-        acc.m = -FLT_MAX;
-        acc.s = 0.f;
-#pragma unroll
-        for (int q = kFusedLdsVec; q < kFusedVec; ++q) fold(q);
-        wait_lds_fill();
-#pragma unroll
-        for (int q = 0; q < kFusedLdsVec; ++q) fold(q);
-    }
-    while (r < n_rows) {
-        const FusedPos where = fused_where<PACKED>(a, r);
-        const int64_t o = where.o, i = where.i;
-        const int64_t tok = o * a.n_inner + i;
-        const char* row = in_row(r);
-        char* ov = out_row(r);
-        const Lse tot = block_lse<kFusedWaves>(acc, sm_l);
-        const int64_t tg = a.targets[where.tgt];
-        const int64_t tloc = (tg >= a.vstart && tg < a.vend) ? tg - a.vstart : -1;
-        if (tid == 0) {
-            const float log_s = logf(tot.s);
-            float lp = 0.f;
-            if (tloc >= 0) lp = (scale_logit<DT, TEMP>(Row<DT>::load1(row, tloc), a.tparam) - tot.m) - log_s;
-            SeqStats st;
-            st.seq_den = a.seq_stats[o * 3]; st.seq_ratio = 1.f; st.seq_w = a.seq_stats[o * 3 + 1]; st.seq_keep = a.seq_stats[o * 3 + 2];
-            TokenIn ti;
-            ti.lp = lp; ti.lpu = lp;
-            ti.prev = c.force_on_policy_ratio ? lp : in.prev[o * in.prev_stride + i];
-            ti.gen = in.gen[o * in.gen_stride + i];
-            ti.ref = c.has_kl ? in.ref[o * in.ref_stride + i] : 0.f;
-            ti.adv = in.adv[o * in.adv_stride + i];
-            ti.tm = mask_at(in, o, i);
-            ti.smv = in.sample_mask[o];
-            ti.correct = 0.f;
-            ti.den_s = valid_seqs(in) + 1e-8f;
-            ti.den_t = valid_toks(in) + 1e-8f;
-            const TokenOut out = token_eval<false>(c, st, ti);
-            float* rec = a.terms + tok * T_COUNT;
-#pragma unroll
-            for (int k = 0; k < P_SAMPLE_MASK; ++k) rec[k] = out.term[k];
-            rec[T_RATIO] = out.ratio;
-            rec[T_RATIO_CL] = out.ratio_cl;
-            rec[T_SELECTED] = out.selected ? 1.f : 0.f;
-            a.lp_out[tok] = lp;
-            sh_g = (out.d_actor + out.d_lpu) * a.loss_scale;
-            sh_lse = tot.m + log_s;
-        }
-        __syncthreads();
-        const float g = sh_g, lse = sh_lse;
-        const int64_t rn = advance(r + step);
-        const char* nx = rn < n_rows ? in_row(rn) : row;
-        const int tvec = tloc >= 0 ? static_cast<int>(tloc / EPV) : -1;
-        const int tsub = tloc >= 0 ? static_cast<int>(tloc % EPV) : -1;
-        const RowGrad rg(lse, g, a.tparam);
-        acc.m = -FLT_MAX;
-        acc.s = 0.f;
-        // The LDS slots first: once all of them are consumed they are refilled for the next row (after
-        // the last row the refills and loads re-read the current row and are ignored).
-#pragma unroll
-        for (int q = 0; q < kFusedLdsVec; ++q) {
-            const int vc = slot_cl(q);
-            const u32x4 d = grad_vec<DT, TEMP>(stash[q * kFusedBlock + tid], vc == tvec ? tsub : -1, rg);
-            __builtin_nontemporal_store(d, const_cast<u32x4*>(vec_at(ov, vc)));
-        }
-#pragma unroll
-        for (int q = 0; q < kFusedLdsVec; ++q) lds_fill(nx, q);
-#pragma unroll
-        for (int q = kFusedLdsVec; q < kFusedVec; ++q) {
-            const int vc = slot_cl(q);
-            const u32x4 d = grad_vec<DT, TEMP>(regs[q - kFusedLdsVec], vc == tvec ? tsub : -1, rg);
-            __builtin_nontemporal_store(d, const_cast<u32x4*>(vec_at(ov, vc)));
-            regs[q - kFusedLdsVec] = __builtin_nontemporal_load(vec_at(nx, vc));
-            __builtin_amdgcn_sched_barrier(0);  // keep the fold behind this slot's memory operations ...
-            if (q >= kFusedLdsVec + kFusedLag) {
-                fold(q - kFusedLag);
-                asm volatile("" : "+v"(acc.m), "+v"(acc.s));  // a use right here, so the fold is not sunk past the loop
-            }
-            __builtin_amdgcn_sched_barrier(0);  // ... and ahead of the next slot's
-        }
-#pragma unroll
-        for (int q = kFusedVec - kFusedLag; q < kFusedVec; ++q) fold(q);
-        wait_lds_fill();
-#pragma unroll
-        for (int q = 0; q < kFusedLdsVec; ++q) fold(q);
-        // sh_g / sh_lse are rewritten only after the next block_lse, whose barriers every thread passes
-        // after reading them above
-        r = rn;
-    }
-}
-
-// Token term records -> sums over shares of kTermsBlock tokens, one workgroup each: a record per thread, read as ten 8-byte
-// pairs.  A sequence in one workgroup reads its records at what one compute unit gets, 23 us for 7 packed sequences (16384
+// Logprobs -> the terms of the loss and the metrics, summed over shares of kTermsBlock tokens, one workgroup each and a token
+// per thread.  A sequence per workgroup is bound by the chain of one compute unit, 23 us for 7 packed sequences (16384
 // tokens); spread out 6 us, 4 sequences of 1024 tokens 9.6 -> 5.7 us.  The shares are added up, in order, by the
 // launch that finishes the metrics: done here by the workgroup that arrives last, the device-scope fence in front of its
 // arrival waits for the L2 to write back what the pass left there, 13 - 25 us.
 constexpr int kTermsBlock = 256, kTermsWaves = kTermsBlock / kWave;
-__global__ __launch_bounds__(kTermsBlock) void grpo_terms_reduce_kernel(FusedArgs a, int64_t chunks) {
+__global__ __launch_bounds__(kTermsBlock) void grpo_terms_reduce_kernel(FusedArgs a, int64_t chunks, int64_t n_rows) {
     __shared__ double sm_d[kTermsWaves * P_R_MIN];
     __shared__ float sm_f[kTermsWaves];
-    static_assert(T_COUNT % 2 == 0, "records are read as 8-byte pairs");
-    constexpr int kPairs = T_COUNT / 2;
+    const nrl_grpo_cfg& c = a.cfg;
+    const nrl_grpo_inputs& in = a.in;
     const int64_t b = blockIdx.x / chunks, q = blockIdx.x - b * chunks, t = q * kTermsBlock + threadIdx.x;
     double acc[P_R_MIN];
 #pragma unroll
     for (int k = 0; k < P_R_MIN; ++k) acc[k] = 0;
     float r_min = INFINITY, r_max = -INFINITY, rc_min = INFINITY, rc_max = -INFINITY;
-    if (t < a.n_inner) {
-        float rec[T_COUNT];
-        const float2* p = reinterpret_cast<const float2*>(a.terms + (b * a.n_inner + t) * T_COUNT);  // 8-byte aligned: T_COUNT is even
+    bool live = t < a.n_inner;
+    if (live && a.cu) {  // a position that has a packed row
+        const int64_t start = a.cu[b], len = a.cu[b + 1] - start;
+        live = t + 1 < len && start + t >= 0 && start + t < n_rows;
+    }
+    const float tm = live ? mask_at(in, b, t) : 0.f, smv = in.sample_mask[b];
+    if (tm * smv != 0.f) {
+        const float lp = a.lp_out[b * a.n_inner + t];
+        SeqStats st;
+        st.seq_den = a.seq_stats[b * 3]; st.seq_ratio = 1.f; st.seq_w = a.seq_stats[b * 3 + 1]; st.seq_keep = a.seq_stats[b * 3 + 2];
+        TokenIn ti;
+        ti.lp = lp; ti.lpu = lp;
+        ti.prev = c.force_on_policy_ratio ? lp : in.prev[b * in.prev_stride + t];
+        ti.gen = in.gen[b * in.gen_stride + t];
+        ti.ref = c.has_kl ? in.ref[b * in.ref_stride + t] : 0.f;
+        ti.adv = in.adv[b * in.adv_stride + t];
+        ti.tm = tm; ti.smv = smv; ti.correct = 0.f;
+        ti.den_s = valid_seqs(in) + 1e-8f;
+        ti.den_t = valid_toks(in) + 1e-8f;
+        const TokenOut out = token_eval<false>(c, st, ti);
 #pragma unroll
-        for (int k = 0; k < kPairs; ++k) { const float2 v = p[k]; rec[2 * k] = v.x; rec[2 * k + 1] = v.y; }
-#pragma unroll
-        for (int k = 0; k < P_SAMPLE_MASK; ++k) acc[k] = rec[k];
-        if (rec[T_SELECTED] != 0.f) { r_min = r_max = rec[T_RATIO]; rc_min = rc_max = rec[T_RATIO_CL]; }
+        for (int k = 0; k < P_SAMPLE_MASK; ++k) acc[k] = out.term[k];
+        if (out.selected) { r_min = r_max = out.ratio; rc_min = rc_max = out.ratio_cl; }
     }
     store_parts<kTermsWaves>(a.parts + blockIdx.x * static_cast<int64_t>(P_COUNT), acc, r_min, r_max, rc_min, rc_max, sm_d, sm_f);
 }
@@ -994,13 +811,17 @@ static int64_t align8(int64_t v) { return (v + 7) / 8 * 8; }
 
 static int64_t terms_chunks(int64_t n) { return n < 1 ? 1 : (n + kTermsBlock - 1) / kTermsBlock; }
 
-extern "C" int64_t nrl_fused_workspace_bytes(int64_t batch, int64_t n_inner) {
+// statistics, partial sums, one record per row (16-byte aligned)
+static int64_t fused_workspace(int64_t batch, int64_t n_inner, int64_t n_rows) {
     const int64_t b = batch < 1 ? 1 : batch, n = n_inner < 1 ? 1 : n_inner;
-    return align8(b * 3 * 4) + align8(b * n * T_COUNT * 4) + b * terms_chunks(n) * P_COUNT * 8;
+    return align8(b * 3 * 4) + b * terms_chunks(n) * P_COUNT * 8 + 16 + (n_rows < 1 ? 1 : n_rows) * R_WORDS * 4;
 }
-
+extern "C" int64_t nrl_fused_workspace_bytes(int64_t batch, int64_t n_inner) {
+    // (the gradient may have more rows per sequence than the loss has tokens; they have no record)
+    return fused_workspace(batch, n_inner, (batch < 1 ? 1 : batch) * (n_inner < 1 ? 1 : n_inner));
+}
 extern "C" int64_t nrl_fused_packed_workspace_bytes(int64_t n_seq, int64_t n_inner, int64_t total) {
-    return nrl_fused_workspace_bytes(n_seq, n_inner) + 16 + (total < 1 ? 1 : total) * 16;
+    return fused_workspace(n_seq, n_inner, total);
 }
 
 // rows describes the logits; with cu != NULL it is one packed row of rows->n_inner positions (n_outer 1) and
@@ -1028,7 +849,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     if (seq_weights && in->batch * in->sm1 > 0 && !in->prev) return fail(NRL_E_INVALID, "prev_logprobs is NULL");
     if (cfg->kl_type < 1 || cfg->kl_type > 3 || cfg->tis_type < 0 || cfg->tis_type > 3) return fail(NRL_E_INVALID, "bad kl_type or tis_type");
     const int bytes = rows->dtype == NRL_F32 ? 4 : 2, epv = 16 / bytes;
-    if (rows->vocab % epv || rows->vocab / epv > static_cast<int64_t>(kFusedMaxVec) * kFusedBlock)
+    if (rows->vocab % epv || rows->vocab / epv > static_cast<int64_t>(kFusedMaxVec) * 1024)
         return fail(NRL_E_UNSUPPORTED, "row does not fit the on-chip path (vocab %lld)", (long long)rows->vocab);
     if ((reinterpret_cast<uintptr_t>(rows->logits) & 15) || (reinterpret_cast<uintptr_t>(dlogits) & 15) ||
         (rows->stride_outer * bytes) % 16 || (rows->stride_inner * bytes) % 16 || (d_stride_outer * bytes) % 16 ||
@@ -1061,9 +882,8 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     a.lp_out = logprob_out;
     char* ws = static_cast<char*>(workspace);
     a.seq_stats = reinterpret_cast<float*>(ws); ws += align8(in->batch * 3 * 4);
-    a.terms = reinterpret_cast<float*>(ws); ws += align8(in->batch * (in->sm1 < 1 ? 1 : in->sm1) * T_COUNT * 4);
     a.parts = reinterpret_cast<double*>(ws); ws += in->batch * terms_chunks(in->sm1) * P_COUNT * 8;
-    a.row_pos = cu ? reinterpret_cast<int4*>(ws + ((16 - (reinterpret_cast<uintptr_t>(ws) & 15)) & 15)) : nullptr;
+    a.rec = reinterpret_cast<uint32_t*>(ws + ((16 - (reinterpret_cast<uintptr_t>(ws) & 15)) & 15));
     int tc = 0;
     a.tparam = 1.f;
     if (rows->temperature != 1.0f) {
@@ -1072,35 +892,17 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     const unsigned nb = static_cast<unsigned>(in->batch);
-    const int64_t fill = cu ? (n_rows > in->batch * in->sm1 * 4 ? n_rows : in->batch * in->sm1 * 4) : 0;
-    const unsigned more = static_cast<unsigned>(fill + kSeqBlock - 1 < 256ll * kSeqBlock ? (fill + kSeqBlock - 1) / kSeqBlock : 256);
-    if (nb + more > 0) fused_prep_kernel<<<dim3(nb + more), dim3(kSeqBlock), 0, s>>>(a, n_rows);
+    const int64_t items = n_rows > in->batch * in->sm1 ? n_rows : in->batch * in->sm1;
+    const unsigned more = static_cast<unsigned>(items < 1024ll * kSeqBlock ? (items + kSeqBlock - 1) / kSeqBlock : 1024);
+    if (nb + more > 0) fused_prep_kernel<<<dim3(nb + more), dim3(kSeqBlock), 0, s>>>(a, n_rows, rows->dtype, tc);
     if (n_rows > 0) {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             return fail(NRL_E_LAUNCH, "cannot read the device's compute-unit count");
-        // one resident workgroup per compute unit (64 KiB of LDS and 1024 threads each)
-        const dim3 grid((unsigned)(n_rows < cus ? n_rows : cus)), block(kFusedBlock);
-        const int64_t slots = (rows->vocab / epv + kFusedBlock - 1) / kFusedBlock;
-        const int nreg = slots <= 8 ? 4 : slots <= 12 ? 8 : slots <= 16 ? 12 : 16;
-#define NRL_FUSED_LAUNCH(DT_, TC_, NR_)                                                                           \
-    if (cu) fused_logits_loss_kernel<DT_, TC_, NR_, true><<<grid, block, 0, s>>>(a, n_rows);                      \
-    else fused_logits_loss_kernel<DT_, TC_, NR_, false><<<grid, block, 0, s>>>(a, n_rows)
-#define NRL_FUSED_CASE(DT_, TC_)                                                                                  \
-    case DT_ * 3 + TC_:                                                                                           \
-        if (nreg == 4) { NRL_FUSED_LAUNCH(DT_, TC_, 4); }                                                         \
-        else if (nreg == 8) { NRL_FUSED_LAUNCH(DT_, TC_, 8); }                                                    \
-        else if (nreg == 12) { NRL_FUSED_LAUNCH(DT_, TC_, 12); }                                                  \
-        else { NRL_FUSED_LAUNCH(DT_, TC_, 16); }                                                                  \
-        break;
-        switch (rows->dtype * 3 + tc) {
-            NRL_FUSED_CASE(NRL_F32, 0) NRL_FUSED_CASE(NRL_F32, 1) NRL_FUSED_CASE(NRL_F32, 2)
-            NRL_FUSED_CASE(NRL_BF16, 0) NRL_FUSED_CASE(NRL_BF16, 1) NRL_FUSED_CASE(NRL_BF16, 2)
-            NRL_FUSED_CASE(NRL_F16, 0) NRL_FUSED_CASE(NRL_F16, 1) NRL_FUSED_CASE(NRL_F16, 2)
-            default: return fail(NRL_E_INVALID, "unknown logits dtype");
-        }
-#undef NRL_FUSED_CASE
-#undef NRL_FUSED_LAUNCH
+        const FusedLaunch l{a, tc, cu != nullptr, n_rows, cus, s};
+        if (rows->dtype == NRL_F32) launch_fused_f32(l);
+        else if (rows->dtype == NRL_BF16) launch_fused_bf16(l);
+        else launch_fused_f16(l);
     }
     GrpoArgs fa;
     fa.cfg = *cfg;
@@ -1108,7 +910,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     fa.dlp = nullptr; fa.dlpu = nullptr;
     fa.parts = a.parts;
     fa.seq_stats = a.seq_stats; fa.chunks = terms_chunks(in->sm1);
-    if (nb > 0) grpo_terms_reduce_kernel<<<dim3((unsigned)(nb * fa.chunks)), dim3(kTermsBlock), 0, s>>>(a, fa.chunks);
+    if (nb > 0) grpo_terms_reduce_kernel<<<dim3((unsigned)(nb * fa.chunks)), dim3(kTermsBlock), 0, s>>>(a, fa.chunks, n_rows);
     grpo_finish_kernel<<<dim3(1), dim3(kSeqBlock), 0, s>>>(fa, loss_out, metrics_out);
     return check_launch("fused_logits_grpo_loss");
 }

@@ -451,3 +451,29 @@ def test_metrics_over_shares_of_a_sequence(cfg, b, s):
     assert _close(got.item(), want.item(), rel=1e-4, abs_=1e-6)
     for k in wm:
         assert _close(float(gm[k]), float(wm[k])), (k, gm[k], wm[k])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("vectors", [1, 255, 2048, 2049, 3073, 4097, 5120, 5121, 8193, 10240, 10241, 16385, 20480])
+def test_workgroup_sizes_and_slot_counts(dtype, vectors):
+    """16-byte vectors per row around every change of workgroup size and register slots, against the three-pass path: lse of the
+    two differs by the order of fp32 sums (about 1e-6), so gradients by that and one rounding."""
+    vocab = vectors * (16 // torch.empty(0, dtype=dtype).element_size())
+    b, s = (2, 1300) if vectors == 1 else (3, 5)  # the short rows outnumber the resident workgroups
+    logits, data, gs, gt = _batch(b, s, vocab, dtype, seed=vectors)
+    ddev = {k: v.to(DEV) for k, v in data.items()}
+    gs, gt = gs.to(DEV), gt.to(DEV)
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    xf, xu = (logits.to(DEV).requires_grad_(True) for _ in range(2))
+    got, gm = fused_logits_clipped_pg_loss(xf, ddev, fn, gs, gt)
+    got.backward()
+    loss_input, d2 = prepare_loss_input(xu, dict(ddev), fn)
+    want, wm = fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)
+    want.backward()
+    assert _close(got.item(), want.item(), rel=1e-4)
+    for k in wm:
+        assert _close(float(gm[k]), float(wm[k])), k
+    gf, gu = xf.grad.float(), xu.grad.float()
+    scale = gu.abs().max().item()
+    step = 0.0 if dtype == torch.float32 else 2.0 ** -7  # neighbouring 16-bit values
+    assert bool(((gf - gu).abs() <= gu.abs() * (step + 1e-4) + 1e-4 * scale * (1.0 if dtype == torch.float32 else 2.0 ** -8)).all())
