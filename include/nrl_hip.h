@@ -314,6 +314,21 @@ int nrl_fused_packed_logits_grpo_loss(const nrl_rows* rows, int32_t target_is_pr
                                       float* loss_out, float* metrics_out, void* workspace, int64_t workspace_bytes,
                                       void* stream);
 
+/* Both of the above (cu_seqlens NULL: the first) for rows that need not lie on the 16-byte grid nor fit on the chip: 1 KiB to
+ * NRL_FUSED_ANY_ROW_MAX bytes, logits and gradient rows alike modulo 16 bytes, not in place, temperature as a multiplication.
+ * row_grad_out: fp32 [n_outer * d_n_inner, 4], 16-byte aligned: what nrl_rows_grad needs to write the gradient again.  The gradient
+ * is written for an upstream factor of 1. */
+#define NRL_FUSED_ANY_ROW_MIN 1024
+#define NRL_FUSED_ANY_ROW_MAX (1 << 20)
+int nrl_fused_any_row_grpo_loss(const nrl_rows* rows, int32_t target_is_pre_rolled, const int32_t* cu_seqlens, int64_t n_seq,
+                                const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float* row_grad_out, void* dlogits,
+                                int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out,
+                                float* loss_out, float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream);
+/* dlogits = *factor times the gradient described by row_grad, over all n_outer * n_inner rows; *factor is read from the device and
+ * nothing is done when it equals `written`, the factor dlogits holds already (NaN: always write). */
+int nrl_rows_grad(const nrl_rows* rows, const float* row_grad, const float* factor, float written, void* dlogits,
+                  int64_t d_stride_outer, int64_t d_stride_inner, void* stream);
+
 /* NLLLossFn scalar branch (loss_functions.py:818-842): loss = -sum(lp*mask)/(Gt+1e-8);
  * metrics_out[0..2] = {loss, num_unmasked_tokens, num_valid_samples}; dlp_out = -mask/(Gt+1e-8). */
 int nrl_nll_loss_fwd_bwd(const nrl_grpo_inputs* in, float* loss_out, float* dlp_out,

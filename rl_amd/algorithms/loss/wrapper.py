@@ -105,21 +105,25 @@ class SequencePackingFusionLossWrapper:
         self.context_parallel_group = context_parallel_group
 
     def __call__(self, next_token_logits, data, global_valid_seqs, global_valid_toks):
-        from .fused import fused_packed_logits_clipped_pg_loss, why_not_fusable_packed
+        from .fused import _single_pass_packed, any_row_fusable_packed, fused_packed_logits_clipped_pg_loss, why_not_fusable_packed
         from .utils import prepare_packed_loss_input
 
         # a ClippedPGLossFn whose token gradient needs no other token's logprob: logits -> loss -> gradient
         # in one pass over the packed row, as in wrap_loss_fn_with_input_preparation
         bound = _bound_keywords(self.prepare_fn, prepare_packed_loss_input, ("sampling_params", "chunk_size"))
         if (bound is not None and torch.is_grad_enabled()
-                and isinstance(next_token_logits, torch.Tensor) and next_token_logits.requires_grad
-                and why_not_fusable_packed(self.loss_fn, next_token_logits, data, bound.get("sampling_params")) is None):
+                and isinstance(next_token_logits, torch.Tensor) and next_token_logits.requires_grad):
             from ...distributed.model_utils import _group_size
 
             if _group_size(self.vocab_parallel_group) == 1 and _group_size(self.context_parallel_group) == 1:
-                return fused_packed_logits_clipped_pg_loss(
-                    next_token_logits, data, self.loss_fn, self.cu_seqlens_q, self.cu_seqlens_q_padded,
-                    global_valid_seqs, global_valid_toks)
+                params = bound.get("sampling_params")
+                if why_not_fusable_packed(self.loss_fn, next_token_logits, data, params) is None:
+                    return fused_packed_logits_clipped_pg_loss(
+                        next_token_logits, data, self.loss_fn, self.cu_seqlens_q, self.cu_seqlens_q_padded,
+                        global_valid_seqs, global_valid_toks)
+                if any_row_fusable_packed(self.loss_fn, next_token_logits, data, params):
+                    return _single_pass_packed(next_token_logits, data, self.loss_fn, self.cu_seqlens_q, self.cu_seqlens_q_padded,
+                                               global_valid_seqs, global_valid_toks, 1.0, True)
         loss_input, prepared = self.prepare_fn(
             logits=next_token_logits, data=data, loss_fn=self.loss_fn, cu_seqlens_q=self.cu_seqlens_q,
             cu_seqlens_q_padded=self.cu_seqlens_q_padded, vocab_parallel_rank=self.vocab_parallel_rank,
@@ -138,19 +142,22 @@ def wrap_loss_fn_with_input_preparation(next_token_logits, data, global_valid_se
     """``wrapper.py:292-322``: prepare, then call the loss.  When the loss is a ``ClippedPGLossFn`` whose
     per-token gradient does not need other tokens' logprobs and the logits are a plain GPU tensor, both
     steps (and the later backward through the logprob op) run as one fused pass over the logits."""
-    from .fused import fused_logits_clipped_pg_loss, why_not_fusable
+    from .fused import _single_pass, any_row_fusable, fused_logits_clipped_pg_loss, why_not_fusable
     from .utils import prepare_loss_input
 
     # chunk_size only bounds the reference's working set and d2t belongs to the draft-model loss: neither changes
     # what the single pass computes, top-k / top-p filtering (checked by why_not_fusable) does
     bound = _bound_keywords(prepare_fn, prepare_loss_input, ("sampling_params", "d2t", "chunk_size"))
     if (bound is not None and bound.get("d2t") is None and torch.is_grad_enabled()
-            and isinstance(next_token_logits, torch.Tensor) and next_token_logits.requires_grad
-            and why_not_fusable(loss_fn, next_token_logits, data, bound.get("sampling_params")) is None):
+            and isinstance(next_token_logits, torch.Tensor) and next_token_logits.requires_grad):
         from ...distributed.model_utils import _group_size
 
         if _group_size(vocab_parallel_group) == 1 and _group_size(context_parallel_group) == 1:
-            return fused_logits_clipped_pg_loss(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks)
+            params = bound.get("sampling_params")
+            if why_not_fusable(loss_fn, next_token_logits, data, params) is None:
+                return fused_logits_clipped_pg_loss(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks)
+            if any_row_fusable(loss_fn, next_token_logits, data, params):
+                return _single_pass(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks, 1.0, False, True)
     loss_input, data = prepare_fn(
         logits=next_token_logits, data=data, loss_fn=loss_fn, vocab_parallel_rank=vocab_parallel_rank,
         vocab_parallel_group=vocab_parallel_group, context_parallel_group=context_parallel_group,

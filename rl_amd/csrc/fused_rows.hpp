@@ -39,6 +39,8 @@ struct FusedArgs {
     const int32_t* cu;
     int64_t n_seq;
     int pre_rolled;
+    float4* row_grad;  // NULL or [rows]: (d loss / d logprob at loss_scale 1, log-sum-exp, target or -1 as bits, 0) of every row, from
+                       // which the gradient can be written again; zeros for rows without a token
 };
 
 struct FusedLaunch {
@@ -46,6 +48,7 @@ struct FusedLaunch {
     int temp;  // 0, 1 (divide), 2 (multiply)
     bool packed;
     int64_t n_rows;
+    bool any_row;  // rows off the 16-byte grid, or longer than the chip holds
     int compute_units;
     hipStream_t stream;
 };
@@ -76,20 +79,29 @@ __device__ __forceinline__ void load_to_lds(const char* base, int bytes, int off
 // What lies between two rows is kept short: the row's inputs come in one load a row ahead, every wave evaluates the token
 // by itself (no broadcast, no second barrier), and only what the gradient needs is evaluated; the terms of the metrics
 // follow in the reduction behind the pass (4 x 1024 rows: 538 -> 520 us for the whole call).
-// Slot order q = 0 .. kVec-1: the LDS slots come first (vector NREG + q), then the register slots (vector q - kFusedLdsVec).
-// NREG is the number of register slots the instantiation carries (the row must fit NREG + kFusedLdsVec
+// Slot order q = 0 .. kVec-1: the LDS slots come first (vector NREG + q), then the register slots (vector q - NLDS).
+// NREG is the number of register slots the instantiation carries (the row must fit NREG + NLDS
 // slots); shorter rows take a smaller instantiation instead of idling through unused slots, and smaller workgroups of which
 // several share a compute unit, so that one's stretch between rows is covered by the others' memory operations.
-template <int DT, int TEMP, int BLOCK, int NREG, bool PACKED>
+//
+// EDGE: rows need not start or end on 16 bytes.  The vectors of a row begin at its first 16-byte boundary; the up to 7 elements
+// before it and the tail shorter than a vector are one element each of the first 32 lanes.  (Input and output rows sit alike.)
+// LONG (1024 threads): vectors past the on-chip slots are read twice.  They are the last ones read of a row and the first
+// ones its gradient needs, in reverse order, so the second read finds them in the 256 MB cache: at most 256 rows' excess
+// lies between the two (85 MB at V = 151936 fp32).
+// Both against the three passes (logprobs, loss, gradient) such rows took before, whole calls: 2 x 1024 rows of V = 151936 fp32
+// 710 -> 498 us, of V = 262144 bf16 577 -> 478, 2 x 512 of V = 262144 fp32 574 -> 447; 3 x 701 rows of V = 50257 bf16 152 -> 144,
+// 4 x 2048 of V = 20001 200 -> 156; 128 rows of V = 262143 fp32 186 -> 105.
+template <int DT, int TEMP, int BLOCK, int NREG, int NLDS, bool EDGE, bool LONG, bool PACKED>
 __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a, int64_t n_rows) {
     constexpr int EPV = Row<DT>::EPV;
-    constexpr int NLDS = kFusedLdsVec, kVec = NREG + NLDS;
+    constexpr int kVec = NREG + NLDS;
     constexpr int kWavesPerBlock = BLOCK / kWave;
     __shared__ u32x4 stash[NLDS * BLOCK];
     __shared__ Lse sm_l[kWavesPerBlock];
     const nrl_grpo_cfg& c = a.cfg;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int nvec = static_cast<int>(a.vocab / EPV);
+    int nvec = static_cast<int>(a.vocab / EPV), head = 0;  // of the row at hand
     const int64_t step = gridDim.x;
     const u32x4 zero = {0u, 0u, 0u, 0u};
 
@@ -114,6 +126,18 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
     auto vec_at = [&](const char* base, int vc) -> const u32x4* {  // uniform base + 32-bit lane offset
         return reinterpret_cast<const u32x4*>(base + static_cast<uint32_t>(vc) * 16u);
     };
+    auto place = [&](const char* row) {  // head and nvec of a row, which its output shares
+        if (!EDGE) return;
+        head = static_cast<int>(((16 - (reinterpret_cast<uintptr_t>(row) & 15)) & 15) / Row<DT>::BYTES);
+        nvec = (static_cast<int>(a.vocab) - head) / EPV;
+    };
+    // this lane's element outside the vectors, or -1
+    auto edge_at = [&]() -> int {
+        if (tid < head) return tid;
+        const int t = head + nvec * EPV + tid - 16;
+        return tid >= 16 && t < static_cast<int>(a.vocab) ? t : -1;
+    };
+    float edge_x = 0.f;
     auto load_rec = [&](int64_t r) -> uint32_t {
         if (r >= n_rows) return 0u;
         if (!PACKED) {  // a record per token: rows behind a sequence's last token have none
@@ -128,9 +152,12 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
     // r's on entry.  Rows passed over are dropped positions or masked tokens: zero gradient, nothing read.
     auto advance = [&](int64_t r, uint32_t& rec) -> int64_t {
         while (r < n_rows && word(rec, R_LIVE) == 0u) {
-            u32x4* ov = reinterpret_cast<u32x4*>(out_row(r));
+            char* out = out_row(r);
+            place(out);
+            u32x4* ov = reinterpret_cast<u32x4*>(out + head * Row<DT>::BYTES);
             rec = load_rec(r + step);
             for (int v = tid; v < nvec; v += BLOCK) ov[v] = zero;
+            if (EDGE && edge_at() >= 0) Row<DT>::store1(out, edge_at(), 0.f);
             r += step;
         }
         return r;
@@ -146,24 +173,32 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
         u32x4* dst = stash + q * BLOCK + (tid & ~(kWave - 1));
         load_to_lds(base, nvec * 16, slot_cl(q) * 16, dst);
     };
-    auto fold = [&](int q) {  // slot q of the incoming row -> running sum; lanes past the row add nothing
-        u32x4 raw = q < NLDS ? stash[(q < NLDS ? q : 0) * BLOCK + tid] : regs[q < NLDS ? 0 : q - NLDS];
-        if (slot_vec(q) >= nvec) raw = u32x4{Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD};
+    auto fold_vec = [&](u32x4 raw, int v) {  // vector v of the incoming row -> running sum; lanes past the row add nothing
+        if (v >= nvec) raw = u32x4{Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD, Row<DT>::NEG_INF_WORD};
         float t[EPV];
         Row<DT>::decode(raw, t);
 #pragma unroll
         for (int k = 0; k < EPV; ++k) t[k] = scale_logit<DT, TEMP>(t[k], a.tparam);
         lse_push<EPV>(acc, t);
     };
+    auto fold = [&](int q) {
+        fold_vec(q < NLDS ? stash[(q < NLDS ? q : 0) * BLOCK + tid] : regs[q < NLDS ? 0 : q - NLDS], slot_vec(q));
+    };
+    constexpr int kAhead = 4;                    // vectors past the slots in flight per lane
+    constexpr int kStride = kAhead * BLOCK;
+    const int past = kVec * BLOCK;
     // the direct-to-LDS loads are not tracked against later LDS reads by the compiler: wait for them
     // (and everything older) by hand before the first read of a refilled LDS slot
     auto wait_lds_fill = [&]() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
 
-    auto load_row = [&](const char* base) {  // the row onto the chip, and its (max, sum)
+    auto load_row = [&](const char* row) {  // the row onto the chip, and its (max, sum)
+        place(row);
+        const char* base = row + head * Row<DT>::BYTES;
 #pragma unroll
         for (int q = 0; q < NLDS; ++q) lds_fill(base, q);
 #pragma unroll
         for (int q = NLDS; q < kVec; ++q) regs[q - NLDS] = __builtin_nontemporal_load(vec_at(base, slot_cl(q)));
+        if (EDGE && edge_at() >= 0) edge_x = Row<DT>::load1(row, edge_at());
         __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first is waited for
         acc.m = -FLT_MAX;
         acc.s = 0.f;
@@ -172,6 +207,16 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
         wait_lds_fill();
 #pragma unroll
         for (int q = 0; q < NLDS; ++q) fold(q);
+        if (EDGE && edge_at() >= 0) lse_push1(acc, scale_logit<DT, TEMP>(edge_x, a.tparam));
+        if (LONG) {
+            for (int v0 = past; v0 < nvec; v0 += kStride) {
+                u32x4 x[kAhead];
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) x[j] = *vec_at(base, min(v0 + j * BLOCK + tid, nvec - 1));
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) fold_vec(x[j], v0 + j * BLOCK + tid);
+            }
+        }
     };
 
     uint32_t rec = load_rec(blockIdx.x);
@@ -184,7 +229,8 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
         load_row(in_row(r));
     }
     while (r < n_rows) {
-        char* ov = out_row(r);
+        char* const out = out_row(r);
+        char* const ov = out + head * Row<DT>::BYTES;
         const Lse tot = block_lse<kWavesPerBlock>(acc, sm_l);
         const int tloc = static_cast<int>(word(rec, R_TLOC));
         const float log_s = logf(tot.s), lse = tot.m + log_s;
@@ -202,17 +248,28 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
             ti.correct = 0.f;
             ti.den_s = valid_seqs(a.in) + 1e-8f;
             ti.den_t = valid_toks(a.in) + 1e-8f;
-            const TokenOut out = token_eval<false>(c, st, ti);
-            g = (out.d_actor + out.d_lpu) * a.loss_scale;
+            const TokenOut tok = token_eval<false>(c, st, ti);
+            g = (tok.d_actor + tok.d_lpu) * a.loss_scale;
+            if (EDGE && tid == 0 && a.row_grad) a.row_grad[r] = make_float4(g, lse, __int_as_float(tloc), 0.f);
             if (tid == 0) a.lp_out[static_cast<int64_t>(word(rec, R_SEQ)) * a.n_inner + word(rec, R_POS)] = lp;
         }
-        uint32_t rec_n = ahead;
-        const int64_t rn = advance(r + step, rec_n);
-        const float stats_n = load_stats(rn < n_rows ? rec_n : rec);
-        ahead = load_rec(rn + step);
-        const int tvec = tloc >= 0 ? tloc / EPV : -1;
-        const int tsub = tloc >= 0 ? tloc % EPV : -1;
+        const int tvec = tloc >= head ? (tloc - head) / EPV : -1;  // (of a target in the tail: no vector of the row)
+        const int tsub = tloc >= head ? (tloc - head) % EPV : -1;
         const RowGrad rg(lse, g, a.tparam);
+        if (EDGE && edge_at() >= 0) Row<DT>::store1(out, edge_at(), grad_elem<DT, TEMP>(edge_x, edge_at() == tloc, rg));
+        if (LONG) {
+            const char* base = in_row(r) + head * Row<DT>::BYTES;
+            for (int v0 = past + (nvec - 1 - past) / kStride * kStride; v0 >= past; v0 -= kStride) {
+                u32x4 x[kAhead];
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) x[j] = __builtin_nontemporal_load(vec_at(base, min(v0 + j * BLOCK + tid, nvec - 1)));
+#pragma unroll
+                for (int j = 0; j < kAhead; ++j) {
+                    const int v = v0 + j * BLOCK + tid;
+                    if (v < nvec) __builtin_nontemporal_store(grad_vec<DT, TEMP>(x[j], v == tvec ? tsub : -1, rg), const_cast<u32x4*>(vec_at(ov, v)));
+                }
+            }
+        }
 #pragma unroll
         for (int q = 0; q < kVec; ++q) {
             const int vc = slot_cl(q);
@@ -221,6 +278,10 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
             __builtin_nontemporal_store(d, const_cast<u32x4*>(vec_at(ov, vc)));
         }
         __builtin_amdgcn_sched_barrier(0);  // the stores stay together, and ahead of the loads
+        uint32_t rec_n = ahead;
+        const int64_t rn = advance(r + step, rec_n);
+        const float stats_n = load_stats(rn < n_rows ? rec_n : rec);
+        ahead = load_rec(rn + step);
         if (rn < n_rows) load_row(in_row(rn));
         // sm_l is rewritten only behind the first barrier of the next block_lse, which every thread passes after reading it
         r = rn;
@@ -229,17 +290,22 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
     }
 }
 
-template <int DT, int TEMP, int BLOCK, int NREG> void fused_launch(const FusedLaunch& l) {
-    // as many workgroups as are resident together: 1024 threads per compute unit at 128 registers, 64 KiB of LDS
+template <int DT, int TEMP, int BLOCK, int NREG, int NLDS = kFusedLdsVec, bool EDGE = false, bool LONG = false> void fused_launch(const FusedLaunch& l) {
+    // as many workgroups as are resident together: 1024 threads per compute unit at 128 registers, 64 (LONG: 128) KiB of LDS
     const int64_t resident = static_cast<int64_t>(l.compute_units) * (1024 / BLOCK);
     const dim3 grid(static_cast<unsigned>(l.n_rows < resident ? l.n_rows : resident)), block(BLOCK);
-    if (l.packed) fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, true><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
-    else fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, false><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
+    if (l.packed) fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, NLDS, EDGE, LONG, true><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
+    else fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, NLDS, EDGE, LONG, false><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
 }
 template <int DT, int TEMP, int BLOCK> void fused_launch(const FusedLaunch& l, int64_t slots) {
     if (slots <= 12) fused_launch<DT, TEMP, BLOCK, 8>(l);
     else if (slots <= 16) fused_launch<DT, TEMP, BLOCK, 12>(l);
     else fused_launch<DT, TEMP, BLOCK, 16>(l);
+}
+template <int DT, int TEMP, int BLOCK> void fused_launch_edge(const FusedLaunch& l, int64_t slots) {
+    if (slots <= 12) fused_launch<DT, TEMP, BLOCK, 8, kFusedLdsVec, true>(l);
+    else if (slots <= 16) fused_launch<DT, TEMP, BLOCK, 12, kFusedLdsVec, true>(l);
+    else fused_launch<DT, TEMP, BLOCK, 16, kFusedLdsVec, true>(l);
 }
 template <int DT, int TEMP> void fused_launch(const FusedLaunch& l) {
     const int64_t nvec = l.a.vocab / Row<DT>::EPV;
@@ -250,7 +316,20 @@ template <int DT, int TEMP> void fused_launch(const FusedLaunch& l) {
     else if (slots(512) <= kFusedMaxVec) fused_launch<DT, TEMP, 512>(l, slots(512));
     else fused_launch<DT, TEMP, 1024>(l, slots(1024));
 }
+template <int DT, int TEMP> void fused_launch_edge(const FusedLaunch& l) {
+    const int64_t nvec = l.a.vocab / Row<DT>::EPV;
+    auto slots = [&](int block) { return (nvec + block - 1) / block; };
+    if (slots(256) <= kFusedMaxVec) fused_launch_edge<DT, TEMP, 256>(l, slots(256));
+    else if (slots(512) <= kFusedMaxVec) fused_launch_edge<DT, TEMP, 512>(l, slots(512));
+    else if (slots(1024) <= kFusedMaxVec) fused_launch_edge<DT, TEMP, 1024>(l, slots(1024));
+    else fused_launch<DT, TEMP, 1024, 12, 8, true, true>(l);  // the larger LDS share leaves registers for the vectors past it
+}
 template <int DT> void fused_launch(const FusedLaunch& l) {
+    if (l.any_row) {  // (no divide: the caller's own is a multiplication)
+        if (l.temp == 0) fused_launch_edge<DT, 0>(l);
+        else fused_launch_edge<DT, 2>(l);
+        return;
+    }
     if (l.temp == 0) fused_launch<DT, 0>(l);
     else if (l.temp == 1) fused_launch<DT, 1>(l);
     else fused_launch<DT, 2>(l);

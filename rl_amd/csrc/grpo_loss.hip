@@ -20,6 +20,7 @@
 #include "common.hpp"
 #include "fused_rows.hpp"
 #include "grpo_token.hpp"
+#include "row_grad.hpp"
 
 namespace nrl {
 
@@ -353,6 +354,7 @@ __global__ __launch_bounds__(kSeqBlock) void fused_prep_kernel(FusedArgs a, int6
         const int64_t first = (b - in.batch) * kSeqBlock + threadIdx.x, step = (gridDim.x - in.batch) * kSeqBlock;
         for (int64_t i = first; i < in.batch * n; i += step) a.lp_out[i] = 0.f;
         for (int64_t r = first; r < n_rows; r += step) {
+            if (a.row_grad) a.row_grad[r] = make_float4(0.f, 0.f, 0.f, 0.f);
             FusedPos q;
             int64_t off;
             if (a.cu) {
@@ -826,7 +828,7 @@ extern "C" int64_t nrl_fused_packed_workspace_bytes(int64_t n_seq, int64_t n_inn
 
 // rows describes the logits; with cu != NULL it is one packed row of rows->n_inner positions (n_outer 1) and
 // the loss inputs are [n_seq, in->sm1]
-static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float loss_scale, void* dlogits,
+static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float loss_scale, float* row_grad, void* dlogits,
                       int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out, float* loss_out,
                       float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream, const int32_t* cu,
                       int64_t n_seq, int pre_rolled) {
@@ -849,12 +851,22 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     if (seq_weights && in->batch * in->sm1 > 0 && !in->prev) return fail(NRL_E_INVALID, "prev_logprobs is NULL");
     if (cfg->kl_type < 1 || cfg->kl_type > 3 || cfg->tis_type < 0 || cfg->tis_type > 3) return fail(NRL_E_INVALID, "bad kl_type or tis_type");
     const int bytes = rows->dtype == NRL_F32 ? 4 : 2, epv = 16 / bytes;
-    if (rows->vocab % epv || rows->vocab / epv > static_cast<int64_t>(kFusedMaxVec) * 1024)
-        return fail(NRL_E_UNSUPPORTED, "row does not fit the on-chip path (vocab %lld)", (long long)rows->vocab);
-    if ((reinterpret_cast<uintptr_t>(rows->logits) & 15) || (reinterpret_cast<uintptr_t>(dlogits) & 15) ||
-        (rows->stride_outer * bytes) % 16 || (rows->stride_inner * bytes) % 16 || (d_stride_outer * bytes) % 16 ||
-        (d_stride_inner * bytes) % 16)
-        return fail(NRL_E_UNSUPPORTED, "rows must be 16-byte aligned");
+    const uintptr_t xa = reinterpret_cast<uintptr_t>(rows->logits), da = reinterpret_cast<uintptr_t>(dlogits);
+    if (row_grad) {
+        if (rows->vocab * bytes < NRL_FUSED_ANY_ROW_MIN || rows->vocab * bytes > NRL_FUSED_ANY_ROW_MAX)
+            return fail(NRL_E_UNSUPPORTED, "row of %lld bytes", (long long)(rows->vocab * bytes));
+        if (((xa - da) & 15) || ((rows->stride_outer - d_stride_outer) * bytes) % 16 || ((rows->stride_inner - d_stride_inner) * bytes) % 16 || xa % bytes)
+            return fail(NRL_E_UNSUPPORTED, "logits and gradient rows sit differently on the 16-byte grid");
+        if (xa && xa == da) return fail(NRL_E_UNSUPPORTED, "the gradient cannot be written over the logits");
+        if (rows->temperature != 1.0f && rows->temp_mode != NRL_TEMP_RCP) return fail(NRL_E_UNSUPPORTED, "temperature as a divide");
+        if (reinterpret_cast<uintptr_t>(row_grad) & 15) return fail(NRL_E_INVALID, "row_grad must be 16-byte aligned");
+    } else {
+        if (rows->vocab % epv || rows->vocab / epv > static_cast<int64_t>(kFusedMaxVec) * 1024)
+            return fail(NRL_E_UNSUPPORTED, "row does not fit the on-chip path (vocab %lld)", (long long)rows->vocab);
+        if ((xa & 15) || (da & 15) || (rows->stride_outer * bytes) % 16 || (rows->stride_inner * bytes) % 16 ||
+            (d_stride_outer * bytes) % 16 || (d_stride_inner * bytes) % 16)
+            return fail(NRL_E_UNSUPPORTED, "rows must be 16-byte aligned");
+    }
     const int64_t n_rows = rows->n_outer * d_n_inner;
     if (n_rows >= (1ll << 31)) return fail(NRL_E_INVALID, "more than 2^31 rows in one launch");
     if (in->batch * terms_chunks(in->sm1) >= (1ll << 31)) return fail(NRL_E_INVALID, "more than 2^31 shares of sequences");
@@ -873,6 +885,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     a.in = *in;
     a.in.lp = nullptr; a.in.lpu = nullptr;
     a.cu = cu; a.n_seq = n_seq; a.pre_rolled = pre_rolled;
+    a.row_grad = reinterpret_cast<float4*>(row_grad);
     a.logits = rows->logits; a.n_inner = in->sm1; a.d_n_inner = d_n_inner; a.vocab = rows->vocab;
     a.stride_outer = rows->stride_outer; a.stride_inner = rows->stride_inner;
     a.targets = rows->targets; a.ts_outer = rows->tgt_stride_outer; a.ts_inner = rows->tgt_stride_inner;
@@ -899,7 +912,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             return fail(NRL_E_LAUNCH, "cannot read the device's compute-unit count");
-        const FusedLaunch l{a, tc, cu != nullptr, n_rows, cus, s};
+        const FusedLaunch l{a, tc, cu != nullptr, n_rows, row_grad != nullptr, cus, s};
         if (rows->dtype == NRL_F32) launch_fused_f32(l);
         else if (rows->dtype == NRL_BF16) launch_fused_bf16(l);
         else launch_fused_f16(l);
@@ -919,7 +932,7 @@ extern "C" int nrl_fused_logits_grpo_loss(const nrl_rows* rows, const nrl_grpo_c
                                           float loss_scale, void* dlogits, int64_t d_n_inner, int64_t d_stride_outer,
                                           int64_t d_stride_inner, float* logprob_out, float* loss_out, float* metrics_out,
                                           void* workspace, int64_t workspace_bytes, void* stream) {
-    return fused_impl(rows, cfg, in, loss_scale, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
+    return fused_impl(rows, cfg, in, loss_scale, nullptr, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
                       metrics_out, workspace, workspace_bytes, stream, nullptr, 0, 0);
 }
 
@@ -930,6 +943,72 @@ extern "C" int nrl_fused_packed_logits_grpo_loss(const nrl_rows* rows, int32_t t
                                                  void* stream) {
     if (!cu_seqlens) return fail(NRL_E_INVALID, "cu_seqlens is NULL");
     if (rows && rows->tgt_stride_inner != 1) return fail(NRL_E_INVALID, "packed targets must be contiguous");
-    return fused_impl(rows, cfg, in, loss_scale, dlogits, rows ? rows->n_inner : 0, 0, d_row_stride, logprob_out, loss_out,
+    return fused_impl(rows, cfg, in, loss_scale, nullptr, dlogits, rows ? rows->n_inner : 0, 0, d_row_stride, logprob_out, loss_out,
                       metrics_out, workspace, workspace_bytes, stream, cu_seqlens, n_seq, target_is_pre_rolled);
+}
+
+extern "C" int nrl_fused_any_row_grpo_loss(const nrl_rows* rows, int32_t target_is_pre_rolled, const int32_t* cu_seqlens, int64_t n_seq,
+                                           const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float* row_grad_out, void* dlogits,
+                                           int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out,
+                                           float* loss_out, float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream) {
+    if (!row_grad_out) return fail(NRL_E_INVALID, "row_grad_out is NULL");
+    if (cu_seqlens && rows && rows->tgt_stride_inner != 1) return fail(NRL_E_INVALID, "packed targets must be contiguous");
+    return fused_impl(rows, cfg, in, 1.f, row_grad_out, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
+                      metrics_out, workspace, workspace_bytes, stream, cu_seqlens, n_seq, target_is_pre_rolled);
+}
+
+// The gradient of the rows again, for another upstream factor than the one it was written for (read from the device: with the
+// same factor nothing is done).  The factor multiplies d loss / d logprob before the row is formed, so a gradient is rounded
+// once whatever it is.
+struct RowsGradArgs {
+    const void* logits;
+    int64_t n_inner, vocab, stride_outer, stride_inner;
+    void* d;
+    int64_t ds_outer, ds_inner;
+    const float4* row_grad;
+    const float* factor;
+    float written;
+    float tparam;
+};
+template <int DT, int TEMP> __global__ __launch_bounds__(kBlock) void rows_grad_kernel(RowsGradArgs a, int64_t n_rows) {
+    const float f = *a.factor;
+    if (f == a.written) return;
+    for (int64_t r = blockIdx.x; r < n_rows; r += gridDim.x) {
+        const int64_t o = r / a.n_inner, i = r - o * a.n_inner;
+        char* out = static_cast<char*>(a.d) + (o * a.ds_outer + i * a.ds_inner) * Row<DT>::BYTES;
+        const float4 w = a.row_grad[r];
+        const float g = w.x * f;
+        if (g == 0.f) {
+            row_zero<DT>(out, a.vocab);
+            continue;
+        }
+        const char* row = static_cast<const char*>(a.logits) + (o * a.stride_outer + i * a.stride_inner) * Row<DT>::BYTES;
+        row_write_grad<DT, TEMP>(row, out, a.vocab, w.y, g, __float_as_int(w.z), a.tparam);
+    }
+}
+
+extern "C" int nrl_rows_grad(const nrl_rows* rows, const float* row_grad, const float* factor, float written, void* dlogits,
+                             int64_t d_stride_outer, int64_t d_stride_inner, void* stream) {
+    if (!rows) return fail(NRL_E_INVALID, "rows_grad: null argument");
+    if (rows->dtype != NRL_F32 && rows->dtype != NRL_BF16 && rows->dtype != NRL_F16) return fail(NRL_E_INVALID, "unknown logits dtype");
+    if (rows->n_outer < 0 || rows->n_inner < 0 || rows->vocab <= 0 || rows->vocab >= (1ll << 31)) return fail(NRL_E_INVALID, "bad shape");
+    if (!(rows->temperature > 0.f) || (rows->temperature != 1.0f && rows->temp_mode != NRL_TEMP_RCP))
+        return fail(NRL_E_UNSUPPORTED, "rows_grad: temperature must be a positive multiplication");
+    const int64_t n_rows = rows->n_outer * rows->n_inner;
+    if (n_rows == 0) return NRL_OK;
+    if (!rows->logits || !row_grad || !factor || !dlogits) return fail(NRL_E_INVALID, "rows_grad: null pointer");
+    const bool temp = rows->temperature != 1.0f;
+    const RowsGradArgs a{rows->logits, rows->n_inner, rows->vocab, rows->stride_outer, rows->stride_inner, dlogits, d_stride_outer, d_stride_inner,
+                         reinterpret_cast<const float4*>(row_grad), factor, written, temp ? 1.0f / rows->temperature : 1.f};
+    const dim3 grid((unsigned)(n_rows < 2048 ? n_rows : 2048)), block(kBlock);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    switch (rows->dtype * 2 + (temp ? 1 : 0)) {
+        case NRL_F32 * 2: rows_grad_kernel<NRL_F32, 0><<<grid, block, 0, s>>>(a, n_rows); break;
+        case NRL_F32 * 2 + 1: rows_grad_kernel<NRL_F32, 2><<<grid, block, 0, s>>>(a, n_rows); break;
+        case NRL_BF16 * 2: rows_grad_kernel<NRL_BF16, 0><<<grid, block, 0, s>>>(a, n_rows); break;
+        case NRL_BF16 * 2 + 1: rows_grad_kernel<NRL_BF16, 2><<<grid, block, 0, s>>>(a, n_rows); break;
+        case NRL_F16 * 2: rows_grad_kernel<NRL_F16, 0><<<grid, block, 0, s>>>(a, n_rows); break;
+        default: rows_grad_kernel<NRL_F16, 2><<<grid, block, 0, s>>>(a, n_rows); break;
+    }
+    return check_launch("rows_grad");
 }

@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <limits>
 #include <memory>
 #include <optional>
 #include <string>
@@ -283,11 +284,11 @@ GrpoOut grpo_loss(const Tensor& lp_in, const Tensor& lpu_in, const LossData& d, 
 }
 
 struct FusedOut {
-    Tensor loss, dlogits, lp, metrics;
+    Tensor loss, dlogits, lp, metrics, row_grad;
 };
 // cu not defined: logits [B, S, V], targets [B, >= n_inner]; otherwise packed logits [T, V] and targets [>= T]
 FusedOut fused_loss(const Tensor& logits, const Tensor& targets, int64_t n_inner, const Tensor& cu, bool pre_rolled, const LossData& d,
-                    const nrl_grpo_cfg& cfg, double loss_scale, double temperature, int64_t mode, bool in_place) {
+                    const nrl_grpo_cfg& cfg, double loss_scale, double temperature, int64_t mode, bool in_place, bool any_row = false) {
     need_gpu(logits, targets, cu);
     const bool packed = cu.defined();
     nrl_rows rows;
@@ -309,12 +310,18 @@ FusedOut fused_loss(const Tensor& logits, const Tensor& targets, int64_t n_inner
     }
     const c10::OptionalDeviceGuard guard(logits.device());
     const LossInputs l = loss_inputs(d, logits, b, n_inner);
-    FusedOut o{f32({}, logits), in_place ? logits : grad_buffer(logits.sizes(), logits), f32({b, n_inner}, logits), f32({NRL_GRPO_N_METRICS}, logits)};
+    FusedOut o{f32({}, logits), in_place ? logits : grad_buffer(logits.sizes(), logits), f32({b, n_inner}, logits), f32({NRL_GRPO_N_METRICS}, logits), Tensor()};
     const int64_t bytes = packed ? nrl_fused_packed_workspace_bytes(b, n_inner, logits.size(0)) : nrl_fused_workspace_bytes(b, n_inner);
     const Tensor ws = workspace(bytes, logits);
     const float scale = static_cast<float>(loss_scale);
     Timed timed(packed ? "fused_packed_logits_loss" : "fused_logits_loss");
-    if (packed)
+    if (any_row) {
+        const int64_t per = packed ? logits.size(0) : logits.size(1);
+        o.row_grad = f32({packed ? per : b * per, 4}, logits);
+        check(nrl_fused_any_row_grpo_loss(&rows, pre_rolled, packed ? ptr<int32_t>(cu) : nullptr, packed ? b : 0, &cfg, &l.in, ptr(o.row_grad),
+                                          ptr<void>(o.dlogits), per, packed ? 0 : o.dlogits.stride(0), o.dlogits.stride(packed ? 0 : 1), ptr(o.lp),
+                                          ptr(o.loss), ptr(o.metrics), ws.data_ptr(), ws.numel() * 8, stream_of(logits)), "nrl_fused_any_row_grpo_loss");
+    } else if (packed)
         check(nrl_fused_packed_logits_grpo_loss(&rows, pre_rolled, ptr<int32_t>(cu), b, &cfg, &l.in, scale, ptr<void>(o.dlogits), o.dlogits.stride(0),
                                                 ptr(o.lp), ptr(o.loss), ptr(o.metrics), ws.data_ptr(), ws.numel() * 8, stream_of(logits)),
               "nrl_fused_packed_logits_grpo_loss");
@@ -537,6 +544,46 @@ struct FusedLoss : torch::autograd::Function<FusedLoss> {
     }
 };
 
+// The single pass over rows off the 16-byte grid or longer than the chip holds.  Here the logits are saved, with 16 bytes per row:
+// the gradient can be written again, which an upstream factor other than 1 and a second backward through the same graph need.
+struct FusedRowsLoss : torch::autograd::Function<FusedRowsLoss> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, const FusedArgs& a) {
+        ctx->set_materialize_grads(false);
+        const Tensor logits = logits_in.detach();
+        FusedOut o = fused_loss(logits, a.targets, a.n_inner, a.cu, true, a.data, a.cfg, 1.0, a.temperature, a.mode, false, true);
+        ctx->save_for_backward({logits, o.row_grad});
+        ctx->saved_data["dlogits"] = o.dlogits;
+        ctx->saved_data["temperature"] = a.temperature;
+        ctx->saved_data["mode"] = a.mode;
+        ctx->mark_non_differentiable({o.metrics});
+        return {o.loss, o.metrics};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        variable_list out(2);
+        if (!grads[0].defined()) return out;
+        const auto saved = ctx->get_saved_variables();
+        const Tensor logits = saved[0].dim() == 3 ? saved[0] : saved[0].unsqueeze(0);
+        const Tensor factor = to_f32(grads[0].detach(), logits);
+        const c10::OptionalDeviceGuard guard(logits.device());
+        Tensor d;
+        float written = 1.f;
+        const auto it = ctx->saved_data.find("dlogits");
+        if (it != ctx->saved_data.end()) {
+            d = it->second.toTensor();
+            ctx->saved_data.erase(it);
+        } else {
+            d = grad_buffer(saved[0].sizes(), saved[0]);
+            written = std::numeric_limits<float>::quiet_NaN();
+        }
+        const nrl_rows rows = make_rows(logits, Tensor(), logits.size(1), 0, logits.size(2), ctx->saved_data["temperature"].toDouble(), ctx->saved_data["mode"].toInt());
+        Timed timed("rows_grad");
+        check(nrl_rows_grad(&rows, ptr(saved[1]), ptr(factor), written, ptr<void>(d), d.dim() == 3 ? d.stride(0) : 0, d.stride(d.dim() - 2), stream_of(logits)),
+              "nrl_rows_grad");
+        out[0] = d;
+        return out;
+    }
+};
+
 // filtered logprobs (and, when asked for, the unfiltered ones the KL term needs, without a gradient)
 struct RowsLogprobSampled : torch::autograd::Function<RowsLogprobSampled> {
     static Tensor forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& targets, int64_t n_inner, int64_t top_k, double top_p, bool inference_only,
@@ -743,12 +790,12 @@ PYBIND11_MODULE(_host, m) {
     m.def("fused_clipped_pg", [](const Tensor& logits, const Tensor& targets, int64_t shift, int64_t n_inner, const OptTensor& cu, const OptTensor& prev,
                                  const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
                                  const Tensor& seqs, const Tensor& toks, const std::vector<int64_t>& iflags, const std::vector<double>& fparams,
-                                 double loss_scale, double temperature, int64_t mode, bool in_place) {
+                                 double loss_scale, double temperature, int64_t mode, bool in_place, bool any_row) {
         Tensor t = targets.device() == logits.device() && targets.scalar_type() == at::kLong ? targets : targets.to(logits.device(), at::kLong);
         if (shift) t = t.narrow(1, shift, t.size(1) - shift);
         const FusedArgs a{t, opt(cu), n_inner, loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, seqs, toks, 1), make_cfg(iflags, fparams),
                           loss_scale, temperature, mode, in_place};
-        const variable_list o = FusedLoss::apply(logits, a);
+        const variable_list o = any_row ? FusedRowsLoss::apply(logits, a) : FusedLoss::apply(logits, a);
         return std::make_tuple(o[0], o[1]);
     });
     m.def("gather_entropy", [](const Tensor& logits, const Tensor& indices, int64_t n, bool entropy) {

@@ -1,0 +1,138 @@
+"""The single pass over rows off the 16-byte grid or longer than the chip holds, reached through the wrappers, against the
+three-pass path.  The two sum a row's exponentials in different orders (about 1e-6 in the log-sum-exp), and round a gradient
+element to its type once: neighbouring 16-bit values may differ, fp32 values by 1e-4 of the largest as in test_gpu_fused."""
+
+import pytest
+import torch
+
+from rl_amd.algorithms.logits_sampling_utils import TrainingSamplingParams
+from rl_amd.algorithms.loss import (
+    ClippedPGLossConfig,
+    ClippedPGLossFn,
+    SequencePackingFusionLossWrapper,
+    prepare_loss_input,
+    prepare_packed_loss_input,
+    wrap_loss_fn_with_input_preparation,
+)
+from rl_amd.algorithms.loss.fused import any_row_fusable, why_not_fusable
+from rl_amd.temperature import apply_temperature_scaling, deferred_temperature
+from test_gpu_fused import _batch, _close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _same_gradient(got, want, dtype):
+    got, want = got.float(), want.float()
+    scale = want.abs().max().item()
+    step = 0.0 if dtype == torch.float32 else 2.0 ** -7
+    assert bool(((got - want).abs() <= want.abs() * (step + 1e-4) + 1e-4 * scale * (1.0 if dtype == torch.float32 else 2.0 ** -8)).all())
+
+
+def _three_pass(x, data, fn, gs, gt, **kw):
+    loss_input, d2 = prepare_loss_input(x, dict(data), fn, **kw)
+    return fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)
+
+
+def _setup(b, s, vocab, dtype):
+    logits, data, gs, gt = _batch(b, s, vocab, dtype, seed=vocab)
+    return logits.to(DEV), {k: v.to(DEV) for k, v in data.items()}, gs.to(DEV), gt.to(DEV)
+
+
+SHAPES = [
+    (torch.bfloat16, 513), (torch.bfloat16, 4103), (torch.bfloat16, 24581), (torch.bfloat16, 40961), (torch.bfloat16, 50257),
+    (torch.bfloat16, 81927), (torch.bfloat16, 98305), (torch.bfloat16, 163841), (torch.bfloat16, 163848), (torch.bfloat16, 262144),
+    (torch.bfloat16, 229381), (torch.float16, 50257), (torch.float16, 170003), (torch.float32, 257), (torch.float32, 20483),
+    (torch.float32, 81921), (torch.float32, 81924), (torch.float32, 98308), (torch.float32, 151936), (torch.float32, 262143),
+]
+
+
+@pytest.mark.parametrize("dtype,vocab", SHAPES)
+def test_rows_of_any_length_and_alignment(dtype, vocab):
+    logits, data, gs, gt = _setup(3, 7, vocab, dtype)
+    data["input_ids"][0, 4] = vocab - 1  # a target in the tail, and one in front of the first boundary of its row
+    data["input_ids"][0, 5] = 0
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    xf, xu = (logits.clone().requires_grad_(True) for _ in range(2))
+    assert why_not_fusable(fn, xf, data) is not None and any_row_fusable(fn, xf, data)
+    got, gm = wrap_loss_fn_with_input_preparation(xf, data, gs, gt, fn, prepare_loss_input)
+    want, wm = _three_pass(xu, data, fn, gs, gt)
+    assert _close(got.item(), want.item(), rel=1e-4)
+    for k in wm:
+        assert _close(float(gm[k]), float(wm[k])), k
+    got.backward()
+    want.backward()
+    _same_gradient(xf.grad, xu.grad, dtype)
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1027), (torch.float32, 90001)])
+def test_more_rows_than_workgroups_and_other_factors(dtype, vocab):
+    """An upstream factor that is no power of two (rounded once), and a second backward through the same graph."""
+    logits, data, gs, gt = _setup(4, 300 if vocab < 2000 else 90, vocab, dtype)
+    fn = ClippedPGLossFn(ClippedPGLossConfig(reference_policy_kl_penalty=0.0, ratio_clip_min=0.2, ratio_clip_max=0.28))
+    xf, xu = (logits.clone().requires_grad_(True) for _ in range(2))
+    got, _ = wrap_loss_fn_with_input_preparation(xf, data, gs, gt, fn, prepare_loss_input)
+    want, _ = _three_pass(xu, data, fn, gs, gt)
+    for factor in (1.0, 0.3, 1.0):
+        (df,) = torch.autograd.grad(got * factor, xf, retain_graph=True)
+        (du,) = torch.autograd.grad(want * factor, xu, retain_graph=True)
+        _same_gradient(df, du, dtype)
+    (0.7 * got).backward()
+    (0.7 * want).backward()
+    _same_gradient(xf.grad, xu.grad, dtype)
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 4099), (torch.float32, 81930)])
+def test_temperature_strides_and_refusals(dtype, vocab):
+    logits, data, gs, gt = _setup(3, 7, vocab, dtype)
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    params = TrainingSamplingParams(temperature=0.7)
+    xf, xu = (logits.clone().requires_grad_(True) for _ in range(2))
+    with deferred_temperature():
+        zf = apply_temperature_scaling(xf * 1.0, params)
+        got, _ = wrap_loss_fn_with_input_preparation(zf, data, gs, gt, fn, prepare_loss_input)
+    want, _ = _three_pass(apply_temperature_scaling(xu * 1.0, params), data, fn, gs, gt)
+    got.backward()
+    want.backward()
+    assert _close(got.item(), want.item(), rel=1e-4)
+    _same_gradient(xf.grad, xu.grad, dtype)
+    # rows inside a wider buffer: alike modulo 16 bytes when the padding is a multiple of that, the general path otherwise
+    per = 16 // logits.element_size()
+    for pad, route in ((2 * per, True), (1, False)):
+        wide = torch.zeros(3, 7, vocab + pad, dtype=dtype, device=DEV)
+        wide[..., :vocab] = logits
+        xw = wide[..., :vocab].requires_grad_(True)
+        assert any_row_fusable(fn, xw, data) is route
+        got, _ = wrap_loss_fn_with_input_preparation(xw, data, gs, gt, fn, prepare_loss_input)
+        (dw,) = torch.autograd.grad(got, xw)
+        xu = logits.clone().requires_grad_(True)
+        (du,) = torch.autograd.grad(_three_pass(xu, data, fn, gs, gt)[0], xu)
+        _same_gradient(dw, du, dtype)
+    assert not any_row_fusable(fn, logits[..., 1:], data) and not any_row_fusable(fn, logits[..., :100], data)
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 1029), (torch.bfloat16, 180003), (torch.float32, 82001)])
+def test_packed_rows(dtype, vocab):
+    logits, data, gs, gt = _setup(3, 8, vocab, dtype)
+    lens, cuts = [8, 5, 1], [12, 6, 3]
+    cu = torch.tensor([0, 8, 13, 14], dtype=torch.int32, device=DEV)
+    cup = torch.tensor([0, 12, 18, 21], dtype=torch.int32, device=DEV)
+    data["sample_mask"][:] = 1
+    data["token_mask"][:] = 1
+    for i, n in enumerate(lens):
+        data["token_mask"][i, n:] = 0
+    gt = data["token_mask"][:, 1:].sum()
+    g = torch.Generator().manual_seed(3)
+    x = (torch.randn(1, sum(cuts) + 2, vocab, generator=g) * 2).to(dtype).to(DEV)
+    fn = ClippedPGLossFn(ClippedPGLossConfig(token_level_loss=False, reference_policy_kl_penalty=0.001))
+    xf, xu = (x.clone().requires_grad_(True) for _ in range(2))
+    got, gm = SequencePackingFusionLossWrapper(fn, prepare_packed_loss_input, cu, cup)(xf, data, gs, gt)
+    loss_input, d2 = prepare_packed_loss_input(xu, dict(data), fn, cu, cup)
+    want, wm = fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)
+    assert _close(got.item(), want.item(), rel=1e-4)
+    for k in wm:
+        assert _close(float(gm[k]), float(wm[k])), k
+    for factor in (1.0, 0.3):
+        (df,) = torch.autograd.grad(got * factor, xf, retain_graph=True)
+        (du,) = torch.autograd.grad(want * factor, xu, retain_graph=True)
+        _same_gradient(df, du, dtype)
