@@ -47,6 +47,7 @@ constexpr int kChunks = kSelBlock * kSub;    // 2048
 constexpr int kCap = 4096;                   // candidate capacity (LDS); rows under a small top-k use kCapSmall
 constexpr int kCapSmall = 2048;              // ... which lets six workgroups share a compute unit instead of three
 constexpr int kSmallTopK = 512;
+constexpr int kSeqList = 512;                // top-p alone: longer candidate lists are summed in double
 
 struct Lse2 {
     float m, s;
@@ -141,6 +142,13 @@ __device__ __forceinline__ float wave_seq_sum_desc(const float* e, int n) {
         for (int i = kWave - 1; i >= 0; --i) s += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), i));
     }
     return s;
+}
+
+// sum of e[0 .. n) in double; called by every lane of one wave, which all return it
+__device__ __forceinline__ float wave_sum_list(const float* e, int n) {
+    double s = 0.0;
+    for (int i = threadIdx.x & (kWave - 1); i < n; i += kWave) s += static_cast<double>(e[i]);
+    return static_cast<float>(wave_sum_double(s));
 }
 
 // descending bitonic sort of sh.cand[0 .. n_pad)
@@ -605,10 +613,15 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
     for (int i = tid; i < n_k; i += kSelBlock)
         sh.expv[i] = expf(key_value(static_cast<uint32_t>(sh.cand[i] >> 32)) - m);
     __syncthreads();
+    // Short lists are summed element by element, in the order of a sorted cumulative sum in fp32.  Over thousands of elements
+    // that order means nothing any more (every implementation of the sum takes its own), and it costs one dependent addition
+    // per element, three times.  Long lists under top-p alone are summed in double, by the lanes side by side: 1500 rows of
+    // V = 151936 under top_p 0.95, kept sets from a few tokens to thousands: 509 -> 476 us.
+    const bool long_list = PONLY && n_k > kSeqList;
     if (tid < kWave) {  // one wave; every lane computes the same scalars, lane 0 writes them
         int n_keep = n_k;
         if (use_p) {
-            float s_k = wave_seq_sum_desc(sh.expv, n_k);
+            float s_k = long_list ? wave_sum_list(sh.expv, n_k) : wave_seq_sum_desc(sh.expv, n_k);
             // ascending cumulative probability, smallest kept value first; keep while it exceeds 1 - p
             const float cut = 1.0f - a.top_p;
             float cum = 0.f;
@@ -625,7 +638,21 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
             // under the cut and is taken off again), index 0 is always kept and never enters the sum.
             const int top_blk = (n_k - 1) / kWave;
             int steps_under = 0;
-            for (int blk = top_blk; blk >= 0; --blk) {
+            double run = cum;
+            if (long_list) {
+                for (int blk = top_blk; blk >= 0 && run <= cut; --blk) {
+                    const int idx = blk * kWave + tid;
+                    double v = (idx >= 1 && idx < n_k) ? static_cast<double>(sh.expv[idx] / s_k) : 0.0;
+#pragma unroll
+                    for (int off = 1; off < kWave; off <<= 1) {
+                        const double up = __shfl_down(v, off, kWave);
+                        if (tid + off < kWave) v += up;
+                    }
+                    steps_under += __popcll(__ballot(run + v <= cut));
+                    run += lane_double(v, 0);
+                }
+            }
+            for (int blk = long_list ? -1 : top_blk; blk >= 0; --blk) {
                 const int idx = blk * kWave + tid;
                 const float v = (idx >= 1 && idx < n_k) ? sh.expv[idx] / s_k : 0.f;
 #pragma unroll
@@ -640,7 +667,7 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
             if (n_keep < 1) n_keep = 1;
             if (n_keep > n_k) n_keep = n_k;
         }
-        const float s = wave_seq_sum_desc(sh.expv, n_keep);
+        const float s = long_list ? wave_sum_list(sh.expv, n_keep) : wave_seq_sum_desc(sh.expv, n_keep);
         const unsigned long long last = sh.cand[n_keep - 1];
         const uint32_t last_key = static_cast<uint32_t>(last >> 32);
         int tie = 0;

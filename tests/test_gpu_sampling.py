@@ -474,3 +474,28 @@ def test_wide_rows_come_out_the_same_every_time():
         again = ops.topk_topp_logprob_fwd(x, t, n, 0, 0.95, 0.7, NRL_TEMP_RCP, True)
         for a, b in zip(first, again):
             assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("nucleus", [500, 512, 513, 700, 1300, 3900])
+def test_nuclei_around_the_length_that_is_summed_in_double(nucleus):
+    """Top-p alone with about `nucleus` kept ids, against 64-bit sums: the kept set is the heaviest ids, holds top_p of the mass and
+    would not without its lightest (both up to 1e-5, the fp32 rounding of the log-sum-exp and of thousands of quotients), and
+    logprobs are normalised over exactly that set."""
+    from rl_amd.distributed.sampling_logprob import filter_logits, rows_logprob_sampled
+
+    g = torch.Generator(device="cuda").manual_seed(nucleus)
+    rows, vocab, top_p = 24, 30000, 0.95
+    x = torch.randn(1, rows, vocab, generator=g, device="cuda") * 0.3 - 9.0
+    heavy = torch.rand(rows, vocab, generator=g, device="cuda").topk(nucleus + 40, dim=-1).indices
+    x[0].scatter_(1, heavy, torch.randn(rows, nucleus + 40, generator=g, device="cuda") * 0.3)
+    _, keep = filter_logits(x, None, top_p)
+    x64, keep = x[0].double(), keep[0]
+    p = x64.softmax(-1)
+    mass, lightest = (p * keep).sum(-1), p.masked_fill(~keep, 2.0).amin(-1)
+    assert int(keep.sum(-1).amin()) > nucleus // 2
+    assert bool((mass >= top_p - 1e-5).all()) and bool((mass - lightest <= top_p + 1e-5).all())
+    assert bool((x64.masked_fill(keep, -1e9).amax(-1) <= x64.masked_fill(~keep, 1e9).amin(-1)).all())
+    ids = x[0].argmax(-1)
+    lp = rows_logprob_sampled(x, ids[None], rows, None, top_p, inference_only=True)[0]
+    want = x64.gather(-1, ids[:, None])[:, 0] - x64.masked_fill(~keep, float("-inf")).logsumexp(-1)
+    torch.testing.assert_close(lp.double(), want, rtol=0, atol=3e-6)  # fp32 logarithm and difference of values up to 9
