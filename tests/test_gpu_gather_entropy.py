@@ -76,3 +76,33 @@ def test_minus_infinity_logits_have_no_entropy_and_no_gradient():
     assert abs(h.item() - (p * p.log()).sum().item()) <= 1e-6
     d = _ops().gather_entropy_bwd(x, idx, 1, lse, h, torch.ones(1, 1, device=DEV), torch.ones(1, 1, 1, device=DEV))
     assert bool(torch.isfinite(d).all()) and d[0, 0, 1].item() == 0.0 and d[0, 0, 3].item() == 0.0
+
+
+@pytest.mark.parametrize("dtype,value", [(torch.float32, v) for v in (-1e6, 1e12, -1e12, -6e29, -1e30, 3e38, torch.finfo(torch.float32).min)]
+                         + [(torch.bfloat16, v) for v in (1e12, -7e29, -1e30, torch.finfo(torch.bfloat16).min)]
+                         + [(torch.float16, torch.finfo(torch.float16).min)])
+@pytest.mark.parametrize("vocab", [8192, 8201])
+def test_flat_rows_of_any_magnitude(dtype, value, vocab):
+    """A row whose logits are all alike, as one masked whole is, and the same with one ordinary logit."""
+    x = torch.full((1, 2, vocab), value, dtype=dtype, device=DEV)
+    x[0, 1, 5] = 1.0 if value < 0 else torch.finfo(dtype).max
+    idx = torch.tensor([[[0, 5], [0, 5]]], device=DEV)
+    out, h, lse = _ops().gather_entropy_fwd(x, idx, 2, True)
+    flat, log_v = x[0, 0, 0].double().item(), torch.tensor(float(vocab)).log().item()
+    unit = abs(flat) * 2.0 ** -23  # the log-sum-exp is one fp32 number of this size, the logprobs are differences from it
+    assert abs(h[0, 0].item() + log_v) <= 1e-5 and abs(lse[0, 0].double().item() - flat - log_v) <= unit + 1e-5
+    assert bool(((out[0, 0].double() + log_v).abs() <= max(unit, log_v if unit > 1 else 0.0) + 1e-5).all())
+    assert h[0, 1].item() == 0.0 and lse[0, 1].item() == x[0, 1, 5].float().item() and out[0, 1, 1].item() == 0.0
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_long_rows_keep_the_precision_of_fp32(dtype):
+    """2-norm of the error against 64 bits: the log-sum-exp and the difference from it round once each, 2^-24 of numbers up to
+    1.5 times the results; sums of 262144 terms must not add to that."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = (torch.randn(1, 64, 262144, generator=g, device=DEV) * torch.linspace(2, 6, 64, device=DEV).view(1, 64, 1)).to(dtype)
+    idx = torch.randint(0, 262144, (1, 64, 32), generator=g, device=DEV)
+    out, h, _ = _ops().gather_entropy_fwd(x, idx, 64, True)
+    lp = x.double().log_softmax(-1)
+    for got, want in ((out, lp.gather(-1, idx)), (h, (lp.exp() * lp).sum(-1))):
+        assert ((got.double() - want).norm() / want.norm()).item() <= 2.0 ** -23
