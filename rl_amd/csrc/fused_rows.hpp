@@ -39,6 +39,7 @@ struct FusedArgs {
     const int32_t* cu;
     int64_t n_seq;
     int pre_rolled;
+    int any_row;       // rows off the 16-byte grid, or longer than the chip holds
     float4* row_grad;  // NULL or [rows]: (d loss / d logprob at loss_scale 1, log-sum-exp, target or -1 as bits, 0) of every row, from
                        // which the gradient can be written again; zeros for rows without a token
 };

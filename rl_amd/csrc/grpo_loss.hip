@@ -442,7 +442,10 @@ __global__ __launch_bounds__(kTermsBlock) void grpo_terms_reduce_kernel(FusedArg
     for (int k = 0; k < P_R_MIN; ++k) acc[k] = 0;
     float r_min = INFINITY, r_max = -INFINITY, rc_min = INFINITY, rc_max = -INFINITY;
     bool live = t < a.n_inner;
-    if (live && a.cu) {  // a position that has a packed row
+    // Packed sequences may hold fewer rows than the loss inputs have columns.  On any_row rows a token of the mask beyond its
+    // sequence's rows counts with a logprob of 0 (what lp_out holds there), as the unpacked logprobs of the general path
+    // make it count; on aligned rows it does not count.
+    if (live && a.cu && !a.any_row) {
         const int64_t start = a.cu[b], len = a.cu[b + 1] - start;
         live = t + 1 < len && start + t >= 0 && start + t < n_rows;
     }
@@ -885,7 +888,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     a.in = *in;
     a.in.lp = nullptr; a.in.lpu = nullptr;
     a.cu = cu; a.n_seq = n_seq; a.pre_rolled = pre_rolled;
-    a.row_grad = reinterpret_cast<float4*>(row_grad);
+    a.row_grad = reinterpret_cast<float4*>(row_grad); a.any_row = row_grad != nullptr;
     a.logits = rows->logits; a.n_inner = in->sm1; a.d_n_inner = d_n_inner; a.vocab = rows->vocab;
     a.stride_outer = rows->stride_outer; a.stride_inner = rows->stride_inner;
     a.targets = rows->targets; a.ts_outer = rows->tgt_stride_outer; a.ts_inner = rows->tgt_stride_inner;

@@ -14,7 +14,7 @@ from rl_amd.algorithms.loss import (
     prepare_packed_loss_input,
     wrap_loss_fn_with_input_preparation,
 )
-from rl_amd.algorithms.loss.fused import any_row_fusable, why_not_fusable
+from rl_amd.algorithms.loss.fused import any_row_fusable, any_row_fusable_packed, why_not_fusable
 from rl_amd.temperature import apply_temperature_scaling, deferred_temperature
 from test_gpu_fused import _batch, _close
 
@@ -136,3 +136,29 @@ def test_packed_rows(dtype, vocab):
         (df,) = torch.autograd.grad(got * factor, xf, retain_graph=True)
         (du,) = torch.autograd.grad(want * factor, xu, retain_graph=True)
         _same_gradient(df, du, dtype)
+
+
+@pytest.mark.parametrize("vocab", [4099, 164000])
+def test_masked_in_positions_beyond_a_packed_sequence(vocab):
+    """They have no row: their logprob is 0 and they count in the loss and the metrics, as on the general path."""
+    logits, data, gs, _ = _setup(4, 9, vocab, torch.bfloat16)
+    data["token_mask"][:] = 1
+    data["sample_mask"][:] = 1
+    gt = data["token_mask"][:, 1:].sum()
+    cu = torch.tensor([0, 8, 13, 13, 14], dtype=torch.int32, device=DEV)
+    cup = torch.tensor([0, 12, 18, 18, 21], dtype=torch.int32, device=DEV)
+    g = torch.Generator().manual_seed(4)
+    x = (torch.randn(1, 23, vocab, generator=g) * 2).to(torch.bfloat16).to(DEV)
+    for cfg in (dict(), dict(token_level_loss=False, reference_policy_kl_penalty=0.001), dict(reference_policy_kl_penalty=0.0)):
+        fn = ClippedPGLossFn(ClippedPGLossConfig(**cfg))
+        xf, xu = (x.clone().requires_grad_(True) for _ in range(2))
+        assert any_row_fusable_packed(fn, xf, data)
+        got, gm = SequencePackingFusionLossWrapper(fn, prepare_packed_loss_input, cu, cup)(xf, data, gs, gt)
+        loss_input, d2 = prepare_packed_loss_input(xu, dict(data), fn, cu, cup)
+        want, wm = fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)
+        assert _close(got.item(), want.item(), rel=1e-4)
+        for k in wm:
+            assert _close(float(gm[k]), float(wm[k])), k
+        got.backward()
+        want.backward()
+        _same_gradient(xf.grad, xu.grad, torch.bfloat16)
