@@ -316,8 +316,8 @@ int nrl_fused_packed_logits_grpo_loss(const nrl_rows* rows, int32_t target_is_pr
 
 /* Both of the above (cu_seqlens NULL: the first) for rows that need not lie on the 16-byte grid nor fit on the chip: 1 KiB to
  * NRL_FUSED_ANY_ROW_MAX bytes, logits and gradient rows alike modulo 16 bytes, not in place, temperature as a multiplication.
- * row_grad_out: fp32 [n_outer * d_n_inner, 4], 16-byte aligned: what nrl_rows_grad needs to write the gradient again.  The gradient
- * is written for an upstream factor of 1. */
+ * row_grad_out: fp32 [n_outer * d_n_inner, 4], 16-byte aligned (NULL without rows): what nrl_rows_grad needs to write the gradient
+ * again.  The gradient is written for an upstream factor of 1. */
 #define NRL_FUSED_ANY_ROW_MIN 1024
 #define NRL_FUSED_ANY_ROW_MAX (1 << 20)
 int nrl_fused_any_row_grpo_loss(const nrl_rows* rows, int32_t target_is_pre_rolled, const int32_t* cu_seqlens, int64_t n_seq,

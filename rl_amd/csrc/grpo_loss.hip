@@ -831,7 +831,7 @@ extern "C" int64_t nrl_fused_packed_workspace_bytes(int64_t n_seq, int64_t n_inn
 
 // rows describes the logits; with cu != NULL it is one packed row of rows->n_inner positions (n_outer 1) and
 // the loss inputs are [n_seq, in->sm1]
-static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float loss_scale, float* row_grad, void* dlogits,
+static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float loss_scale, bool any_row, float* row_grad, void* dlogits,
                       int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out, float* loss_out,
                       float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream, const int32_t* cu,
                       int64_t n_seq, int pre_rolled) {
@@ -855,7 +855,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     if (cfg->kl_type < 1 || cfg->kl_type > 3 || cfg->tis_type < 0 || cfg->tis_type > 3) return fail(NRL_E_INVALID, "bad kl_type or tis_type");
     const int bytes = rows->dtype == NRL_F32 ? 4 : 2, epv = 16 / bytes;
     const uintptr_t xa = reinterpret_cast<uintptr_t>(rows->logits), da = reinterpret_cast<uintptr_t>(dlogits);
-    if (row_grad) {
+    if (any_row) {
         if (rows->vocab * bytes < NRL_FUSED_ANY_ROW_MIN || rows->vocab * bytes > NRL_FUSED_ANY_ROW_MAX)
             return fail(NRL_E_UNSUPPORTED, "row of %lld bytes", (long long)(rows->vocab * bytes));
         if (((xa - da) & 15) || ((rows->stride_outer - d_stride_outer) * bytes) % 16 || ((rows->stride_inner - d_stride_inner) * bytes) % 16 || xa % bytes)
@@ -877,9 +877,14 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     const int64_t need = cu ? nrl_fused_packed_workspace_bytes(in->batch, in->sm1, n_rows) : nrl_fused_workspace_bytes(in->batch, in->sm1);
     if (workspace_bytes < need) return fail(NRL_E_WORKSPACE, "workspace too small");
     if (reinterpret_cast<uintptr_t>(workspace) & 7) return fail(NRL_E_INVALID, "workspace must be 8-byte aligned");
-    if (n_rows > 0) {
-        if (!rows->logits || !rows->targets || !dlogits || !logprob_out) return fail(NRL_E_INVALID, "null logits, targets or output");
-        if (!in->gen || !in->adv || !in->token_mask || !in->sample_mask || !in->global_valid) return fail(NRL_E_INVALID, "null loss input");
+    // (empty inputs come without memory: sequences of one token have rows but no token that carries a loss, a microbatch may
+    // have no row at all)
+    const bool tokens = in->batch * in->sm1 > 0;
+    if (!in->global_valid || (in->batch > 0 && !in->sample_mask)) return fail(NRL_E_INVALID, "null sample_mask or global_valid");
+    if (n_rows > 0 && (!rows->logits || !dlogits || (any_row && !row_grad))) return fail(NRL_E_INVALID, "null logits, gradient or row_grad");
+    if (tokens) {
+        if ((n_rows > 0 && !rows->targets) || !logprob_out) return fail(NRL_E_INVALID, "null targets or logprob output");
+        if (!in->gen || !in->adv || !in->token_mask) return fail(NRL_E_INVALID, "null loss input");
         if (!cfg->force_on_policy_ratio && !in->prev) return fail(NRL_E_INVALID, "prev_logprobs is NULL");
         if (cfg->has_kl && !in->ref) return fail(NRL_E_INVALID, "reference_policy_logprobs is NULL");
     }
@@ -888,7 +893,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
     a.in = *in;
     a.in.lp = nullptr; a.in.lpu = nullptr;
     a.cu = cu; a.n_seq = n_seq; a.pre_rolled = pre_rolled;
-    a.row_grad = reinterpret_cast<float4*>(row_grad); a.any_row = row_grad != nullptr;
+    a.row_grad = reinterpret_cast<float4*>(row_grad); a.any_row = any_row;
     a.logits = rows->logits; a.n_inner = in->sm1; a.d_n_inner = d_n_inner; a.vocab = rows->vocab;
     a.stride_outer = rows->stride_outer; a.stride_inner = rows->stride_inner;
     a.targets = rows->targets; a.ts_outer = rows->tgt_stride_outer; a.ts_inner = rows->tgt_stride_inner;
@@ -915,7 +920,7 @@ static int fused_impl(const nrl_rows* rows, const nrl_grpo_cfg* cfg, const nrl_g
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
             return fail(NRL_E_LAUNCH, "cannot read the device's compute-unit count");
-        const FusedLaunch l{a, tc, cu != nullptr, n_rows, row_grad != nullptr, cus, s};
+        const FusedLaunch l{a, tc, cu != nullptr, n_rows, any_row, cus, s};
         if (rows->dtype == NRL_F32) launch_fused_f32(l);
         else if (rows->dtype == NRL_BF16) launch_fused_bf16(l);
         else launch_fused_f16(l);
@@ -935,7 +940,7 @@ extern "C" int nrl_fused_logits_grpo_loss(const nrl_rows* rows, const nrl_grpo_c
                                           float loss_scale, void* dlogits, int64_t d_n_inner, int64_t d_stride_outer,
                                           int64_t d_stride_inner, float* logprob_out, float* loss_out, float* metrics_out,
                                           void* workspace, int64_t workspace_bytes, void* stream) {
-    return fused_impl(rows, cfg, in, loss_scale, nullptr, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
+    return fused_impl(rows, cfg, in, loss_scale, false, nullptr, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
                       metrics_out, workspace, workspace_bytes, stream, nullptr, 0, 0);
 }
 
@@ -946,7 +951,7 @@ extern "C" int nrl_fused_packed_logits_grpo_loss(const nrl_rows* rows, int32_t t
                                                  void* stream) {
     if (!cu_seqlens) return fail(NRL_E_INVALID, "cu_seqlens is NULL");
     if (rows && rows->tgt_stride_inner != 1) return fail(NRL_E_INVALID, "packed targets must be contiguous");
-    return fused_impl(rows, cfg, in, loss_scale, nullptr, dlogits, rows ? rows->n_inner : 0, 0, d_row_stride, logprob_out, loss_out,
+    return fused_impl(rows, cfg, in, loss_scale, false, nullptr, dlogits, rows ? rows->n_inner : 0, 0, d_row_stride, logprob_out, loss_out,
                       metrics_out, workspace, workspace_bytes, stream, cu_seqlens, n_seq, target_is_pre_rolled);
 }
 
@@ -954,9 +959,8 @@ extern "C" int nrl_fused_any_row_grpo_loss(const nrl_rows* rows, int32_t target_
                                            const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float* row_grad_out, void* dlogits,
                                            int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out,
                                            float* loss_out, float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream) {
-    if (!row_grad_out) return fail(NRL_E_INVALID, "row_grad_out is NULL");
     if (cu_seqlens && rows && rows->tgt_stride_inner != 1) return fail(NRL_E_INVALID, "packed targets must be contiguous");
-    return fused_impl(rows, cfg, in, 1.f, row_grad_out, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
+    return fused_impl(rows, cfg, in, 1.f, true, row_grad_out, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
                       metrics_out, workspace, workspace_bytes, stream, cu_seqlens, n_seq, target_is_pre_rolled);
 }
 

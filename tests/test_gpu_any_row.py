@@ -162,3 +162,33 @@ def test_masked_in_positions_beyond_a_packed_sequence(vocab):
         got.backward()
         want.backward()
         _same_gradient(xf.grad, xu.grad, torch.bfloat16)
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 4099), (torch.bfloat16, 4096), (torch.float32, 90000)])
+@pytest.mark.parametrize("b,s", [(0, 9), (3, 1), (0, 1)])
+def test_empty_microbatches(dtype, vocab, b, s):
+    """No sequence, and sequences of one token: a zero loss and a zero gradient."""
+    logits, data, gs, gt = _setup(3, 9, vocab, dtype)
+    data = {k: v[:b] if v.dim() == 1 else v[:b, :s] for k, v in data.items()}
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    x = logits[:b, :s].clone().requires_grad_(True)
+    got, gm = wrap_loss_fn_with_input_preparation(x, data, gs, gt, fn, prepare_loss_input)
+    want, wm = _three_pass(x, data, fn, gs, gt)
+    assert got.item() == want.item() == 0.0
+    for k in wm:
+        assert float(gm[k]) == float(wm[k]) or (float(gm[k]) != float(gm[k]) and float(wm[k]) != float(wm[k])), k
+    (d,) = torch.autograd.grad(got * 0.3, x)
+    assert d.shape == x.shape and not bool(d.any())
+
+
+@pytest.mark.parametrize("vocab", [4099, 4096])
+def test_empty_packed_microbatches(vocab):
+    logits, data, gs, gt = _setup(3, 9, vocab, torch.bfloat16)
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    one = {k: v if v.dim() == 1 else v[:, :1] for k, v in data.items()}
+    cu = torch.tensor([0, 1, 2, 3], dtype=torch.int32, device=DEV)
+    x = logits[0, :4].clone().unsqueeze(0).requires_grad_(True)
+    assert any_row_fusable_packed(fn, x, one)
+    got, _ = SequencePackingFusionLossWrapper(fn, prepare_packed_loss_input, cu, cu)(x, one, gs, gt)
+    (d,) = torch.autograd.grad(got, x)
+    assert got.item() == 0.0 and d.shape == x.shape and not bool(d.any())
