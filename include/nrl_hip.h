@@ -317,11 +317,11 @@ int nrl_fused_packed_logits_grpo_loss(const nrl_rows* rows, int32_t target_is_pr
 /* Both of the above (cu_seqlens NULL: the first) for rows that need not lie on the 16-byte grid nor fit on the chip: 1 KiB to
  * NRL_FUSED_ANY_ROW_MAX bytes, logits and gradient rows alike modulo 16 bytes, not in place, temperature as a multiplication.
  * row_grad_out: fp32 [n_outer * d_n_inner, 4], 16-byte aligned (NULL without rows): what nrl_rows_grad needs to write the gradient
- * again.  The gradient is written for an upstream factor of 1. */
+ * again.  The gradient is written for an upstream factor of loss_scale, row_grad_out for one of 1. */
 #define NRL_FUSED_ANY_ROW_MIN 1024
 #define NRL_FUSED_ANY_ROW_MAX (1 << 20)
 int nrl_fused_any_row_grpo_loss(const nrl_rows* rows, int32_t target_is_pre_rolled, const int32_t* cu_seqlens, int64_t n_seq,
-                                const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float* row_grad_out, void* dlogits,
+                                const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float loss_scale, float* row_grad_out, void* dlogits,
                                 int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out,
                                 float* loss_out, float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream);
 /* dlogits = *factor times the gradient described by row_grad, over all n_outer * n_inner rows; *factor is read from the device and

@@ -91,7 +91,7 @@ SIGNATURES = {
     "nrl_fused_packed_logits_grpo_loss": (C.c_int, [C.POINTER(NrlRows), C.c_int32, _P, _I64, C.POINTER(NrlGrpoCfg),
                                                     C.POINTER(NrlGrpoInputs), _F, _P, _I64, _P, _P, _P, _P, _I64, _P]),
     "nrl_fused_any_row_grpo_loss": (C.c_int, [C.POINTER(NrlRows), C.c_int32, _P, _I64, C.POINTER(NrlGrpoCfg), C.POINTER(NrlGrpoInputs),
-                                              _P, _P, _I64, _I64, _I64, _P, _P, _P, _P, _I64, _P]),
+                                              _F, _P, _P, _I64, _I64, _I64, _P, _P, _P, _P, _I64, _P]),
     "nrl_rows_grad": (C.c_int, [C.POINTER(NrlRows), _P, _P, _F, _P, _I64, _I64, _P]),
     "nrl_nll_loss_fwd_bwd": (C.c_int, [C.POINTER(NrlGrpoInputs), _P, _P, _P, _P, _I64, _P]),
     "nrl_calculate_kl": (C.c_int, [_P, _P, _P, _I64, _I32, _I32, _F, _I32, _F, _P, _P]),
@@ -133,7 +133,7 @@ SIGNATURES = {
 _lib = None
 
 
-ABI_VERSION = 115  # nrl_version() of the library these signatures describe
+ABI_VERSION = 116  # nrl_version() of the library these signatures describe
 
 
 def load() -> C.CDLL:

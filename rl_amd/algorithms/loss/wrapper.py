@@ -104,7 +104,8 @@ class SequencePackingFusionLossWrapper:
         self.vocab_parallel_group = vocab_parallel_group
         self.context_parallel_group = context_parallel_group
 
-    def __call__(self, next_token_logits, data, global_valid_seqs, global_valid_toks):
+    def __call__(self, next_token_logits, data, global_valid_seqs, global_valid_toks, *, loss_scale: float = 1.0):
+        """``loss_scale``: see ``wrap_loss_fn_with_input_preparation``."""
         from .fused import _single_pass_packed, any_row_fusable_packed, fused_packed_logits_clipped_pg_loss, why_not_fusable_packed
         from .utils import prepare_packed_loss_input
 
@@ -120,10 +121,10 @@ class SequencePackingFusionLossWrapper:
                 if why_not_fusable_packed(self.loss_fn, next_token_logits, data, params) is None:
                     return fused_packed_logits_clipped_pg_loss(
                         next_token_logits, data, self.loss_fn, self.cu_seqlens_q, self.cu_seqlens_q_padded,
-                        global_valid_seqs, global_valid_toks)
+                        global_valid_seqs, global_valid_toks, loss_scale=loss_scale)
                 if any_row_fusable_packed(self.loss_fn, next_token_logits, data, params):
                     return _single_pass_packed(next_token_logits, data, self.loss_fn, self.cu_seqlens_q, self.cu_seqlens_q_padded,
-                                               global_valid_seqs, global_valid_toks, 1.0, True)
+                                               global_valid_seqs, global_valid_toks, loss_scale, True)
         loss_input, prepared = self.prepare_fn(
             logits=next_token_logits, data=data, loss_fn=self.loss_fn, cu_seqlens_q=self.cu_seqlens_q,
             cu_seqlens_q_padded=self.cu_seqlens_q_padded, vocab_parallel_rank=self.vocab_parallel_rank,
@@ -138,10 +139,14 @@ def wrap_loss_fn_with_input_preparation(next_token_logits, data, global_valid_se
                                         loss_fn: LossFunction, prepare_fn: Callable[..., Any],
                                         vocab_parallel_rank: Optional[int] = None,
                                         vocab_parallel_group: Optional[Any] = None,
-                                        context_parallel_group: Optional[Any] = None):
+                                        context_parallel_group: Optional[Any] = None, *, loss_scale: float = 1.0):
     """``wrapper.py:292-322``: prepare, then call the loss.  When the loss is a ``ClippedPGLossFn`` whose
     per-token gradient does not need other tokens' logprobs and the logits are a plain GPU tensor, both
-    steps (and the later backward through the logprob op) run as one fused pass over the logits."""
+    steps (and the later backward through the logprob op) run as one fused pass over the logits.
+
+    ``loss_scale`` is the factor the caller expects autograd to deliver to the returned loss (``1 / n`` when it divides by
+    ``n`` before ``backward()``).  The fused pass writes the gradient for it; whatever factor comes is honoured, but another
+    one than named costs a second pass over the gradient."""
     from .fused import _single_pass, any_row_fusable, fused_logits_clipped_pg_loss, why_not_fusable
     from .utils import prepare_loss_input
 
@@ -155,9 +160,9 @@ def wrap_loss_fn_with_input_preparation(next_token_logits, data, global_valid_se
         if _group_size(vocab_parallel_group) == 1 and _group_size(context_parallel_group) == 1:
             params = bound.get("sampling_params")
             if why_not_fusable(loss_fn, next_token_logits, data, params) is None:
-                return fused_logits_clipped_pg_loss(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks)
+                return fused_logits_clipped_pg_loss(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks, loss_scale=loss_scale)
             if any_row_fusable(loss_fn, next_token_logits, data, params):
-                return _single_pass(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks, 1.0, False, True)
+                return _single_pass(next_token_logits, data, loss_fn, global_valid_seqs, global_valid_toks, loss_scale, False, True)
     loss_input, data = prepare_fn(
         logits=next_token_logits, data=data, loss_fn=loss_fn, vocab_parallel_rank=vocab_parallel_rank,
         vocab_parallel_group=vocab_parallel_group, context_parallel_group=context_parallel_group,

@@ -250,8 +250,9 @@ __global__ __launch_bounds__(BLOCK, 4) void fused_logits_loss_kernel(FusedArgs a
             ti.den_s = valid_seqs(a.in) + 1e-8f;
             ti.den_t = valid_toks(a.in) + 1e-8f;
             const TokenOut tok = token_eval<false>(c, st, ti);
-            g = (tok.d_actor + tok.d_lpu) * a.loss_scale;
-            if (EDGE && tid == 0 && a.row_grad) a.row_grad[r] = make_float4(g, lse, __int_as_float(tloc), 0.f);
+            const float g1 = tok.d_actor + tok.d_lpu;
+            g = g1 * a.loss_scale;
+            if (EDGE && tid == 0 && a.row_grad) a.row_grad[r] = make_float4(g1, lse, __int_as_float(tloc), 0.f);
             if (tid == 0) a.lp_out[static_cast<int64_t>(word(rec, R_SEQ)) * a.n_inner + word(rec, R_POS)] = lp;
         }
         const int tvec = tloc >= head ? (tloc - head) / EPV : -1;  // (of a target in the tail: no vector of the row)

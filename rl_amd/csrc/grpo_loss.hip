@@ -956,11 +956,11 @@ extern "C" int nrl_fused_packed_logits_grpo_loss(const nrl_rows* rows, int32_t t
 }
 
 extern "C" int nrl_fused_any_row_grpo_loss(const nrl_rows* rows, int32_t target_is_pre_rolled, const int32_t* cu_seqlens, int64_t n_seq,
-                                           const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float* row_grad_out, void* dlogits,
+                                           const nrl_grpo_cfg* cfg, const nrl_grpo_inputs* in, float loss_scale, float* row_grad_out, void* dlogits,
                                            int64_t d_n_inner, int64_t d_stride_outer, int64_t d_stride_inner, float* logprob_out,
                                            float* loss_out, float* metrics_out, void* workspace, int64_t workspace_bytes, void* stream) {
     if (cu_seqlens && rows && rows->tgt_stride_inner != 1) return fail(NRL_E_INVALID, "packed targets must be contiguous");
-    return fused_impl(rows, cfg, in, 1.f, true, row_grad_out, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
+    return fused_impl(rows, cfg, in, loss_scale, true, row_grad_out, dlogits, d_n_inner, d_stride_outer, d_stride_inner, logprob_out, loss_out,
                       metrics_out, workspace, workspace_bytes, stream, cu_seqlens, n_seq, target_is_pre_rolled);
 }
 

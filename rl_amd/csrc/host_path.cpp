@@ -318,7 +318,7 @@ FusedOut fused_loss(const Tensor& logits, const Tensor& targets, int64_t n_inner
     if (any_row) {
         const int64_t per = packed ? logits.size(0) : logits.size(1);
         o.row_grad = f32({packed ? per : b * per, 4}, logits);
-        check(nrl_fused_any_row_grpo_loss(&rows, pre_rolled, packed ? ptr<int32_t>(cu) : nullptr, packed ? b : 0, &cfg, &l.in, ptr(o.row_grad),
+        check(nrl_fused_any_row_grpo_loss(&rows, pre_rolled, packed ? ptr<int32_t>(cu) : nullptr, packed ? b : 0, &cfg, &l.in, scale, ptr(o.row_grad),
                                           ptr<void>(o.dlogits), per, packed ? 0 : o.dlogits.stride(0), o.dlogits.stride(packed ? 0 : 1), ptr(o.lp),
                                           ptr(o.loss), ptr(o.metrics), ws.data_ptr(), ws.numel() * 8, stream_of(logits)), "nrl_fused_any_row_grpo_loss");
     } else if (packed)
@@ -545,14 +545,17 @@ struct FusedLoss : torch::autograd::Function<FusedLoss> {
 };
 
 // The single pass over rows off the 16-byte grid or longer than the chip holds.  Here the logits are saved, with 16 bytes per row:
-// the gradient can be written again, which an upstream factor other than 1 and a second backward through the same graph need.
+// the gradient can be written again, which an upstream factor other than loss_scale and a second backward through the same graph
+// need.  Written again it costs another read and write of every live row (2 x 1024 rows of V = 151936 fp32: 504 us with the
+// factor named, 936 without, 675 in three passes), so whoever knows the factor names it.
 struct FusedRowsLoss : torch::autograd::Function<FusedRowsLoss> {
     static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, const FusedArgs& a) {
         ctx->set_materialize_grads(false);
         const Tensor logits = logits_in.detach();
-        FusedOut o = fused_loss(logits, a.targets, a.n_inner, a.cu, true, a.data, a.cfg, 1.0, a.temperature, a.mode, false, true);
+        FusedOut o = fused_loss(logits, a.targets, a.n_inner, a.cu, true, a.data, a.cfg, a.loss_scale, a.temperature, a.mode, false, true);
         ctx->save_for_backward({logits, o.row_grad});
         ctx->saved_data["dlogits"] = o.dlogits;
+        ctx->saved_data["loss_scale"] = a.loss_scale;
         ctx->saved_data["temperature"] = a.temperature;
         ctx->saved_data["mode"] = a.mode;
         ctx->mark_non_differentiable({o.metrics});
@@ -566,7 +569,7 @@ struct FusedRowsLoss : torch::autograd::Function<FusedRowsLoss> {
         const Tensor factor = to_f32(grads[0].detach(), logits);
         const c10::OptionalDeviceGuard guard(logits.device());
         Tensor d;
-        float written = 1.f;
+        float written = static_cast<float>(ctx->saved_data["loss_scale"].toDouble());
         const auto it = ctx->saved_data.find("dlogits");
         if (it != ctx->saved_data.end()) {
             d = it->second.toTensor();

@@ -142,6 +142,10 @@ class LossPostProcessor:
         self.sampling_params = sampling_params
         _need_single_gpu(cp_size, "LossPostProcessor")
 
+    def _loss_scale(self) -> float:
+        """What this worker's loop multiplies the loss by before ``backward()`` (``train.py:547-548``)."""
+        return float((self.dp_size or 1) * (self.cp_size or 1))
+
     def __call__(self, logits: torch.Tensor, data_dict: Any, processed_inputs: Any, global_valid_seqs: torch.Tensor,
                  global_valid_toks: torch.Tensor, sequence_dim: int = 1):
         from functools import partial
@@ -161,7 +165,7 @@ class LossPostProcessor:
                                                  cu_seqlens_q_padded=cu)
             return wrapped(logits, data_dict, global_valid_seqs, global_valid_toks)
         loss, metrics = wrap_loss_fn_with_input_preparation(logits, data_dict, global_valid_seqs, global_valid_toks,
-                                                            self.loss_fn, prepare)
+                                                            self.loss_fn, prepare, loss_scale=self._loss_scale())
         if hasattr(metrics, "defer_scaling"):
             # this worker's loop divides every metric by the number of global batches before it calls backward()
             # (``train.py:525-547``): let the mapping record that instead of waiting for the device

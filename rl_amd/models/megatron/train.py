@@ -32,9 +32,9 @@ class LossPostProcessor:
     ``prepare_loss_input`` is bound to ``sampling_params`` / ``d2t`` / ``chunk_size`` with ``functools.partial``
     exactly as the reference binds it, so the wrappers below see what a real worker hands them; a
     ``ClippedPGLossFn`` the single pass covers then runs logits -> loss -> gradient as one kernel.  The loss is
-    multiplied by ``num_microbatches`` (``:583-594``, undoing the schedule's averaging); the gradient the single
-    pass has already written is rescaled on the device by whatever factor autograd delivers.  The draft-model
-    wrapper (``student_logits`` in the data) is not part of this path."""
+    multiplied by ``num_microbatches`` (``:583-594``, undoing the schedule's averaging); the single pass writes the
+    gradient for what the two leave (``_loss_scale``) and rescales it on the device if autograd delivers another
+    factor.  The draft-model wrapper (``student_logits`` in the data) is not part of this path."""
 
     def __init__(self, loss_fn: Any, cfg: Any, num_microbatches: int = 1, cp_normalize: bool = True,
                  sampling_params: Optional[TrainingSamplingParams] = None, draft_model: Any = None,
@@ -48,6 +48,12 @@ class LossPostProcessor:
         self.sampling_params = sampling_params
         self.prepare_fn = prepare_fn
         self.d2t = None
+
+    def _loss_scale(self) -> float:
+        """The schedule's division by ``num_microbatches`` and this class's multiplication, as autograd rounds them in fp32:
+        not always 1 (41, 47, 55, ... microbatches)."""
+        n = self.num_microbatches
+        return 1.0 if not n or n == 1 else float(torch.ones((), dtype=torch.float32, device="cpu") / n * n)
 
     def __call__(self, data_dict: Any, packed_seq_params: Any = None, global_valid_seqs: Optional[torch.Tensor] = None,
                  global_valid_toks: Optional[torch.Tensor] = None) -> Callable[[torch.Tensor], Tuple[torch.Tensor, Dict[str, Any]]]:
@@ -68,6 +74,7 @@ class LossPostProcessor:
             prepare = partial(prepare_loss_input, sampling_params=self.sampling_params, d2t=self.d2t, chunk_size=chunk)
         if "student_logits" in data_dict:
             raise NotImplementedError("LossPostProcessor: the draft-model loss is outside this build")
+        scale = {"loss_scale": self._loss_scale()}
         if self.cfg["sequence_packing"]["enabled"] and packed_seq_params is not None:
             if self.cfg.get("sequence_packing", {}).get("fuse_loss", False):
                 assert self.prepare_fn is None, (
@@ -78,13 +85,14 @@ class LossPostProcessor:
                 prepare = partial(prepare_packed_loss_input, sampling_params=self.sampling_params, chunk_size=chunk)
             else:
                 wrapper_cls = SequencePackingLossWrapper
+                scale = {}  # a loss per sequence, no single pass
             wrapped = wrapper_cls(loss_fn=self.loss_fn, prepare_fn=prepare, cu_seqlens_q=packed_seq_params.cu_seqlens_q,
                                   cu_seqlens_q_padded=packed_seq_params.cu_seqlens_q_padded, vocab_parallel_rank=0,
                                   vocab_parallel_group=None, context_parallel_group=None)
         else:
             wrapped = partial(wrap_loss_fn_with_input_preparation, loss_fn=self.loss_fn, prepare_fn=prepare,
                               vocab_parallel_rank=0, vocab_parallel_group=None, context_parallel_group=None)
-        wrapped = partial(wrapped, data=data_dict, global_valid_seqs=global_valid_seqs, global_valid_toks=global_valid_toks)
+        wrapped = partial(wrapped, data=data_dict, global_valid_seqs=global_valid_seqs, global_valid_toks=global_valid_toks, **scale)
         num_microbatches = self.num_microbatches
 
         def counteract_schedule_averaging(*args, **kwargs):

@@ -192,3 +192,67 @@ def test_empty_packed_microbatches(vocab):
     got, _ = SequencePackingFusionLossWrapper(fn, prepare_packed_loss_input, cu, cu)(x, one, gs, gt)
     (d,) = torch.autograd.grad(got, x)
     assert got.item() == 0.0 and d.shape == x.shape and not bool(d.any())
+
+
+def _untouched_by_backward(x, loss, factor, want):
+    """The gradient is the one the forward wrote: the logits it could be written again from are gone by then."""
+    x.data.zero_()
+    (d,) = torch.autograd.grad(loss, x)
+    _same_gradient(d, want * factor, d.dtype)
+
+
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 4099), (torch.float32, 82001)])
+def test_a_named_factor_is_written_by_the_forward(dtype, vocab):
+    from types import SimpleNamespace
+
+    from rl_amd.models.automodel.train import LossPostProcessor as DTensorPost
+    from rl_amd.models.megatron.train import LossPostProcessor as MegatronPost
+
+    logits, data, gs, gt = _setup(3, 7, vocab, dtype)
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    xu = logits.clone().requires_grad_(True)
+    (want,) = torch.autograd.grad(_three_pass(xu, data, fn, gs, gt)[0], xu)
+    want = want.float()
+
+    def fresh():
+        return logits.clone().requires_grad_(True)
+
+    x = fresh()
+    loss, _ = wrap_loss_fn_with_input_preparation(x, data, gs, gt, fn, prepare_loss_input, loss_scale=0.3)
+    (again,) = torch.autograd.grad(loss * 0.7, x, retain_graph=True)  # not the one that was named
+    _same_gradient(again, want * 0.7, dtype)
+    x = fresh()
+    loss, _ = wrap_loss_fn_with_input_preparation(x, data, gs, gt, fn, prepare_loss_input, loss_scale=0.3)
+    _untouched_by_backward(x, loss * 0.3, 0.3, want)
+
+    x = fresh()
+    post = DTensorPost(fn, {}, None, None, None, 1, 4)
+    loss, _ = post(x, dict(data), SimpleNamespace(), gs, gt)
+    _untouched_by_backward(x, loss * post.dp_size * post.cp_size, 4.0, want)
+
+    for n in (1, 8, 41):
+        x = fresh()
+        cfg = {"sequence_packing": {"enabled": False}}
+        loss, _ = MegatronPost(fn, cfg, num_microbatches=n)(dict(data), None, gs, gt)(x)
+        _untouched_by_backward(x, loss / n, 1.0, want)
+
+
+def test_a_named_factor_of_packed_rows():
+    from types import SimpleNamespace
+
+    from rl_amd.models.megatron.train import LossPostProcessor
+
+    logits, data, gs, gt = _setup(3, 8, 1029, torch.bfloat16)
+    cu = torch.tensor([0, 8, 16, 24], dtype=torch.int32, device=DEV)
+    flat = logits.reshape(1, 24, 1029)
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    xu = flat.clone().requires_grad_(True)
+    loss_input, d2 = prepare_packed_loss_input(xu, dict(data), fn, cu, cu)
+    (want,) = torch.autograd.grad(fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)[0], xu)
+    x = flat.clone().requires_grad_(True)
+    loss, _ = SequencePackingFusionLossWrapper(fn, prepare_packed_loss_input, cu, cu)(x, data, gs, gt, loss_scale=0.3)
+    _untouched_by_backward(x, loss * 0.3, 0.3, want.float())
+    x = flat.clone().requires_grad_(True)
+    post = LossPostProcessor(fn, {"sequence_packing": {"enabled": True, "fuse_loss": True}}, num_microbatches=41)
+    loss, _ = post(dict(data), SimpleNamespace(cu_seqlens_q=cu, cu_seqlens_q_padded=cu), gs, gt)(x)
+    _untouched_by_backward(x, loss / 41, 1.0, want.float())
