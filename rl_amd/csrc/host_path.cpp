@@ -60,7 +60,6 @@ void need_gpu(const Tensor& t) {
 }
 template <typename... T> void need_gpu(const Tensor& t, const T&... more) { need_gpu(t); need_gpu(more...); }
 
-Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 template <typename T = float> T* ptr(const Tensor& t) { return t.defined() && t.numel() > 0 ? static_cast<T*>(t.data_ptr()) : nullptr; }
 
 int dtype_code(const Tensor& t) {
@@ -188,6 +187,14 @@ struct LossData {
     Tensor prev, gen, ref, adv, token_mask, sample_mask, correct, seqs, toks;
     int64_t shift = 1;  // columns in front of the first one that is read
 };
+Tensor opt(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
+LossData loss_data(const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
+                   const OptTensor& correct, const Tensor& seqs, const Tensor& toks, int64_t shift) {
+    LossData d;
+    d.prev = opt(prev); d.gen = gen; d.ref = opt(ref); d.adv = adv; d.token_mask = token_mask; d.sample_mask = sample_mask; d.correct = opt(correct);
+    d.seqs = seqs; d.toks = toks; d.shift = shift;
+    return d;
+}
 
 LossInputs loss_inputs(const LossData& d, const Tensor& like, int64_t b, int64_t n) {
     LossInputs l;
@@ -463,6 +470,9 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> group_baseline_std(const Tensor& prom
 // ---------------------------------------------------------------------------------------------
 // autograd nodes
 // ---------------------------------------------------------------------------------------------
+// Every tensor a node reads is an argument of its own, also those without a gradient: autograd looks at the arguments to refuse
+// forward-mode differentiation and to tell whether the result depends on a tensor that requires a gradient.
+
 // logits [B, S, V], targets [B, >= n_inner] (already aligned to the rows) -> fp32 [B, n_inner].  Saved for the backward:
 // the logits (no copy), the targets and one fp32 log-sum-exp per row; the softmax is never materialised.
 struct RowsLogprob : torch::autograd::Function<RowsLogprob> {
@@ -490,15 +500,18 @@ struct RowsLogprob : torch::autograd::Function<RowsLogprob> {
 
 // loss and metrics of given logprobs; the kernel also returns d loss / d lp (and / d lpu), so the backward is a scalar multiply
 struct ClippedPg : torch::autograd::Function<ClippedPg> {
-    static variable_list forward(AutogradContext* ctx, const Tensor& lp, const OptTensor& lpu, const LossData& d, const nrl_grpo_cfg& cfg) {
+    static variable_list forward(AutogradContext* ctx, const Tensor& lp, const OptTensor& lpu, const OptTensor& prev, const Tensor& gen, const OptTensor& ref,
+                                 const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask, const OptTensor& correct, const Tensor& seqs,
+                                 const Tensor& toks, const nrl_grpo_cfg& cfg) {
         ctx->set_materialize_grads(false);
-        GrpoOut o = grpo_loss(lp.detach(), lpu.has_value() ? lpu->detach() : Tensor(), d, cfg);
+        GrpoOut o = grpo_loss(lp.detach(), lpu.has_value() ? lpu->detach() : Tensor(),
+                              loss_data(prev, gen, ref, adv, token_mask, sample_mask, correct, seqs, toks, 1), cfg);
         ctx->save_for_backward({o.dlp, o.dlpu});
         ctx->mark_non_differentiable({o.metrics});
         return {o.loss, o.metrics};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        variable_list out(4);
+        variable_list out(12);
         if (!grads[0].defined()) return out;
         const auto saved = ctx->get_saved_variables();
         if (ctx->needs_input_grad(0)) out[0] = saved[0] * grads[0];
@@ -512,18 +525,20 @@ struct ClippedPg : torch::autograd::Function<ClippedPg> {
 // host never waits for its value, no second [B, S, V] tensor exists, and when the two agree (the normal case) the kernel
 // touches no memory.
 struct FusedArgs {
-    Tensor targets, cu;
     int64_t n_inner;
-    LossData data;
     nrl_grpo_cfg cfg;
     double loss_scale, temperature;
     int64_t mode;
     bool in_place;
 };
+constexpr int kFusedInputs = 12;  // of the two nodes below
 struct FusedLoss : torch::autograd::Function<FusedLoss> {
-    static variable_list forward(AutogradContext* ctx, const Tensor& logits, const FusedArgs& a) {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, const OptTensor& cu, const OptTensor& prev, const Tensor& gen,
+                                 const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask, const Tensor& seqs,
+                                 const Tensor& toks, const FusedArgs& a) {
         ctx->set_materialize_grads(false);
-        FusedOut o = fused_loss(logits.detach(), a.targets, a.n_inner, a.cu, true, a.data, a.cfg, a.loss_scale, a.temperature, a.mode, a.in_place);
+        FusedOut o = fused_loss(logits.detach(), targets, a.n_inner, opt(cu), true, loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, seqs, toks, 1),
+                                a.cfg, a.loss_scale, a.temperature, a.mode, a.in_place);
         // (an intermediate, neither input nor output: held directly so that it can be rescaled in place)
         ctx->saved_data["dlogits"] = o.dlogits;
         ctx->saved_data["loss_scale"] = a.loss_scale;
@@ -531,8 +546,9 @@ struct FusedLoss : torch::autograd::Function<FusedLoss> {
         return {o.loss, o.metrics};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        variable_list out(2);
+        variable_list out(kFusedInputs);
         if (!grads[0].defined()) return out;
+        if (!ctx->needs_input_grad(0)) return out;
         const auto it = ctx->saved_data.find("dlogits");
         TORCH_CHECK(it != ctx->saved_data.end(), "the single-pass loss hands its gradient buffer to autograd once; a second backward "
                     "through the same loss needs a new forward");
@@ -549,10 +565,13 @@ struct FusedLoss : torch::autograd::Function<FusedLoss> {
 // need.  Written again it costs another read and write of every live row (2 x 1024 rows of V = 151936 fp32: 504 us with the
 // factor named, 936 without, 675 in three passes), so whoever knows the factor names it.
 struct FusedRowsLoss : torch::autograd::Function<FusedRowsLoss> {
-    static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, const FusedArgs& a) {
+    static variable_list forward(AutogradContext* ctx, const Tensor& logits_in, const Tensor& targets, const OptTensor& cu, const OptTensor& prev, const Tensor& gen,
+                                 const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask, const Tensor& seqs,
+                                 const Tensor& toks, const FusedArgs& a) {
         ctx->set_materialize_grads(false);
         const Tensor logits = logits_in.detach();
-        FusedOut o = fused_loss(logits, a.targets, a.n_inner, a.cu, true, a.data, a.cfg, a.loss_scale, a.temperature, a.mode, false, true);
+        FusedOut o = fused_loss(logits, targets, a.n_inner, opt(cu), true, loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, seqs, toks, 1), a.cfg,
+                                a.loss_scale, a.temperature, a.mode, false, true);
         ctx->save_for_backward({logits, o.row_grad});
         ctx->saved_data["dlogits"] = o.dlogits;
         ctx->saved_data["loss_scale"] = a.loss_scale;
@@ -562,8 +581,9 @@ struct FusedRowsLoss : torch::autograd::Function<FusedRowsLoss> {
         return {o.loss, o.metrics};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        variable_list out(2);
+        variable_list out(kFusedInputs);
         if (!grads[0].defined()) return out;
+        if (!ctx->needs_input_grad(0)) return out;
         const auto saved = ctx->get_saved_variables();
         const Tensor logits = saved[0].dim() == 3 ? saved[0] : saved[0].unsqueeze(0);
         const Tensor factor = to_f32(grads[0].detach(), logits);
@@ -705,17 +725,6 @@ class Fetch {
     hipEvent_t done_ = nullptr;
 };
 
-// ---------------------------------------------------------------------------------------------
-// entry points
-// ---------------------------------------------------------------------------------------------
-LossData loss_data(const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
-                   const OptTensor& correct, const Tensor& seqs, const Tensor& toks, int64_t shift) {
-    LossData d;
-    d.prev = opt(prev); d.gen = gen; d.ref = opt(ref); d.adv = adv; d.token_mask = token_mask; d.sample_mask = sample_mask; d.correct = opt(correct);
-    d.seqs = seqs; d.toks = toks; d.shift = shift;
-    return d;
-}
-
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -787,7 +796,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("clipped_pg", [](const Tensor& lp, const OptTensor& lpu, const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv,
                            const Tensor& token_mask, const Tensor& sample_mask, const OptTensor& correct, const Tensor& seqs, const Tensor& toks,
                            const std::vector<int64_t>& iflags, const std::vector<double>& fparams) {
-        const variable_list o = ClippedPg::apply(lp, lpu, loss_data(prev, gen, ref, adv, token_mask, sample_mask, correct, seqs, toks, 1), make_cfg(iflags, fparams));
+        const variable_list o = ClippedPg::apply(lp, lpu, prev, gen, ref, adv, token_mask, sample_mask, correct, seqs, toks, make_cfg(iflags, fparams));
         return std::make_tuple(o[0], o[1]);
     });
     m.def("fused_clipped_pg", [](const Tensor& logits, const Tensor& targets, int64_t shift, int64_t n_inner, const OptTensor& cu, const OptTensor& prev,
@@ -796,9 +805,9 @@ PYBIND11_MODULE(_host, m) {
                                  double loss_scale, double temperature, int64_t mode, bool in_place, bool any_row) {
         Tensor t = targets.device() == logits.device() && targets.scalar_type() == at::kLong ? targets : targets.to(logits.device(), at::kLong);
         if (shift) t = t.narrow(1, shift, t.size(1) - shift);
-        const FusedArgs a{t, opt(cu), n_inner, loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, seqs, toks, 1), make_cfg(iflags, fparams),
-                          loss_scale, temperature, mode, in_place};
-        const variable_list o = any_row ? FusedRowsLoss::apply(logits, a) : FusedLoss::apply(logits, a);
+        const FusedArgs a{n_inner, make_cfg(iflags, fparams), loss_scale, temperature, mode, in_place};
+        const variable_list o = any_row ? FusedRowsLoss::apply(logits, t, cu, prev, gen, ref, adv, token_mask, sample_mask, seqs, toks, a)
+                                        : FusedLoss::apply(logits, t, cu, prev, gen, ref, adv, token_mask, sample_mask, seqs, toks, a);
         return std::make_tuple(o[0], o[1]);
     });
     m.def("gather_entropy", [](const Tensor& logits, const Tensor& indices, int64_t n, bool entropy) {

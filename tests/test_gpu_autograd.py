@@ -1,0 +1,48 @@
+"""What autograd sees of the nodes of the C++ host path."""
+
+import pytest
+import torch
+
+from rl_amd.algorithms.loss import ClippedPGLossConfig, ClippedPGLossFn, prepare_loss_input, wrap_loss_fn_with_input_preparation
+from test_gpu_fused import _batch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _setup(vocab):
+    logits, data, gs, gt = _batch(3, 9, vocab, torch.bfloat16, seed=vocab)
+    return logits.to(DEV), {k: v.to(DEV) for k, v in data.items()}, gs.to(DEV), gt.to(DEV)
+
+
+def _loss(route, logits, data, gs, gt):
+    fn = ClippedPGLossFn(ClippedPGLossConfig())
+    if route == "general":
+        loss_input, data = prepare_loss_input(logits, dict(data), fn)
+        return fn(data=data, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)[0]
+    return wrap_loss_fn_with_input_preparation(logits, data, gs, gt, fn, prepare_loss_input)[0]
+
+
+ROUTES = [("general", 4096), ("single pass", 4096), ("single pass", 4099)]
+
+
+@pytest.mark.parametrize("route,vocab", ROUTES)
+@pytest.mark.parametrize("key", ["advantages", "prev_logprobs", "generation_logprobs", "reference_policy_logprobs"])
+def test_loss_inputs_are_inputs_of_the_node(route, vocab, key):
+    """Forward-mode differentiation through any of them is refused; one that requires a gradient is part of the graph and
+    receives none."""
+    import torch.autograd.forward_ad as fad
+
+    logits, data, gs, gt = _setup(vocab)
+    x = logits.clone().requires_grad_(True)
+    with fad.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        _loss(route, x, {**data, key: fad.make_dual(data[key], torch.ones_like(data[key]))}, gs, gt)
+    leaf = data[key].clone().requires_grad_(True)
+    want = _loss(route, x, data, gs, gt)
+    (dx,) = torch.autograd.grad(want, x)
+    got = _loss(route, x, {**data, key: leaf}, gs, gt)
+    dx2, dleaf = torch.autograd.grad(got, (x, leaf), allow_unused=True)
+    assert torch.equal(dx, dx2) and dleaf is None
+    if route == "general":  # (the single pass is taken for logits that require a gradient)
+        got = _loss(route, logits, {**data, key: leaf}, gs, gt)
+        assert got.requires_grad and torch.autograd.grad(got, leaf, allow_unused=True) == (None,)
