@@ -473,6 +473,22 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> group_baseline_std(const Tensor& prom
 // Every tensor a node reads is an argument of its own, also those without a gradient: autograd looks at the arguments to refuse
 // forward-mode differentiation and to tell whether the result depends on a tensor that requires a gradient.
 
+// A gradient whose own gradient the kernels cannot give: under create_graph it depends on the upstream one, so that
+// differentiating it again says what is missing instead of taking it for a constant.
+struct FirstOrder : torch::autograd::Function<FirstOrder> {
+    static Tensor forward(AutogradContext*, const Tensor&, const Tensor& d) { return d; }
+    static variable_list backward(AutogradContext*, variable_list) {
+        TORCH_WARN("rl_amd: the gradient of this operation has no gradient of its own; what flows into it here is dropped");
+        return variable_list(2);
+    }
+};
+Tensor first_order(const variable_list& grads, const Tensor& d) {
+    if (at::GradMode::is_enabled())
+        for (const Tensor& g : grads)
+            if (g.defined() && g.requires_grad()) return FirstOrder::apply(g, d);
+    return d;
+}
+
 // logits [B, S, V], targets [B, >= n_inner] (already aligned to the rows) -> fp32 [B, n_inner].  Saved for the backward:
 // the logits (no copy), the targets and one fp32 log-sum-exp per row; the softmax is never materialised.
 struct RowsLogprob : torch::autograd::Function<RowsLogprob> {
@@ -493,7 +509,7 @@ struct RowsLogprob : torch::autograd::Function<RowsLogprob> {
         const auto saved = ctx->get_saved_variables();
         Tensor d = logprob_bwd(saved[0], saved[1], saved[2], to_f32(grads[0], saved[0]), a[0], a[1], a[2], ctx->saved_data["temperature"].toDouble(), a[3], false);
         variable_list out(8);
-        out[0] = d;
+        out[0] = first_order(grads, d);
         return out;
     }
 };
@@ -602,7 +618,7 @@ struct FusedRowsLoss : torch::autograd::Function<FusedRowsLoss> {
         Timed timed("rows_grad");
         check(nrl_rows_grad(&rows, ptr(saved[1]), ptr(factor), written, ptr<void>(d), d.dim() == 3 ? d.stride(0) : 0, d.stride(d.dim() - 2), stream_of(logits)),
               "nrl_rows_grad");
-        out[0] = d;
+        out[0] = first_order(grads, d);
         return out;
     }
 };
@@ -627,7 +643,7 @@ struct RowsLogprobSampled : torch::autograd::Function<RowsLogprobSampled> {
         Kept k;
         k.thr = s[2]; k.tie = s[3]; k.lse = s[4]; k.n = s[5]; k.idx = s[6]; k.x = s[7];
         variable_list out(9);
-        out[0] = topk_topp_bwd(s[0], s[1], k, to_f32(grads[0], s[0]), a[0], ctx->saved_data["temperature"].toDouble(), a[1]);
+        out[0] = first_order(grads, topk_topp_bwd(s[0], s[1], k, to_f32(grads[0], s[0]), a[0], ctx->saved_data["temperature"].toDouble(), a[1]));
         return out;
     }
 };
@@ -686,8 +702,8 @@ struct GatherEntropy : torch::autograd::Function<GatherEntropy> {
         const auto s = ctx->get_saved_variables();
         const bool entropy = ctx->saved_data["entropy"].toBool();
         variable_list out(4);
-        out[0] = gather_entropy_bwd(s[0], s[1], ctx->saved_data["n"].toInt(), s[2], entropy ? OptTensor(s[3]) : OptTensor(),
-                                    entropy ? OptTensor(to_f32(grads[1], s[0])) : OptTensor(), to_f32(grads[0], s[0]));
+        out[0] = first_order(grads, gather_entropy_bwd(s[0], s[1], ctx->saved_data["n"].toInt(), s[2], entropy ? OptTensor(s[3]) : OptTensor(),
+                                                       entropy ? OptTensor(to_f32(grads[1], s[0])) : OptTensor(), to_f32(grads[0], s[0])));
         return out;
     }
 };

@@ -46,3 +46,27 @@ def test_loss_inputs_are_inputs_of_the_node(route, vocab, key):
     if route == "general":  # (the single pass is taken for logits that require a gradient)
         got = _loss(route, logits, {**data, key: leaf}, gs, gt)
         assert got.requires_grad and torch.autograd.grad(got, leaf, allow_unused=True) == (None,)
+
+
+@pytest.mark.parametrize("op", ["logprobs", "filtered", "gather", "single pass"])
+def test_a_second_derivative_is_not_taken_for_zero(op):
+    """Under create_graph the gradient depends on the upstream one, and differentiating it warns."""
+    from rl_amd.algorithms.logits_sampling_utils import TrainingSamplingParams
+    from rl_amd.distributed import model_utils as MU
+
+    logits, data, gs, gt = _setup(4099)
+    x = logits.float().requires_grad_(True)
+    if op == "gather":
+        ids = data["input_ids"].unsqueeze(-1).contiguous()
+        y = MU.get_distillation_topk_logprobs_from_logits(x, torch.zeros_like(ids, dtype=torch.float32), ids, True, True)[0].square().sum()
+    elif op == "single pass":
+        y = _loss(op, x, data, gs, gt).square()
+    else:
+        params = TrainingSamplingParams(top_k=4000, top_p=1.0, temperature=1.0) if op == "filtered" else None
+        y = MU.from_parallel_logits_to_logprobs(x, data["input_ids"], 0, 4099, None, sampling_params=params).clamp(min=-50).square().sum()
+    (d,) = torch.autograd.grad(y, x, create_graph=True)
+    assert d.requires_grad
+    with pytest.warns(UserWarning, match="autograd|no gradient of its own"):
+        torch.autograd.grad(d.sum(), x, allow_unused=True)
+    (d,) = torch.autograd.grad(_loss("general", x, data, gs, gt), x)
+    assert not d.requires_grad
