@@ -178,6 +178,11 @@ def host():
         spec = importlib.util.spec_from_file_location("rl_amd.lib._host", HOST_PATH)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
+        built = getattr(module, "abi_version", None)
+        if built != ABI_VERSION:  # it would hand the library structures of another layout
+            raise RuntimeError(
+                f"{HOST_PATH} has ABI version {built}, this package is for {ABI_VERSION}: rebuild it with `python -m rl_amd.build`"
+            )
         _host = module
     return _host
 

@@ -27,6 +27,6 @@ int check_launch(const char* what) {
 
 }  // namespace nrl
 
-extern "C" int nrl_version(void) { return 116; }
+extern "C" int nrl_version(void) { return NRL_ABI_VERSION; }
 
 extern "C" const char* nrl_last_error(void) { return nrl::error_slot(); }

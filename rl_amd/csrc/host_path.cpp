@@ -745,6 +745,7 @@ class Fetch {
 
 PYBIND11_MODULE(_host, m) {
     m.doc() = "host path of the rl_amd training calls";
+    m.attr("abi_version") = NRL_ABI_VERSION;  // of the structures it hands to the library
     m.def("set_kernel_timer", [](py::object t) {
         delete g_timer;
         g_timer = t.is_none() ? nullptr : new py::object(t);

@@ -49,6 +49,20 @@ def test_cpu_tensors_fail_loudly():
         torch.ops.rl_amd.logprob_fwd(torch.randn(1, 2, 8), torch.zeros(1, 2, dtype=torch.long), 2, 0, 8, 1.0, 1, False)
 
 
+def test_host_path_of_another_abi_version_is_refused(monkeypatch, tmp_path):
+    """As an extension left over from a build whose second link failed: it fills structures of another layout."""
+    from rl_amd import _lib
+
+    assert _lib.host().abi_version == _lib.load().nrl_version()
+    for text in ("", f"abi_version = {_lib.ABI_VERSION - 1}"):
+        stale = tmp_path / "_host.py"
+        stale.write_text(text)
+        monkeypatch.setattr(_lib, "_host", None)
+        monkeypatch.setattr(_lib, "HOST_PATH", str(stale))
+        with pytest.raises(RuntimeError, match="rebuild"):
+            _lib.host()
+
+
 def test_missing_library_raises(monkeypatch):
     from rl_amd import _lib
 
