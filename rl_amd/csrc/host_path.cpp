@@ -101,6 +101,10 @@ Tensor grad_buffer(at::IntArrayRef shape, const Tensor& like) {
     return flat.narrow(0, off, bytes).view(like.scalar_type()).view(shape);
 }
 
+int64_t vocab_of(const Tensor& logits) {
+    TORCH_CHECK_VALUE(logits.dim() == 3, "expected logits [B,S,V], got ", logits.sizes());
+    return logits.size(2);
+}
 nrl_rows make_rows(const Tensor& logits, const Tensor& targets, int64_t n_inner, int64_t v0, int64_t v1, double temperature, int64_t mode) {
     TORCH_CHECK_VALUE(logits.dim() == 3 && (!targets.defined() || targets.dim() == 2), "expected logits [B,S,V] and targets [B,S'], got ",
                       logits.sizes());
@@ -312,7 +316,7 @@ FusedOut fused_loss(const Tensor& logits, const Tensor& targets, int64_t n_inner
         rows.tgt_stride_outer = 0;
         b = cu.size(0) - 1;
     } else {
-        rows = make_rows(logits, targets, n_inner, 0, logits.size(2), temperature, mode);
+        rows = make_rows(logits, targets, n_inner, 0, vocab_of(logits), temperature, mode);
         b = logits.size(0);
     }
     const c10::OptionalDeviceGuard guard(logits.device());
@@ -345,7 +349,7 @@ struct Kept {  // what a filtered forward leaves for its backward, with the reco
 Kept topk_topp_fwd(const Tensor& logits, const Tensor& targets, int64_t n_inner, int64_t top_k, double top_p, double temperature, int64_t mode,
                    bool want_unfiltered, int64_t capacity) {
     need_gpu(logits, targets);
-    const nrl_rows rows = make_rows(logits, targets, n_inner, 0, logits.size(2), temperature, mode);
+    const nrl_rows rows = make_rows(logits, targets, n_inner, 0, vocab_of(logits), temperature, mode);
     const int64_t b = logits.size(0);
     const c10::OptionalDeviceGuard guard(logits.device());
     const auto i32 = logits.options().dtype(at::kInt);
@@ -368,7 +372,7 @@ Kept topk_topp_fwd(const Tensor& logits, const Tensor& targets, int64_t n_inner,
 
 Tensor topk_topp_bwd(const Tensor& logits, const Tensor& targets, const Kept& k, const Tensor& grad, int64_t n_inner, double temperature, int64_t mode) {
     need_gpu(logits, targets, k.thr, k.tie, k.lse, grad, k.n, k.idx, k.x);
-    const nrl_rows rows = make_rows(logits, targets, n_inner, 0, logits.size(2), temperature, mode);
+    const nrl_rows rows = make_rows(logits, targets, n_inner, 0, vocab_of(logits), temperature, mode);
     const int64_t b = logits.size(0);
     for (const Tensor* t : {&k.thr, &k.tie, &k.lse})
         TORCH_CHECK_VALUE(t->sizes() == at::IntArrayRef({b, n_inner}) && t->is_contiguous(), "thr, tie and lse_kept must be contiguous [B, n_inner] tensors");
@@ -403,7 +407,7 @@ Tensor gather_indices(const Tensor& logits, const Tensor& indices) {
 // `entropy`) and the log-sum-exps, from one pass over the logits.
 std::tuple<Tensor, Tensor, Tensor> gather_entropy_fwd(const Tensor& logits, const Tensor& indices, int64_t n_inner, bool entropy) {
     need_gpu(logits, indices);
-    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, logits.size(2), 1.0, NRL_TEMP_RCP);
+    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, vocab_of(logits), 1.0, NRL_TEMP_RCP);
     const Tensor idx = gather_indices(logits, indices);
     const int64_t b = logits.size(0), s = logits.size(1), k = idx.size(2);
     const c10::OptionalDeviceGuard guard(logits.device());
@@ -418,7 +422,7 @@ Tensor gather_entropy_bwd(const Tensor& logits, const Tensor& indices, int64_t n
                           const OptTensor& grad_h_in, const Tensor& grad_in) {
     Tensor h = opt(h_in), grad_h = opt(grad_h_in);
     need_gpu(logits, indices, lse, h, grad_h, grad_in);
-    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, logits.size(2), 1.0, NRL_TEMP_RCP);
+    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, vocab_of(logits), 1.0, NRL_TEMP_RCP);
     const Tensor idx = gather_indices(logits, indices);
     const int64_t b = logits.size(0), s = logits.size(1), k = idx.size(2);
     auto scalar = [&](const Tensor& t, const char* name) {

@@ -70,3 +70,21 @@ def test_a_second_derivative_is_not_taken_for_zero(op):
         torch.autograd.grad(d.sum(), x, allow_unused=True)
     (d,) = torch.autograd.grad(_loss("general", x, data, gs, gt), x)
     assert not d.requires_grad
+
+
+def test_logits_of_another_rank_are_a_value_error():
+    from rl_amd.algorithms.logits_sampling_utils import TrainingSamplingParams
+    from rl_amd.distributed import model_utils as MU
+
+    logits, data, _, _ = _setup(4096)
+    flat, ids = logits[0], data["input_ids"]
+    params = TrainingSamplingParams(top_k=20, top_p=0.9, temperature=1.0)
+    ops = torch.ops.rl_amd
+    for call in (
+        lambda: MU.from_parallel_logits_to_logprobs(flat, ids, 0, 4096, None, sampling_params=params),
+        lambda: MU.from_parallel_logits_to_logprobs(flat, ids, 0, 4096, None),
+        lambda: ops.topk_topp_logprob_fwd(flat, ids, 8, 20, 0.9, 1.0, 1, False),
+        lambda: ops.gather_entropy_fwd(flat, ids.unsqueeze(-1), 8, True),
+    ):
+        with pytest.raises(ValueError, match="logits"):
+            call()
