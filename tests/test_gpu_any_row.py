@@ -1,10 +1,12 @@
 """The single pass over rows off the 16-byte grid or longer than the chip holds, reached through the wrappers, against the
-three-pass path.  The two sum a row's exponentials in different orders (about 1e-6 in the log-sum-exp), and round a gradient
+CPU oracle and the three-pass path.  They sum a row's exponentials in different orders (about 1e-6 in the log-sum-exp), and round a gradient
 element to its type once: neighbouring 16-bit values may differ, fp32 values by 1e-4 of the largest as in test_gpu_fused."""
 
 import pytest
 import torch
 
+from oracle import logprob as OL
+from oracle import loss as O
 from rl_amd.algorithms.logits_sampling_utils import TrainingSamplingParams
 from rl_amd.algorithms.loss import (
     ClippedPGLossConfig,
@@ -256,3 +258,69 @@ def test_a_named_factor_of_packed_rows():
     post = LossPostProcessor(fn, {"sequence_packing": {"enabled": True, "fuse_loss": True}}, num_microbatches=41)
     loss, _ = post(dict(data), SimpleNamespace(cu_seqlens_q=cu, cu_seqlens_q_padded=cu), gs, gt)(x)
     _untouched_by_backward(x, loss / 41, 1.0, want.float())
+
+
+# one length for every workgroup size and number of register slots, the form for rows longer than the chip holds last
+@pytest.mark.parametrize("dtype,vocab", [(torch.bfloat16, 20003), (torch.bfloat16, 30001), (torch.bfloat16, 40961), (torch.bfloat16, 50257),
+                                         (torch.bfloat16, 65003), (torch.bfloat16, 81919), (torch.bfloat16, 98305), (torch.bfloat16, 131075),
+                                         (torch.bfloat16, 163841), (torch.float16, 50257), (torch.float32, 32003), (torch.float32, 151936)])
+def test_rows_of_any_length_against_the_oracle(dtype, vocab):
+    logits, data, gs, gt = _batch(4, 7, vocab, dtype, seed=vocab + 1)
+    cfg = dict(reference_policy_kl_penalty=0.05)
+    xo = logits.float().clone().requires_grad_(True)
+    want, _ = O.clipped_pg_loss(O.LossConfig(**cfg), OL.next_token_logprobs(data["input_ids"], xo), data, gs, gt)
+    want.backward()
+    x = logits.to(DEV).requires_grad_(True)
+    fn = ClippedPGLossFn(ClippedPGLossConfig(**cfg))
+    dev = {k: v.to(DEV) for k, v in data.items()}
+    assert any_row_fusable(fn, x, dev) and why_not_fusable(fn, x, dev) is not None
+    got, _ = wrap_loss_fn_with_input_preparation(x, dev, gs.to(DEV), gt.to(DEV), fn, prepare_loss_input)
+    got.backward()
+    assert _close(got.item(), want.item(), rel=1e-4)
+    # (the oracle's gradient is fp32: an fp16 one is rounded to multiples of 2^-24 where it is subnormal, half of that off)
+    wanted = xo.grad if dtype != torch.float16 else torch.where((xo.grad - x.grad.cpu().float()).abs() <= 2.0 ** -25, x.grad.cpu().float(), xo.grad)
+    _same_gradient(x.grad.cpu(), wanted, dtype)
+
+
+def _many_rows(b, s, vocab, dtype, seed):
+    """As ``_batch``, made on the GPU: every sequence but one carries tokens, behind a prompt of its own length."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    x = (torch.randn(b, s, vocab, generator=g, device=DEV) * 2.5).to(dtype)
+    ids = torch.randint(0, vocab, (b, s), generator=g, device=DEV)
+    lp = torch.stack([x[i, :-1].float().log_softmax(-1).gather(-1, ids[i, 1:, None]).squeeze(-1) for i in range(b)])
+    cur = torch.cat([torch.zeros(b, 1, device=DEV), lp], 1)
+    noise = lambda: 0.05 * torch.randn(b, s, generator=g, device=DEV)  # noqa: E731
+    prompt = torch.randint(1, s // 3, (b, 1), generator=g, device=DEV)
+    data = {"input_ids": ids, "token_mask": (torch.arange(s, device=DEV) >= prompt).long(), "sample_mask": torch.ones(b, device=DEV),
+            "advantages": torch.randn(b, 1, generator=g, device=DEV).expand(b, s).contiguous(), "prev_logprobs": cur + noise(),
+            "generation_logprobs": cur + noise(), "reference_policy_logprobs": cur + noise()}
+    data["sample_mask"][b // 2] = 0
+    return x, data, data["sample_mask"].sum(), (data["token_mask"][:, 1:] * data["sample_mask"][:, None]).sum()
+
+
+# more rows than workgroups are resident (1024 of 256 threads, 512 of 512, 256 of 1024), so that a workgroup goes from one row to
+# others with another head and tail; the aligned lengths are the longest of their workgroup size
+WALKS = [(1100, 20003), (600, 50257), (600, 81919), (300, 98305), (300, 163003), (300, 164001), (1100, 40960), (600, 81920), (300, 163840)]
+
+
+@pytest.mark.parametrize("rows,vocab", WALKS)
+@pytest.mark.parametrize("packed", [False, True])
+def test_a_workgroup_walks_several_rows(rows, vocab, packed):
+    b = 4
+    logits, data, gs, gt = _many_rows(b, rows // b, vocab, torch.bfloat16, seed=vocab)
+    fn = ClippedPGLossFn(ClippedPGLossConfig(reference_policy_kl_penalty=0.05))
+    if packed:
+        cu = torch.arange(0, rows + 1, rows // b, dtype=torch.int32, device=DEV)
+        xf, xu = (logits.reshape(1, rows, vocab).clone().requires_grad_(True) for _ in range(2))
+        got, _ = SequencePackingFusionLossWrapper(fn, prepare_packed_loss_input, cu, cu)(xf, data, gs, gt)
+        loss_input, d2 = prepare_packed_loss_input(xu, dict(data), fn, cu, cu)
+        want, _ = fn(data=d2, global_valid_seqs=gs, global_valid_toks=gt, **loss_input)
+    else:
+        xf, xu = (logits.clone().requires_grad_(True) for _ in range(2))
+        got, _ = wrap_loss_fn_with_input_preparation(xf, data, gs, gt, fn, prepare_loss_input)
+        want, _ = _three_pass(xu, data, fn, gs, gt)
+    assert _close(got.item(), want.item(), rel=1e-4)
+    got.backward()
+    want.backward()
+    _same_gradient(xf.grad, xu.grad, torch.bfloat16)
+    assert bool((xf.grad.reshape(b, rows // b, vocab)[:, -1] == 0).all()) and bool((xf.grad.float().abs().sum(-1) > 0).float().mean() > 0.4)
