@@ -27,39 +27,46 @@ if ROOT not in sys.path:
 HBM_PEAK_GBS = 8000.0  # MI355X published HBM3E bandwidth
 
 def source_fingerprint(name):
-    """First 12 hex digits of the SHA-256 of ``rl_amd/csrc/<name>``: what a row of the traffic table is tied to."""
+    """First 12 hex digits of the SHA-256 of the files ``rl_amd/csrc/<name>``, several joined with ``+``: what a row of the
+    traffic table is tied to."""
     import hashlib
 
+    digest = hashlib.sha256()
     try:
-        with open(os.path.join(ROOT, "rl_amd", "csrc", name), "rb") as fh:
-            return hashlib.sha256(fh.read()).hexdigest()[:12]
+        for part in name.split("+"):
+            with open(os.path.join(ROOT, "rl_amd", "csrc", part.strip()), "rb") as fh:
+                digest.update(fh.read())
     except OSError:
         return None
+    return digest.hexdigest()[:12]
+
+
+def traffic_rows():
+    """The cells of every row of the traffic table."""
+    try:
+        with open(os.path.join(ROOT, "profiles", "measured_traffic.md")) as fh:
+            lines = fh.read().splitlines()
+    except OSError:
+        return []
+    rows = ([c.strip() for c in line.strip().strip("|").split("|")] for line in lines)
+    return [c for c in rows if len(c) == 7 and c[0] != "key" and not set(c[0]) <= set("-")]
 
 
 def load_measured_traffic():
     """HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, from the committed table
     ``profiles/measured_traffic.md`` (key -> dict(kernel, read, write, profile)).  Each row names the profile summary
-    it was taken from and the kernel's source file with that file's fingerprint at the time of the measurement; a
+    it was taken from and the kernel's source files with their fingerprint at the time of the measurement; a
     row whose source has changed since is dropped here, so the JSON line says ``traffic: null`` instead of quoting
     bytes that belong to another version of the kernel."""
     table = {}
-    path = os.path.join(ROOT, "profiles", "measured_traffic.md")
-    try:
-        with open(path) as fh:
-            for line in fh:
-                cells = [c.strip() for c in line.strip().strip("|").split("|")]
-                if len(cells) == 7 and cells[0] not in ("key", "---") and not set(cells[0]) <= set("-"):
-                    try:
-                        name, _, stamp = cells[5].partition("@")
-                        if source_fingerprint(name.strip()) != stamp.strip():
-                            continue
-                        table[cells[0]] = dict(kernel=cells[1], shape=cells[2], read=float(cells[3]), write=float(cells[4]),
-                                               profile=cells[6])
-                    except ValueError:
-                        pass
-    except OSError:
-        pass
+    for cells in traffic_rows():
+        name, _, stamp = cells[5].partition("@")
+        if source_fingerprint(name.strip()) != stamp.strip():
+            continue
+        try:
+            table[cells[0]] = dict(kernel=cells[1], shape=cells[2], read=float(cells[3]), write=float(cells[4]), profile=cells[6])
+        except ValueError:
+            pass
     return table
 
 
@@ -968,10 +975,8 @@ def main():
 def _main():
     args = parse_args()
     if args.source_fingerprints:
-        import glob
-
-        for path in sorted(glob.glob(os.path.join(ROOT, "rl_amd", "csrc", "*.hip"))):
-            print("%s@%s" % (os.path.basename(path), source_fingerprint(os.path.basename(path))), file=_JSON_OUT)
+        for name in sorted({cells[5].partition("@")[0].strip() for cells in traffic_rows()}):
+            print("%s@%s" % (name, source_fingerprint(name)), file=_JSON_OUT)
         return
     if args.gpus != 1:
         print("bench.py: this build runs on ONE GPU; --gpus must be 1 (no multi-GPU path exists)", file=sys.stderr)

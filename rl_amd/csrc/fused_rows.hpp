@@ -88,8 +88,11 @@ __device__ __forceinline__ void load_to_lds(const char* base, int bytes, int off
 // EDGE: rows need not start or end on 16 bytes.  The vectors of a row begin at its first 16-byte boundary; the up to 7 elements
 // before it and the tail shorter than a vector are one element each of the first 32 lanes.  (Input and output rows sit alike.)
 // LONG (1024 threads): vectors past the on-chip slots are read twice.  They are the last ones read of a row and the first
-// ones its gradient needs, in reverse order, so the second read finds them in the 256 MB cache: at most 256 rows' excess
-// lies between the two (85 MB at V = 151936 fp32).
+// ones its gradient needs, in reverse order, so that the second read finds them in the 256 MB cache: at most 256 rows' excess
+// lies between the two (72 MB at V = 151936 fp32, 185 MB in the longest rows taken, 1 MiB; gradient stores of other rows pass
+// through the same cache meanwhile).  The counters of L2 fills see both reads alike; what speaks for the cache is the rate
+// with the second read counted: whole calls at 5.2, 5.6 and 5.85 TB/s for V = 151936, 200000 and 262144 fp32, where rows that
+// fit are served at 4.9 - 5.1.
 // Both against the three passes (logprobs, loss, gradient) such rows took before, whole calls: 2 x 1024 rows of V = 151936 fp32
 // 710 -> 498 us, of V = 262144 bf16 577 -> 478, 2 x 512 of V = 262144 fp32 574 -> 447; 3 x 701 rows of V = 50257 bf16 152 -> 144,
 // 4 x 2048 of V = 20001 200 -> 156; 128 rows of V = 262143 fp32 186 -> 105.
@@ -299,6 +302,11 @@ template <int DT, int TEMP, int BLOCK, int NREG, int NLDS = kFusedLdsVec, bool E
     if (l.packed) fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, NLDS, EDGE, LONG, true><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
     else fused_logits_loss_kernel<DT, TEMP, BLOCK, NREG, NLDS, EDGE, LONG, false><<<grid, block, 0, l.stream>>>(l.a, l.n_rows);
 }
+// Slots past the end of a row are loaded, computed and stored all the same, so a row takes the form with the fewest that
+// hold it.  Whole calls of bf16 rows against the 16-slot form of the same workgroup size, on the 16-byte grid and off it:
+// 8 register slots, at V = 24576 / 49152 / 98304: 9 and 12 % faster (256 threads), 14 and 21 % (512), 17 and 16 % (1024); 12: 256
+// threads 8 and 11 % at V = 25600, 3 and 6 at 28672, 0 and 3 at 30720, 3 and 2 % slower at 32768; 512 threads 1 and 10 % at
+// 65536; 1024 threads 4 and 8 % at 131072; 4 at V = 16384: 31 %.
 template <int DT, int TEMP, int BLOCK> void fused_launch(const FusedLaunch& l, int64_t slots) {
     if (slots <= 12) fused_launch<DT, TEMP, BLOCK, 8>(l);
     else if (slots <= 16) fused_launch<DT, TEMP, BLOCK, 12>(l);
@@ -333,7 +341,7 @@ template <int DT> void fused_launch(const FusedLaunch& l) {
         return;
     }
     if (l.temp == 0) fused_launch<DT, 0>(l);
-    else if (l.temp == 1) fused_launch<DT, 1>(l);
+    else if (l.temp == 1) fused_launch<DT, 1>(l);  // NRL_TEMP_DIV, for direct callers: the wrappers' divide is PyTorch's on the GPU, a multiplication
     else fused_launch<DT, 2>(l);
 }
 
