@@ -745,6 +745,22 @@ class Fetch {
     hipEvent_t done_ = nullptr;
 };
 
+// The registered operators take what the kernels take: fp32 on the GPU.  (The calls of a training step convert and move.)
+template <typename T> const T& operator_input(const T& t_in, const char* name) {
+    const Tensor t = OptTensor(t_in).value_or(Tensor());
+    need_gpu(t);
+    TORCH_CHECK_VALUE(!t.defined() || t.scalar_type() == at::kFloat, name, " must be fp32, got ", t.scalar_type(), " ", t.sizes());
+    return t_in;
+}
+LossData operator_data(const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
+                       const OptTensor& correct, const Tensor& global_valid) {
+    TORCH_CHECK_VALUE(operator_input(global_valid, "global_valid").dim() == 1 && global_valid.size(0) == 2,
+                      "global_valid must be fp32 [2] = (valid_seqs, valid_toks)");
+    return loss_data(operator_input(prev, "prev"), operator_input(gen, "gen"), operator_input(ref, "ref"), operator_input(adv, "adv"),
+                     operator_input(token_mask, "token_mask"), operator_input(sample_mask, "sample_mask"), operator_input(correct, "correct_mask"),
+                     global_valid[0], global_valid[1], 0);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -766,21 +782,17 @@ PYBIND11_MODULE(_host, m) {
     m.def("grpo_loss", [](const Tensor& lp, const OptTensor& lpu, const OptTensor& prev, const Tensor& gen, const OptTensor& ref, const Tensor& adv,
                           const Tensor& token_mask, const Tensor& sample_mask, const OptTensor& correct, const Tensor& global_valid,
                           const std::vector<int64_t>& iflags, const std::vector<double>& fparams) {
-        TORCH_CHECK_VALUE(global_valid.scalar_type() == at::kFloat && global_valid.dim() == 1 && global_valid.size(0) == 2,
-                          "global_valid must be fp32 [2] = (valid_seqs, valid_toks)");
-        const GrpoOut o = grpo_loss(lp, opt(lpu), loss_data(prev, gen, ref, adv, token_mask, sample_mask, correct, global_valid[0], global_valid[1], 0),
-                                    make_cfg(iflags, fparams));
+        const GrpoOut o = grpo_loss(operator_input(lp, "lp"), opt(operator_input(lpu, "lpu")),
+                                    operator_data(prev, gen, ref, adv, token_mask, sample_mask, correct, global_valid), make_cfg(iflags, fparams));
         return std::make_tuple(o.loss, o.dlp, o.dlpu, o.metrics);
     });
     m.def("fused_loss", [](const Tensor& logits, const Tensor& targets, int64_t n_inner, const OptTensor& cu, bool pre_rolled, const OptTensor& prev,
                            const Tensor& gen, const OptTensor& ref, const Tensor& adv, const Tensor& token_mask, const Tensor& sample_mask,
                            const Tensor& global_valid, const std::vector<int64_t>& iflags, const std::vector<double>& fparams, double loss_scale,
                            double temperature, int64_t mode, bool in_place) {
-        TORCH_CHECK_VALUE(global_valid.scalar_type() == at::kFloat && global_valid.dim() == 1 && global_valid.size(0) == 2,
-                          "global_valid must be fp32 [2] = (valid_seqs, valid_toks)");
         const FusedOut o = fused_loss(logits, targets, n_inner, opt(cu), pre_rolled,
-                                      loss_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, global_valid[0], global_valid[1], 0),
-                                      make_cfg(iflags, fparams), loss_scale, temperature, mode, in_place);
+                                      operator_data(prev, gen, ref, adv, token_mask, sample_mask, std::nullopt, global_valid), make_cfg(iflags, fparams),
+                                      loss_scale, temperature, mode, in_place);
         return std::make_tuple(o.loss, o.dlogits, o.lp, o.metrics);
     });
     m.def("topk_topp_fwd", [](const Tensor& logits, const OptTensor& targets, int64_t n_inner, int64_t top_k, double top_p, double temperature, int64_t mode,

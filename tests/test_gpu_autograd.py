@@ -1,4 +1,4 @@
-"""What autograd sees of the nodes of the C++ host path."""
+"""The C++ host path: what autograd sees of its nodes, and what its operators refuse."""
 
 import pytest
 import torch
@@ -88,3 +88,28 @@ def test_logits_of_another_rank_are_a_value_error():
     ):
         with pytest.raises(ValueError, match="logits"):
             call()
+
+
+@pytest.mark.parametrize("name", ["lp", "prev", "gen", "ref", "adv", "token_mask", "sample_mask", "global_valid"])
+def test_loss_operators_take_fp32_on_the_gpu_only(name):
+    ops = torch.ops.rl_amd
+    logits, data, _, _ = _setup(4096)
+    iflags, fparams = ClippedPGLossFn(ClippedPGLossConfig())._kernel_config(False)
+    rows = lambda k: data[k][:, 1:].float().contiguous()  # noqa: E731
+    good = dict(lp=-torch.rand(3, 8, device=DEV), prev=rows("prev_logprobs"), gen=rows("generation_logprobs"), ref=rows("reference_policy_logprobs"),
+                adv=rows("advantages"), token_mask=rows("token_mask"), sample_mask=data["sample_mask"].float(),
+                global_valid=torch.tensor([2.0, 9.0], device=DEV))
+
+    def general(a):
+        return ops.grpo_loss(a["lp"], None, a["prev"], a["gen"], a["ref"], a["adv"], a["token_mask"], a["sample_mask"], None,
+                             a["global_valid"], iflags, fparams)
+
+    def single_pass(a):
+        return ops.fused_logits_grpo_loss(logits, data["input_ids"][:, 1:], 8, a["prev"], a["gen"], a["ref"], a["adv"], a["token_mask"],
+                                          a["sample_mask"], a["global_valid"], iflags, fparams, 1.0, 1.0, 1)
+
+    for call in (general, single_pass)[: 1 if name == "lp" else 2]:
+        call(good)
+        for bad in (good[name].double(), good[name].long(), good[name].cpu()):
+            with pytest.raises((ValueError, RuntimeError), match="fp32|GPU only"):
+                call({**good, name: bad})
