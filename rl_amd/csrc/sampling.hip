@@ -25,6 +25,8 @@
 // alone, thousands of exact ties, or a top_k in the thousands) are marked and finished by
 // topk_topp_wide_kernel, which finds the same predicate by a radix descent over the row's order keys
 // (a histogram pass per key digit: two to three passes for 16-bit logits).
+//
+// bf16 rows under top-p alone take none of this: nucleus_count_kernel counts the elements of every value.
 
 #include <float.h>
 #include <math.h>
@@ -151,8 +153,8 @@ __device__ __forceinline__ float wave_sum_list(const float* e, int n) {
     return static_cast<float>(wave_sum_double(s));
 }
 
-// descending bitonic sort of sh.cand[0 .. n_pad)
-template <int CAP> __device__ __forceinline__ void sort_candidates_desc(SelShared<CAP>& sh, int n_pad) {
+// descending bitonic sort of list[0 .. n_pad) in LDS by a workgroup of THREADS; n_pad is a power of two
+template <int THREADS> __device__ __forceinline__ void sort_list_desc(unsigned long long* list, int n_pad) {
     const int tid = threadIdx.x;
     if (n_pad <= 2 * kWave) {
         // short lists (the usual case under top-k) are sorted by one wave alone: its LDS operations execute
@@ -166,8 +168,8 @@ template <int CAP> __device__ __forceinline__ void sort_candidates_desc(SelShare
                         const int lo = ((i / stride) * (stride << 1)) + (i % stride);
                         const int hi = lo + stride;
                         const bool desc = ((lo & size) == 0);
-                        const unsigned long long a = sh.cand[lo], b = sh.cand[hi];
-                        if ((a < b) == desc) { sh.cand[lo] = b; sh.cand[hi] = a; }
+                        const unsigned long long a = list[lo], b = list[hi];
+                        if ((a < b) == desc) { list[lo] = b; list[hi] = a; }
                     }
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                     __builtin_amdgcn_wave_barrier();
@@ -181,12 +183,12 @@ template <int CAP> __device__ __forceinline__ void sort_candidates_desc(SelShare
     for (int size = 2; size <= n_pad; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
             __syncthreads();
-            for (int i = tid; i < (n_pad >> 1); i += kSelBlock) {
+            for (int i = tid; i < (n_pad >> 1); i += THREADS) {
                 const int lo = ((i / stride) * (stride << 1)) + (i % stride);
                 const int hi = lo + stride;
                 const bool desc = ((lo & size) == 0);
-                const unsigned long long a = sh.cand[lo], b = sh.cand[hi];
-                if ((a < b) == desc) { sh.cand[lo] = b; sh.cand[hi] = a; }
+                const unsigned long long a = list[lo], b = list[hi];
+                if ((a < b) == desc) { list[lo] = b; list[hi] = a; }
             }
         }
     }
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
             if (pos < CAP) sh.cand[pos] = (static_cast<unsigned long long>(key) << 32) | static_cast<uint32_t>(index);
         }
     };
-    auto push_raw = [&](const u32x4& q, int64_t vi) {
+    auto push_raw = [&](const u32x4& q, int vi) {
         float t[EPV];
         Row<DT>::decode(q, t);
 #pragma unroll
@@ -597,7 +599,7 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
     int n_pad = 1;
     while (n_pad < n) n_pad <<= 1;
     for (int i = n + tid; i < n_pad; i += kSelBlock) sh.cand[i] = 0ull;  // sorts last
-    sort_candidates_desc(sh, n_pad);
+    sort_list_desc<kSelBlock>(sh.cand, n_pad);
 
     // ---- top-k threshold (ties kept), softmax over the kept values ----
     int n_k = n;
@@ -698,6 +700,480 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
                 a.logprob[r] = lp;
                 if (a.logprob_full) a.logprob_full[r] = lpf;
             }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// top-p alone over bf16 rows: nothing is sorted and no exponential is taken per element.  A bf16 row has few distinct
+// values, so the number of elements per value says everything: one pass over the row counts them in LDS, one bin per
+// value, and the bins (count x exp(value - max), in double, walked from the smallest value) give the log-sum-exp, the
+// threshold, how many of the elements that tie with it fall, and the kept log-sum-exp.  A second pass, from cache, runs
+// only to find the first survivor among such ties or to record a small kept set.
+//
+// The 16384 bins hold the magnitudes in [2^-31, 2^33), 64 binades of 128 values for either sign.  Smaller magnitudes
+// weigh exp(0) to well below an fp32 rounding and share one count; a row whose threshold is among them, or that holds a
+// larger value, is left to the wide kernel.  Larger negative values weigh nothing next to any value of the bins.
+// Counts are integers and every sum runs in a fixed order, so a row comes out the same every time.
+//
+// What bounds it: the LDS atomics of the first pass, about 15 cycles per 64 elements and compute unit, where the row
+// itself would arrive in 11; then the latency of the steps between two passes, which two workgroups of 1024 threads per
+// compute unit cover for each other (workgroups of 512, of which the bins admit two as well: 195 us).  With a kept-set
+// record, top_p 0.95, standard deviations 2 - 6, against candidate lists, a sort and the radix descent of the wide kernel:
+// 1499 rows of V = 151 936 145 us (62 to read the rows) and 726; 180 rows of V = 205 350 47 and 470; 4000 rows of 32 000
+// with a temperature 158 and 408; 800 rows of 9001 37 and 185.
+// ---------------------------------------------------------------------------------------------
+constexpr int kNucThreads = 1024, kNucWaves = kNucThreads / kWave;
+constexpr int kNucLow = 0x3000;                     // bf16 bits of 2^-31, the smallest magnitude with a bin of its own
+constexpr int kNucSide = 0x2000;                    // bins per sign: magnitudes 0x3000 .. 0x4fff
+constexpr int kNucBins = 2 * kNucSide;
+constexpr int kNucChunks = kNucBins / kWave;        // the bins in ascending order of the value, a wave's lanes at a time
+constexpr int kNucList = 4096;                      // entries of the list a small kept set is collected in (over the bins)
+constexpr int kNucLoads = 4;                        // 16-byte loads in flight per thread
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short i16x2 __attribute__((ext_vector_type(2)));
+
+struct NucShared {
+    union {
+        uint32_t bin[kNucBins];
+        struct {
+            unsigned long long list[kNucList];
+            uint16_t hit[kNucThreads];  // threads that saw an element of the kept set
+        };
+        uint32_t block[kNucThreads];  // elements equal to the threshold, per block of indices
+    };
+    double chunk_mass[kNucChunks];
+    int chunk_n[kNucChunks];
+    int key_w[kNucWaves];          // largest value of a wave, as a number that ascends with it
+    uint32_t block_w[kNucWaves], step_n[3];
+    int n_small, odd;
+    int n_list, n_hit, tie;
+};
+
+// bin number in ascending order of the value -> its place in LDS; -> the value
+__device__ __forceinline__ int nuc_bin(int rank) { return rank < kNucSide ? kNucBins - 1 - rank : rank - kNucSide; }
+__device__ __forceinline__ float nuc_value(int rank) {
+    const uint32_t bits = rank < kNucSide ? 0x8000u | static_cast<uint32_t>(kNucSide - 1 - rank + kNucLow) : static_cast<uint32_t>(rank - kNucSide + kNucLow);
+    return bf16_bits_to_f32(bits);
+}
+
+// sum and maximum of an int (>= 0) over a wave, by lane moves
+template <typename F> __device__ __forceinline__ int wave_fold_int(int v, F f) {
+    v = f(v, __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
+    v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
+    v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false));  // row_half_mirror
+    v = f(v, __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, false));  // row_mirror
+    return f(f(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)), f(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+__device__ __forceinline__ int wave_sum_int(int v) { return wave_fold_int(v, [](int p, int q) { return p + q; }); }
+__device__ __forceinline__ int wave_max_int(int v) { return wave_fold_int(v, [](int p, int q) { return p > q ? p : q; }); }
+
+// inclusive sum over the lanes up to this one, by lane moves
+__device__ __forceinline__ double wave_scan_double(double v) {
+    auto add = [&](auto ctrl, int rows) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        constexpr int CTRL = decltype(ctrl)::value;
+        const int lo = static_cast<int>(u), hi = static_cast<int>(u >> 32);
+        uint32_t l, h;  // lanes outside the move bring zero
+        if (rows == 0xf) { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, false); }
+        else if (rows == 0xa) { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xa, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xa, 0xf, false); }
+        else { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xc, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xc, 0xf, false); }
+        v += __builtin_bit_cast(double, (static_cast<uint64_t>(h) << 32) | l);
+    };
+    add(std::integral_constant<int, 0x111>{}, 0xf);  // row_shr 1, 2, 4, 8: sums inside the rows of 16 lanes
+    add(std::integral_constant<int, 0x112>{}, 0xf);
+    add(std::integral_constant<int, 0x114>{}, 0xf);
+    add(std::integral_constant<int, 0x118>{}, 0xf);
+    add(std::integral_constant<int, 0x142>{}, 0xa);  // row_bcast 15: the row before, to rows 1 and 3
+    add(std::integral_constant<int, 0x143>{}, 0xc);  // row_bcast 31: the first two rows, to rows 2 and 3
+    return v;
+}
+
+constexpr int kOddNan = 1, kOddLarge = 2;  // a NaN or +inf; a finite value above the bins
+
+template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_count_kernel(SelArgs a) {
+    using R = Row<NRL_BF16>;
+    __shared__ NucShared sh;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const int64_t r = blockIdx.x;
+    const uint32_t o = blockIdx.x / static_cast<uint32_t>(a.n_inner);  // (fewer than 2^31 rows)
+    const int64_t i_in = blockIdx.x - o * static_cast<uint32_t>(a.n_inner);
+    const char* row = static_cast<const char*>(a.logits) + (o * a.stride_outer + i_in * a.stride_inner) * R::BYTES;
+    const int64_t vocab = a.vocab;
+    const int64_t head = sel_row_head<NRL_BF16>(row, vocab);
+    const int64_t nvec = (vocab - head) / R::EPV;
+    const int64_t tail0 = head + nvec * R::EPV;
+    const u32x4* xv = reinterpret_cast<const u32x4*>(row + head * R::BYTES);
+
+    // a vector of scaled logits, still as bf16 bits
+    auto scaled_bits = [&](const u32x4& q) -> u32x4 {
+        if constexpr (TEMP == 0) return q;
+        float t[R::EPV];
+        R::decode(q, t);
+#pragma unroll
+        for (int k = 0; k < R::EPV; ++k) t[k] = TEMP == 1 ? __fdiv_rn(t[k], a.tparam) : t[k] * a.tparam;
+        return R::encode(t);
+    };
+    auto load_scaled = [&](int64_t e) { return scale_logit<NRL_BF16, TEMP>(R::load1(row, e), a.tparam); };
+    // f(scaled vector, its index) over the kNucStep vectors from `base` on, or over the row
+    const int n_vec = static_cast<int>(nvec);
+    constexpr int kNucStep = kNucLoads * kNucThreads;
+    auto for_step = [&](int base, auto f) {
+        if (base >= n_vec) return;
+        u32x4 q[kNucLoads];
+#pragma unroll
+        for (int u = 0; u < kNucLoads; ++u) q[u] = xv[base + u * kNucThreads < n_vec ? base + u * kNucThreads : n_vec - 1];
+#pragma unroll
+        for (int u = 0; u < kNucLoads; ++u)
+            if (base + u * kNucThreads < n_vec) f(scaled_bits(q[u]), base + u * kNucThreads);
+    };
+    auto for_vectors = [&](auto f) {
+        for (int base = tid; base < n_vec; base += kNucStep) for_step(base, f);
+    };
+
+    // the target's logit, on its way while the row is counted
+    int64_t tg = -1;
+    float x_tg = 0.f;
+    if (a.targets && a.logprob) {
+        tg = a.targets[o * a.ts_outer + i_in * a.ts_inner];
+        if (tg >= 0 && tg < vocab) x_tg = R::load1(row, tg);
+    }
+
+    // ---- count the elements of every value ----
+#pragma unroll
+    for (int i = tid; i < kNucBins / 4; i += kNucThreads) reinterpret_cast<u32x4*>(sh.bin)[i] = u32x4{0u, 0u, 0u, 0u};
+    if (tid == 0) { sh.n_small = 0; sh.odd = 0; sh.n_list = 0; sh.n_hit = 0; }
+    __syncthreads();
+    int n_small = 0, odd = 0;
+    // the largest of this thread's bits as signed numbers, which is its largest value if that is not negative, and the
+    // smallest as unsigned ones, which is its largest value if all are negative; by halves of the words
+    i16x2 largest = {-32768, -32768};
+    u16x2 least = {65535, 65535};
+    // t: bits - kNucLow.  Its top four bits tell the ranges apart: 0, 1 and 8, 9 the bins of either sign, 2 - 4 larger
+    // (also NaN), 5 - 7 and 13 - 15 smaller magnitudes, 10 - 12 larger negative ones (also NaN).
+    auto count_one = [&](uint32_t t) {
+        if (!(t & 0x6000u)) { atomicAdd(&sh.bin[(t & 0x1fffu) | ((t >> 2) & 0x2000u)], 1u); return; }
+        const uint32_t bits = (t + kNucLow) & 0xffffu, mag = bits & 0x7fffu;
+        if (mag > 0x7f80u || bits == 0x7f80u) odd |= kOddNan;
+        else if (mag < static_cast<uint32_t>(kNucLow)) ++n_small;
+        else if (!(bits & 0x8000u)) odd |= kOddLarge;
+    };
+    for_vectors([&](const u32x4& q, int) {
+        uint32_t t[4], outside = 0u;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const uint32_t pair = q[w];  // (__builtin_bit_cast straight from q[w] reads element 0 whatever w is)
+            largest = __builtin_elementwise_max(largest, __builtin_bit_cast(i16x2, pair));
+            least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, pair));
+            t[w] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, pair) - u16x2{kNucLow, kNucLow});
+            outside |= t[w] & 0x60006000u;
+        }
+        if (outside == 0u) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const u16x2 up = __builtin_bit_cast(u16x2, t[w]) >> 2;
+                const uint32_t at = (t[w] & 0x1fff1fffu) | (__builtin_bit_cast(uint32_t, up) & 0x20002000u);
+                atomicAdd(&sh.bin[at & 0xffffu], 1u);
+                atomicAdd(&sh.bin[at >> 16], 1u);
+            }
+        } else {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) { count_one(t[w] & 0xffffu); count_one(t[w] >> 16); }
+        }
+    });
+    auto count_scalar = [&](int64_t e) {
+        const uint32_t bits = f32_to_bf16_bits(load_scaled(e));
+        count_one((bits - kNucLow) & 0xffffu);
+        largest.x = static_cast<short>(bits) > largest.x ? static_cast<short>(bits) : largest.x;
+        least.x = static_cast<unsigned short>(bits) < least.x ? static_cast<unsigned short>(bits) : least.x;
+    };
+    if (tid < head) count_scalar(tid);
+    if (tail0 + tid < vocab) count_scalar(tail0 + tid);
+    if (n_small) atomicAdd(&sh.n_small, n_small);
+    if (odd) atomicOr(&sh.odd, odd);
+    {
+        const int high = largest.x > largest.y ? largest.x : largest.y;
+        const int low = least.x < least.y ? least.x : least.y;
+        const int key = wave_max_int(high >= 0 ? 0x8000 | high : 0xffff & ~low);  // ascending with the value
+        if (lane == 0) sh.key_w[wave] = key;
+    }
+    __syncthreads();
+    n_small = sh.n_small;
+    odd = sh.odd;
+    uint32_t max_bits;  // of the row
+    {
+        int key = sh.key_w[0];
+#pragma unroll
+        for (int w = 1; w < kNucWaves; ++w) key = sh.key_w[w] > key ? sh.key_w[w] : key;
+        max_bits = static_cast<uint32_t>(key & 0x8000 ? key & 0x7fff : 0xffff & ~key);
+    }
+    const uint32_t max_mag = max_bits & 0x7fffu;
+    const bool max_binned = max_mag - kNucLow < static_cast<uint32_t>(kNucSide);
+    const float m = max_binned ? bf16_bits_to_f32(max_bits) : 0.f;  // (a maximum under the bins counts as 0)
+    // (every wave finds the same values from here on: what they rest on is read from LDS by all)
+    int pick = -1, n_eq = 0, above = 0;
+    float e_thr = 0.f;
+    double z = 0.0, below = 0.0, cut = 0.0;
+    if (!odd && (max_binned || n_small > 0)) {
+        // ---- mass and elements of every chunk of bins, the waves taking turns: what is not empty lies close together ----
+#pragma unroll 4
+        for (int c = wave; c < kNucChunks; c += kNucWaves) {
+            const int rank = c * kWave + lane, n = static_cast<int>(sh.bin[nuc_bin(rank)]);
+            double mass = 0.0;
+            int elems = 0;
+            if (__ballot(n != 0)) {
+                if (n) mass = static_cast<double>(n) * static_cast<double>(expf(nuc_value(rank) - m));
+                mass = wave_sum_double(mass);
+                elems = wave_sum_int(n);
+            }
+            if (lane == 0) { sh.chunk_mass[c] = mass; sh.chunk_n[c] = elems; }
+        }
+        __syncthreads();
+        // ---- the chunk, then the bin, in which the running sum from the smallest value passes (1 - p) Z ----
+        static_assert(kNucChunks == 4 * kWave, "four chunks per lane, the lower half of the lanes has the negative values");
+        double four[4];
+        double own = 0.0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) { four[k] = sh.chunk_mass[4 * lane + k]; own += four[k]; }
+        const double upto = wave_scan_double(own);
+        const double small = n_small > 0 ? static_cast<double>(n_small) * static_cast<double>(expf(-m)) : 0.0;  // between the two signs
+        z = lane_double(upto, kWave - 1) + small;
+        cut = static_cast<double>(1.0f - a.top_p) * z;
+        double from = upto - own + (lane >= kWave / 2 ? small : 0.0);
+        const double next = __shfl_down(from, 1, kWave);
+        const double to = lane == kWave / 2 - 1 ? next - small : lane == kWave - 1 ? z : next;  // the next lane starts where this one ends
+        const unsigned long long who = __ballot(own > 0.0 && from <= cut && cut < to);
+        int chunk = -1;
+        if (who) {
+            int k_at = -1;
+            double k_from = 0.0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                // (the last one with mass stays where rounding leaves the sum just short of the cut)
+                if (four[k] > 0.0 && (k_at < 0 || from <= cut)) { k_at = k; k_from = from; }
+                from += four[k];
+            }
+            const int src = __builtin_ctzll(who);
+            chunk = 4 * src + __builtin_amdgcn_readlane(k_at, src);
+            below = lane_double(k_from, src);
+        } else if (!(cut < z) && max_binned) {
+            chunk = ((max_bits & 0x8000u) ? kNucSide - 1 - static_cast<int>(max_mag - kNucLow) : kNucSide + static_cast<int>(max_mag - kNucLow)) / kWave;
+        }
+        if (chunk >= 0) {
+            const int rank = chunk * kWave + lane, n = static_cast<int>(sh.bin[nuc_bin(rank)]);
+            const float e = n ? expf(nuc_value(rank) - m) : 0.f;
+            const double mass = static_cast<double>(n) * static_cast<double>(e), sum = wave_scan_double(mass);
+            unsigned long long with = __ballot(mass > 0.0);
+            const unsigned long long past = who ? __ballot(mass > 0.0 && below + sum > cut) : 0ull;
+            // (none past the cut: rounding again, or nothing at all may fall short of it: the largest value stays)
+            const int at = past ? __builtin_ctzll(past) : with ? 63 - __builtin_clzll(with) : -1;
+            if (at >= 0) {
+                pick = chunk * kWave + at;
+                n_eq = __builtin_amdgcn_readlane(n, at);
+                e_thr = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(e), at));
+                const double eq_mass = static_cast<double>(n_eq) * static_cast<double>(e_thr);
+                below = who ? below + (lane_double(sum, at) - eq_mass) : z - eq_mass;
+                if (a.kept_n) {
+                    above = lane > at ? n : 0;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) above += 4 * lane + k > chunk ? sh.chunk_n[4 * lane + k] : 0;
+                    above = wave_sum_int(above) + (pick < kNucSide ? n_small : 0);
+                }
+            }
+        }
+    }
+    if (pick < 0) {
+        // NaN and +inf make every result NaN, and so does a row of -inf; the wide kernel finishes the other rows, and finds
+        // the row's largest (scaled) logit in thr
+        const float row_max = bf16_bits_to_f32(max_bits);
+        const bool wide = !(odd & kOddNan) && row_max > -INFINITY;
+        if (tid == 0) {
+            const float nan = __builtin_nanf("");
+            a.thr[r] = wide ? row_max : nan;
+            a.tie[r] = wide ? kTieUnresolved : 0;
+            a.lse_kept[r] = nan;
+            if (a.logprob) a.logprob[r] = nan;
+            if (a.lse_full) a.lse_full[r] = (odd & kOddNan) ? nan : -INFINITY;
+            if (a.logprob_full) a.logprob_full[r] = nan;
+            if (a.kept_n) a.kept_n[r] = -1;
+        }
+        return;
+    }
+    const float thr = nuc_value(pick);
+    const double at_or_above = z - below;
+    double drop_d = floor((cut - below) / static_cast<double>(e_thr));
+    drop_d = drop_d < 0.0 ? 0.0 : drop_d > n_eq - 1 ? n_eq - 1 : drop_d;
+    const int drop = static_cast<int>(drop_d);  // elements equal to the threshold that fall: those with the smallest indices
+    const float lse_kept = m + logf(static_cast<float>(at_or_above - drop_d * static_cast<double>(e_thr)));
+    const float lse_full = m + logf(static_cast<float>(z));
+    int tie = 0, n_keep = -1;
+    if (a.kept_n && above + n_eq <= kNucList && above + n_eq - drop <= a.kept_cap) n_keep = above + n_eq - drop;
+    if (n_keep >= 0) {
+        // the kept set and the ties that fall, in descending order of (value, index)
+        __syncthreads();
+        auto push = [&](float x, int64_t index) {
+            if (x < thr) return;
+            const int pos = atomicAdd(&sh.n_list, 1);
+            if (pos < kNucList) sh.list[pos] = (static_cast<unsigned long long>(order_key(x)) << 32) | static_cast<uint32_t>(index);
+        };
+        auto push_vector = [&](const u32x4& q, int vi) {
+            float t[R::EPV];
+            R::decode(q, t);
+            float vm = t[0];
+#pragma unroll
+            for (int k = 1; k < R::EPV; ++k) vm = fmaxf(vm, t[k]);
+            if (vm >= thr) {
+#pragma unroll
+                for (int k = 0; k < R::EPV; ++k) push(t[k], head + static_cast<int64_t>(vi) * R::EPV + k);
+            }
+        };
+        if (thr > 0.f) {
+            // only what the threads read that saw such an element is read again, dealt out over all of them
+            const int bits = static_cast<int>(f32_to_bf16_bits(thr));
+            if (largest.x >= bits || largest.y >= bits) sh.hit[atomicAdd(&sh.n_hit, 1)] = static_cast<uint16_t>(tid);
+            __syncthreads();
+            const int per = (n_vec + kNucThreads - 1) / kNucThreads, n_items = sh.n_hit * per;
+            for (int item = tid; item < n_items; item += 2 * kNucThreads) {
+                int vi[2];
+                u32x4 q[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int it = item + u * kNucThreads, h = it / per;
+                    vi[u] = it < n_items ? sh.hit[h] + (it - h * per) * kNucThreads : n_vec;
+                    if (vi[u] < n_vec) q[u] = xv[vi[u]];
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (vi[u] < n_vec) push_vector(scaled_bits(q[u]), vi[u]);
+            }
+        } else {
+            for_vectors(push_vector);
+        }
+        if (tid < head) push(load_scaled(tid), tid);
+        if (tail0 + tid < vocab) push(load_scaled(tail0 + tid), tail0 + tid);
+        __syncthreads();
+        const int n = sh.n_list < kNucList ? sh.n_list : kNucList;
+        auto record = [&](unsigned long long c, int at) {
+            if (at < n_keep) {
+                a.kept_idx[r * a.kept_cap + at] = static_cast<int32_t>(c & 0xffffffffu);
+                a.kept_x[r * a.kept_cap + at] = key_value(static_cast<uint32_t>(c >> 32));
+            }
+            if (at == n_keep - 1) sh.tie = static_cast<int>(c & 0xffffffffu);
+        };
+        if (n <= kNucThreads) {
+            // an element's place is the number of larger ones (no two are equal): n LDS reads in a row, all lanes the same
+            // word, where a sort takes a barrier or an LDS round trip for each of its steps
+            if (tid < n) {
+                const unsigned long long c = sh.list[tid];
+                int at = 0;
+#pragma unroll 8
+                for (int i = 0; i < n; ++i) at += sh.list[i] > c ? 1 : 0;
+                record(c, at);
+            }
+        } else {
+            int n_pad = 1;
+            while (n_pad < n) n_pad <<= 1;
+            for (int i = n + tid; i < n_pad; i += kNucThreads) sh.list[i] = 0ull;
+            sort_list_desc<kNucThreads>(sh.list, n_pad);
+            for (int q = tid; q < n; q += kNucThreads) record(sh.list[q], q);
+        }
+        __syncthreads();
+        if (drop > 0) tie = sh.tie;
+    } else if (drop > 0) {
+        // the element with `drop` equal ones before it: equal elements are counted per block of indices, from the front of
+        // the row until there are more than that (half of the row on average), then one look at the block that holds it
+        const uint32_t want = static_cast<uint32_t>(drop);
+        __syncthreads();
+        sh.block[tid] = 0u;
+        if (tid < 3) sh.step_n[tid] = 0;
+        __syncthreads();
+        int shift = 0;
+        while ((static_cast<int64_t>(kNucThreads) << shift) < vocab) ++shift;
+        const uint32_t bits = f32_to_bf16_bits(thr), both = bits | (bits << 16);
+        uint32_t seen_n = 0u;
+        // (steps take turns at three counters: the one cleared in a step was last read two barriers ago)
+        for (int base = 0, step = 0; base == 0 || base < n_vec; base += kNucStep, step = step == 2 ? 0 : step + 1) {
+            int mine = 0;
+            auto count = [&](int64_t index) {
+                atomicAdd(&sh.block[index >> shift], 1u);
+                ++mine;
+            };
+            if (base == 0 && tid < head && load_scaled(tid) == thr) count(tid);
+            for_step(base + tid, [&](const u32x4& q, int vi) {
+                uint32_t differ = 0u;  // elements that are not equal, by halves
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t pair = q[w] ^ both;
+                    const u16x2 one = __builtin_elementwise_min(__builtin_bit_cast(u16x2, pair), u16x2{1, 1});
+                    differ += __builtin_bit_cast(uint32_t, one);
+                }
+                if (differ != 0x00040004u) {
+#pragma unroll
+                    for (int k = 0; k < R::EPV; ++k)
+                        if (((q[k >> 1] >> (16 * (k & 1))) & 0xffffu) == bits) count(head + static_cast<int64_t>(vi) * R::EPV + k);
+                }
+            });
+            if (mine) atomicAdd(&sh.step_n[step], static_cast<uint32_t>(mine));
+            if (tid == 0) sh.step_n[step == 2 ? 0 : step + 1] = 0;
+            __syncthreads();
+            seen_n += sh.step_n[step];
+            if (seen_n > want) break;
+        }
+        if (seen_n <= want && tail0 + tid < vocab && load_scaled(tail0 + tid) == thr) atomicAdd(&sh.block[(tail0 + tid) >> shift], 1u);
+        __syncthreads();
+        const uint32_t here = sh.block[tid];
+        uint32_t upto = here;
+#pragma unroll
+        for (int off = 1; off < kWave; off <<= 1) {
+            const uint32_t low = __shfl_up(upto, off, kWave);
+            if (lane >= off) upto += low;
+        }
+        if (lane == kWave - 1) sh.block_w[wave] = upto;
+        __syncthreads();
+        uint32_t before = upto - here;
+        for (int w = 0; w < wave; ++w) before += sh.block_w[w];
+        const bool holder = before <= want && want < before + here;
+        const unsigned long long who = __ballot(holder);
+        if (who) {  // one wave: it walks the block
+            const int src = __builtin_ctzll(who);
+            uint32_t seen = __builtin_amdgcn_readlane(before, src);
+            const int64_t first = static_cast<int64_t>(wave * kWave + src) << shift;
+            int64_t stop = first + (int64_t{1} << shift);
+            stop = stop < vocab ? stop : vocab;
+            for (int64_t j0 = first; j0 < stop && seen <= want; j0 += 4 * kWave) {
+                bool eq[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int64_t j = j0 + u * kWave + lane;
+                    eq[u] = load_scaled(j < stop ? j : stop - 1) == thr && j < stop;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const unsigned long long bal = __ballot(eq[u]);
+                    if (eq[u] && seen + __popcll(bal & ((1ull << lane) - 1ull)) == want) sh.tie = static_cast<int>(j0 + u * kWave + lane);
+                    seen += __popcll(bal);
+                }
+            }
+        }
+        __syncthreads();
+        tie = sh.tie;
+    }
+    if (tid == 0) {
+        if (a.kept_n) a.kept_n[r] = n_keep;
+        a.thr[r] = thr;
+        a.tie[r] = tie;
+        a.lse_kept[r] = lse_kept;
+        if (a.lse_full) a.lse_full[r] = lse_full;
+        if (a.targets && a.logprob) {
+            float lp = -INFINITY, lpf = 0.f;
+            if (tg >= 0 && tg < vocab) {
+                const float xt = scale_logit<NRL_BF16, TEMP>(x_tg, a.tparam);
+                if (xt > thr || (xt == thr && tg >= tie)) lp = xt - lse_kept;
+                lpf = xt - lse_full;
+            }
+            a.logprob[r] = lp;
+            if (a.logprob_full) a.logprob_full[r] = lpf;
         }
     }
 }
@@ -1287,8 +1763,14 @@ extern "C" int nrl_topk_topp_logprob_fwd(const nrl_rows* rows, int64_t top_k, fl
     const bool full = !use_k || logprob_unfiltered_out != nullptr || lse_full_out != nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool small = use_k && a.top_k <= kSmallTopK;
-    if (!use_k) {
-        NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_fwd_kernel<DT, TEMP, true, kCap, true><<<dim3((unsigned)n), dim3(kSelBlock), 0, s>>>(a));
+    if (!use_k && rows->dtype == NRL_BF16) {
+        // (values of fp16 and fp32 are too many for a bin each)
+        if (tc == 0) nucleus_count_kernel<0><<<dim3((unsigned)n), dim3(kNucThreads), 0, s>>>(a);
+        else if (tc == 1) nucleus_count_kernel<1><<<dim3((unsigned)n), dim3(kNucThreads), 0, s>>>(a);
+        else nucleus_count_kernel<2><<<dim3((unsigned)n), dim3(kNucThreads), 0, s>>>(a);
+    } else if (!use_k) {
+        NRL_SEL_DISPATCH(rows->dtype, tc, if constexpr (DT != NRL_BF16)
+                             topk_topp_fwd_kernel<DT, TEMP, true, kCap, true><<<dim3((unsigned)n), dim3(kSelBlock), 0, s>>>(a));
     } else if (full && small) {
         NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_fwd_kernel<DT, TEMP, true, kCapSmall><<<dim3((unsigned)n), dim3(kSelBlock), 0, s>>>(a));
     } else if (full) {

@@ -1,0 +1,141 @@
+"""Top-p alone over bf16 rows (values counted in LDS): thresholds, ties, log-sum-exps and kept-set records against 64-bit sums."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _check(x, top_p, temperature=1.0, div=False, capacity=128):
+    """``x``: bf16 [B, n + 1, V] on the GPU.  Every row's kept set holds top_p of the mass and would not without its lightest
+    element, whose smallest indices fell first (both up to 1e-6: each element's exponential carries a rounding of 2^-24, so
+    do their sums); the log-sum-exps are those of the whole row and of the kept set, to two roundings of fp32."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_DIV, NRL_TEMP_RCP
+
+    b, s, vocab = x.shape
+    n = s - 1
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    t = torch.where(torch.rand(b, n, generator=g, device=DEV) < 0.5, x[:, :n].float().nan_to_num(nan=-1e30).argmax(-1),
+                    torch.randint(0, vocab, (b, n), generator=g, device=DEV))
+    lp, thr, tie, lse, lpu, cnt, idx, val = torch.ops.rl_amd.topk_topp_logprob_fwd_rec(
+        x, t, n, 0, top_p, temperature, NRL_TEMP_DIV if div else NRL_TEMP_RCP, True, capacity)
+    z = x[:, :n].float()
+    if temperature != 1.0:
+        z = (z / torch.tensor(temperature, device=DEV) if div else z * (torch.tensor(1.0) / temperature).to(DEV)).to(torch.bfloat16).float()
+    bad = (z.isnan() | (z == math.inf)).any(-1) | ~z.isfinite().any(-1)
+    assert bool(thr[bad].isnan().all()) and bool(lse[bad].isnan().all()) and bool(lp[bad].isnan().all()) and bool((cnt[bad] == -1).all())
+    assert bool((tie >= 0).all())
+    z64 = z.double()
+    index = torch.arange(vocab, device=DEV)
+    keep = (z > thr[..., None]) | ((z == thr[..., None]) & (index >= tie[..., None]))
+    p = z64.softmax(-1)
+    mass, lightest = (p * keep).sum(-1), p.masked_fill(~keep, 2.0).amin(-1)
+    ok = ~bad
+    cut = 1.0 - float(torch.tensor(1.0) - torch.tensor(top_p))  # 1 - p as fp32 holds it
+    assert bool(keep.any(-1)[ok].all())
+    assert bool((mass >= cut - 1e-6)[ok].all())
+    assert bool(((mass - lightest <= cut + 1e-6) | (keep.sum(-1) == 1))[ok].all())
+    want = z64.masked_fill(~keep, -math.inf).logsumexp(-1)
+    tol = 2.0 ** -23 * (2 + want.abs() + z64.amax(-1).abs())
+    assert bool(((lse.double() - want).abs() <= tol)[ok].all())
+    xt = z64.gather(-1, t[..., None])[..., 0]
+    kept_t = keep.gather(-1, t[..., None])[..., 0]
+    fin = ok & kept_t
+    tol_t = tol + 2.0 ** -23 * xt.abs()
+    assert bool(((lp.double() - (xt - want)).abs() <= tol_t)[fin].all())
+    assert bool((lp == -math.inf)[ok & ~kept_t].all())
+    fin = ok & xt.isfinite()
+    full = z64.logsumexp(-1)
+    tol_f = 2.0 ** -23 * (2 + full.abs() + z64.amax(-1).abs() + xt.abs())   # the same two roundings, of the whole row's sum
+    assert bool(((lpu.double() - (xt - full)).abs() <= tol_f)[fin].all())
+    kept_n = keep.sum(-1)
+    on = cnt >= 0
+    assert torch.equal(cnt[on].long(), kept_n[on])
+    for bi, i in on.nonzero().tolist():
+        c = int(cnt[bi, i])
+        ids = idx[bi, i, :c].long()
+        assert bool(keep[bi, i, ids].all()) and ids.unique().numel() == c
+        v = z[bi, i, ids]
+        assert torch.equal(v, val[bi, i, :c])
+        assert bool(((v[1:] < v[:-1]) | ((v[1:] == v[:-1]) & (ids[1:] < ids[:-1]))).all())   # descending (value, index)
+    return cnt, kept_n
+
+
+@pytest.mark.parametrize("vocab", [1, 7, 64, 1025, 8191, 32775, 151936])
+@pytest.mark.parametrize("top_p", [1e-9, 0.3, 0.95, 0.9999])
+def test_rows_of_every_spread(vocab, top_p):
+    """Standard deviations from nearly flat (thousands of ties at the threshold) to nearly certain, shifted to either side of zero;
+    rows start off the 16-byte grid where the vocabulary is odd."""
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    sd = torch.tensor([0.02, 0.5, 2.0, 3.0, 4.5, 8.0, 1.0, 3.0, 1.0], device=DEV).view(1, -1, 1)
+    shift = torch.tensor([0.0, 0.0, 0.0, 0.0, 0.0, 0.0, -20.0, 40.0, 0.0], device=DEV).view(1, -1, 1)
+    x = (torch.randn(2, 9, vocab, generator=g, device=DEV) * sd + shift).to(torch.bfloat16)
+    cnt, kept_n = _check(x, top_p)
+    assert bool((cnt >= 0)[kept_n <= 4].all())
+
+
+@pytest.mark.parametrize("div", [False, True])
+@pytest.mark.parametrize("temperature", [0.7, 1.3])
+def test_temperatures_and_layouts(temperature, div):
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = (torch.randn(3, 6, 20010, generator=g, device=DEV) * 3).to(torch.bfloat16)
+    _check(x, 0.9, temperature, div)
+    _check(x.transpose(0, 1), 0.9, temperature, div)      # rows of a batch far apart, batches close together
+    _check(x[..., 3:20001], 0.9, temperature, div)        # rows longer apart than they are, off the 16-byte grid
+    _check(x[:, ::2], 0.9, temperature, div)
+
+
+@pytest.mark.parametrize("capacity", [1, 128, 2048])
+def test_records_up_to_their_capacity(capacity):
+    """Kept sets on either side of the capacity, with ties that fall: coarse values (steps of 1/8) tie by the dozen."""
+    g = torch.Generator(device=DEV).manual_seed(capacity)
+    x = torch.randn(1, 33, 4099, generator=g, device=DEV) * torch.linspace(0.5, 6.0, 33, device=DEV).view(1, -1, 1)
+    x = (x * 8).round() / 8 + 0.0   # (no negative zeros: they come before the positive ones in the order of the values)
+    cnt, kept_n = _check(x.to(torch.bfloat16), 0.9, capacity=capacity)
+    n = cnt.shape[1]
+    assert bool((cnt == kept_n)[kept_n <= capacity].all()) and bool((cnt == -1)[kept_n > capacity].all()) and n == 32
+
+
+def test_values_outside_the_bins():
+    """Masked vocabulary (-inf, finfo.min, -1e9), zeros and magnitudes under 2^-31 among ordinary values, a maximum of zero, thresholds
+    among the zeros, values above 2^33, rows of nothing but -inf, NaN and +inf."""
+    g = torch.Generator(device=DEV).manual_seed(11)
+    vocab = 5003
+    x = torch.randn(1, 16, vocab, generator=g, device=DEV) * 3
+    part = torch.rand(1, 16, vocab, generator=g, device=DEV) < 0.4
+    for i, fill in enumerate((-math.inf, -3.3e38, -1e9, 0.0, -0.0, 1e-12, -1e-30)):
+        x[0, i] = x[0, i].masked_fill(part[0, i], fill)
+    x[0, 7] = -x[0, 7].abs() - 1.0
+    x[0, 7, 100:103] = 0.0                     # the maximum is zero, three times
+    x[0, 8] = 0.0                              # the threshold is among the zeros
+    x[0, 9] = x[0, 9] * 1e-12
+    x[0, 10, 17] = 2.0 ** 40                   # above the bins
+    x[0, 11] = -math.inf
+    x[0, 12, 5] = math.nan
+    x[0, 13, 6] = math.inf
+    x[0, 14] = -2.0 ** 40                      # every value below the bins, and one that is not
+    x[0, 14, 9] = -2.0 ** 39
+    _check(x.to(torch.bfloat16), 0.95)
+    y = torch.full((1, 3, vocab), -1.5, device=DEV)
+    y[0, 1] = torch.where(torch.arange(vocab, device=DEV) % 3 == 0, 2.0, -5.0)
+    _check(y.to(torch.bfloat16), 0.75)         # one giant tie; a tie of a third of the row
+
+
+def test_repeats_bit_for_bit():
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = (torch.randn(1, 40, 151936, generator=g, device=DEV) * torch.linspace(1.0, 6.0, 40, device=DEV).view(1, -1, 1)).to(torch.bfloat16)
+    t = torch.randint(0, 151936, (1, 39), generator=g, device=DEV)
+    first = torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, 39, 0, 0.95, 1.0, NRL_TEMP_RCP, True)
+    for _ in range(3):
+        for a, b in zip(first, torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, 39, 0, 0.95, 1.0, NRL_TEMP_RCP, True)):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
