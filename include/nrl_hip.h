@@ -519,7 +519,7 @@ int nrl_seq_logprob_error(const float* prev, int64_t prev_stride, const float* g
  * matmul does.  logprob_out / lse_out: fp32 [N] (lse_out may be NULL).
  * Backward: grad fp32 [N] -> dhidden_out fp32 [N, H] (row stride ld_dh) and dweight_out bf16 [V, H]
  * (row stride ld_dw), accumulated in fp32 and narrowed once.  Tokens are processed in chunks of 16384:
- * per chunk the gradient of the logits exists as bf16 [chunk, V] (twice, one transposed).
+ * per chunk the gradient of the logits exists as bf16 [chunk, V].
  * Kept logits (a choice of the caller, who has the memory or not): with logits_out not NULL the forward
  * also writes the bf16 logits into that buffer (16-byte aligned, nrl_lmhead_kept_logits_bytes(N, V) bytes:
  * 2 bytes per token and id, both rounded up to multiples of 32); handed back as logits_kept the backward reads

@@ -1,12 +1,12 @@
 // K6: fused lm_head -> token logprob (hidden @ W^T, never materialising the full logits) and its
 // backward (dH, dW), on the gfx950 matrix cores.
 //
-// Three bf16 MFMA GEMM cores, C[M,N] = A[M,K] * B[N,K]^T with fp32 accumulation (v_mfma_f32_32x32x16_bf16,
+// Three bf16 MFMA GEMM cores, C[M,N] = A[M,K] * B[N,K]^T (core T: A[K,M]^T) with fp32 accumulation (v_mfma_f32_32x32x16_bf16,
 // 4 wave64, one per SIMD, 256 accumulator registers each), serve every product:
 //   * core B (K a multiple of 64; forward and recomputing gradient): 256 x 256 tile, waves 2 x 2 with 128 x 128
 //     each, both operands double-buffered in LDS by direct global-to-LDS loads;
-//   * core C (K a multiple of 64; the backward's dH and dW products): 256 x 256 tile, waves side by side with
-//     256 x 64 each, operand A through LDS, operand B from a fragment-major copy straight into registers;
+//   * core T (K a multiple of 64; the backward's dH and dW products): 256 x 256 tile, waves side by side with
+//     256 x 64 each, operand A, k across its rows, through LDS, operand B, laid out by fragments, straight into registers;
 //   * core A, the general one (K a multiple of 8): 256 x 128 tile, operands staged through registers
 //     into one padded LDS buffer.
 // Workgroups are numbered so that the 32 that share an XCD (and its L2) cover a 4 x 8 patch of tiles.
@@ -16,14 +16,13 @@
 //          bf16) and folded into a running (max, sum-exp) per token column without any cross-lane
 //          traffic while the workgroup walks its vocabulary tiles; the target's logit is captured on the
 //          way.  Only [tokens] sized partials leave the chip.
-//   GRAD   backward: recomputed tile -> the softmax part -g * exp(x - lse) of the logits' gradient, written as
-//          bf16 row-major (for dH = G W) and, with the one-hot term g at the target added, transposed (for
-//          dW = G^T hidden), for one token chunk at a time.  The one-hot term of dH, g * W[target], is added
-//          in fp32 by its own kernel: it is the one large element of a row of G, and narrowing it to bf16
-//          would put its rounding error (up to 2^-8, coherent over the row) straight into dH.
+//   GRAD   backward: recomputed tile -> the logits' gradient G, g * (onehot - softmax), as bf16 in the layout of core T's
+//          fragments, which dH = G W and dW = G^T hidden both read, for one token chunk at a time.  The element at the
+//          target is the one large element of a row of G: what its rounding to bf16 loses (up to 2^-8 of it, coherent over
+//          the row) is kept in fp32 and added to dH with the target's row of W by its own kernel.
 //   STORE / ACCUM  plain fp32 C = or C += for dH and dW.
 // The vocabulary is walked in tiles while the token chunk bounds what is materialised:
-// chunk x V bf16 for G and G^T (5 GB each at chunk 16384, V 151936) instead of N x V.
+// chunk x V bf16 for G (5 GB at chunk 16384, V 151936) instead of N x V.
 
 #include <float.h>
 #include <stdlib.h>
@@ -40,24 +39,28 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int GB_THREADS = 256;  // 4 wave64, whatever the core
 
 struct GemmOperands {
-    const uint16_t* a;  // [M, K] row stride lda
-    const uint16_t* b;  // [N, K] row stride ldb
-    int64_t lda, ldb, m, n, k;  // k multiple of 8; slabs beyond k read as zero
+    const uint16_t* a;  // [M, K] row stride lda; core T: [K, M], of which the first rows_a rows exist (those past them count
+                        // as the last one, against zeros of b), or G fragment-major (lda: its ids)
+    const uint16_t* b;  // [N, K] row stride ldb; core T: fragment-major, ldb its k extent
+    int64_t lda, ldb = 0, m, n, k;  // k multiple of 8; slabs beyond k read as zero
     // An extent that only the device knows (the number of tokens that carry a gradient): when `live` is set, the
-    // kernel replaces m (live_dim 1) or k (live_dim 2, rounded up to 64) by clamp(live[0] - live_from, 0, that
+    // kernel replaces m (live_dim 1), k (live_dim 2, rounded up to 64) or n (live_dim 3) by clamp(live[0] - live_from, 0, that
     // extent) before it starts, and leaves at once when nothing is left.
     const int32_t* live = nullptr;
     int64_t live_from = 0;
     int live_dim = 0;
+    int64_t rows_a = 0;
 };
 
 // applies the device-side extent; false when the product is empty
 __device__ __forceinline__ bool resolve_live(GemmOperands& op) {
     if (op.live) {
-        int64_t r = static_cast<int64_t>(op.live[0]) - op.live_from;
+        int64_t r = static_cast<int64_t>(__builtin_amdgcn_readfirstlane(op.live[0])) - op.live_from;
         r = r < 0 ? 0 : r;
-        if (op.live_dim == 1) op.m = r < op.m ? r : op.m;
-        else { r = (r + 63) / 64 * 64; op.k = r < op.k ? r : op.k; }
+        const int64_t slabs = (r + 63) / 64 * 64;
+        op.m = op.live_dim == 1 && r < op.m ? r : op.m;
+        op.n = op.live_dim == 3 && r < op.n ? r : op.n;
+        op.k = op.live_dim == 2 && slabs < op.k ? slabs : op.k;
     }
     return op.m > 0 && op.k > 0 && op.n > 0;
 }
@@ -328,36 +331,69 @@ struct CoreB {
 };
 
 // ---------------------------------------------------------------------------------------------
-// Core C: 256 x 256 tile, the four waves side by side along N (wave tile 256 x 64: NI = 8, NJ = 2), K a multiple
-// of 64.  Only operand A goes through LDS (four 32 KiB buffers filled by direct global-to-LDS loads, three slabs
-// ahead); each wave reads its own operand-B fragments straight from memory into registers, one slab ahead.  For
-// that B is stored "fragment-major": the 1 KiB that the 64 lanes of a wave feed to one matrix instruction (32 rows
-// x 16 k) is contiguous, lane by lane, and the blocks of a 32-row group follow each other along k -- a wave's load
-// of a fragment is then one fully used 1 KiB burst.  Per 16-wide k step a wave issues 8 LDS fragment reads for 16
-// MFMAs like core B, but the workgroup writes half as much into LDS and no wave reads B from it.
-//   element (n, k) of B sits at ((n / 32 * K16 + k / 16) * 64 + n % 32 + 32 * (k % 16 / 8)) * 8 + k % 8,
-//   K16 = ldb / 16 (ldb: the allocated k extent, a multiple of 64); row groups are allocated up to a multiple of 256 rows.
+// Core T: the backward's products C[M, N] = A^T B, 256 x 256 tile, the four waves side by side along N (wave tile 256 x 64: NI =
+// 8, NJ = 2), K a multiple of 64.  Both products read the gradient of the logits as the gradient kernels write it, and dH
+// reads W as it lies: no operand is laid out anew but the hidden states (W^T of [151936, 4096] alone took 430 us and 1.2 GB).
+//
+// "Fragment-major" [N, K]: the 1 KiB that the 64 lanes of a wave feed to one matrix instruction (32 rows x 16 k) is a block,
+// lane by lane, and the blocks of a 32-row group follow each other along k:
+//   element (n, k) sits at ((n / 32 * K16 + k / 16) * 64 + n % 32 + 32 * (k % 16 / 8)) * 8 + k % 8
+// with K16 = ldb / 16 (ldb: the allocated k extent, a multiple of 64); row groups are allocated up to a multiple of 256 rows.
+// G (tokens x ids) and the hidden states (h x tokens) lie like that.
+//   * Operand B is fragment-major and goes straight from memory into registers, a fully used 1 KiB burst per fragment, one
+//     slab ahead; no wave reads it from LDS.
+//   * Operand A goes through LDS, four 32 KiB buffers filled by direct global-to-LDS loads, three slabs ahead.  Its k runs
+//     across memory, so its fragments are read by ds_read_b64_tr_b16: each 16 lanes read 4 k x 16 columns and every lane
+//     receives one column of that block, 4 consecutive k; two reads are a lane's 8 k.
+//       dH (GA false): A = W [K, M], a slab is 64 rows of 512 bytes; the 16-byte chunk c of row r sits at c ^ ((r & 3) << 1).
+//       dW (GA true): A = G, K the tokens: a slab is 2 x 16 blocks, each copied as it is but for the order of its 16-byte
+//         units: unit (token t, ids 8 h ..) of the block of ids 16 b .. sits at t ^ 4 h ^ 8 (b & 1) of half h.
+//     Either way the 16 lanes of a read fall on different banks (4.1 cycles per read and wave; 8.1 unswizzled; full rate 4).
+// Bound by the matrix cores under the power limit, for short batches by the stores of dW.  H 4096, V 151936, us for (dH, dW, the
+// gradient and the layout kernels), against products from W^T and G^T laid out in memory (a [M, K] operand A through LDS):
+// 6912 tokens 6615 + 6290 + 830 and 6863 + 6040 + 1985; 2048: 1830 + 2035 + 240 and 1800 + 2098 + 810; 448: 490 + 773 + 65 and 483
+// + 725 + 535; 64: 234 + 435 + 25 and 313 + 456 + 460.  With both operands through LDS by 64-deep slabs in two buffers (core B's
+// scheme) dH of 6912 tokens took 6744, dW 6535, and 7300 and 6800 in a loop with the forward, at a lower clock.
 // ---------------------------------------------------------------------------------------------
-template <int SPREAD> struct CoreCT {
-    static constexpr int BM = 256, BN = 256, NI = 8, NJ = 2, BK = 64, WAVES_N = 4;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ int64_t frag_major(int64_t n, int64_t k, int64_t k16) {  // k a multiple of 8: a 16-byte unit
+    return (((n >> 5) * k16 + (k >> 4)) * 64 + (n & 31) + 32 * ((k >> 3) & 1)) * 8;
+}
+
+template <bool GA> struct CoreT {
+    static constexpr int BM = 256, BN = 256, NI = 8, NJ = 2, BK = 64;
     static constexpr int KS = BK / 16;
     static constexpr int NBUF = 4;
     static constexpr int TILE_BYTES = 256 * BK * 2;
     static constexpr int LDS_BYTES = NBUF * TILE_BYTES;
     static constexpr int ROUNDS = 256 * BK / 8 / GB_THREADS;  // 8 direct loads per lane and slab
 
+    struct SlabA {              // GA false: its first row, and the offset of the last row there is; GA true: its first block
+        const char* p;
+        uint32_t last;
+    };
     struct Ctx {
-        const char* pa;
-        uint32_t voa[ROUNDS];
-        uint32_t aoff[2][KS];   // lane's fragment address for each k step: buffers 0/1 and buffers 2/3 (tile row group 0)
+        uint32_t row_a, chunk_a, step_a;  // GA false: lane's row and chunk in a round of direct loads, bytes; rows of a round apart
+        uint32_t lane_a, block0;          // GA true: lane's unit in a block, bytes; first block of ids (of k16)
+        uint32_t k16_a;
+        uint32_t aaddr[2][2];   // lane's address of a read, buffers 0/1 and 2/3: GA false: even and odd column groups, GA true: low, high k
         uint64_t pb[NJ];        // this wave's two row groups of B at k = 0 (uniform)
         uint32_t vlane;         // lane * 16
         int wave;
     };
 
-    __device__ static __forceinline__ void issue_a(const Ctx& c, unsigned char* lds, int buf, int64_t k0, int j) {
+    __device__ static __forceinline__ void issue_a(const Ctx& c, unsigned char* lds, int buf, const SlabA& s, int j) {
         unsigned char* dst = lds + buf * TILE_BYTES + (j * GB_THREADS + c.wave * 64) * 16;
-        const char* src = c.pa + k0 * 2 + c.voa[j];
+        const char* src;
+        if constexpr (GA) {
+            // block j * 4 + wave of the slab: 16 blocks of ids for each of two groups of tokens; past the last, the last again
+            const uint32_t b = static_cast<uint32_t>((j & 3) * 4 + c.wave) + c.block0;
+            src = s.p + (static_cast<uint64_t>(j >> 2) * c.k16_a + (b < c.k16_a ? b : c.k16_a - 1)) * 1024u + c.lane_a;
+        } else {
+            const uint32_t row = c.row_a + j * c.step_a;
+            src = s.p + ((row < s.last ? row : s.last) + c.chunk_a);
+        }
         __builtin_amdgcn_global_load_lds(reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(src)),
                                          (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
     }
@@ -369,14 +405,35 @@ template <int SPREAD> struct CoreCT {
         asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(v) : "v"(c.vlane), "s"(base), "n"(KSTEP * 1024));
         return v;
     }
-    __device__ static __forceinline__ bf16x8 lds_read16(uint32_t addr, int imm) {
-        bf16x8 v;
-        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(imm));
+    struct FragsA {
+        u32x2 lo[NI], hi[NI];
+        __device__ __forceinline__ bf16x8 get(int f) const {
+            return __builtin_bit_cast(bf16x8, u32x4{lo[f].x, lo[f].y, hi[f].x, hi[f].y});
+        }
+    };
+    __device__ static __forceinline__ u32x2 lds_read_tr(uint32_t addr, int imm) {
+        u32x2 v;
+        asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(imm));
         return v;
     }
-    __device__ static __forceinline__ void wait_a(bf16x8 (&a)[NI]) {
+    // both reads of fragment f of k step ks out of buffer `slot`
+    __device__ static __forceinline__ void read_a(const Ctx& c, FragsA& a, int slot, int ks, int f) {
+        const uint32_t(&at)[2] = c.aaddr[slot >> 1];
+        if constexpr (GA) {
+            const int imm = (slot & 1) * TILE_BYTES + (ks >> 1) * 16 * 1024 + f * 2 * 1024 + (ks & 1) * 256;
+            a.lo[f] = lds_read_tr(at[0], imm);
+            a.hi[f] = lds_read_tr(at[1], imm);
+        } else {
+            const int imm = (slot & 1) * TILE_BYTES + ks * 16 * 512 + (f >> 1) * 128;
+            a.lo[f] = lds_read_tr(at[f & 1], imm);
+            a.hi[f] = lds_read_tr(at[f & 1], imm + 4 * 512);
+        }
+    }
+    // every LDS read issued so far has returned; the operands tie the wait to the fragments it guards
+    __device__ static __forceinline__ void wait_a(FragsA& a) {
         asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]));
+                     : "+v"(a.lo[0]), "+v"(a.lo[1]), "+v"(a.lo[2]), "+v"(a.lo[3]), "+v"(a.lo[4]), "+v"(a.lo[5]), "+v"(a.lo[6]), "+v"(a.lo[7]));
+        asm volatile("" : "+v"(a.hi[0]), "+v"(a.hi[1]), "+v"(a.hi[2]), "+v"(a.hi[3]), "+v"(a.hi[4]), "+v"(a.hi[5]), "+v"(a.hi[6]), "+v"(a.hi[7]));
     }
     template <int N> __device__ static __forceinline__ void wait_b(bf16x8 (&b)[KS][NJ]) {
         asm volatile("s_waitcnt vmcnt(%8)"
@@ -396,7 +453,7 @@ template <int SPREAD> struct CoreCT {
     }
 
     // One slab out of LDS buffer SLOT; its B fragments are in register set SLOT & 1 of a ring of 2 KS k steps.  On
-    // entry the A fragments of k step 0 are in flight into af[0].  Every k step issues four vector-memory operations,
+    // entry the A fragments of k step 0 are in af[0].  Every k step issues four vector-memory operations,
     // behind its first MFMAs: the two B fragments of the k step LEAD steps ahead (into the registers that the k
     // step before this one has just finished with), then two of the eight direct loads of the slab three ahead
     // (into the buffer that the previous slab's barrier freed).  Memory operations complete in order, so at the
@@ -405,15 +462,11 @@ template <int SPREAD> struct CoreCT {
     // issued two slabs ago or, for a tile's second slab, up to 20 operations before this point, hence vmcnt(20),
     // and the barrier frees SLOT for the slab four ahead.
     template <int SLOT>
-    __device__ static __forceinline__ void compute(const Ctx& c, unsigned char* lds, f32x16 (&acc)[NI][NJ], bf16x8 (&af)[2][NI],
-                                                   bf16x8 (&bfr)[2][KS][NJ], int64_t k_b1, int64_t k_b2, int64_t k_a) {
+    __device__ static __forceinline__ void compute(const Ctx& c, unsigned char* lds, f32x16 (&acc)[NI][NJ], FragsA (&af)[2],
+                                                   bf16x8 (&bfr)[2][KS][NJ], int64_t k_b1, int64_t k_b2, const SlabA& s_a) {
         constexpr int SET = SLOT & 1, NEXT = (SLOT + 1) % NBUF;
-        auto frag_a = [&](int slot, int ks, int set, int f) {
-            af[set][f] = lds_read16(c.aoff[slot >> 1][ks], (slot & 1) * TILE_BYTES + f * 32 * BK * 2);
-        };
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
-            wait_a(af[ks & 1]);
             if (ks == KS - 1) {
                 wait_b<20>(bfr[SET]);
                 asm volatile("s_barrier" ::: "memory");
@@ -426,24 +479,28 @@ template <int SPREAD> struct CoreCT {
                 for (int j = 0; j < NJ; ++j) {
                     const int idx = i * NJ + j;
                     __builtin_amdgcn_sched_barrier(0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1][i], bfr[SET][ks][j], acc[i][j], 0, 0, 0);
-                    if (idx == 0 || idx == SPREAD) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks & 1].get(i), bfr[SET][ks][j], acc[i][j], 0, 0, 0);
+                    if (idx == 0 || idx == 2) {
                         __builtin_amdgcn_sched_barrier(0);
                         // k step ks + LEAD: ks == 0 -> next slab's last k step, otherwise the slab after it
-                        if (ks == 0) fetch_b(c, bfr, SET ^ 1, KS - 1, k_b1, idx / SPREAD);
-                        else fetch_b(c, bfr, SET, ks - 1, k_b2, idx / SPREAD);
+                        if (ks == 0) fetch_b(c, bfr, SET ^ 1, KS - 1, k_b1, idx / 2);
+                        else fetch_b(c, bfr, SET, ks - 1, k_b2, idx / 2);
                     }
-                    if (idx == 2 * SPREAD || idx == 3 * SPREAD) {
+                    if (idx == 4 || idx == 6) {
                         __builtin_amdgcn_sched_barrier(0);
-                        issue_a(c, lds, (SLOT + 3) % NBUF, k_a, ks * 2 + idx / SPREAD - 2);
+                        issue_a(c, lds, (SLOT + 3) % NBUF, s_a, ks * 2 + idx / 2 - 2);
                     }
                     if (idx < NI) {
                         __builtin_amdgcn_sched_barrier(0);
-                        if (ks + 1 < KS) frag_a(SLOT, ks + 1, (ks + 1) & 1, idx);
-                        else frag_a(NEXT, 0, 0, idx);
+                        if (ks + 1 < KS) read_a(c, af[(ks + 1) & 1], SLOT, ks + 1, idx);
+                        else read_a(c, af[0], NEXT, 0, idx);
                     }
                 }
             }
+            // (at the end of the k step, not at the start of the next one: no register whose read is under way may be live
+            // where the slab loop turns, or the compiler could move it there)
+            __builtin_amdgcn_sched_barrier(0);
+            wait_a(af[(ks + 1) & 1]);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -456,65 +513,82 @@ template <int SPREAD> struct CoreCT {
         Ctx c;
         c.wave = wave;
         c.vlane = static_cast<uint32_t>(lane * 16);
-        c.pa = reinterpret_cast<const char*>(op.a + row0 * op.lda);
         const int64_t k16 = op.ldb / 16;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
             c.pb[j] = reinterpret_cast<uint64_t>(op.b) + static_cast<uint64_t>(((col0 >> 5) + wave * NJ + j) * k16) * 1024u;
-        const int lr = tid >> 3, cg = (tid & 7) ^ ((lr >> 1) & 7);
-        const int last_a = static_cast<int>(op.m - 1 - row0 < 255 ? op.m - 1 - row0 : 255);
-#pragma unroll
-        for (int j = 0; j < ROUNDS; ++j) {
-            const int r = j * 32 + lr;
-            c.voa[j] = static_cast<uint32_t>((r < last_a ? r : last_a) * op.lda + cg * 8) * 2u;
-        }
-        const int fr = lane & 31, fh = lane >> 5;
+        const char* pa;
         const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
+        const int g = lane >> 4, i4 = (lane & 15) >> 2, i = lane & 3;  // a read's block of 16 columns (g & 1) and 8 k (g >> 1), k and piece in it
+        if constexpr (GA) {
+            pa = reinterpret_cast<const char*>(op.a);
+            c.k16_a = static_cast<uint32_t>(op.lda / 16);
+            c.block0 = static_cast<uint32_t>(row0 / 16);
+            c.lane_a = static_cast<uint32_t>(lane ^ ((lane >> 5) << 2) ^ ((wave & 1) << 3)) * 16u;
+            const uint32_t unit = static_cast<uint32_t>(((g >> 1) * 8 + i4) ^ ((i >> 1) << 2) ^ ((g & 1) << 3));
+            c.aaddr[0][0] = lds_base + static_cast<uint32_t>((g & 1) * 1024 + (i >> 1) * 512 + (i & 1) * 8) + unit * 16u;
+            c.aaddr[0][1] = lds_base + static_cast<uint32_t>((g & 1) * 1024 + (i >> 1) * 512 + (i & 1) * 8) + (unit ^ 4u) * 16u;
+        } else {
+            // 8 rows a round, 32 chunks a row, chunks past the operand's end clamped
+            pa = reinterpret_cast<const char*>(op.a + row0);
+            const int chunk = (tid & 31) ^ (((tid >> 5) & 3) << 1);
+            const int64_t left = op.m - row0;
+            const int last = static_cast<int>(left < 256 ? (left + 7) / 8 : 32) - 1;
+            c.row_a = static_cast<uint32_t>(tid >> 5) * static_cast<uint32_t>(op.lda) * 2u;
+            c.chunk_a = static_cast<uint32_t>(chunk < last ? chunk : last) * 16u;
+            c.step_a = static_cast<uint32_t>(op.lda) * 16u;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const uint32_t sw = static_cast<uint32_t>(((ks * 2 + fh) ^ ((fr >> 1) & 7)) * 16);
-            c.aoff[0][ks] = lds_base + static_cast<uint32_t>(fr * BK * 2) + sw;
-            c.aoff[1][ks] = c.aoff[0][ks] + 2 * TILE_BYTES;
+            for (int odd = 0; odd < 2; ++odd)
+                c.aaddr[0][odd] = lds_base + static_cast<uint32_t>(((g >> 1) * 8 + i4) * 512 + (i & 1) * 8) +
+                                  static_cast<uint32_t>(((4 * odd + (g & 1) * 2 + (i >> 1)) ^ (i4 << 1)) * 16);
         }
-        const int64_t nk = op.k / BK;
-        const int64_t k_last = (nk - 1) * BK;
-        auto slab_k = [&](int64_t kt) { return kt < nk ? kt * BK : k_last; };
-        bf16x8 af[2][NI], bfr[2][KS][NJ];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) c.aaddr[1][q] = c.aaddr[0][q] + 2 * TILE_BYTES;
+        const int nk = __builtin_amdgcn_readfirstlane(static_cast<int>(op.k / BK));
+        auto slab_k = [&](int kt) { return static_cast<int64_t>(kt < nk ? kt : nk - 1) * BK; };  // past the end: the last slab again, unused
+        auto slab_a = [&](int kt) {
+            const int64_t k0 = slab_k(kt);
+            if constexpr (GA) return SlabA{pa + (k0 >> 5) * static_cast<int64_t>(c.k16_a) * 1024, 0u};
+            else return SlabA{pa + k0 * op.lda * 2, op.rows_a - k0 < BK ? static_cast<uint32_t>((op.rows_a - k0 - 1) * op.lda * 2) : 0xffffffffu};
+        };
+        FragsA af[2];
+        bf16x8 bfr[2][KS][NJ];
         // order: the B fragments of the first LEAD k steps, then slabs 0, 1, 2 of A (the waits count on it)
 #pragma unroll
-        for (int g = 0; g < LEAD; ++g)
+        for (int q = 0; q < LEAD; ++q)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) fetch_b(c, bfr, g / KS, g % KS, g < KS ? 0 : slab_k(1), j);
+            for (int j = 0; j < NJ; ++j) fetch_b(c, bfr, q / KS, q % KS, q < KS ? 0 : slab_k(1), j);
         __builtin_amdgcn_sched_barrier(0);
+        {
+            const SlabA s0 = slab_a(0), s1 = slab_a(1), s2 = slab_a(2);
 #pragma unroll
-        for (int j = 0; j < ROUNDS; ++j) issue_a(c, lds, 0, 0, j);
+            for (int j = 0; j < ROUNDS; ++j) issue_a(c, lds, 0, s0, j);
 #pragma unroll
-        for (int j = 0; j < ROUNDS; ++j) issue_a(c, lds, 1, slab_k(1), j);
+            for (int j = 0; j < ROUNDS; ++j) issue_a(c, lds, 1, s1, j);
 #pragma unroll
-        for (int j = 0; j < ROUNDS; ++j) issue_a(c, lds, 2, slab_k(2), j);
+            for (int j = 0; j < ROUNDS; ++j) issue_a(c, lds, 2, s2, j);
+        }
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * ROUNDS) : "memory");  // slab 0 of A has landed everywhere
 #pragma unroll
-        for (int f = 0; f < NI; ++f) af[0][f] = lds_read16(c.aoff[0][0], f * 32 * BK * 2);
-        int64_t kt = 0;
+        for (int f = 0; f < NI; ++f) read_a(c, af[0], 0, 0, f);
+        wait_a(af[0]);
+        int kt = 0;
         for (; kt + 3 < nk; kt += 4) {
-            compute<0>(c, lds, acc, af, bfr, slab_k(kt + 1), slab_k(kt + 2), slab_k(kt + 3));
-            compute<1>(c, lds, acc, af, bfr, slab_k(kt + 2), slab_k(kt + 3), slab_k(kt + 4));
-            compute<2>(c, lds, acc, af, bfr, slab_k(kt + 3), slab_k(kt + 4), slab_k(kt + 5));
-            compute<3>(c, lds, acc, af, bfr, slab_k(kt + 4), slab_k(kt + 5), slab_k(kt + 6));
+            compute<0>(c, lds, acc, af, bfr, slab_k(kt + 1), slab_k(kt + 2), slab_a(kt + 3));
+            compute<1>(c, lds, acc, af, bfr, slab_k(kt + 2), slab_k(kt + 3), slab_a(kt + 4));
+            compute<2>(c, lds, acc, af, bfr, slab_k(kt + 3), slab_k(kt + 4), slab_a(kt + 5));
+            compute<3>(c, lds, acc, af, bfr, slab_k(kt + 4), slab_k(kt + 5), slab_a(kt + 6));
         }
-        if (kt < nk) compute<0>(c, lds, acc, af, bfr, slab_k(kt + 1), slab_k(kt + 2), slab_k(kt + 3));
-        if (kt + 1 < nk) compute<1>(c, lds, acc, af, bfr, slab_k(kt + 2), slab_k(kt + 3), slab_k(kt + 4));
-        if (kt + 2 < nk) compute<2>(c, lds, acc, af, bfr, slab_k(kt + 3), slab_k(kt + 4), slab_k(kt + 5));
+        if (kt < nk) compute<0>(c, lds, acc, af, bfr, slab_k(kt + 1), slab_k(kt + 2), slab_a(kt + 3));
+        if (kt + 1 < nk) compute<1>(c, lds, acc, af, bfr, slab_k(kt + 2), slab_k(kt + 3), slab_a(kt + 4));
+        if (kt + 2 < nk) compute<2>(c, lds, acc, af, bfr, slab_k(kt + 3), slab_k(kt + 4), slab_a(kt + 5));
         // what the last slabs fetched ahead is never used, but its registers and buffers must stay untouched until it
         // has arrived
-        wait_a(af[0]);
         wait_b<0>(bfr[0]);
         wait_b<0>(bfr[1]);
         asm volatile("s_barrier" ::: "memory");
     }
 };
-
-using CoreC = CoreCT<2>;
 
 template <class Core> __device__ __forceinline__ void zero_acc(f32x16 (&acc)[Core::NI][Core::NJ]) {
 #pragma unroll
@@ -568,6 +642,36 @@ __device__ __forceinline__ bool patch_tile(const Patches& p, uint32_t w, int64_t
     by = __builtin_amdgcn_readfirstlane(static_cast<int>(iy * p.py + (t - tx * p.py)));
     split = __builtin_amdgcn_readfirstlane(static_cast<int>(sp));
     return tx < p.px && split < p.splits && bx < nbx && by < nby;
+}
+
+// How a product of the backward covers its tiles.  The tiles (of every k range, one range after the other) are numbered along
+// strips px wide, row by row within a strip, and every XCD takes an eighth of the numbers in a row: the 32 tiles that its
+// compute units hold at a time are px x 32 / px, which share their panels through its L2, every compute unit has a tile until
+// the last few, and no workgroup is launched for a place without one.  (Fixed patches of 4 x 8 slots did that: a grid of 16 x 1
+// tiles filled every eighth slot of a patch, and as consecutive workgroups go to the shader engines in turn, the work of an XCD
+// went to 8 of its 32 compute units: dH of 64 tokens, H 4096, V 151936 750 us, 448 tokens 860; 1371 x 2624 x 258550, 6 x 11
+// tiles in 3 ranges, put 44 tiles on one XCD and 22 on others.)
+struct Strips {
+    uint32_t px = 4;
+    int splits = 1;
+    __host__ __device__ uint32_t units(int64_t nbx, int64_t nby) const { return static_cast<uint32_t>(nbx * nby * splits); }
+    uint32_t grid(int64_t nbx, int64_t nby) const { return (units(nbx, nby) + 7) / 8 * 8; }
+    double rounds(int64_t nbx, int64_t nby) const { return static_cast<double>(((units(nbx, nby) + 7) / 8 + 31) / 32); }
+};
+
+// Tile coordinates (and k range) of workgroup w; false for the few past the last tile.
+__device__ __forceinline__ bool strip_tile(const Strips& p, uint32_t w, int64_t nbx, int64_t nby, int64_t& bx, int64_t& by, int& split) {
+    const uint32_t nx = static_cast<uint32_t>(nbx), ny = static_cast<uint32_t>(nby), all = p.units(nbx, nby), per = (all + 7) / 8;
+    const uint32_t unit = (w & 7) * per + (w >> 3);
+    const uint32_t sp = unit / (nx * ny), u = unit - sp * nx * ny;
+    const uint32_t strip = u / (p.px * ny), in = u - strip * p.px * ny;
+    const uint32_t left = nx - strip * p.px, width = left < p.px ? left : p.px;
+    const uint32_t row = in / width;
+    // the divisions run on the vector unit; hand the (uniform) results back to scalar registers
+    bx = __builtin_amdgcn_readfirstlane(static_cast<int>(strip * p.px + (in - row * width)));
+    by = __builtin_amdgcn_readfirstlane(static_cast<int>(row));
+    split = __builtin_amdgcn_readfirstlane(static_cast<int>(sp));
+    return (w >> 3) < per && unit < all;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -823,11 +927,19 @@ struct LmGradArgs {
     int64_t vocab_start;
     const float* lse;        // [chunk]
     const float* grad;       // [chunk] upstream d loss / d logprob
-    uint16_t* g;             // [chunk_pad, ldg] row-major, columns >= V zero
+    uint16_t* g;             // fragment-major (tokens, ids), ids V .. ldg - 1 zero
     int64_t ldg;
-    uint16_t* gt;            // [V, ldgt] transposed, columns >= chunk zero
-    int64_t ldgt;
+    float* resid;            // [chunk] what the rounding of the one-hot element to bf16 lost (written where the target is here)
 };
+
+// The element of G at the target: g + the softmax part, rounded to bf16 like every other; what that rounding loses (up to
+// 2^-8 of g, which would be the largest error of the whole row) goes to `resid` and into dH with the fp32 weight row.
+__device__ __forceinline__ uint32_t one_hot_element(float g, uint32_t softmax_bits, float& resid) {
+    const float whole = g + bf16_bits_to_f32(softmax_bits);
+    const uint32_t bits = f32_to_bf16_bits(whole);
+    resid = whole - bf16_bits_to_f32(bits);
+    return bits;
+}
 
 // XCD patch of the recomputing gradient kernel, 8 token tiles x 4 vocabulary tiles: 1.7 % faster than 4 x 8
 constexpr Patches kGradPatches{8, 4, 1};
@@ -861,29 +973,25 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
     zero_acc<Core>(acc);
     Core::tile(a.op, row0, col0, acc, lds);
     const int64_t m_pad = ((a.op.m + 63) / 64) * 64;
-    // gradient of the lane's 4 consecutive tokens (accumulator rows) of tile (i, j), group q, as two bf16 pairs:
-    // s01 / s23 the softmax part alone (for G), p01 / p23 with the one-hot term (for G^T)
-    auto grad4 = [&](int i, int j, int q, uint32_t& p01, uint32_t& p23, uint32_t& s01, uint32_t& s23) {
+    // gradient of the lane's 4 consecutive tokens (accumulator rows) of tile (i, j), group q, as two bf16 pairs
+    auto grad4 = [&](int i, int j, int q, uint32_t& p01, uint32_t& p23) {
         const int64_t c = col0 + wn * (NJ * 32) + j * 32 + (lane & 31);
         const bool col_ok = c < a.op.n;
-        float gv[4], sv[4];
+        uint32_t bits[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int e = q * 4 + u;
             const int rl = wm * 128 + i * 32 + acc_row(e, lane);
             const bool row_ok = row0 + rl < a.op.m;
-            gv[u] = sv[u] = 0.f;
+            bits[u] = 0u;
             if (row_ok && col_ok && g_l[rl] != 0.f) {
                 const float x = round_bf16(acc[i][j][e]);
-                const float p = fast_exp2(__builtin_fmaf(x, kLog2e, -lse_l[rl]));
-                sv[u] = -p * g_l[rl];
-                gv[u] = tgt_local[rl] == c ? g_l[rl] + round_bf16(sv[u]) : sv[u];
+                bits[u] = f32_to_bf16_bits(-fast_exp2(__builtin_fmaf(x, kLog2e, -lse_l[rl])) * g_l[rl]);
+                if (tgt_local[rl] == c) bits[u] = one_hot_element(g_l[rl], bits[u], a.resid[row0 + rl]);
             }
         }
-        p01 = pack_bf16x2(gv[0], gv[1]);
-        p23 = pack_bf16x2(gv[2], gv[3]);
-        s01 = pack_bf16x2(sv[0], sv[1]);
-        s23 = pack_bf16x2(sv[2], sv[3]);
+        p01 = bits[0] | (bits[1] << 16);
+        p23 = bits[2] | (bits[3] << 16);
     };
     // The softmax part of the whole tile's gradients as bf16 pairs.  A group of 4 accumulator rows is the same for
     // every j, so its per-token values are read from LDS once; columns past the vocabulary become zero by a select.
@@ -916,43 +1024,12 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
         }
     };
     if constexpr (Core::LDS_BYTES >= BM * BN * 2) {
-        // Both layouts leave through LDS so that every global store is a 16-byte piece of a 512-byte run.
+        // G leaves through LDS so that every global store is a 16-byte piece of a 512-byte run: 2-byte writes; the 16-byte
+        // chunk C of token row t sits at C ^ ((t >> 2) & 7).
         static_assert(BM == GB_THREADS, "one thread per token row patches the one-hot term");
-        // Pass 1, [vocab][token]: a lane's 4 tokens are one 8-byte unit; unit U of row v sits at U ^ (v & 63).
-        // Pass 2, [token][vocab]: 2-byte writes; the 16-byte chunk C of row t sits at C ^ ((t >> 2) & 7).
         constexpr int RV = BN / 8;  // 16-byte pieces per token row of the tile
         uint32_t p01[NI][NJ][4], p23[NI][NJ][4];
         grad_all(p01, p23);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int v = wn * (NJ * 32) + j * 32 + (lane & 31);
-#pragma unroll
-            for (int i = 0; i < NI; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int t0 = wm * 128 + i * 32 + acc_row(q * 4, lane);
-                    const int unit = (t0 >> 2) ^ (v & 63);
-                    *reinterpret_cast<uint2*>(lds + v * (BM * 2) + unit * 8) = uint2{p01[i][j][q], p23[i][j][q]};
-                }
-        }
-        __syncthreads();
-        {   // the one-hot term of G^T: token `tid` adds its g at its target's row, if that row is in this tile
-            const int v = tgt_local[tid] - static_cast<int>(col0);
-            if (tgt_local[tid] >= 0 && v >= 0 && v < BN) {
-                uint16_t* cell = reinterpret_cast<uint16_t*>(lds + v * (BM * 2) + (((tid >> 2) ^ (v & 63)) * 8) + (tid & 3) * 2);
-                *cell = static_cast<uint16_t>(f32_to_bf16_bits(g_l[tid] + bf16_bits_to_f32(*cell)));
-            }
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int it = 0; it < BN * 32 / GB_THREADS; ++it) {
-            const int idx = it * GB_THREADS + tid, v = idx >> 5, m = idx & 31;
-            const uint2 lo = *reinterpret_cast<const uint2*>(lds + v * (BM * 2) + (((2 * m) ^ (v & 63)) * 8));
-            const uint2 hi = *reinterpret_cast<const uint2*>(lds + v * (BM * 2) + (((2 * m + 1) ^ (v & 63)) * 8));
-            const int64_t c = col0 + v, r = row0 + 8 * m;
-            if (c < a.op.n && r < a.ldgt) *reinterpret_cast<u32x4*>(a.gt + c * a.ldgt + r) = u32x4{lo.x, lo.y, hi.x, hi.y};
-        }
-        __syncthreads();
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int v = wn * (NJ * 32) + j * 32 + (lane & 31);
@@ -972,37 +1049,39 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
                 }
         }
         __syncthreads();
+        {   // the one-hot term: token `tid` adds its g at its target's column, if that column is in this tile
+            const int v = tgt_local[tid] - static_cast<int>(col0);
+            if (tgt_local[tid] >= 0 && v >= 0 && v < BN) {
+                uint16_t* cell = reinterpret_cast<uint16_t*>(lds + tid * (BN * 2) + (((v >> 3) ^ ((tid >> 2) & 7)) * 16) + (v & 7) * 2);
+                *cell = static_cast<uint16_t>(one_hot_element(g_l[tid], *cell, a.resid[row0 + tid]));
+            }
+        }
+        __syncthreads();
 #pragma unroll 4
         for (int it = 0; it < BM * RV / GB_THREADS; ++it) {
-            const int idx = it * GB_THREADS + tid, t = idx / RV, m = idx % RV;
+            // 32 tokens of one chunk are 512 bytes of G
+            const int idx = it * GB_THREADS + tid, t = (idx & 31) + 32 * (idx / (32 * RV)), m = (idx >> 5) % RV;
             const u32x4 x = *reinterpret_cast<const u32x4*>(lds + t * (BN * 2) + ((m ^ ((t >> 2) & 7)) * 16));
             const int64_t r = row0 + t, c = col0 + 8 * m;
-            if (r < m_pad && c < a.ldg) *reinterpret_cast<u32x4*>(a.g + r * a.ldg + c) = x;
+            if (r < m_pad && c < a.ldg) *reinterpret_cast<u32x4*>(a.g + frag_major(r, c, a.ldg / 16)) = x;
         }
     } else {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int64_t c = col0 + wn * (NJ * 32) + j * 32 + (lane & 31);
-            const bool col_ok = c < a.op.n;
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {  // four groups of four consecutive rows
-                    uint32_t p01, p23, s01, s23;
-                    grad4(i, j, q, p01, p23, s01, s23);
+                    uint32_t p01, p23;
+                    grad4(i, j, q, p01, p23);
                     const int64_t r_first = row0 + wm * 128 + i * 32 + acc_row(q * 4, lane);
                     if (c < a.ldg) {
-                        uint16_t* gp = a.g + r_first * a.ldg + c;
-                        if (r_first + 0 < m_pad) gp[0] = static_cast<uint16_t>(s01);
-                        if (r_first + 1 < m_pad) gp[a.ldg] = static_cast<uint16_t>(s01 >> 16);
-                        if (r_first + 2 < m_pad) gp[2 * a.ldg] = static_cast<uint16_t>(s23);
-                        if (r_first + 3 < m_pad) gp[3 * a.ldg] = static_cast<uint16_t>(s23 >> 16);
-                    }
-                    if (col_ok && r_first < a.ldgt) {
-                        uint2 v;
-                        v.x = p01;
-                        v.y = p23;
-                        *reinterpret_cast<uint2*>(a.gt + c * a.ldgt + r_first) = v;
+                        uint16_t* gp = a.g + frag_major(r_first, c, a.ldg / 16) + (c & 7);  // (four tokens of one group)
+                        if (r_first + 0 < m_pad) gp[0] = static_cast<uint16_t>(p01);
+                        if (r_first + 1 < m_pad) gp[8] = static_cast<uint16_t>(p01 >> 16);
+                        if (r_first + 2 < m_pad) gp[16] = static_cast<uint16_t>(p23);
+                        if (r_first + 3 < m_pad) gp[24] = static_cast<uint16_t>(p23 >> 16);
                     }
                 }
             }
@@ -1011,13 +1090,11 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// backward from kept logits: the same G and G^T without the product.  One workgroup turns a tile of 128 tokens x
-// 128 vocabulary ids: a thread reads 16 bytes of 4 consecutive live tokens (two runs of 4 ids, 8 ids apart: what a
-// lane of the forward held; the neighbouring thread holds the runs in between, and the two swap a run each so that
-// both end up with 8 consecutive ids), writes its part of G
-// straight back (16 bytes of a 256-byte run), and hands the 4 tokens' values of each id to LDS as one 8-byte unit
-// of the transposed tile (unit U of row v at U ^ swizzle(v)), from where G^T leaves in 16-byte pieces after the
-// one-hot term was added to the tokens' target cells.
+// backward from kept logits: the same G without the product.  A wave owns 32 live tokens, one per lane of either half, and
+// walks blocks of 16 ids: the lane reads the 16 bytes that a lane of the forward held (ids 4 h .. and 8 + 4 h .. of the block,
+// h its half), swaps a run of 4 ids with its partner in the other half so that both hold 8 consecutive ids, and the wave
+// writes the block of G as it lies, 1 KiB.  Bound by HBM (read + write): 6912 tokens, V 151936: 800 us, 5.3 TB/s (by tiles of 128
+// tokens x 128 ids with G^T written too, through LDS: 1520).
 // ---------------------------------------------------------------------------------------------
 struct LmGradKeptArgs {
     const unsigned char* logits;  // bf16 logits as the forward left them (kept_block)
@@ -1032,131 +1109,90 @@ struct LmGradKeptArgs {
     const float* grad;
     uint16_t* g;              // as in LmGradArgs
     int64_t ldg;
-    uint16_t* gt;
-    int64_t ldgt;
+    float* resid;
 };
 
-constexpr int KT = 128;  // tile side of lmhead_grad_kept_kernel
+constexpr int kKeptBlocks = 16;  // blocks of 16 ids that a wave of lmhead_grad_kept_kernel walks
+constexpr int kKeptInFlight = 4;
 
 __global__ __launch_bounds__(256) void lmhead_grad_kept_kernel(LmGradKeptArgs a) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[KT * KT * 2];
-    __shared__ int tgt_l[KT];
-    __shared__ float lse_l[KT], g_l[KT];
-    __shared__ int64_t row_l[KT];
-    const int tid = threadIdx.x;
+    const int lane = threadIdx.x & 63, half = lane >> 5;
     int64_t m = static_cast<int64_t>(a.live[0]) - a.live_from;
     m = m < 0 ? 0 : (m > a.rows ? a.rows : m);
-    const int64_t row0 = static_cast<int64_t>(blockIdx.y) * KT, col0 = static_cast<int64_t>(blockIdx.x) * KT;
-    if (row0 >= m) return;
-    const int64_t m_pad = (m + 63) / 64 * 64;
-    if (tid < KT) {
-        const int64_t r = row0 + tid;
-        int64_t t = -1, src = 0;
-        float l = 128.f, g = 0.f;  // rows past the live ones: a finite exponent and a zero gradient
-        if (r < m) { t = a.targets[r] - a.vocab_start; l = a.lse[r]; g = a.grad[r]; src = a.row_map[r]; }
-        tgt_l[tid] = (t >= 0 && t < a.vocab && g != 0.f) ? static_cast<int>(t) : -1;
-        lse_l[tid] = l * kLog2e;
-        g_l[tid] = g;
-        row_l[tid] = src;
+    const int64_t row = static_cast<int64_t>(blockIdx.y) * 32 + (lane & 31), m_pad = (m + 63) / 64 * 64;
+    if (static_cast<int64_t>(blockIdx.y) * 32 >= m_pad) return;
+    int64_t src = 0;
+    int tgt = -1;
+    float ls = 128.f * kLog2e, g = 0.f;  // rows past the live ones: a finite exponent and a zero gradient
+    if (row < m) {
+        const int64_t t = a.targets[row] - a.vocab_start;
+        ls = a.lse[row] * kLog2e;
+        g = a.grad[row];
+        src = a.row_map[row];
+        tgt = (t >= 0 && t < a.vocab && g != 0.f) ? static_cast<int>(t) : -1;
     }
-    __syncthreads();
-    auto swz = [](int v) { return (v ^ (v >> 5)) & 31; };
+    const bool live = g != 0.f;
+    const unsigned char* from = a.logits + kept_block(src >> 5, 0, a.n_vb) + half * 512 + (src & 31) * 16;
+    const int64_t blocks = a.ldg / 16;
+    uint16_t* to = a.g + frag_major(row, 8 * half, blocks);
+    const int64_t b0 = (static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6)) * kKeptBlocks;
+#pragma unroll 1
+    for (int64_t b = b0; b < b0 + kKeptBlocks && b < blocks; b += kKeptInFlight) {
+        u32x4 raw[kKeptInFlight];
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-        const int item = pass * 256 + tid, piece = item & 15, t4 = item >> 4;  // 8 ids x 4 tokens
-        const int64_t c = col0 + piece * 8;
-        uint32_t w[4][4];  // [token][pair of ids]
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int t = t4 * 4 + u;
-            float sv[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) sv[k] = 0.f;
-            // (the swap below runs in every lane: whether a token is live is the same for both partners, whether the
-            // ids exist is not)
-            u32x4 raw = u32x4{0u, 0u, 0u, 0u};
-            const bool live = row0 + t < m && g_l[t] != 0.f;
-            if (live && (c & ~15) < a.vocab) {
-                // piece = 4 * (block of the tile) + 2 * (half p) + h
-                const int64_t src = row_l[t];
-                raw = *reinterpret_cast<const u32x4*>(a.logits + kept_block(src >> 5, (col0 >> 5) + (piece >> 2), a.n_vb) +
-                                                     ((piece >> 1) & 1) * 1024 + ((piece & 1) * 32 + (src & 31)) * 16);
-            }
-            {
-                // this lane (h) holds the ids 16 p + 4 h + {0..3} and + 8 + {0..3}; the lane with the other h sits next
-                // to it.  h = 0 keeps its first run and takes the partner's first run, h = 1 takes the partner's
-                // second run and keeps its own second: 8 consecutive ids, the ids c .. c + 7 of the tile.
-                const bool hi = piece & 1;
-                const uint32_t give0 = hi ? raw.x : raw.z, give1 = hi ? raw.y : raw.w;
-                const uint32_t got0 = __shfl_xor(give0, 1, kWave), got1 = __shfl_xor(give1, 1, kWave);
-                raw = hi ? u32x4{got0, got1, raw.z, raw.w} : u32x4{raw.x, raw.y, got0, got1};
-            }
-            if (live && c < a.vocab) {
-                float x[8];
-                Row<NRL_BF16>::decode(raw, x);
-                const float ng = -g_l[t], ls = lse_l[t];
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    sv[k] = c + k < a.vocab ? fast_exp2(__builtin_fmaf(x[k], kLog2e, -ls)) * ng : 0.f;
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) w[u][q] = pack_bf16x2(sv[2 * q], sv[2 * q + 1]);
-            if (row0 + t < m_pad && c < a.ldg)
-                *reinterpret_cast<u32x4*>(a.g + (row0 + t) * a.ldg + c) = u32x4{w[u][0], w[u][1], w[u][2], w[u][3]};
+        for (int u = 0; u < kKeptInFlight; ++u) {
+            raw[u] = u32x4{0u, 0u, 0u, 0u};
+            if (live && (b + u) * 16 < a.vocab) raw[u] = *reinterpret_cast<const u32x4*>(from + (b + u) * 1024);
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int v = piece * 8 + k, q = k >> 1;
-            uint2 unit;
-            if (k & 1) {
-                unit.x = (w[0][q] >> 16) | (w[1][q] & 0xffff0000u);
-                unit.y = (w[2][q] >> 16) | (w[3][q] & 0xffff0000u);
-            } else {
-                unit.x = (w[0][q] & 0xffffu) | (w[1][q] << 16);
-                unit.y = (w[2][q] & 0xffffu) | (w[3][q] << 16);
-            }
-            *reinterpret_cast<uint2*>(lds + v * (KT * 2) + ((t4 ^ swz(v)) * 8)) = unit;
-        }
-    }
-    __syncthreads();
-    if (tid < KT) {  // the one-hot term of G^T: token `tid` adds its g at its target's row, if that row is in this tile
-        const int v = tgt_l[tid] - static_cast<int>(col0);
-        if (tgt_l[tid] >= 0 && v >= 0 && v < KT) {
-            uint16_t* cell = reinterpret_cast<uint16_t*>(lds + v * (KT * 2) + (((tid >> 2) ^ swz(v)) * 8) + (tid & 3) * 2);
-            *cell = static_cast<uint16_t>(f32_to_bf16_bits(g_l[tid] + bf16_bits_to_f32(*cell)));
-        }
-    }
-    __syncthreads();
+        for (int u = 0; u < kKeptInFlight; ++u) {
+            if (b + u >= blocks) break;
+            // half 0 keeps its first run and takes the partner's first, half 1 takes the partner's second and keeps its own
+            const uint32_t give0 = half ? raw[u].x : raw[u].z, give1 = half ? raw[u].y : raw[u].w;
+            const uint32_t got0 = __shfl_xor(give0, 32, kWave), got1 = __shfl_xor(give1, 32, kWave);
+            const u32x4 bits = half ? u32x4{got0, got1, raw[u].z, raw[u].w} : u32x4{raw[u].x, raw[u].y, got0, got1};
+            const int64_t c = (b + u) * 16 + 8 * half;  // this lane's 8 ids
+            float x[8], sv[8];
+            Row<NRL_BF16>::decode(bits, x);
 #pragma unroll
-    for (int it = 0; it < KT * 16 / 256; ++it) {
-        const int item = it * 256 + tid, v = item >> 4, mq = item & 15;
-        const uint2 lo = *reinterpret_cast<const uint2*>(lds + v * (KT * 2) + (((2 * mq) ^ swz(v)) * 8));
-        const uint2 hi = *reinterpret_cast<const uint2*>(lds + v * (KT * 2) + (((2 * mq + 1) ^ swz(v)) * 8));
-        const int64_t c = col0 + v, r = row0 + 8 * mq;
-        if (c < a.vocab && r < a.ldgt) *reinterpret_cast<u32x4*>(a.gt + c * a.ldgt + r) = u32x4{lo.x, lo.y, hi.x, hi.y};
+            for (int k = 0; k < 8; ++k) sv[k] = live && c + k < a.vocab ? fast_exp2(__builtin_fmaf(x[k], kLog2e, -ls)) * -g : 0.f;
+            u32x4 out;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out[q] = pack_bf16x2(sv[2 * q], sv[2 * q + 1]);
+            const int at = tgt < 0 ? -1 : tgt - static_cast<int>(c);
+            if (at >= 0 && at < 8) {  // the token's target is among these ids (one lane of the whole launch)
+                const int q = at >> 1, up = (at & 1) * 16;
+                uint32_t pair = q == 0 ? out.x : q == 1 ? out.y : q == 2 ? out.z : out.w;
+                const uint32_t one = one_hot_element(g, (pair >> up) & 0xffffu, a.resid[row]);
+                pair = (pair & (0xffff0000u >> up)) | (one << up);
+                if (q == 0) out.x = pair;
+                if (q == 1) out.y = pair;
+                if (q == 2) out.z = pair;
+                if (q == 3) out.w = pair;
+            }
+            *reinterpret_cast<u32x4*>(to + (b + u) * 512) = out;
+        }
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// plain GEMM with fp32 accumulation: C = A B^T or C += A B^T.  MODE bit 0 (ACCUM): the product is added to what c
-// holds; bit 1 (NARROW): the result goes to cb, bf16 with c's row stride, instead of to c.  The two are not
-// combined: with the prior values in flight next to the narrowing stores the compiler spills accumulators inside the
-// K loop.  A product whose k extent turns out empty on the device still delivers zeros without ACCUM; with ACCUM there
-// is nothing to do.
-// Splits: with patches.splits > 1 workgroup and split compute a k range of their own and store the partial product at
+// The backward's products on core T, fp32: C = A^T B (GA: dW, rows m of c) or its transpose (dH: column n of the product is
+// row row_map[n] of c, if there is a row_map).  MODE bit 0 (ACCUM): the product is added to what c holds; bit 1 (NARROW): the
+// result goes to cb, bf16 with c's row stride, instead of to c.  The two are not combined.  A product whose k extent turns
+// out empty on the device still delivers zeros without ACCUM; with ACCUM there is nothing to do.
+// Splits: with strips.splits > 1 workgroup and split compute a k range of their own and store the partial product at
 // c + split * split_stride (MODE 0); the reduction kernels below add the partials in order.  A split whose range turns
 // out empty stores zeros.
 // ---------------------------------------------------------------------------------------------
 constexpr int GEMM_ACCUM = 1, GEMM_NARROW = 2;
-template <class Core, int MODE>
-__global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, Patches patches, float* c, int64_t ldc,
+template <bool GA, int MODE>
+__global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, Strips strips, float* c, int64_t ldc,
                                                               const int32_t* row_map, uint16_t* cb, int64_t split_stride) {
     constexpr bool ACCUM = (MODE & GEMM_ACCUM) != 0, NARROW = (MODE & GEMM_NARROW) != 0;
     static_assert(!(ACCUM && NARROW), "accumulate in fp32, narrow in a pass of its own");
+    using Core = CoreT<GA>;
     constexpr int NI = Core::NI, NJ = Core::NJ, BM = Core::BM, BN = Core::BN;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[Core::LDS_BYTES];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave / Core::WAVES_N, wn = wave % Core::WAVES_N;
     bool runs = resolve_live(op);
     if (!runs) {
         // only an empty k extent leaves anything to write, and only where the output is not simply kept as it is
@@ -1164,12 +1200,14 @@ __global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, P
     }
     int64_t bx, by;
     int split;
-    // (the accumulating product is never split and always takes 4 x 8 patches: with more live across its K loop it spills)
-    if (!patch_tile(ACCUM ? Patches{} : patches, blockIdx.x, (op.m + BM - 1) / BM, (op.n + BN - 1) / BN, bx, by, split)) return;
-    if (!ACCUM && patches.splits > 1) {
-        const int64_t per = ((op.k + patches.splits - 1) / patches.splits + 63) / 64 * 64, k0 = per * split;
-        op.a += k0;
-        op.b += k0 / 16 * 512;  // operand B is fragment-major: 16 k of a 32-row group are one block of 512 elements
+    if (!strip_tile(strips, blockIdx.x, (op.m + BM - 1) / BM, (op.n + BN - 1) / BN, bx, by, split)) return;
+    if (!ACCUM && strips.splits > 1) {
+        // (as in patch_tile: the result of the division goes back to a scalar register, and with it all that follows)
+        const int64_t per = __builtin_amdgcn_readfirstlane(static_cast<int>(((op.k + strips.splits - 1) / strips.splits + 63) / 64 * 64));
+        const int64_t k0 = per * split;
+        op.a += k0 * op.lda;  // (fragment-major, k a multiple of 32: the groups of 32 tokens are 32 lda apart)
+        op.b += k0 * 32;      // 16 k of a 32-row group are one block of 512 elements
+        op.rows_a -= k0;
         op.k = op.k - k0 < per ? op.k - k0 : per;
         runs = runs && op.k > 0;
         c += split * split_stride;
@@ -1180,86 +1218,93 @@ __global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, P
     if (runs) Core::tile(op, row0, col0, acc, lds);
     // (the write-back reads the accumulators with instructions the compiler does not look into: the wait a matrix
     // instruction's result needs before another unit reads it is spelled out)
-    asm volatile("s_nop 15\n s_nop 7" ::: "memory");
-    if (row_map) {
-        // rows of the product are scattered: row r of C goes to row row_map[r] of the output (plain store only)
+    int tid = threadIdx.x;
+    asm volatile("s_nop 15\n s_nop 7" : "+v"(tid)::"memory");
+    const int lane = tid & 63, wn = tid >> 6;
+    const int64_t m0 = row0 + 4 * (lane >> 5);               // element e of block i is row m0 + 32 i + 8 (e / 4) + e % 4
+    const int64_t n0 = col0 + wn * (NJ * 32) + (lane & 31);  // and of block j column n0 + 32 j
+    if constexpr (GA) {
+        // (a wave's store is two runs of 32 columns; four rows of 8 bytes a lane, as below, are 9 us slower a tile)
+        const bool interior = row0 + BM <= op.m && col0 + BN <= op.n;
+        auto write_back = [&](auto interior_tag) {
+            constexpr bool INTERIOR = decltype(interior_tag)::value;
+            // Half of the tile's 16 blocks at a time: with an accumulating epilogue all 128 loads of a half go out before
+            // the first is used, so a tile pays two memory latencies, not one per block.
+            constexpr int HI = NI / 2;
 #pragma unroll
-        for (int i = 0; i < NI; ++i)
+            for (int i0 = 0; i0 < NI; i0 += HI) {
+                float prior[HI][NJ][16];
+                if (ACCUM) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int64_t r = row0 + wm * (NI * 32) + i * 32 + acc_row(e, lane);
-                if (r >= op.m) continue;
-                float* out = c + static_cast<int64_t>(row_map[r]) * ldc;
+                    for (int i = i0; i < i0 + HI; ++i)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    const int64_t col = col0 + wn * (NJ * 32) + j * 32 + (lane & 31);
-                    if (col < op.n) out[col] = acc[i][j][e];
+                        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                            for (int e = 0; e < 16; ++e) {
+                                const int64_t r = m0 + i * 32 + 8 * (e >> 2) + (e & 3), n = n0 + j * 32;
+                                if (INTERIOR || (r < op.m && n < op.n)) prior[i - i0][j][e] = c[r * ldc + n];
+                            }
                 }
-            }
-        return;
-    }
-    // an interior tile takes the path without per-element bounds (no divergent branch between the loads)
-    const bool interior = row0 + BM <= op.m && col0 + BN <= op.n;
-    auto write_back = [&](auto interior_tag) {
-        constexpr bool INTERIOR = decltype(interior_tag)::value;
-        // Half of the tile's 16 blocks at a time: with an accumulating epilogue all 128 loads of a half go out before
-        // the first is used, so a tile pays two memory latencies, not one per block.  The accumulators are read one
-        // by one where they are used (plain uses would have the compiler copy them all to vector registers, which
-        // are taken by the loaded values).
-        constexpr int HI = NI / 2 > 0 ? NI / 2 : 1;
-#pragma unroll
-        for (int i0 = 0; i0 < NI; i0 += HI) {
-            float prior[HI][NJ][16];
-            if (ACCUM) {
 #pragma unroll
                 for (int i = i0; i < i0 + HI; ++i)
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
-                        const int64_t col = col0 + wn * (NJ * 32) + j * 32 + (lane & 31);
-                        const float* base = c + (row0 + wm * (NI * 32) + i * 32) * ldc + col;
+                        float* base = c + (m0 + i * 32) * ldc + n0 + j * 32;
+                        uint16_t* base_b = cb + (m0 + i * 32) * ldc + n0 + j * 32;
 #pragma unroll
                         for (int e = 0; e < 16; ++e) {
-                            const int r = acc_row(e, lane);
-                            prior[i - i0][j][e] =
-                                (INTERIOR || (row0 + wm * (NI * 32) + i * 32 + r < op.m && col < op.n)) ? base[r * ldc] : 0.f;
+                            const int r = 8 * (e >> 2) + (e & 3);
+                            const float v = acc_read(acc[i][j][e]);
+                            if (INTERIOR || (m0 + i * 32 + r < op.m && n0 + j * 32 < op.n)) {
+                                if (NARROW) base_b[r * ldc] = static_cast<uint16_t>(f32_to_bf16_bits(v));
+                                else base[r * ldc] = ACCUM ? prior[i - i0][j][e] + v : v;
+                            }
                         }
                     }
             }
+        };
+        if (interior) write_back(std::true_type{});
+        else write_back(std::false_type{});
+    } else {
+        static_assert(GA || MODE == 0, "the transposed product is stored as it is");
+        // four values leave together where the rows of c are aligned for that (m is a multiple of 8)
+        const bool quads = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(c) & 15) == 0;
 #pragma unroll
-            for (int i = i0; i < i0 + HI; ++i)
+        for (int j = 0; j < NJ; ++j) {
+            const int64_t n = n0 + j * 32;
+            if (n >= op.n) continue;
+            float* out = c + (row_map ? static_cast<int64_t>(row_map[n]) : n) * ldc + m0;
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    const int64_t col = col0 + wn * (NJ * 32) + j * 32 + (lane & 31);
-                    // (cb has c's row stride: one set of offsets serves the prior values and the narrowed result)
-                    float* base = c + (row0 + wm * (NI * 32) + i * 32) * ldc + col;
-                    uint16_t* base_b = cb + (row0 + wm * (NI * 32) + i * 32) * ldc + col;
+            for (int i = 0; i < NI; ++i)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        const int r = acc_row(e, lane);
-                        const float v = acc_read(acc[i][j][e]);
-                        if (INTERIOR || (row0 + wm * (NI * 32) + i * 32 + r < op.m && col < op.n)) {
-                            if (NARROW) base_b[r * ldc] = static_cast<uint16_t>(f32_to_bf16_bits(ACCUM ? prior[i - i0][j][e] + v : v));
-                            else base[r * ldc] = ACCUM ? prior[i - i0][j][e] + v : v;
-                        }
+                for (int q = 0; q < 4; ++q) {
+                    const int off = i * 32 + 8 * q;
+                    if (m0 + off >= op.m) continue;
+                    float v[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) v[u] = acc_read(acc[i][j][4 * q + u]);
+                    if (quads) {
+                        *reinterpret_cast<float4*>(out + off) = float4{v[0], v[1], v[2], v[3]};
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) out[off + u] = v[u];
                     }
                 }
         }
-    };
-    if (interior) write_back(std::true_type{});
-    else write_back(std::false_type{});
+    }
 }
 
 // dH of a chunk's live tokens: the partial products of its k splits added in order (SUM; otherwise the product is
-// already in place), plus the one-hot term g_r * W[target_r, :] in fp32, which is kept out of the bf16 product.  Row r is
-// token row_map[r]; a target outside the shard adds nothing.  One workgroup per row.
+// already in place), plus resid_r * W[target_r, :] in fp32: what the rounding of the one-hot element of G to bf16 lost (zero
+// where the target lies outside the shard).  Row r is token row_map[r].  One workgroup per row.
 template <bool SUM>
 __global__ __launch_bounds__(256) void lmhead_finish_dh_kernel(float* dh, int64_t ld_dh, const float* parts, int n_splits,
                                                               int64_t split_stride, const int32_t* row_map, const int32_t* live,
-                                                              int64_t live_from, const float* grad, const int64_t* targets,
+                                                              int64_t live_from, const float* resid, const int64_t* targets,
                                                               int64_t vocab_start, int64_t vocab, const uint16_t* w, int64_t ldw, int64_t h) {
     const int64_t r = blockIdx.x;
     if (r >= static_cast<int64_t>(live[0]) - live_from) return;
-    const float g = grad[r];
+    const float g = resid[r];
     const int64_t t = targets[r] - vocab_start;
     const bool hot = g != 0.f && t >= 0 && t < vocab;
     if (!SUM && !hot) return;
@@ -1331,7 +1376,7 @@ __global__ __launch_bounds__(1024) void live_tokens_kernel(const float* grad, in
 __global__ __launch_bounds__(256) void gather_live_kernel(const uint16_t* hidden, int64_t ldh, int64_t h, const int64_t* targets,
                                                          const float* lse, const float* grad, const int32_t* idx,
                                                          const int32_t* count, int64_t n, uint16_t* hidden_c, int64_t* targets_c,
-                                                         float* lse_c, float* grad_c) {
+                                                         float* lse_c, float* grad_c, float* resid_c) {
     const int64_t i = blockIdx.x;
     const bool live = i < count[0];
     const int64_t src = live ? idx[i] : 0;
@@ -1343,15 +1388,16 @@ __global__ __launch_bounds__(256) void gather_live_kernel(const uint16_t* hidden
         targets_c[i] = live ? targets[src] : 0;
         lse_c[i] = live ? lse[src] : 0.f;
         grad_c[i] = live ? grad[src] : 0.f;
+        resid_c[i] = 0.f;
     }
 }
 
-// B[n, k] = src[k, n] in core C's fragment-major layout (k extent ldk, a multiple of 64): k < rows and n < cols are
+// B[n, k] = src[k, n] in the fragment-major layout (k extent ldk, a multiple of 64): k < rows and n < cols are
 // copied, everything else up to pad_k and up to the launch's n tiles is zero.  cols and the source's row stride are
 // multiples of 8.  One wave per tile of 64 k x 64 n, four of them side by side along n in a workgroup: a lane loads 16
 // bytes of 8 rows (8 lanes share a 128-byte line), turns its 8 x 8 block in registers, and the wave's 16-byte units
-// leave through LDS so that every store is 1 KiB contiguous.  Bound by HBM (read + write); W [151936, 4096]: 430 us,
-// 5.8 TB/s (element by element through a 64 x 64 LDS tile: 900 us).
+// leave through LDS so that every store is 1 KiB contiguous.  Bound by HBM (read + write); hidden states of 8192
+// tokens, H 4096: 24 us.
 __global__ __launch_bounds__(256) void transpose_to_frag_kernel(const uint16_t* src, int64_t rows, int64_t cols, int64_t lds_,
                                                                uint16_t* dst, int64_t ldk, int64_t pad_k) {
     __shared__ __attribute__((aligned(16))) u32x4 units[4][512];
@@ -1463,18 +1509,21 @@ template <class Core> static FwdPlan fwd_plan(int64_t n, int64_t v, bool save) {
 // whose partial products are added afterwards.  Costs in microseconds: a 256 x 256 x 64 slab takes 1.4, a tile about 5
 // more for its start and write-back, and the partials are written and read at about 4 TB/s.  dH of 512 tokens (32 tiles,
 // V 151936 along k): 2519 us unsplit, 470 in 8 ranges.  `room`: floats available for partial products.
-static Patches gemm_plan(int64_t m, int64_t n, int64_t k, int64_t room) {
-    const int64_t nbx = (m + CoreC::BM - 1) / CoreC::BM, nby = (n + CoreC::BN - 1) / CoreC::BN, slabs = (k + 63) / 64;
-    Patches best;
+static Strips gemm_plan(int64_t m, int64_t n, int64_t k, int64_t room) {
+    const int64_t nbx = (m + CoreT<true>::BM - 1) / CoreT<true>::BM, nby = (n + CoreT<true>::BN - 1) / CoreT<true>::BN, slabs = (k + 63) / 64;
+    Strips best;
+    double fewest = 1e300;  // operand panels that the 32 tiles of an XCD read, per tile
+    for (uint32_t px = 1; px <= 32; px *= 2) {
+        const double x = static_cast<double>(px < nbx ? px : nbx), y = static_cast<double>(32 / px < nby ? 32 / px : nby);
+        if ((x + y) / (x * y) < fewest) { fewest = (x + y) / (x * y); best.px = px; }
+    }
     double best_cost = 1e300;
-    for (int splits = 1; splits <= 16 && (splits == 1 || (splits * m * n <= room && slabs >= 8 * splits)); ++splits)
-        for (uint32_t px = 1; px <= 8; px *= 2) {
-            const Patches p{px, 32 / px, splits};
-            double cost = p.rounds(nbx, nby) * (1.4 * static_cast<double>((slabs + splits - 1) / splits) + 5.0);
-            cost *= 1.0 + 0.002 * (px + 32.0 / px - 12.0);
-            if (splits > 1) cost += 8.0 + static_cast<double>(splits) * m * n * 8 / 4e6;
-            if (cost < best_cost) { best_cost = cost; best = p; }
-        }
+    for (int splits = 1; splits <= 16 && (splits == 1 || (splits * m * n <= room && slabs >= 8 * splits)); ++splits) {
+        const Strips p{best.px, splits};
+        double cost = p.rounds(nbx, nby) * (1.4 * static_cast<double>((slabs + splits - 1) / splits) + 5.0);
+        if (splits > 1) cost += 8.0 + static_cast<double>(splits) * m * n * 8 / 4e6;
+        if (cost < best_cost) { best_cost = cost; best.splits = splits; }
+    }
     return best;
 }
 
@@ -1548,11 +1597,12 @@ template <class Core> static void launch_grad(const LmGradArgs& a, hipStream_t s
                                dim3(GB_THREADS), 0, s>>>(a);
 }
 
-// C = or += A B^T with B in core C's fragment-major layout (op.ldb: its k extent); op.k a multiple of 64
-template <int MODE> static void launch_gemm(const GemmOperands& op, const Patches& p, float* c, int64_t ldc, hipStream_t s,
-                                            const int32_t* row_map = nullptr, uint16_t* cb = nullptr) {
-    gemm_f32_kernel<CoreC, MODE><<<dim3((unsigned)p.grid((op.m + CoreC::BM - 1) / CoreC::BM, (op.n + CoreC::BN - 1) / CoreC::BN)),
-                                   dim3(GB_THREADS), 0, s>>>(op, p, c, ldc, row_map, cb, op.m * ldc);
+// C = or += (A^T B)^T on core T (see gemm_f32_kernel); op.k a multiple of 64
+template <bool GA, int MODE> static void launch_gemm(const GemmOperands& op, const Strips& p, float* c, int64_t ldc, hipStream_t s,
+                                                     const int32_t* row_map = nullptr, uint16_t* cb = nullptr) {
+    using Core = CoreT<GA>;
+    gemm_f32_kernel<GA, MODE><<<dim3(p.grid((op.m + Core::BM - 1) / Core::BM, (op.n + Core::BN - 1) / Core::BN)),
+                                      dim3(GB_THREADS), 0, s>>>(op, p, c, ldc, row_map, cb, (GA ? op.m : op.n) * ldc);
 }
 
 extern "C" int64_t nrl_lmhead_kept_logits_bytes(int64_t n_tokens, int64_t vocab) {
@@ -1590,14 +1640,13 @@ extern "C" int nrl_lmhead_logprob_fwd(const void* hidden, int64_t n_tokens, int6
 // tokens per backward chunk: long enough that the dW product (K = chunk) amortises its fp32 read-modify-write
 static constexpr int64_t kBwdChunk = 16384;
 static int64_t bwd_chunk(int64_t n) { return n < kBwdChunk ? round_up(n < 1 ? 1 : n, 64) : kBwdChunk; }
-// Row stride (elements) of the two operands of the dW product, whose rows hold a chunk's tokens: one 128-byte line
-// more than the chunk, because rows a power of two apart (16384 tokens = 32 KiB) fall on the same memory channels
-// (measured on the dW product: 1.6 % faster than unpadded; two lines more is 5 % slower, three as good as one).
+// k extent of hidden^T: one 128-byte line more than the chunk, because row groups a power of two apart (16384 tokens = 1 MiB)
+// fall on the same memory channels (the dW product 1.6 % faster than unpadded).
 static int64_t bwd_ld_t(int64_t chunk) { return chunk + 64; }
 // dH of a chunk of `rows` tokens, with room for partial products of up to 32768 rows in all (0.5 GB at H 4096)
-static Patches dh_plan(int64_t rows, int64_t h, int64_t vp) { return gemm_plan(rows, h, vp, 32768 * h); }
+static Strips dh_plan(int64_t rows, int64_t h, int64_t vp) { return gemm_plan(h, rows, vp, 32768 * h); }
 // dW of a batch that is one chunk, with room for partial products of up to 1 GiB
-static Patches dw_plan(int64_t vocab, int64_t h, int64_t rows) { return gemm_plan(vocab, h, rows, (1ll << 30) / 4); }
+static Strips dw_plan(int64_t vocab, int64_t h, int64_t rows) { return gemm_plan(vocab, h, rows, (1ll << 30) / 4); }
 static int64_t dh_parts_bytes(int64_t rows, int64_t h, int64_t vp) {
     const int splits = rows > 0 ? dh_plan(rows, h, vp).splits : 1;
     return splits > 1 ? splits * rows * h * 4 : 0;
@@ -1607,17 +1656,15 @@ extern "C" int64_t nrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t hidd
     const int64_t n = n_tokens < 1 ? 1 : n_tokens;
     const int64_t chunk = bwd_chunk(n_tokens), vp = round_up(vocab, 64), n_pad = round_up(n, chunk);
     int64_t b = 0;
-    b += round_up(hidden_size, 256) * vp * 2;        // W^T, fragment-major
-    b += chunk * vp * 2;              // G
-    b += vocab * bwd_ld_t(chunk) * 2;        // G^T
-    b += round_up(hidden_size, 256) * bwd_ld_t(chunk) * 2;  // hidden chunk^T, fragment-major
+    b += round_up(chunk, 256) * vp * 2;                    // G, fragment-major
+    b += round_up(hidden_size, 256) * bwd_ld_t(chunk) * 2; // hidden chunk^T, fragment-major
     // dW: the fp32 accumulator of the chunks, or the partial products of a single chunk
     b += vocab * hidden_size * 4 * (n <= chunk ? dw_plan(vocab, hidden_size, round_up(n, 64)).splits : 1);
     // partial products of dH, of a whole chunk or of the last, shorter one
     const int64_t whole = n >= chunk ? dh_parts_bytes(chunk, hidden_size, vp) : 0, rest = dh_parts_bytes(n % chunk, hidden_size, vp);
     b += whole > rest ? whole : rest;
     b += n_pad * hidden_size * 2;     // hidden rows of the tokens that carry a gradient
-    b += n_pad * (8 + 4 + 4 + 4);     // their targets, log-sum-exps, gradients and token indices
+    b += n_pad * (8 + 4 + 4 + 4 + 4); // their targets, log-sum-exps, gradients, one-hot roundings and token indices
     return b + 4096;
 }
 
@@ -1642,15 +1689,12 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     const int64_t n_pad = round_up(n_tokens < 1 ? 1 : n_tokens, chunk);
     char* ws = static_cast<char*>(workspace);
     auto take = [&](int64_t bytes) { char* p = ws; ws += (bytes + 255) / 256 * 256; return p; };
+    uint16_t* g = reinterpret_cast<uint16_t*>(take(round_up(chunk, 256) * vp * 2));
     const int64_t h_pad = round_up(h, 256);
-    uint16_t* wt = reinterpret_cast<uint16_t*>(take(h_pad * vp * 2));
-    uint16_t* g = reinterpret_cast<uint16_t*>(take(chunk * vp * 2));
-    const int64_t ld_t = bwd_ld_t(chunk);
-    uint16_t* gt = reinterpret_cast<uint16_t*>(take(vocab * ld_t * 2));
-    uint16_t* ht = reinterpret_cast<uint16_t*>(take(h_pad * ld_t * 2));
+    uint16_t* ht = reinterpret_cast<uint16_t*>(take(h_pad * bwd_ld_t(chunk) * 2));
     const bool one_chunk = n_tokens <= chunk;
-    const Patches dw_patches = dw_plan(vocab, h, round_up(n_tokens < 1 ? 1 : n_tokens, 64));
-    float* dw = reinterpret_cast<float*>(take(vocab * h * 4 * (one_chunk ? dw_patches.splits : 1)));
+    const Strips dw_strips = dw_plan(vocab, h, round_up(n_tokens < 1 ? 1 : n_tokens, 64));
+    float* dw = reinterpret_cast<float*>(take(vocab * h * 4 * (one_chunk ? dw_strips.splits : 1)));
     float* dh_parts;
     {
         const int64_t n = n_tokens < 1 ? 1 : n_tokens;
@@ -1661,13 +1705,12 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     int64_t* tgt_c = reinterpret_cast<int64_t*>(take(n_pad * 8));
     float* lse_c = reinterpret_cast<float*>(take(n_pad * 4));
     float* grad_c = reinterpret_cast<float*>(take(n_pad * 4));
+    float* resid_c = reinterpret_cast<float*>(take(n_pad * 4));
     int32_t* idx = reinterpret_cast<int32_t*>(take(n_pad * 4 + 256));
     int32_t* count = idx + n_pad;
     const uint16_t* hid = static_cast<const uint16_t*>(hidden);
     const uint16_t* w = static_cast<const uint16_t*>(weight);
 
-    // W^T [H, vp] (zero-padded, fragment-major: operand B of the dH product)
-    transpose_to_frag_kernel<<<dim3((unsigned)(h_pad / 256), (unsigned)(vp / 64)), dim3(256), 0, s>>>(w, vocab, h, ldw, wt, vp, vp);
     if (n_tokens == 0) {
         // no token: dW is zero (rows of h bf16 = h / 2 words, row stride ld_dw / 2 words: both are multiples of 8)
         for (int64_t r = 0; r < vocab; r += 65535)
@@ -1679,7 +1722,7 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
         // device; the launches are sized for all tokens and the workgroups beyond the live ones leave at once.
         live_tokens_kernel<<<dim3(1), dim3(1024), 0, s>>>(grad, n_tokens, idx, count);
         gather_live_kernel<<<dim3((unsigned)n_pad), dim3(256), 0, s>>>(hid, ldh, h, targets, lse, grad, idx, count, n_tokens, hid_c, tgt_c,
-                                                                        lse_c, grad_c);
+                                                                        lse_c, grad_c, resid_c);
         for (int64_t r = 0; r < n_tokens; r += 65535)  // dH rows of the other tokens are zero
             fill_zero_rows_kernel<<<dim3((unsigned)(n_tokens - r < 65535 ? n_tokens - r : 65535)), dim3(256), 0, s>>>(
                 dhidden_out + r * ld_dh, ld_dh, h);
@@ -1692,47 +1735,47 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     for (int64_t t0 = 0; t0 < n_tokens; t0 += chunk) {
         const int64_t rows = n_tokens - t0 < chunk ? n_tokens - t0 : chunk;   // upper bound: the live rows of this chunk
         const int64_t rows_pad = round_up(rows, 64);
-        // G / G^T for this chunk of live tokens
+        // G for this chunk of live tokens
         LmGradArgs ga;
         ga.op.a = hid_c + t0 * h; ga.op.b = w; ga.op.lda = h; ga.op.ldb = ldw; ga.op.m = rows; ga.op.n = vocab; ga.op.k = h;
         ga.op.live = count; ga.op.live_from = t0; ga.op.live_dim = 1;
         ga.targets = tgt_c + t0; ga.vocab_start = vocab_start; ga.lse = lse_c + t0; ga.grad = grad_c + t0;
-        ga.g = g; ga.ldg = vp; ga.gt = gt; ga.ldgt = ld_t;
+        ga.g = g; ga.ldg = vp; ga.resid = resid_c + t0;
         if (logits_kept) {
             LmGradKeptArgs ka;
             ka.logits = static_cast<const unsigned char*>(logits_kept); ka.n_vb = (vocab + 31) / 32; ka.row_map = idx + t0; ka.live = count;
             ka.live_from = t0; ka.rows = rows; ka.vocab = vocab; ka.targets = ga.targets; ka.vocab_start = vocab_start;
-            ka.lse = ga.lse; ka.grad = ga.grad; ka.g = g; ka.ldg = vp; ka.gt = gt; ka.ldgt = ld_t;
-            lmhead_grad_kept_kernel<<<dim3((unsigned)((vp + KT - 1) / KT), (unsigned)((rows + KT - 1) / KT)), dim3(256), 0, s>>>(ka);
+            ka.lse = ga.lse; ka.grad = ga.grad; ka.g = g; ka.ldg = vp; ka.resid = ga.resid;
+            lmhead_grad_kept_kernel<<<dim3((unsigned)((vp / 16 + 4 * kKeptBlocks - 1) / (4 * kKeptBlocks)), (unsigned)(rows_pad / 32)), dim3(256), 0, s>>>(ka);
         } else if (h % CoreB::BK == 0) launch_grad<CoreB>(ga, s);
         else launch_grad<CoreA>(ga, s);
-        // dH[token of row r] = G [rows, V] * (W^T [H, V])^T, written to the tokens' own rows
+        // dH[token of row r] = G [rows, V] W [V, H], written to the tokens' own rows (columns of G past V are zero)
         GemmOperands dh;
-        dh.a = g; dh.lda = vp; dh.b = wt; dh.ldb = vp; dh.m = rows; dh.n = h; dh.k = vp;
-        dh.live = count; dh.live_from = t0; dh.live_dim = 1;
-        const Patches dh_patches = dh_plan(rows, h, vp);
-        if (dh_patches.splits > 1) {
-            launch_gemm<0>(dh, dh_patches, dh_parts, h, s);
+        dh.a = w; dh.lda = ldw; dh.b = g; dh.ldb = vp; dh.m = h; dh.n = rows; dh.k = vp; dh.rows_a = vocab;
+        dh.live = count; dh.live_from = t0; dh.live_dim = 3;
+        const Strips dh_strips = dh_plan(rows, h, vp);
+        if (dh_strips.splits > 1) {
+            launch_gemm<false, 0>(dh, dh_strips, dh_parts, h, s);
             lmhead_finish_dh_kernel<true><<<dim3((unsigned)rows), dim3(256), 0, s>>>(
-                dhidden_out, ld_dh, dh_parts, dh_patches.splits, rows * h, idx + t0, count, t0, ga.grad, ga.targets, vocab_start, vocab, w, ldw, h);
+                dhidden_out, ld_dh, dh_parts, dh_strips.splits, rows * h, idx + t0, count, t0, ga.resid, ga.targets, vocab_start, vocab, w, ldw, h);
         } else {
-            launch_gemm<0>(dh, dh_patches, dhidden_out, ld_dh, s, idx + t0);
+            launch_gemm<false, 0>(dh, dh_strips, dhidden_out, ld_dh, s, idx + t0);
             lmhead_finish_dh_kernel<false><<<dim3((unsigned)rows), dim3(256), 0, s>>>(
-                dhidden_out, ld_dh, nullptr, 1, 0, idx + t0, count, t0, ga.grad, ga.targets, vocab_start, vocab, w, ldw, h);
+                dhidden_out, ld_dh, nullptr, 1, 0, idx + t0, count, t0, ga.resid, ga.targets, vocab_start, vocab, w, ldw, h);
         }
-        // dW += G^T [V, rows] * (hidden^T [H, rows])^T
+        // dW += G^T [V, rows] hidden [rows, H] (rows of both past the live ones, up to a multiple of 64, are zero)
         transpose_to_frag_kernel<<<dim3((unsigned)(h_pad / 256), (unsigned)(rows_pad / 64)), dim3(256), 0, s>>>(
-            hid_c + t0 * h, rows, h, h, ht, ld_t, rows_pad);
+            hid_c + t0 * h, rows, h, h, ht, bwd_ld_t(chunk), rows_pad);
         GemmOperands dwo;
-        dwo.a = gt; dwo.lda = ld_t; dwo.b = ht; dwo.ldb = ld_t; dwo.m = vocab; dwo.n = h; dwo.k = rows_pad;
+        dwo.a = g; dwo.lda = vp; dwo.b = ht; dwo.ldb = bwd_ld_t(chunk); dwo.m = vocab; dwo.n = h; dwo.k = rows_pad;
         dwo.live = count; dwo.live_from = t0; dwo.live_dim = 2;
         // (the narrowing epilogue writes with the accumulator's row stride)
-        if (single && dw_patches.splits > 1) {
-            launch_gemm<0>(dwo, dw_patches, dw, h, s);
-            lmhead_sum_dw_kernel<<<dim3(2048), dim3(256), 0, s>>>(static_cast<uint16_t*>(dweight_out), dw, dw_patches.splits, vocab * h, vocab * h);
-        } else if (single) launch_gemm<GEMM_NARROW>(dwo, dw_patches, dw, h, s, nullptr, static_cast<uint16_t*>(dweight_out));
-        else if (t0 == 0) launch_gemm<0>(dwo, Patches{}, dw, h, s);
-        else launch_gemm<GEMM_ACCUM>(dwo, Patches{}, dw, h, s);
+        if (single && dw_strips.splits > 1) {
+            launch_gemm<true, 0>(dwo, dw_strips, dw, h, s);
+            lmhead_sum_dw_kernel<<<dim3(2048), dim3(256), 0, s>>>(static_cast<uint16_t*>(dweight_out), dw, dw_strips.splits, vocab * h, vocab * h);
+        } else if (single) launch_gemm<true, GEMM_NARROW>(dwo, dw_strips, dw, h, s, nullptr, static_cast<uint16_t*>(dweight_out));
+        else if (t0 == 0) launch_gemm<true, 0>(dwo, Strips{}, dw, h, s);
+        else launch_gemm<true, GEMM_ACCUM>(dwo, Strips{}, dw, h, s);
     }
     if (n_tokens > 0 && !single) {
         uint16_t* out = static_cast<uint16_t*>(dweight_out);

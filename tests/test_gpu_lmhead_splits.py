@@ -40,6 +40,45 @@ def test_split_products_match_oracle(n, h, v, keep):
     assert torch.equal(again[0], dh) and torch.equal(again[1], dw)  # partial products are added in a fixed order
 
 
+# edges of core T's tiles, slabs and fragments: ids, tokens and hidden sizes on either side of 16, 32, 64 and 256
+@pytest.mark.parametrize("n,h,v", [(1, 8, 1), (31, 8, 17), (33, 72, 63), (64, 264, 65), (65, 248, 255), (257, 256, 257), (255, 8, 1030), (129, 520, 40)])
+@pytest.mark.parametrize("keep", [False, True])
+def test_products_at_the_edges_of_tiles(n, h, v, keep):
+    g = torch.Generator().manual_seed(n * 1000 + v)
+    hid = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    w = (torch.randn(v, h, generator=g) * 0.1).to(torch.bfloat16)
+    tgt = torch.randint(0, v, (n,), generator=g)
+    up = torch.randn(n, generator=g) * 1e-2
+    up[1::4] = 0
+    _, lse, kept = _ops().lmhead_logprob_fwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), 0, v, keep)
+    dh, dw = _ops().lmhead_logprob_bwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), lse, up.to(DEV), 0, v, kept if keep else None)
+    o_dh, o_dw, b_dh, b_dw = narrowing_bounds(hid, w, tgt, up)
+    assert bool(((dh.cpu() - o_dh).abs() <= b_dh).all())
+    assert bool(((dw.float().cpu() - o_dw).abs() <= b_dw).all())
+
+
+def test_products_of_a_shard_leave_other_ranks_targets_out():
+    """A rank that holds ids 100 .. 399: targets elsewhere have a softmax part but no one-hot element and no residual."""
+    g = torch.Generator().manual_seed(9)
+    n, h, v, first = 90, 64, 300, 100
+    hid = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    w = (torch.randn(v, h, generator=g) * 0.1).to(torch.bfloat16)
+    tgt = torch.randint(0, 500, (n,), generator=g)
+    up = torch.randn(n, generator=g) * 1e-2
+    _, lse, kept = _ops().lmhead_logprob_fwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), first, first + v, True)
+    inside = ((tgt >= first) & (tgt < first + v)).float()
+    one = torch.nn.functional.one_hot((tgt - first).clamp(0, v - 1), v).float() * inside.unsqueeze(-1)
+    p = torch.softmax((hid @ w.T).float(), -1)
+    grad = (one - p) * up.unsqueeze(-1)
+    mag = (one + 2 * p) * up.abs().unsqueeze(-1)
+    for k in (kept, None):
+        dh, dw = _ops().lmhead_logprob_bwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), lse, up.to(DEV), first, first + v, k)
+        # G narrowed to bf16 (2^-8) from logits narrowed to bf16 (as much again); dW narrowed once more
+        assert bool(((dh.cpu() - grad @ w.float()).abs() <= 2.0 ** -7 * ((p * up.abs().unsqueeze(-1)) @ w.float().abs()) + 1e-6).all())
+        want = grad.T @ hid.float()
+        assert bool(((dw.float().cpu() - want).abs() <= 2.0 ** -7 * (mag.T @ hid.float().abs()) + 2.0 ** -8 * want.abs() + 1e-6).all())
+
+
 @pytest.mark.parametrize("n,h,v", [(300, 128, 20000), (4096, 64, 600)])
 def test_no_live_token_gives_zero_gradients(n, h, v):
     hid = torch.randn(n, h, device=DEV).to(torch.bfloat16)
