@@ -1570,27 +1570,35 @@ struct SelBwdArgs {
     const int32_t* kept_idx;
     const float* kept_x;
     int kept_cap;
-    int prefilled;  // the record is in use: the whole gradient buffer was zero-filled before this launch, rows on record only add their entries
+    int prefilled;  // the record is in use: rows on record and rows without a gradient were zero-filled before this launch (fill_zero_rows_kernel), rows on record only add their entries
+    int parts;      // workgroups per row
 };
+
+// The number of kept entries on record for gradient row (o, i), or -1: the row is streamed from the logits.  `g` becomes its
+// upstream gradient, 0 for rows that have none (those are zero whatever the record says).
+__device__ __forceinline__ int topk_topp_on_record(const SelBwdArgs& a, int64_t o, int64_t i, float& g) {
+    g = i < a.n_inner ? a.grad[o * a.gs_outer + i * a.gs_inner] : 0.f;
+    if (g == 0.f) return 0;
+    const int n = a.kept_n[o * a.n_inner + i];
+    return n > a.kept_cap ? -1 : n;  // (above the capacity: not a count the forward writes)
+}
 
 // MODE 0: gradient, MODE 1: filtered logits (-inf outside the kept set) + keep mask
 template <int DT, int TEMP, int MODE>
-__device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_t r) {
+__device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_t r, int part) {
     constexpr int EPV = Row<DT>::EPV;
     const int tid = threadIdx.x;
     const int64_t o = r / a.d_n_inner, i_in = r - o * a.d_n_inner;
     char* out = static_cast<char*>(a.out) + (o * a.ds_outer + i_in * a.ds_inner) * Row<DT>::BYTES;
     const int64_t vocab = a.vocab;
     float g = 0.f;
-    if (MODE == 0 && i_in < a.n_inner) g = a.grad[o * a.gs_outer + i_in * a.gs_inner];
     // With the forward's record of the kept set the gradient row is zeros plus the few kept entries, written
     // without reading the logits again.
     int n_rec = -1;
-    if (MODE == 0 && g != 0.f && a.prefilled) {
-        n_rec = a.kept_n[o * a.n_inner + i_in];
-        if (n_rec > a.kept_cap) n_rec = -1;  // not a count the forward writes: stream the row instead
-    }
-    if (MODE == 0 && a.prefilled && (g == 0.f || n_rec >= 0)) {
+    if (MODE == 0 && a.prefilled) n_rec = topk_topp_on_record(a, o, i_in, g);
+    else if (MODE == 0 && i_in < a.n_inner) g = a.grad[o * a.gs_outer + i_in * a.gs_inner];
+    if (MODE == 0 && a.prefilled && n_rec >= 0) {
+        if (part > 0) return;
         // the zeros are there already (an earlier launch on the stream): only the kept entries are written
         const int64_t rec = (o * a.n_inner + i_in) * a.kept_cap;
         if (n_rec > 0) {
@@ -1612,9 +1620,9 @@ __device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_
         const int64_t zn = (vocab - zh) / EPV;
         u32x4* zv = reinterpret_cast<u32x4*>(out + zh * Row<DT>::BYTES);
         const u32x4 z = {0u, 0u, 0u, 0u};
-        for (int64_t v = tid; v < zn; v += kSelBlock) zv[v] = z;
-        if (tid < zh) Row<DT>::store1(out, tid, 0.f);
-        if (zh + zn * EPV + tid < vocab) Row<DT>::store1(out, zh + zn * EPV + tid, 0.f);
+        for (int64_t v = zn * part / a.parts + tid; v < zn * (part + 1) / a.parts; v += kSelBlock) zv[v] = z;
+        if (part == 0 && tid < zh) Row<DT>::store1(out, tid, 0.f);
+        if (part == 0 && zh + zn * EPV + tid < vocab) Row<DT>::store1(out, zh + zn * EPV + tid, 0.f);
         return;
     }
     const int64_t rr = o * a.n_inner + i_in;
@@ -1638,7 +1646,7 @@ __device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_
 
     const int64_t head = sel_row_head<DT>(row, vocab);
     if (sel_row_head<DT>(out, vocab) != head) {
-        for (int64_t e = tid; e < vocab; e += kSelBlock) {
+        for (int64_t e = vocab * part / a.parts + tid; e < vocab * (part + 1) / a.parts; e += kSelBlock) {
             bool keep;
             Row<DT>::store1(out, e, elem(Row<DT>::load1(row, e), e, keep));
             if (keep_row) keep_row[e] = keep ? 1 : 0;
@@ -1654,21 +1662,33 @@ __device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_
     using MaskWord = typename std::conditional<EPV == 8, uint64_t, uint32_t>::type;
     static_assert(sizeof(MaskWord) == EPV, "one mask byte per element of a vector");
     const bool mask_words = keep_row && ((reinterpret_cast<uintptr_t>(keep_row) + head) % EPV) == 0;
-    for (int64_t vi = tid; vi < nvec; vi += kSelBlock) {
-        float t[EPV];
-        Row<DT>::decode(__builtin_nontemporal_load(xv + vi), t);
-        MaskWord bits = 0;
+    const int64_t end = nvec * (part + 1) / a.parts;
+    constexpr int kLoads = 4;  // in flight per thread
+    for (int64_t v0 = nvec * part / a.parts + tid; v0 < end; v0 += kLoads * kSelBlock) {
+        u32x4 q[kLoads];
 #pragma unroll
-        for (int k = 0; k < EPV; ++k) {
-            bool keep;
-            const int64_t idx = head + vi * EPV + k;
-            t[k] = elem(t[k], idx, keep);
-            bits |= static_cast<MaskWord>(keep ? 1 : 0) << (8 * k);
-            if (keep_row && !mask_words) keep_row[idx] = keep ? 1 : 0;
+        for (int u = 0; u < kLoads; ++u)
+            if (v0 + u * kSelBlock < end) q[u] = __builtin_nontemporal_load(xv + v0 + u * kSelBlock);
+#pragma unroll
+        for (int u = 0; u < kLoads; ++u) {
+            const int64_t vi = v0 + u * kSelBlock;
+            if (vi >= end) break;
+            float t[EPV];
+            Row<DT>::decode(q[u], t);
+            MaskWord bits = 0;
+#pragma unroll
+            for (int k = 0; k < EPV; ++k) {
+                bool keep;
+                const int64_t idx = head + vi * EPV + k;
+                t[k] = elem(t[k], idx, keep);
+                bits |= static_cast<MaskWord>(keep ? 1 : 0) << (8 * k);
+                if (keep_row && !mask_words) keep_row[idx] = keep ? 1 : 0;
+            }
+            if (mask_words) *reinterpret_cast<MaskWord*>(keep_row + head + vi * EPV) = bits;
+            __builtin_nontemporal_store(Row<DT>::encode(t), ov + vi);
         }
-        if (mask_words) *reinterpret_cast<MaskWord*>(keep_row + head + vi * EPV) = bits;
-        __builtin_nontemporal_store(Row<DT>::encode(t), ov + vi);
     }
+    if (part > 0) return;
     for (int w = 0; w < 2; ++w) {
         const int64_t e = w == 0 ? (tid < head ? tid : -1) : (tail0 + tid < vocab ? tail0 + tid : -1);
         if (e < 0) continue;
@@ -1678,26 +1698,39 @@ __device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_
     }
 }
 
-// Zero fill of a contiguous buffer by one workgroup per compute unit in 256 KiB spans: 6.0 TB/s, as a memset, where
-// one workgroup per row reaches 5.5.
+// Zero fill of the rows of a contiguous gradient that are not streamed from the logits, by one workgroup per compute unit in
+// 256 KiB spans: 6.0 TB/s where nothing is streamed, as a memset, where one workgroup per row reaches 5.5.  A 16-byte unit that a
+// streamed row shares with its neighbour is cleared too; the row is written later.  (1500 rows of V = 151 936, half of them
+// streamed: 57 us when every row was cleared, 29 now.)
 constexpr int kFillGrid = 256;
 constexpr int64_t kFillSpan = 256 * 1024;
-__global__ __launch_bounds__(256) void fill_zero_flat_kernel(char* out, int64_t total_bytes) {
+template <int DT> __global__ __launch_bounds__(256) void fill_zero_rows_kernel(SelBwdArgs a, int64_t total_bytes) {
     const u32x4 z = {0u, 0u, 0u, 0u};
+    char* out = static_cast<char*>(a.out);
+    const int64_t row_bytes = a.vocab * Row<DT>::BYTES;
     for (int64_t s0 = static_cast<int64_t>(blockIdx.x) * kFillSpan; s0 < total_bytes; s0 += static_cast<int64_t>(gridDim.x) * kFillSpan) {
-        u32x4* zv = reinterpret_cast<u32x4*>(out + s0);
-        const int64_t left = total_bytes - s0;
-        const int64_t nv = (left < kFillSpan ? left : kFillSpan) / 16;
-        for (int64_t v = threadIdx.x; v < nv; v += 256) zv[v] = z;
-        if (left < kFillSpan && threadIdx.x < (left & 15)) out[s0 + nv * 16 + threadIdx.x] = 0;
+        const int64_t s1 = s0 + kFillSpan < total_bytes ? s0 + kFillSpan : total_bytes;
+        for (int64_t r = s0 / row_bytes; r * row_bytes < s1; ++r) {
+            const int64_t o = r / a.d_n_inner;
+            float g;
+            if (topk_topp_on_record(a, o, r - o * a.d_n_inner, g) < 0) continue;
+            const int64_t b0 = r * row_bytes > s0 ? r * row_bytes : s0, b1 = (r + 1) * row_bytes < s1 ? (r + 1) * row_bytes : s1;
+            const int64_t v1 = b1 / 16;  // whole units, from the one that holds the row's first byte
+            for (int64_t v = b0 / 16 + threadIdx.x; v < v1; v += 256) reinterpret_cast<u32x4*>(out)[v] = z;
+            // the row's last bytes: the unit's other bytes are the next row's, or past the buffer's end
+            const int64_t b = (v1 * 16 > b0 ? v1 * 16 : b0) + static_cast<int64_t>(threadIdx.x) * Row<DT>::BYTES;
+            if (b < b1) Row<DT>::store1(out, b / Row<DT>::BYTES, 0.f);
+        }
     }
 }
 
-// One workgroup per row (a fixed set of 512 workgroups walking the rows, which fills memory 10 % faster when it does
-// nothing else, measured no gain here: with few workgroups per compute unit the record staging of a row is exposed).
+// One workgroup per row, or several for few rows (a fixed set of 512 workgroups walking the rows, which fills memory
+// 10 % faster when it does nothing else, measured no gain here: with few workgroups per compute unit the record staging of a
+// row is exposed).
 template <int DT, int TEMP, int MODE>
-__global__ __launch_bounds__(kSelBlock) void topk_topp_stream_kernel(SelBwdArgs a, int64_t n_rows) {
-    for (int64_t r = blockIdx.x; r < n_rows; r += gridDim.x) topk_topp_stream_row<DT, TEMP, MODE>(a, r);
+__global__ __launch_bounds__(kSelBlock) void topk_topp_stream_kernel(SelBwdArgs a) {
+    const uint32_t r = blockIdx.x / static_cast<uint32_t>(a.parts);
+    topk_topp_stream_row<DT, TEMP, MODE>(a, r, static_cast<int>(blockIdx.x - r * a.parts));
 }
 
 static int temp_code3(float temperature, int mode, float* tparam) {
@@ -1828,8 +1861,17 @@ extern "C" int nrl_topk_topp_logprob_bwd(const nrl_rows* rows, const float* thr,
         const uintptr_t l1 = l0 + static_cast<uintptr_t>(((rows->n_outer - 1) * so + (rows->n_inner - 1) * si + rows->vocab) * elt);
         if (d0 < l1 && l0 < d1) a.prefilled = 0;
     }
-    if (a.prefilled) fill_zero_flat_kernel<<<dim3(kFillGrid), dim3(256), 0, s>>>(static_cast<char*>(dlogits), n * rows->vocab * elt);
-    NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_stream_kernel<DT, TEMP, 0><<<dim3((unsigned)n), dim3(kSelBlock), 0, s>>>(a, n));
+    if (a.prefilled) {
+        const int64_t total = n * rows->vocab * elt;
+        if (rows->dtype == NRL_F32) fill_zero_rows_kernel<NRL_F32><<<dim3(kFillGrid), dim3(256), 0, s>>>(a, total);
+        else fill_zero_rows_kernel<NRL_BF16><<<dim3(kFillGrid), dim3(256), 0, s>>>(a, total);  // (zeros of two bytes, either type)
+    }
+    // Parts of at least 32 KiB, as long as the rows alone are too few to keep the chip busy to the end: 1500 rows of V = 151 936,
+    // half of them streamed, 126 -> 110 us; 4096 rows that are all on record only pay for the workgroups (two a row: 11 -> 14).
+    const int64_t most = rows->vocab * elt / 32768;
+    a.parts = static_cast<int>(6144 / n < most ? 6144 / n : most);
+    if (a.parts < 1) a.parts = 1;
+    NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_stream_kernel<DT, TEMP, 0><<<dim3((unsigned)(n * a.parts)), dim3(kSelBlock), 0, s>>>(a));
     return check_launch("topk_topp_logprob_bwd");
 }
 
@@ -1846,9 +1888,9 @@ extern "C" int nrl_topk_topp_filter(const nrl_rows* rows, const float* thr, cons
     a.thr = thr; a.tie = tie; a.lse_kept = thr; a.grad = nullptr; a.gs_outer = 0; a.gs_inner = 0;
     a.out = filtered_out; a.d_n_inner = rows->n_inner; a.ds_outer = f_stride_outer; a.ds_inner = f_stride_inner;
     a.keep_out = keep_out;
-    a.kept_n = nullptr; a.kept_idx = nullptr; a.kept_x = nullptr; a.kept_cap = 0; a.prefilled = 0;
+    a.kept_n = nullptr; a.kept_idx = nullptr; a.kept_x = nullptr; a.kept_cap = 0; a.prefilled = 0; a.parts = 1;
     const int tc = temp_code3(rows->temperature, rows->temp_mode, &a.tparam);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_stream_kernel<DT, TEMP, 1><<<dim3((unsigned)n), dim3(kSelBlock), 0, s>>>(a, n));
+    NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_stream_kernel<DT, TEMP, 1><<<dim3((unsigned)n), dim3(kSelBlock), 0, s>>>(a));
     return check_launch("topk_topp_filter");
 }

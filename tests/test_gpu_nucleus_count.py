@@ -139,3 +139,28 @@ def test_repeats_bit_for_bit():
     for _ in range(3):
         for a, b in zip(first, torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, 39, 0, 0.95, 1.0, NRL_TEMP_RCP, True)):
             assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("vocab", [5, 20003, 131077])
+def test_gradient_rows_cleared_and_streamed_side_by_side(dtype, vocab):
+    """Rows on record, streamed rows and rows without a gradient next to each other, whose ends share 16-byte units (odd
+    vocabularies) and 256 KiB spans; few rows, so that several workgroups stream one.  The same bits as streaming every row."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    n = 13
+    sd = torch.tensor([6.0, 0.3, 6.0, 6.0, 0.3, 0.3, 8.0, 0.3, 5.0, 0.1, 0.1, 9.0, 6.0, 1.0], device=DEV).view(1, -1, 1)
+    x = (torch.randn(2, n + 1, vocab, generator=g, device=DEV) * sd).to(dtype)
+    t = x[:, :n].float().argmax(-1)
+    up = torch.randn(2, n, generator=g, device=DEV)
+    up[:, 2] = 0.0
+    up[:, 7] = 0.0
+    _, thr, tie, lse, _, cnt, idx, val = torch.ops.rl_amd.topk_topp_logprob_fwd_rec(x, t, n, 0, 0.9, 1.0, NRL_TEMP_RCP, False, 128)
+    if vocab > 128:
+        assert int((cnt < 0).sum()) > 4 and int((cnt >= 0).sum()) > 4
+    want = torch.ops.rl_amd.topk_topp_logprob_bwd(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP)
+    got = torch.ops.rl_amd.topk_topp_logprob_bwd(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP, cnt, idx, val)
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    assert torch.equal(got.view(bits), want.view(bits))
