@@ -577,21 +577,6 @@ class DistillationLossConfig(BaseModel, extra="allow"):
     zero_outside_topk: bool = False
 
 
-class _DistillTopk(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, student_lp, teacher_lp, h_all, token_mask, sample_mask, global_valid_toks, kl_type, w, zero_outside, log_inf):
-        loss, d_s, d_h = _OPS.distill_topk_loss(student_lp.detach(), teacher_lp.detach(), None if h_all is None else h_all.detach(),
-                                                token_mask, sample_mask, global_valid_toks, kl_type, w, zero_outside, log_inf)
-        ctx.save_for_backward(d_s, d_h)
-        ctx.has_h = h_all is not None and d_h.numel() > 0
-        return loss
-
-    @staticmethod
-    def backward(ctx, grad_loss):
-        d_s, d_h = ctx.saved_tensors
-        return (d_s * grad_loss, None, d_h * grad_loss if ctx.has_h else None) + (None,) * 7
-
-
 class DistillationLossFn(LossFunction):
     """Top-k distillation loss (``loss_functions.py:1124-1206``): forward, reverse or mixed KL between the
     teacher's and the student's top-k log-probabilities per token, optionally with the correction for the
@@ -619,14 +604,11 @@ class DistillationLossFn(LossFunction):
         dev = _gpu_for(student_topk_logprobs)
         token_mask = sample_mask = valid = None
         if "token_mask" in data and "sample_mask" in data:
-            n = student_topk_logprobs.shape[1]
-            token_mask = _f32(data["token_mask"][:, 1:][:, :n], dev)
-            sample_mask = _f32(data["sample_mask"], dev)
-            valid = _global_valid(1.0, global_valid_toks, dev)[1:]
-        loss = _DistillTopk.apply(
-            _f32(student_topk_logprobs, dev), _f32(teacher_topk_logprobs, dev), None if H_all is None else _f32(H_all, dev),
-            token_mask, sample_mask, valid, self._KL[self.kl_type], float(self.mixed_kl_weight), bool(self.zero_outside_topk),
-            float(self.log_infinitesimal),
+            token_mask, sample_mask = data["token_mask"], data["sample_mask"]
+            valid = _scalar(global_valid_toks, dev)
+        loss = _host().distill_loss(
+            _f32(student_topk_logprobs, dev), teacher_topk_logprobs, H_all, token_mask, sample_mask, valid, self._KL[self.kl_type],
+            float(self.mixed_kl_weight), bool(self.zero_outside_topk), float(self.log_infinitesimal),
         )
         if home != dev:
             loss = loss.to(home)

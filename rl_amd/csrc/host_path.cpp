@@ -446,6 +446,71 @@ Tensor gather_entropy_bwd(const Tensor& logits, const Tensor& indices, int64_t n
     return d;
 }
 
+// log_softmax over the whole last axis of the first n_inner rows of every sequence
+Tensor logsoftmax_rows(const Tensor& logits, int64_t n_inner) {
+    need_gpu(logits);
+    const nrl_rows rows = make_rows(logits, Tensor(), n_inner, 0, vocab_of(logits), 1.0, NRL_TEMP_RCP);
+    const c10::OptionalDeviceGuard guard(logits.device());
+    Tensor out = f32({logits.size(0), n_inner, logits.size(2)}, logits);
+    check(nrl_topk_logsoftmax_fwd(&rows, nullptr, logits.size(2), ptr(out), stream_of(logits)), "nrl_topk_logsoftmax_fwd");
+    return out;
+}
+
+// Top-k distillation loss of fp32 logprobs [B, n, K], d loss / d student [B, n, K] and d loss / d h_all [B, n] (empty without
+// the correction).  The two gradients lie in one buffer, so that an upstream factor is one product.
+struct DistillOut {
+    Tensor loss, both, d_s, d_h;
+};
+struct DistillArgs {
+    int64_t kl;
+    double weight;
+    bool zero_outside;
+    double log_inf;
+};
+DistillOut distill_views(const Tensor& both, at::IntArrayRef shape, bool correct) {
+    const int64_t b = shape[0], n = shape[1], ns = b * n * shape[2], h0 = (ns + 3) / 4 * 4;
+    return {Tensor(), both, both.narrow(0, 0, ns).view(shape), correct ? both.narrow(0, h0, b * n).view({b, n}) : both.narrow(0, 0, 0)};
+}
+DistillOut distill_topk_loss(const Tensor& student_in, const Tensor& teacher_in, const Tensor& h_in, const Tensor& token_mask_in, const Tensor& sample_mask_in,
+                             const Tensor& toks_in, const DistillArgs& a) {
+    need_gpu(student_in, teacher_in, h_in, token_mask_in, sample_mask_in, toks_in);
+    TORCH_CHECK_VALUE(student_in.dim() == 3 && student_in.sizes() == teacher_in.sizes(), "student / teacher logprobs must both be [B, n, K], got ",
+                      student_in.sizes(), " and ", teacher_in.sizes());
+    TORCH_CHECK_VALUE(student_in.scalar_type() == at::kFloat && teacher_in.scalar_type() == at::kFloat, "top-k logprobs must be fp32");
+    const int64_t b = student_in.size(0), n = student_in.size(1), k = student_in.size(2);
+    const Tensor student = student_in.contiguous(), teacher = teacher_in.contiguous();
+    const bool correct = a.zero_outside && a.kl != 0;
+    auto given = [&](const Tensor& t, at::IntArrayRef shape, const char* name) {
+        TORCH_CHECK_VALUE(t.scalar_type() == at::kFloat && t.sizes() == shape, name, " must be fp32 ", shape, ", got ", t.scalar_type(), " ", t.sizes());
+    };
+    Tensor h, token_mask = token_mask_in, sample_mask, toks;
+    if (correct) {
+        TORCH_CHECK_VALUE(h_in.defined(), "H_all is required when zero_outside_topk is set and the KL is not the forward one");
+        given(h_in, {b, n}, "H_all");
+        h = h_in.contiguous();
+    }
+    if (token_mask.defined()) {
+        given(token_mask, {b, n}, "token_mask");
+        if (n > 1 && token_mask.stride(1) != 1) token_mask = token_mask.contiguous();
+    }
+    if (sample_mask_in.defined()) {
+        given(sample_mask_in, {b}, "sample_mask");
+        sample_mask = sample_mask_in.contiguous();
+    }
+    TORCH_CHECK_VALUE(!token_mask.defined() || (sample_mask.defined() && toks_in.defined()), "token_mask needs sample_mask and global_valid_toks");
+    if (toks_in.defined()) toks = toks_in.reshape({-1}).slice(0, 0, 1).to(at::kFloat).contiguous();
+    const c10::OptionalDeviceGuard guard(student.device());
+    const int64_t ns = b * n * k, h0 = (ns + 3) / 4 * 4;
+    DistillOut o = distill_views(f32({correct ? h0 + b * n : ns}, student), student.sizes(), correct);
+    o.loss = f32({}, student);
+    const Tensor ws = workspace(nrl_distill_topk_loss_workspace_bytes(b, n), student);
+    check(nrl_distill_topk_loss_fwd_bwd(ptr(student), ptr(teacher), ptr(h), ptr(token_mask), token_mask.defined() && b > 1 ? token_mask.stride(0) : n,
+                                        ptr(sample_mask), ptr(toks), b, n, k, static_cast<int32_t>(a.kl), static_cast<float>(a.weight), a.zero_outside,
+                                        static_cast<float>(a.log_inf), ptr(o.loss), ptr(o.d_s), ptr(o.d_h), ws.data_ptr(), ws.numel() * 8, stream_of(student)),
+          "nrl_distill_topk_loss_fwd_bwd");
+    return o;
+}
+
 // -> (baseline [B], std [B], advantages [B], group index of every row [B])
 std::tuple<Tensor, Tensor, Tensor, Tensor> group_baseline_std(const Tensor& prompts_in, const Tensor& rewards_in, const Tensor& valid_in,
                                                               const OptTensor& std_rewards_in, bool leave_one_out, bool normalize) {
@@ -712,6 +777,28 @@ struct GatherEntropy : torch::autograd::Function<GatherEntropy> {
     }
 };
 
+// the top-k distillation loss; the kernel also returns its gradients, so the backward is one product with the upstream factor
+struct DistillLoss : torch::autograd::Function<DistillLoss> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& student, const Tensor& teacher, const OptTensor& h, const OptTensor& token_mask,
+                          const OptTensor& sample_mask, const OptTensor& toks, const DistillArgs& a) {
+        const auto plain = [](const OptTensor& t) { return t.has_value() ? t->detach() : Tensor(); };
+        const DistillOut o = distill_topk_loss(student.detach(), teacher.detach(), plain(h), plain(token_mask), plain(sample_mask), plain(toks), a);
+        ctx->save_for_backward({o.both});
+        ctx->saved_data["shape"] = student.sizes().vec();
+        ctx->saved_data["h"] = h.has_value() && o.d_h.numel() > 0;
+        return o.loss;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list grads) {
+        const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+        const bool h = ctx->saved_data["h"].toBool();
+        const DistillOut o = distill_views(ctx->get_saved_variables()[0] * grads[0], shape, h);
+        variable_list out(7);
+        out[0] = o.d_s;
+        if (h) out[2] = o.d_h;
+        return out;
+    }
+};
+
 // ---------------------------------------------------------------------------------------------
 // a small device record on its way to the host
 // ---------------------------------------------------------------------------------------------
@@ -842,6 +929,21 @@ PYBIND11_MODULE(_host, m) {
         const variable_list o = any_row ? FusedRowsLoss::apply(logits, t, cu, prev, gen, ref, adv, token_mask, sample_mask, seqs, toks, a)
                                         : FusedLoss::apply(logits, t, cu, prev, gen, ref, adv, token_mask, sample_mask, seqs, toks, a);
         return std::make_tuple(o[0], o[1]);
+    });
+    m.def("logsoftmax_rows", &logsoftmax_rows);
+    m.def("distill_topk_loss", [](const Tensor& student, const Tensor& teacher, const OptTensor& h, const OptTensor& token_mask, const OptTensor& sample_mask,
+                                  const OptTensor& toks, int64_t kl, double weight, bool zero_outside, double log_inf) {
+        const DistillOut o = distill_topk_loss(student, teacher, opt(h), opt(token_mask), opt(sample_mask), opt(toks), {kl, weight, zero_outside, log_inf});
+        return std::make_tuple(o.loss, o.d_s.clone(), o.d_h.clone());
+    });
+    // of logprobs on the GPU; masks and count in any dtype, anywhere: token_mask [B, >= n + 1], of which the columns 1 .. n count
+    m.def("distill_loss", [](const Tensor& student_in, const Tensor& teacher, const OptTensor& h, const OptTensor& token_mask, const OptTensor& sample_mask,
+                             const OptTensor& toks, int64_t kl, double weight, bool zero_outside, double log_inf) {
+        const auto on = [&](const OptTensor& t) { return t.has_value() ? OptTensor(to_f32(*t, student_in)) : OptTensor(); };
+        const Tensor student = to_f32(student_in, student_in);
+        TORCH_CHECK(!toks.has_value() || toks->numel() == 1, "global_valid_toks must hold one value");
+        const OptTensor mask = token_mask.has_value() ? OptTensor(token_mask->slice(1, 1).slice(1, 0, student.size(1))) : OptTensor();
+        return DistillLoss::apply(student, to_f32(teacher, student), on(h), on(mask), on(sample_mask), on(toks), DistillArgs{kl, weight, zero_outside, log_inf});
     });
     m.def("gather_entropy", [](const Tensor& logits, const Tensor& indices, int64_t n, bool entropy) {
         const variable_list o = GatherEntropy::apply(logits, indices, n, entropy);

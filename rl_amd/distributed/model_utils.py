@@ -665,5 +665,6 @@ def get_distillation_topk_logprobs_from_logits(
         raise ValueError(f"teacher_topk_logits must be [B, S, K], got {tuple(teacher.shape)}")
     if teacher.stride(2) != 1 and teacher.shape[2] > 1:
         teacher = teacher.contiguous()
-    teacher_topk_logprobs = torch.ops.rl_amd.topk_logsoftmax_fwd(teacher.detach()[:, :-1], None)
+    refuse_pending(teacher, "get_distillation_topk_logprobs_from_logits")
+    teacher_topk_logprobs = _host().logsoftmax_rows(teacher.detach(), max(teacher.shape[1] - 1, 0))
     return student_topk_logprobs, teacher_topk_logprobs, H_all

@@ -1,0 +1,81 @@
+"""DistillationLossFn's call: masks and counts of any type and place, upstream factors, and what it refuses."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _case(seed, b=2, s=7, v=300, k=5):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    logits = torch.randn(b, s, v, generator=g, device=DEV)
+    mask = torch.ones(b, s, dtype=torch.int64, device=DEV)
+    mask[:, :2] = 0
+    top, at = torch.randn(b, s, v, generator=g, device=DEV).topk(k, dim=-1)
+    data = {"input_ids": torch.zeros(b, s, dtype=torch.int64, device=DEV), "token_mask": mask, "sample_mask": torch.ones(b, device=DEV),
+            "teacher_topk_logits": top, "teacher_topk_indices": at}
+    return logits, data
+
+
+def _run(logits, data, toks, kl="mixed", factor=1.0, zero=True):
+    from rl_amd.algorithms.loss import DistillationLossConfig, DistillationLossFn, prepare_loss_input
+
+    x = logits.clone().requires_grad_(True)
+    fn = DistillationLossFn(DistillationLossConfig(kl_type=kl, mixed_kl_weight=0.5, zero_outside_topk=zero))
+    kwargs, data = prepare_loss_input(x, dict(data), fn)
+    loss, metrics = fn(data=data, global_valid_seqs=torch.tensor(2.0), global_valid_toks=toks, **kwargs)
+    assert isinstance(metrics["loss"], float) and metrics["loss"] == loss.item()
+    (d,) = torch.autograd.grad(loss * factor, x)
+    return loss.detach(), d
+
+
+@pytest.mark.parametrize("kl", ["forward", "reverse", "mixed"])
+@pytest.mark.parametrize("zero", [True, False])
+def test_masks_counts_and_factors(kl, zero):
+    logits, data = _case(1)
+    toks = torch.tensor(10.0, device=DEV)
+    want, d = _run(logits, data, toks, kl, zero=zero)
+    for other in (10, 10.0, torch.tensor([10.0]), torch.tensor(10)):
+        got, e = _run(logits, data, other, kl, zero=zero)
+        assert torch.equal(got, want) and torch.equal(e, d)
+    for mask in (data["token_mask"].bool(), data["token_mask"].float().cpu(), data["token_mask"].t().contiguous().t()):
+        got, e = _run(logits, {**data, "token_mask": mask, "sample_mask": data["sample_mask"].double().cpu()}, toks, kl, zero=zero)
+        assert torch.equal(got, want) and torch.equal(e, d)
+    _, e = _run(logits, data, toks, kl, factor=0.25, zero=zero)
+    torch.testing.assert_close(e, d * 0.25, rtol=2.0 ** -22, atol=0)   # one rounding of the factor's product each way
+
+
+def test_the_gradient_follows_its_factor_under_create_graph():
+    from rl_amd.algorithms.loss import DistillationLossConfig, DistillationLossFn
+
+    g = torch.Generator(device=DEV).manual_seed(4)
+    student = torch.randn(2, 5, 4, generator=g, device=DEV).log_softmax(-1).requires_grad_(True)
+    teacher = torch.randn(2, 5, 4, generator=g, device=DEV).log_softmax(-1)
+    fn = DistillationLossFn(DistillationLossConfig(kl_type="forward", zero_outside_topk=False))
+    loss, _ = fn(student, teacher, None, {"input_ids": torch.zeros(2, 6)}, None, None)
+    c = torch.tensor(3.0, device=DEV, requires_grad=True)
+    (d,) = torch.autograd.grad(loss * c, student, create_graph=True)
+    (dc,) = torch.autograd.grad(d.sum(), c)
+    torch.testing.assert_close(dc, (d / 3.0).sum().detach())
+
+
+def test_what_is_refused():
+    logits, data = _case(2)
+    with pytest.raises(RuntimeError):
+        _run(logits, data, torch.tensor([10.0, 3.0], device=DEV))
+    with pytest.raises(ValueError):
+        _run(logits, {**data, "token_mask": data["token_mask"][:, :-2]}, torch.tensor(10.0, device=DEV))
+    with pytest.raises(ValueError):
+        _run(logits, {**data, "sample_mask": torch.ones(3, device=DEV)}, torch.tensor(10.0, device=DEV))
+    op = torch.ops.rl_amd.distill_topk_loss
+    lp = torch.randn(2, 5, 4, device=DEV)
+    for bad in ((lp[0], lp[0], None), (lp, lp[:, :-1], None), (lp.double(), lp, None), (lp, lp, None), (lp, lp, lp[:, :, 0][:1])):
+        with pytest.raises(ValueError):
+            op(*bad, None, None, None, 1, 0.5, True, -100.0)
+    with pytest.raises(ValueError):
+        op(lp, lp, None, torch.ones(2, 5, device=DEV), None, None, 0, 0.5, False, -100.0)
+    with pytest.raises(RuntimeError):
+        op(lp.cpu(), lp.cpu(), None, None, None, None, 0, 0.5, False, -100.0)
