@@ -13,7 +13,7 @@
 //                  enough, from the row read once more;
 //   pass 2         re-reads only the chunks whose maximum reaches the bound (about k of 2048) and
 //                  appends the elements above the bound to an LDS list;
-//   finish         bitonic sort of the list by (value, index), top-k threshold with ties kept,
+//   finish         the list put in order by (value, index), top-k threshold with ties kept,
 //                  softmax over the kept values, ascending cumulative mass > 1 - top_p, the
 //                  renormalised log-sum-exp, the target's logprob (-inf when it was filtered).
 // Per row the forward saves (threshold value, tie index, kept log-sum-exp): element v is kept iff
@@ -49,7 +49,6 @@ constexpr int kChunks = kSelBlock * kSub;    // 2048
 constexpr int kCap = 4096;                   // candidate capacity (LDS); rows under a small top-k use kCapSmall
 constexpr int kCapSmall = 2048;              // ... which lets six workgroups share a compute unit instead of three
 constexpr int kSmallTopK = 512;
-constexpr int kSeqList = 512;                // top-p alone: longer candidate lists are summed in double
 
 struct Lse2 {
     float m, s;
@@ -98,15 +97,17 @@ template <int CAP> struct SelShared {
     int n_hit;  // chunks whose maximum reaches the bound (their list lives in expv until the finish phase)
 };
 
-// k-th largest (1-based) of the workgroup's kChunks keys (kSub per thread, in registers); every thread
-// returns it.  Two bits at a time from the top: the answer is the largest v with at least k keys >= v.  A
-// round costs 3 * kSub ballots per wave, three LDS words per wave and one barrier (the buffers alternate), with
+// k-th largest (1-based) of the workgroup's kChunks keys (kSub per thread, in registers), or a little less; every thread
+// returns it.  Two bits at a time from the top: the answer is the largest v with at least k keys >= v, v a multiple of
+// 2^LOW.  Below LOW the keys of a 16-bit type are constant, and for fp32 the bound needs no more than 20 bits (eight, ten and
+// ten rounds for bf16, fp16 and fp32, where all 32 bits take sixteen).  A round costs 3 * kSub ballots per wave, three LDS words per wave and one barrier (the buffers alternate), with
 // no atomics -- chunk maxima share their high bits, so a histogram would serialise on one bin.
-template <int CAP>
+template <int DT> constexpr int kSelectLow = DT == NRL_BF16 ? 16 : 12;
+template <int LOW, int CAP>
 __device__ __forceinline__ uint32_t select_kth_largest(SelShared<CAP>& sh, const uint32_t (&keys)[kSub], int k) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     uint32_t v = 0u;
-    for (int bit = 30; bit >= 0; bit -= 2) {  // two bits per round: three trial values, one barrier
+    for (int bit = 30; bit >= LOW; bit -= 2) {  // two bits per round: three trial values, one barrier
         int cnt[3] = {0, 0, 0};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -129,21 +130,25 @@ __device__ __forceinline__ uint32_t select_kth_largest(SelShared<CAP>& sh, const
     return v;
 }
 
-// sum of e[n-1], e[n-2], ..., e[0] in exactly that order; called by every lane of one wave, which all
-// return the same value (64 elements per LDS read, then lane-to-scalar moves instead of one dependent
-// LDS round trip per element)
-__device__ __forceinline__ float wave_seq_sum_desc(const float* e, int n) {
-    const int lane = threadIdx.x & (kWave - 1);
-    float s = 0.f;
-    for (int blk = (n - 1) / kWave; blk >= 0; --blk) {
-        const int idx = blk * kWave + lane;
-        // lanes past the end hold 0 and come first in this order, where adding them changes nothing; with a
-        // fixed trip count the loop unrolls into 64 lane reads with constant indices
-        const float v = idx < n ? e[idx] : 0.f;
-#pragma unroll
-        for (int i = kWave - 1; i >= 0; --i) s += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), i));
-    }
-    return s;
+// inclusive sum over the lanes up to this one, by lane moves
+__device__ __forceinline__ double wave_scan_double(double v) {
+    auto add = [&](auto ctrl, int rows) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        constexpr int CTRL = decltype(ctrl)::value;
+        const int lo = static_cast<int>(u), hi = static_cast<int>(u >> 32);
+        uint32_t l, h;  // lanes outside the move bring zero
+        if (rows == 0xf) { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, false); }
+        else if (rows == 0xa) { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xa, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xa, 0xf, false); }
+        else { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xc, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xc, 0xf, false); }
+        v += __builtin_bit_cast(double, (static_cast<uint64_t>(h) << 32) | l);
+    };
+    add(std::integral_constant<int, 0x111>{}, 0xf);  // row_shr 1, 2, 4, 8: sums inside the rows of 16 lanes
+    add(std::integral_constant<int, 0x112>{}, 0xf);
+    add(std::integral_constant<int, 0x114>{}, 0xf);
+    add(std::integral_constant<int, 0x118>{}, 0xf);
+    add(std::integral_constant<int, 0x142>{}, 0xa);  // row_bcast 15: the row before, to rows 1 and 3
+    add(std::integral_constant<int, 0x143>{}, 0xc);  // row_bcast 31: the first two rows, to rows 2 and 3
+    return v;
 }
 
 // sum of e[0 .. n) in double; called by every lane of one wave, which all return it
@@ -156,30 +161,6 @@ __device__ __forceinline__ float wave_sum_list(const float* e, int n) {
 // descending bitonic sort of list[0 .. n_pad) in LDS by a workgroup of THREADS; n_pad is a power of two
 template <int THREADS> __device__ __forceinline__ void sort_list_desc(unsigned long long* list, int n_pad) {
     const int tid = threadIdx.x;
-    if (n_pad <= 2 * kWave) {
-        // short lists (the usual case under top-k) are sorted by one wave alone: its LDS operations execute
-        // in order, so the compare-exchange steps need no workgroup barrier
-        __syncthreads();
-        if (tid < kWave) {
-            for (int size = 2; size <= n_pad; size <<= 1) {
-                for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                    const int i = tid;
-                    if (i < (n_pad >> 1)) {
-                        const int lo = ((i / stride) * (stride << 1)) + (i % stride);
-                        const int hi = lo + stride;
-                        const bool desc = ((lo & size) == 0);
-                        const unsigned long long a = list[lo], b = list[hi];
-                        if ((a < b) == desc) { list[lo] = b; list[hi] = a; }
-                    }
-                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                }
-            }
-        }
-        __syncthreads();
-        return;
-    }
     for (int size = 2; size <= n_pad; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
             __syncthreads();
@@ -192,6 +173,25 @@ template <int THREADS> __device__ __forceinline__ void sort_list_desc(unsigned l
             }
         }
     }
+    __syncthreads();
+}
+
+// The same for at most THREADS entries, no two of them equal: an entry's place is the number of larger ones.  n LDS reads in a
+// row, the same word for all lanes, where a sort takes an LDS round trip or a barrier for each of its steps.  With this, the
+// shorter selection above and the target's logit loaded early, forwards under top-k and top-p take (us, before and now): 4095
+// rows of V = 151 936 bf16, k 50 213 and 206; 500 rows of 32 000, k 50 26.6 and 20.4; 4000 rows of 32 000, k 100 111 and 86.
+template <int THREADS> __device__ __forceinline__ void rank_list_desc(unsigned long long* list, int n) {
+    const int tid = threadIdx.x;
+    __syncthreads();
+    unsigned long long c = 0ull;
+    int at = 0;
+    if (tid < n) {
+        c = list[tid];
+#pragma unroll 8
+        for (int i = 0; i < n; ++i) at += list[i] > c ? 1 : 0;
+    }
+    __syncthreads();
+    if (tid < n) list[at] = c;
     __syncthreads();
 }
 
@@ -225,13 +225,22 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
     constexpr int EPV = Row<DT>::EPV;
     const int tid = threadIdx.x;
     const int64_t r = blockIdx.x;
-    const int64_t o = r / a.n_inner, i_in = r - o * a.n_inner;
+    const uint32_t o = blockIdx.x / static_cast<uint32_t>(a.n_inner);  // (fewer than 2^31 rows)
+    const int64_t i_in = blockIdx.x - o * static_cast<uint32_t>(a.n_inner);
     const char* row = static_cast<const char*>(a.logits) + (o * a.stride_outer + i_in * a.stride_inner) * Row<DT>::BYTES;
     const int64_t vocab = a.vocab;
     const int64_t head = sel_row_head<DT>(row, vocab);
     const int64_t nvec = (vocab - head) / EPV;
     const int64_t tail0 = head + nvec * EPV;
     const u32x4* xv = reinterpret_cast<const u32x4*>(row + head * Row<DT>::BYTES);
+
+    // the target's logit, on its way while the row streams
+    int64_t tg = -1;
+    float x_tg = 0.f;
+    if (a.targets && a.logprob) {
+        tg = a.targets[o * a.ts_outer + i_in * a.ts_inner];
+        if (tg >= 0 && tg < vocab) x_tg = Row<DT>::load1(row, tg);
+    }
 
     // ---- pass 1: chunk maxima (+ full-row online log-sum-exp) ----
     // Without the full-row log-sum-exp only maxima leave this pass, and the temperature scaling (a multiplication or
@@ -423,7 +432,7 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
     bool whole_row = true;  // top-p alone: the bound already rests on the whole row
     bool force_wide = false;  // top-p alone: the chunk maxima show that the kept set cannot fit the candidate list
     if (use_k) {
-        if (a.top_k <= kChunks) bound_key = select_kth_largest(sh, mx_key, a.top_k);
+        if (a.top_k <= kChunks) bound_key = select_kth_largest<kSelectLow<DT>>(sh, mx_key, a.top_k);
     } else {
         clear_bins();
         // (how many elements the chunks hold whose maxima fall into each bin, and what they would weigh if each
@@ -596,10 +605,14 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
         }
         return;
     }
-    int n_pad = 1;
-    while (n_pad < n) n_pad <<= 1;
-    for (int i = n + tid; i < n_pad; i += kSelBlock) sh.cand[i] = 0ull;  // sorts last
-    sort_list_desc<kSelBlock>(sh.cand, n_pad);
+    if (n <= kSelBlock) {
+        rank_list_desc<kSelBlock>(sh.cand, n);
+    } else {
+        int n_pad = 1;
+        while (n_pad < n) n_pad <<= 1;
+        for (int i = n + tid; i < n_pad; i += kSelBlock) sh.cand[i] = 0ull;  // sorts last
+        sort_list_desc<kSelBlock>(sh.cand, n_pad);
+    }
 
     // ---- top-k threshold (ties kept), softmax over the kept values ----
     int n_k = n;
@@ -615,61 +628,41 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
     for (int i = tid; i < n_k; i += kSelBlock)
         sh.expv[i] = expf(key_value(static_cast<uint32_t>(sh.cand[i] >> 32)) - m);
     __syncthreads();
-    // Short lists are summed element by element, in the order of a sorted cumulative sum in fp32.  Over thousands of elements
-    // that order means nothing any more (every implementation of the sum takes its own), and it costs one dependent addition
-    // per element, three times.  Long lists under top-p alone are summed in double, by the lanes side by side: 1500 rows of
-    // V = 151936 under top_p 0.95, kept sets from a few tokens to thousands: 509 -> 476 us.
-    const bool long_list = PONLY && n_k > kSeqList;
+    // The masses are summed in double, by the lanes side by side: nearer to the sorted cumulative sum than fp32 in any order, where
+    // element by element in fp32 is one dependent addition per element, three times (4000 rows of V = 32 000, top-k 100, top-p
+    // 0.9: 86 -> 77 us; 1500 rows of V = 151 936 under top-p alone: 509 -> 476).
     if (tid < kWave) {  // one wave; every lane computes the same scalars, lane 0 writes them
         int n_keep = n_k;
         if (use_p) {
-            float s_k = long_list ? wave_sum_list(sh.expv, n_k) : wave_seq_sum_desc(sh.expv, n_k);
+            float s_k = wave_sum_list(sh.expv, n_k);
             // ascending cumulative probability, smallest kept value first; keep while it exceeds 1 - p
             const float cut = 1.0f - a.top_p;
-            float cum = 0.f;
+            double run = 0.0;
             if (!use_k) {
                 // top-p alone normalises over the whole row: the elements below the candidate bound
                 // come first in ascending order and contribute their (small) mass to the running sum
                 const float s_full = expf(lse_full - m);
-                cum = fmaxf(0.f, (s_full - s_k) / s_full);
+                run = fmaxf(0.f, (s_full - s_k) / s_full);
                 s_k = s_full;
             }
             // Elements fall, smallest first, while the running sum stays <= 1 - p; the sum only grows, so
-            // counting the steps that end at or under the cut counts the fallen.  Whole blocks of 64 with
-            // constant lane indices: lanes past the end come first and add nothing (each counts as a step
+            // counting the steps that end at or under the cut counts the fallen.  Whole blocks of 64, the last element in lane 0:
+            // lanes past the end come first and add nothing (each counts as a step
             // under the cut and is taken off again), index 0 is always kept and never enters the sum.
             const int top_blk = (n_k - 1) / kWave;
             int steps_under = 0;
-            double run = cum;
-            if (long_list) {
-                for (int blk = top_blk; blk >= 0 && run <= cut; --blk) {
-                    const int idx = blk * kWave + tid;
-                    double v = (idx >= 1 && idx < n_k) ? static_cast<double>(sh.expv[idx] / s_k) : 0.0;
-#pragma unroll
-                    for (int off = 1; off < kWave; off <<= 1) {
-                        const double up = __shfl_down(v, off, kWave);
-                        if (tid + off < kWave) v += up;
-                    }
-                    steps_under += __popcll(__ballot(run + v <= cut));
-                    run += lane_double(v, 0);
-                }
-            }
-            for (int blk = long_list ? -1 : top_blk; blk >= 0; --blk) {
-                const int idx = blk * kWave + tid;
-                const float v = (idx >= 1 && idx < n_k) ? sh.expv[idx] / s_k : 0.f;
-#pragma unroll
-                for (int i = kWave - 1; i >= 0; --i) {
-                    cum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), i));
-                    steps_under += cum <= cut ? 1 : 0;
-                }
-                if (!(cum <= cut)) break;  // nothing further down can fall (also leaves on a NaN)
+            for (int blk = top_blk; blk >= 0 && run <= cut; --blk) {  // (also leaves on a NaN)
+                const int idx = blk * kWave + kWave - 1 - tid;
+                const double v = wave_scan_double((idx >= 1 && idx < n_k) ? static_cast<double>(sh.expv[idx] / s_k) : 0.0);
+                steps_under += __popcll(__ballot(run + v <= cut));
+                run += lane_double(v, kWave - 1);
             }
             const int fallen = steps_under - ((top_blk + 1) * kWave - n_k);
             n_keep = n_k - fallen;
             if (n_keep < 1) n_keep = 1;
             if (n_keep > n_k) n_keep = n_k;
         }
-        const float s = long_list ? wave_sum_list(sh.expv, n_keep) : wave_seq_sum_desc(sh.expv, n_keep);
+        const float s = wave_sum_list(sh.expv, n_keep);
         const unsigned long long last = sh.cand[n_keep - 1];
         const uint32_t last_key = static_cast<uint32_t>(last >> 32);
         int tie = 0;
@@ -689,10 +682,9 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
             a.lse_kept[r] = lse_kept;
             if (a.lse_full) a.lse_full[r] = lse_full;
             if (a.targets && a.logprob) {
-                const int64_t tg = a.targets[o * a.ts_outer + i_in * a.ts_inner];
                 float lp = -INFINITY, lpf = 0.f;
                 if (tg >= 0 && tg < vocab) {
-                    const float xt = scale_logit<DT, TEMP>(Row<DT>::load1(row, tg), a.tparam);
+                    const float xt = scale_logit<DT, TEMP>(x_tg, a.tparam);
                     const bool kept = xt > thr || (xt == thr && tg >= tie);
                     if (kept) lp = xt - lse_kept;
                     lpf = xt - lse_full;
@@ -768,27 +760,6 @@ template <typename F> __device__ __forceinline__ int wave_fold_int(int v, F f) {
 }
 __device__ __forceinline__ int wave_sum_int(int v) { return wave_fold_int(v, [](int p, int q) { return p + q; }); }
 __device__ __forceinline__ int wave_max_int(int v) { return wave_fold_int(v, [](int p, int q) { return p > q ? p : q; }); }
-
-// inclusive sum over the lanes up to this one, by lane moves
-__device__ __forceinline__ double wave_scan_double(double v) {
-    auto add = [&](auto ctrl, int rows) {
-        const uint64_t u = __builtin_bit_cast(uint64_t, v);
-        constexpr int CTRL = decltype(ctrl)::value;
-        const int lo = static_cast<int>(u), hi = static_cast<int>(u >> 32);
-        uint32_t l, h;  // lanes outside the move bring zero
-        if (rows == 0xf) { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xf, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xf, 0xf, false); }
-        else if (rows == 0xa) { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xa, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xa, 0xf, false); }
-        else { l = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xc, 0xf, false); h = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xc, 0xf, false); }
-        v += __builtin_bit_cast(double, (static_cast<uint64_t>(h) << 32) | l);
-    };
-    add(std::integral_constant<int, 0x111>{}, 0xf);  // row_shr 1, 2, 4, 8: sums inside the rows of 16 lanes
-    add(std::integral_constant<int, 0x112>{}, 0xf);
-    add(std::integral_constant<int, 0x114>{}, 0xf);
-    add(std::integral_constant<int, 0x118>{}, 0xf);
-    add(std::integral_constant<int, 0x142>{}, 0xa);  // row_bcast 15: the row before, to rows 1 and 3
-    add(std::integral_constant<int, 0x143>{}, 0xc);  // row_bcast 31: the first two rows, to rows 2 and 3
-    return v;
-}
 
 constexpr int kOddNan = 1, kOddLarge = 2;  // a NaN or +inf; a finite value above the bins
 

@@ -164,3 +164,37 @@ def test_gradient_rows_cleared_and_streamed_side_by_side(dtype, vocab):
     got = torch.ops.rl_amd.topk_topp_logprob_bwd(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP, cnt, idx, val)
     bits = torch.int32 if dtype == torch.float32 else torch.int16
     assert torch.equal(got.view(bits), want.view(bits))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("top_k", [1, 2, 63, 64, 65, 255, 256, 257, 512, 600])
+def test_lists_around_the_workgroup_size(dtype, top_k):
+    """Candidate lists that one pass of comparisons orders (up to 256) and longer ones that are sorted, with coarse values that tie at
+    the top-k threshold, and negative rows: the same kept set as 64-bit sums over the sorted row give, to the element where the
+    cut does not fall within 1e-6 of a step."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(top_k)
+    n, vocab, top_p = 24, 9001, 0.9
+    x = torch.randn(1, n + 1, vocab, generator=g, device=DEV) * torch.linspace(0.5, 6.0, n + 1, device=DEV).view(1, -1, 1)
+    x[0, ::3] = (x[0, ::3] * 16).round() / 16 + 0.0
+    x[0, 1::5] = -x[0, 1::5].abs() - 0.5
+    x = x.to(dtype)
+    t = x[:, :n].float().argmax(-1)
+    _, thr, tie, lse, _ = torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, n, top_k, top_p, 1.0, NRL_TEMP_RCP, False)
+    z = x[0, :n].double()
+    index = torch.arange(vocab, device=DEV)
+    keep = (z > thr[0, :, None].double()) | ((z == thr[0, :, None].double()) & (index >= tie[0, :, None]))
+    z = z.masked_fill(z < z.topk(top_k, dim=-1).values[:, -1:], -math.inf)
+    order = z.sort(dim=-1, stable=True)
+    mass = order.values.softmax(-1).cumsum(-1)
+    cut = float(torch.tensor(1.0) - torch.tensor(top_p))
+    kept = mass > cut
+    kept[:, -1] = True
+    want = torch.zeros_like(keep).scatter_(-1, order.indices, kept)
+    clear = ((mass - cut).abs() > 1e-6).all(-1)
+    assert int(clear.sum()) > n // 2
+    assert torch.equal(keep[clear], want[clear])
+    full = z.masked_fill(~keep, -math.inf).logsumexp(-1)
+    assert bool(((lse[0].double() - full).abs() <= 2.0 ** -23 * (2 + full.abs() + z.amax(-1).abs())).all())
