@@ -3,7 +3,7 @@
 // Rows belong to one group iff their prompt-token rows are exactly equal.  Launch 1 hashes every
 // prompt row (one workgroup per row).  Launch 2 finds, for every row, the first row with the same
 // content: candidates are pre-filtered by the 64-bit hash and then confirmed with a full
-// element-wise comparison, so a hash collision can never merge two different prompts.  Launch 3
+// element-wise comparison, so a hash collision can never merge two different prompts (small batches: all in one).  Launch 3
 // (one thread per row) accumulates the group statistics in ascending row order in fp32 and
 // evaluates the reference's formula (E[r^2] - E[r]^2 scaled by n/(n-1), NaN -> 0) unchanged, so
 // decisions such as std > 0 come out the same.
@@ -44,36 +44,48 @@ __global__ __launch_bounds__(kAdvBlock) void prompt_group_kernel(const int64_t* 
     const uint64_t hb = hashes[b];
     const int64_t* row = prompts + b * stride;
     int32_t rep = static_cast<int32_t>(b);
-    for (int64_t j = 0; j < b; ++j) {
-        if (hashes[j] != hb) continue;  // uniform across the workgroup
-        const int64_t* other = prompts + j * stride;
-        int differs = 0;
-        for (int64_t i = threadIdx.x; i < len; i += kAdvBlock) differs |= (row[i] != other[i]);
-        if (block_sum<int, kAdvWaves>(differs, sm_flag) == 0) { rep = static_cast<int32_t>(j); break; }
+    // Every wave looks at the same 64 hashes at a time, so the workgroup agrees on the candidates.  (One hash after the
+    // other, each read waited for, and the branch per row of group_row_stats, 64 tokens, all three launches: 64 rows 19.0 us,
+    // 256 48, 1024 191; now 9.0, 20.7, 67.)
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int64_t j0 = 0; j0 < b && rep == b; j0 += kWave) {
+        unsigned long long like = __ballot(j0 + lane < b && hashes[j0 + lane] == hb);
+        for (; like != 0; like &= like - 1) {
+            const int64_t j = j0 + __ffsll(like) - 1;
+            const int64_t* other = prompts + j * stride;
+            int differs = 0;
+            for (int64_t i = threadIdx.x; i < len; i += kAdvBlock) differs |= (row[i] != other[i]);
+            if (block_sum<int, kAdvWaves>(differs, sm_flag) == 0) { rep = static_cast<int32_t>(j); break; }
+        }
     }
     if (threadIdx.x == 0) group[b] = rep;
 }
 
-__global__ void group_stats_kernel(const int32_t* group, int64_t batch, const float* rewards, const float* valid,
-                                   const float* std_rewards, int loo, int normalize, float* baseline, float* stdv,
-                                   float* adv) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= batch) return;
-    const int32_t g = group[i];
-    const float* sr = std_rewards ? std_rewards : rewards;
+// A row's part of the statistics: group id, validity, reward, reward of the deviation.
+struct GroupRow {
+    int32_t group;
+    float valid, reward, sr;
+};
+
+// Row i of the group statistics: the group's rows in ascending order; `at(j)` gives row j.  Rows of other groups are read like
+// the group's own and selected away, so that the reads of several rows are in flight together (a branch per row had every
+// read waited for; figures at prompt_group_kernel).
+template <typename F>
+__device__ __forceinline__ void group_row_stats(int i, int batch, const F& at, int loo, int normalize, float* baseline, float* stdv, float* adv) {
+    const GroupRow own = at(i);
     float n_valid = 0.f, s1 = 0.f, s1s = 0.f, s2 = 0.f;
-    for (int64_t j = 0; j < batch; ++j) {
-        if (group[j] != g) continue;
-        const float v = valid[j];
-        n_valid += v;
-        if (loo && j == i) continue;  // (1 - I) row of the mixing matrix
-        s1 += rewards[j] * v;
-        s1s += sr[j] * v;
-        s2 += (sr[j] * sr[j]) * v;
+#pragma unroll 8
+    for (int j = 0; j < batch; ++j) {
+        const GroupRow q = at(j);
+        const bool same = q.group == own.group, add = same && !(loo && j == i);  // (1 - I) row of the mixing matrix
+        n_valid = same ? n_valid + q.valid : n_valid;
+        s1 = add ? s1 + q.reward * q.valid : s1;
+        s1s = add ? s1s + q.sr * q.valid : s1s;
+        s2 = add ? s2 + (q.sr * q.sr) * q.valid : s2;
     }
     float base, sd = 0.f;
     if (n_valid <= 1.f) {
-        base = rewards[i];
+        base = own.reward;
     } else {
         const float n = n_valid - static_cast<float>(loo);
         base = s1 / n;
@@ -85,10 +97,89 @@ __global__ void group_stats_kernel(const int32_t* group, int64_t batch, const fl
     baseline[i] = base;
     stdv[i] = sd;
     if (adv) {
-        float a = rewards[i] - base;
+        float a = own.reward - base;
         if (normalize && sd > 0.f) a = a / (sd + 1e-6f);
         adv[i] = a;
     }
+}
+
+__global__ void group_stats_kernel(const int32_t* group, int64_t batch, const float* rewards, const float* valid,
+                                   const float* std_rewards, int loo, int normalize, float* baseline, float* stdv,
+                                   float* adv) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= batch) return;
+    const float* sr = std_rewards ? std_rewards : rewards;
+    group_row_stats(static_cast<int>(i), static_cast<int>(batch), [&](int j) { return GroupRow{group[j], valid[j], rewards[j], sr[j]}; }, loo, normalize,
+                    baseline, stdv, adv);
+}
+
+// The three launches in one workgroup, for batches small enough: a wave hashes, then compares, a row at a time; hashes and
+// what the statistics read stay in LDS.  The same comparisons and the same sums in the same order.  Bound by latency, the
+// launches' and that of a wave's rows one after the other.  us, back to back in a graph, groups of 8, against three launches:
+// 8 rows of 64 tokens 4.0 and 6.6, 16 of 256 5.3 and 7.1, 32 of 256 7.9 and 8.0 (and the host launches once).  The limits are
+// where one workgroup stops winning: 32 rows of 512 10.9 and 8.3, 64 of 64 11.9 and 9.0, 8 of 1024 6.5 and 7.4, 16 9.7 and 7.8.
+constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / kWave;
+constexpr int64_t kSmallBatch = 32, kSmallLen = 256;
+
+__global__ __launch_bounds__(kSmallThreads) void group_small_kernel(const int64_t* prompts, int len, int64_t stride, int batch,
+                                                                    const float* rewards, const float* valid, const float* std_rewards,
+                                                                    int loo, int normalize, float* baseline, float* stdv, float* adv,
+                                                                    int32_t* group_out) {
+    constexpr int kLoads = 4;  // in flight per lane; past the end of a row its last token is read
+    __shared__ uint64_t hashes[kSmallBatch];
+    __shared__ GroupRow rows[kSmallBatch];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    if (threadIdx.x < batch) {
+        GroupRow& q = rows[threadIdx.x];
+        q.valid = valid[threadIdx.x];
+        q.reward = rewards[threadIdx.x];
+        q.sr = std_rewards ? std_rewards[threadIdx.x] : q.reward;
+    }
+    for (int b = wave; b < batch; b += kSmallWaves) {
+        const int64_t* row = prompts + b * stride;
+        uint64_t h = 0;
+        for (int i0 = lane; i0 - lane < len; i0 += kLoads * kWave) {
+            uint64_t x[kLoads];
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) x[u] = static_cast<uint64_t>(row[min(i0 + u * kWave, len - 1)]);
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                const int i = i0 + u * kWave;
+                h += i < len ? mix64(static_cast<uint64_t>(i) * 0x100000001b3ull + 1, x[u]) : 0;
+            }
+        }
+        h = wave_sum(h);
+        if (lane == 0) hashes[b] = h;
+    }
+    __syncthreads();
+    for (int b = wave; b < batch; b += kSmallWaves) {
+        const int64_t* row = prompts + b * stride;
+        const uint64_t hb = hashes[b];
+        int rep = b;
+        for (int j0 = 0; j0 < b && rep == b; j0 += kWave) {
+            unsigned long long like = __ballot(j0 + lane < b && hashes[j0 + lane] == hb);
+            for (; like != 0; like &= like - 1) {
+                const int j = j0 + __ffsll(like) - 1;
+                const int64_t* other = prompts + j * stride;
+                uint64_t differs = 0;
+                for (int i0 = lane; i0 - lane < len; i0 += kLoads * kWave) {
+#pragma unroll
+                    for (int u = 0; u < kLoads; ++u) {
+                        const int i = min(i0 + u * kWave, len - 1);
+                        differs |= static_cast<uint64_t>(row[i] ^ other[i]);
+                    }
+                }
+                if (__ballot(differs != 0) == 0) { rep = j; break; }
+            }
+        }
+        if (lane == 0) {
+            rows[b].group = rep;
+            if (group_out) group_out[b] = rep;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < batch)
+        group_row_stats(static_cast<int>(threadIdx.x), batch, [&](int j) { return rows[j]; }, loo, normalize, baseline, stdv, adv);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -230,6 +321,11 @@ extern "C" int nrl_group_baseline_std(const int64_t* prompts, int64_t batch, int
     uint64_t* hashes = static_cast<uint64_t*>(workspace);
     int32_t* group = group_out ? group_out : reinterpret_cast<int32_t*>(hashes + batch);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (batch <= kSmallBatch && prompt_len <= kSmallLen) {
+        group_small_kernel<<<dim3(1), dim3(kSmallThreads), 0, s>>>(prompts, static_cast<int>(prompt_len), prompt_stride, static_cast<int>(batch), rewards, valid,
+                                                                   std_rewards, leave_one_out, normalize, baseline_out, std_out, adv_out, group_out);
+        return check_launch("group_baseline_std");
+    }
     prompt_hash_kernel<<<dim3((unsigned)batch), dim3(kAdvBlock), 0, s>>>(prompts, prompt_len, prompt_stride, hashes);
     prompt_group_kernel<<<dim3((unsigned)batch), dim3(kAdvBlock), 0, s>>>(prompts, prompt_len, prompt_stride, hashes, group);
     group_stats_kernel<<<dim3((unsigned)((batch + 127) / 128)), dim3(128), 0, s>>>(

@@ -312,6 +312,38 @@ def test_groups_and_advantages_match_oracle_bit_exact_decisions(loo):
     torch.testing.assert_close(got_adv, want_adv, rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("batch,plen", [(1, 0), (2, 1), (17, 65), (32, 256), (32, 257), (33, 256), (65, 3), (130, 64), (257, 2)])
+@pytest.mark.parametrize("loo", [True, False])
+def test_group_statistics_around_the_one_workgroup_batches(batch, plen, loo):
+    """Both sides of the limits on rows and tokens, rows that do not fill a wave, equal prompts more than 64 rows apart.
+    Rewards are 0 or 1 and groups have up to 8 rows: sums are exact, the variance (at least 7 / 64 or 0) is off by two
+    roundings of numbers up to 1, so the deviation by 2^-23 / (7 / 64), with its own roundings under 2e-6."""
+    g = torch.Generator().manual_seed(batch * 31 + plen)
+    n_groups = (batch + 7) // 8
+    base = torch.randint(0, 3, (n_groups, plen), generator=g)
+    prompts = torch.cat([base] * 8)[:batch] if plen else torch.zeros(batch, 0, dtype=torch.long)
+    if plen > 4:
+        base[:, 4:] = base[0, 4:].clone()  # rows alike but for the first four tokens
+        prompts = torch.cat([base] * 8)[:batch]
+    rewards = (torch.rand(batch, generator=g) < 0.5).float()
+    valid = (torch.rand(batch, generator=g) < 0.9).float()
+    want_gid = OA.group_ids_by_prompt(prompts).tolist()
+    first = {}
+    for i, v in enumerate(want_gid):
+        first.setdefault(v, i)
+    strided = torch.zeros(batch, plen + 3, dtype=torch.long, device=DEV)
+    strided[:, :plen] = prompts.to(DEV)
+    gb, gs_, ga, gid = torch.ops.rl_amd.group_baseline_std(strided[:, :plen], rewards.to(DEV), valid.to(DEV), None, loo, True)
+    assert gid.cpu().tolist() == [first[v] for v in want_gid]
+    wb, ws = OA.baseline_and_std_per_prompt(prompts, rewards, valid, loo)
+    sizes = torch.bincount(torch.tensor(want_gid))
+    rtol = 2e-6 if int(sizes.max()) <= 8 else 1e-4  # tiny alphabets merge groups: variance at least 1 / size
+    torch.testing.assert_close(gb.cpu(), wb, rtol=2e-7, atol=0)
+    torch.testing.assert_close(gs_.cpu(), ws, rtol=rtol, atol=0)
+    a = rewards - gb.cpu()
+    torch.testing.assert_close(ga.cpu(), torch.where(gs_.cpu() > 0, a / (gs_.cpu() + 1e-6), a), rtol=3e-7, atol=0)
+
+
 def test_config1_end_to_end_small():
     """benchmark config 1 at reduced size: advantages -> logprobs -> loss -> dlogits, fp32 logits."""
     w = synthetic_grpo_batch(4, 4, 64, 2048, seed=1001)
