@@ -647,7 +647,7 @@ def bench_topk(args, torch, w):
         # forward left on record) without reading the logits again
         "algorithmic_bytes_per_token": 2 * row_bytes,
         "hbm_frac_end_to_end": 2 * row_bytes * tokens * args.steps / elapsed / 1e9 / HBM_PEAK_GBS,
-        "roofline": hbm_roofline("fill_zero_flat_kernel + topk_topp_stream_kernel (backward from the kept-set record: write only)", row_bytes * rows,
+        "roofline": hbm_roofline("fill_zero_rows_kernel + topk_topp_stream_kernel (backward from the kept-set record: write only)", row_bytes * rows,
                                  bwd["avg_ms"], "c4" if full else None),
         "roofline_fwd": hbm_roofline("topk_topp_fwd_kernel", row_bytes * w["mb_seqs"] * (w["seq_len"] - 1), fwd["avg_ms"],
                                      "c4_fwd" if full else None),
@@ -674,7 +674,7 @@ def bench_topk(args, torch, w):
     del mbs
     torch.cuda.empty_cache()
     # ---- flat rows: top-p alone over N(0, 1) logits (an early-training policy) -- every row's nucleus is far wider
-    # than the on-chip candidate list, so every row is finished by the radix descent of topk_topp_wide_kernel ----
+    # than an on-chip candidate list; nucleus_count_kernel counts the row's elements by value in one pass ----
     flat_rows = w["mb_seqs"] * w["seq_len"] if full else min(4096, w["mb_seqs"] * w["seq_len"])
     gen = torch.Generator(device=dev).manual_seed(4044)
     flat = torch.empty((1, flat_rows + 1, w["vocab"]), dtype=torch.bfloat16, device=dev).normal_(0.0, 1.0, generator=gen)
@@ -690,12 +690,11 @@ def bench_topk(args, torch, w):
     result["c4_flat"] = {
         "value": flat_rows * args.steps / f_elapsed, "unit": "tokens/s", "ms_per_step": f_elapsed / args.steps * 1e3,
         "rows": flat_rows, "us_per_row": f_ms * 1e3 / flat_rows,
-        "roofline": hbm_roofline("topk_topp_fwd_kernel + topk_topp_wide_kernel (every row wide)", row_bytes * flat_rows, f_ms,
+        "roofline": hbm_roofline("nucleus_count_kernel (every row wide)", row_bytes * flat_rows, f_ms,
                                  "c4_flat" if flat_rows == 65536 and w["vocab"] == 151936 else None),
-        "note": "forward only: top_p=%.2f alone on bf16 N(0,1) logits; the kept set of every row (~10^5 ids) exceeds the "
-                "4096-entry candidate list, so the forward marks the row and the wide kernel finds threshold, tie index and "
-                "kept log-sum-exp in three more passes over the row (two key digits + the tie search); algorithmic bytes = "
-                "one read of the row" % w["top_p"]}
+        "note": "forward only: top_p=%.2f alone on bf16 N(0,1) logits; the kept set of a row is ~10^5 ids: the elements of "
+                "every bf16 value are counted in LDS while the row streams by once, threshold and kept log-sum-exp come from "
+                "the counts, the tie index from a second read as far as it lies; algorithmic bytes = one read of the row" % w["top_p"]}
     del flat
     finish(result, args, torch, w, "topk", cpu_rows=256, gpu_rows=2048)
 
