@@ -16,10 +16,11 @@
 //          bf16) and folded into a running (max, sum-exp) per token column without any cross-lane
 //          traffic while the workgroup walks its vocabulary tiles; the target's logit is captured on the
 //          way.  Only [tokens] sized partials leave the chip.
-//   GRAD   backward: recomputed tile -> the logits' gradient G, g * (onehot - softmax), as bf16 in the layout of core T's
-//          fragments, which dH = G W and dW = G^T hidden both read, for one token chunk at a time.  The element at the
-//          target is the one large element of a row of G: what its rounding to bf16 loses (up to 2^-8 of it, coherent over
-//          the row) is kept in fp32 and added to dH with the target's row of W by its own kernel.
+//   GRAD   backward: recomputed tile -> the softmax part of the logits' gradient, G = -g * softmax, as bf16 in the layout of
+//          core T's fragments, which dH = G W and dW = G^T hidden both read, for one token chunk at a time.  The one-hot term
+//          of dH, g * W[target], is added in fp32 after the product, by the kernel that then puts the term into G for dW: it is
+//          the one large element of a row of G, and in the product its rounding to bf16 (up to 2^-8, coherent over the row)
+//          and its weight in every partial sum after it would be dH's largest error.
 //   STORE / ACCUM  plain fp32 C = or C += for dH and dW.
 // The vocabulary is walked in tiles while the token chunk bounds what is materialised:
 // chunk x V bf16 for G (5 GB at chunk 16384, V 151936) instead of N x V.
@@ -919,27 +920,15 @@ __global__ __launch_bounds__(kFinishTokens * kFinishLanes) void lmhead_fwd_finis
 }
 
 // ---------------------------------------------------------------------------------------------
-// backward: recompute a [chunk, V] slab of logits and emit G = g * (onehot - softmax) in both layouts
+// backward: recompute a [chunk, V] slab of logits and emit its part of G = -g * softmax
 // ---------------------------------------------------------------------------------------------
 struct LmGradArgs {
     GemmOperands op;         // a = hidden chunk [chunk, H], b = W [V, H]
-    const int64_t* targets;  // [chunk]
-    int64_t vocab_start;
     const float* lse;        // [chunk]
     const float* grad;       // [chunk] upstream d loss / d logprob
     uint16_t* g;             // fragment-major (tokens, ids), ids V .. ldg - 1 zero
     int64_t ldg;
-    float* resid;            // [chunk] what the rounding of the one-hot element to bf16 lost (written where the target is here)
 };
-
-// The element of G at the target: g + the softmax part, rounded to bf16 like every other; what that rounding loses (up to
-// 2^-8 of g, which would be the largest error of the whole row) goes to `resid` and into dH with the fp32 weight row.
-__device__ __forceinline__ uint32_t one_hot_element(float g, uint32_t softmax_bits, float& resid) {
-    const float whole = g + bf16_bits_to_f32(softmax_bits);
-    const uint32_t bits = f32_to_bf16_bits(whole);
-    resid = whole - bf16_bits_to_f32(bits);
-    return bits;
-}
 
 // XCD patch of the recomputing gradient kernel, 8 token tiles x 4 vocabulary tiles: 1.7 % faster than 4 x 8
 constexpr Patches kGradPatches{8, 4, 1};
@@ -948,7 +937,6 @@ template <class Core>
 __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
     constexpr int NI = Core::NI, NJ = Core::NJ, BM = Core::BM, BN = Core::BN;
     __shared__ __attribute__((aligned(1024))) unsigned char lds[Core::LDS_BYTES];
-    __shared__ int tgt_local[BM];
     __shared__ float lse_l[BM], g_l[BM];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
@@ -959,12 +947,10 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
     const int64_t row0 = bx * BM, col0 = by * BN;
     {
         const int64_t grow = row0 + tid;
-        int64_t t = -1;
         // rows past the chunk repeat its last row's operand: give them a log-sum-exp that keeps exp(x - lse)
         // finite, and a zero gradient
         float l = 128.f, g = 0.f;
-        if (grow < a.op.m) { t = a.targets[grow] - a.vocab_start; l = a.lse[grow]; g = a.grad[grow]; }
-        tgt_local[tid] = (t >= 0 && t < a.op.n && g != 0.f) ? static_cast<int>(t) : -1;
+        if (grow < a.op.m) { l = a.lse[grow]; g = a.grad[grow]; }
         lse_l[tid] = l * kLog2e;
         g_l[tid] = g;
     }
@@ -987,13 +973,12 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
             if (row_ok && col_ok && g_l[rl] != 0.f) {
                 const float x = round_bf16(acc[i][j][e]);
                 bits[u] = f32_to_bf16_bits(-fast_exp2(__builtin_fmaf(x, kLog2e, -lse_l[rl])) * g_l[rl]);
-                if (tgt_local[rl] == c) bits[u] = one_hot_element(g_l[rl], bits[u], a.resid[row0 + rl]);
             }
         }
         p01 = bits[0] | (bits[1] << 16);
         p23 = bits[2] | (bits[3] << 16);
     };
-    // The softmax part of the whole tile's gradients as bf16 pairs.  A group of 4 accumulator rows is the same for
+    // The whole tile's gradients as bf16 pairs.  A group of 4 accumulator rows is the same for
     // every j, so its per-token values are read from LDS once; columns past the vocabulary become zero by a select.
     auto grad_all = [&](uint32_t (&p01)[NI][NJ][4], uint32_t (&p23)[NI][NJ][4]) {
 #pragma unroll
@@ -1026,7 +1011,6 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
     if constexpr (Core::LDS_BYTES >= BM * BN * 2) {
         // G leaves through LDS so that every global store is a 16-byte piece of a 512-byte run: 2-byte writes; the 16-byte
         // chunk C of token row t sits at C ^ ((t >> 2) & 7).
-        static_assert(BM == GB_THREADS, "one thread per token row patches the one-hot term");
         constexpr int RV = BN / 8;  // 16-byte pieces per token row of the tile
         uint32_t p01[NI][NJ][4], p23[NI][NJ][4];
         grad_all(p01, p23);
@@ -1047,14 +1031,6 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
                             static_cast<uint16_t>(w[u >> 1] >> ((u & 1) * 16));
                     }
                 }
-        }
-        __syncthreads();
-        {   // the one-hot term: token `tid` adds its g at its target's column, if that column is in this tile
-            const int v = tgt_local[tid] - static_cast<int>(col0);
-            if (tgt_local[tid] >= 0 && v >= 0 && v < BN) {
-                uint16_t* cell = reinterpret_cast<uint16_t*>(lds + tid * (BN * 2) + (((v >> 3) ^ ((tid >> 2) & 7)) * 16) + (v & 7) * 2);
-                *cell = static_cast<uint16_t>(one_hot_element(g_l[tid], *cell, a.resid[row0 + tid]));
-            }
         }
         __syncthreads();
 #pragma unroll 4
@@ -1103,13 +1079,10 @@ struct LmGradKeptArgs {
     const int32_t* live;      // device count of live tokens
     int64_t live_from, rows;  // this chunk's live rows are [live_from, live_from + rows) clamped to *live
     int64_t vocab;
-    const int64_t* targets;   // the live rows' targets, log-sum-exps and upstream gradients
-    int64_t vocab_start;
-    const float* lse;
+    const float* lse;         // the live rows' log-sum-exps and upstream gradients
     const float* grad;
     uint16_t* g;              // as in LmGradArgs
     int64_t ldg;
-    float* resid;
 };
 
 constexpr int kKeptBlocks = 16;  // blocks of 16 ids that a wave of lmhead_grad_kept_kernel walks
@@ -1122,14 +1095,11 @@ __global__ __launch_bounds__(256) void lmhead_grad_kept_kernel(LmGradKeptArgs a)
     const int64_t row = static_cast<int64_t>(blockIdx.y) * 32 + (lane & 31), m_pad = (m + 63) / 64 * 64;
     if (static_cast<int64_t>(blockIdx.y) * 32 >= m_pad) return;
     int64_t src = 0;
-    int tgt = -1;
     float ls = 128.f * kLog2e, g = 0.f;  // rows past the live ones: a finite exponent and a zero gradient
     if (row < m) {
-        const int64_t t = a.targets[row] - a.vocab_start;
         ls = a.lse[row] * kLog2e;
         g = a.grad[row];
         src = a.row_map[row];
-        tgt = (t >= 0 && t < a.vocab && g != 0.f) ? static_cast<int>(t) : -1;
     }
     const bool live = g != 0.f;
     const unsigned char* from = a.logits + kept_block(src >> 5, 0, a.n_vb) + half * 512 + (src & 31) * 16;
@@ -1159,17 +1129,6 @@ __global__ __launch_bounds__(256) void lmhead_grad_kept_kernel(LmGradKeptArgs a)
             u32x4 out;
 #pragma unroll
             for (int q = 0; q < 4; ++q) out[q] = pack_bf16x2(sv[2 * q], sv[2 * q + 1]);
-            const int at = tgt < 0 ? -1 : tgt - static_cast<int>(c);
-            if (at >= 0 && at < 8) {  // the token's target is among these ids (one lane of the whole launch)
-                const int q = at >> 1, up = (at & 1) * 16;
-                uint32_t pair = q == 0 ? out.x : q == 1 ? out.y : q == 2 ? out.z : out.w;
-                const uint32_t one = one_hot_element(g, (pair >> up) & 0xffffu, a.resid[row]);
-                pair = (pair & (0xffff0000u >> up)) | (one << up);
-                if (q == 0) out.x = pair;
-                if (q == 1) out.y = pair;
-                if (q == 2) out.z = pair;
-                if (q == 3) out.w = pair;
-            }
             *reinterpret_cast<u32x4*>(to + (b + u) * 512) = out;
         }
     }
@@ -1295,19 +1254,25 @@ __global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, S
 }
 
 // dH of a chunk's live tokens: the partial products of its k splits added in order (SUM; otherwise the product is
-// already in place), plus resid_r * W[target_r, :] in fp32: what the rounding of the one-hot element of G to bf16 lost (zero
-// where the target lies outside the shard).  Row r is token row_map[r].  One workgroup per row.
+// already in place), plus the one-hot term g_r * W[target_r, :] in fp32, which is not in the product's G.  It goes into G here,
+// where the dH product is done with it and the dW product has not read it: one bf16 rounding of g + the softmax part.  Row r is
+// token row_map[r]; a target outside the shard adds nothing.  One workgroup per row.
 template <bool SUM>
 __global__ __launch_bounds__(256) void lmhead_finish_dh_kernel(float* dh, int64_t ld_dh, const float* parts, int n_splits,
                                                               int64_t split_stride, const int32_t* row_map, const int32_t* live,
-                                                              int64_t live_from, const float* resid, const int64_t* targets,
-                                                              int64_t vocab_start, int64_t vocab, const uint16_t* w, int64_t ldw, int64_t h) {
+                                                              int64_t live_from, const float* grad, const int64_t* targets,
+                                                              int64_t vocab_start, int64_t vocab, const uint16_t* w, int64_t ldw, int64_t h,
+                                                              uint16_t* g_frag, int64_t ldg) {
     const int64_t r = blockIdx.x;
     if (r >= static_cast<int64_t>(live[0]) - live_from) return;
-    const float g = resid[r];
+    const float g = grad[r];
     const int64_t t = targets[r] - vocab_start;
     const bool hot = g != 0.f && t >= 0 && t < vocab;
     if (!SUM && !hot) return;
+    if (hot && threadIdx.x == 0) {  // (a 16-byte unit of G belongs to one token)
+        uint16_t* cell = g_frag + frag_major(r, t, ldg / 16) + (t & 7);
+        *cell = static_cast<uint16_t>(f32_to_bf16_bits(g + bf16_bits_to_f32(*cell)));
+    }
     const uint16_t* wr = w + (hot ? t : 0) * ldw;
     float* out = dh + static_cast<int64_t>(row_map[r]) * ld_dh;
     for (int64_t c = threadIdx.x * 4; c < h; c += 256 * 4) {  // h is a multiple of 8, the partials are 16-byte aligned
@@ -1376,7 +1341,7 @@ __global__ __launch_bounds__(1024) void live_tokens_kernel(const float* grad, in
 __global__ __launch_bounds__(256) void gather_live_kernel(const uint16_t* hidden, int64_t ldh, int64_t h, const int64_t* targets,
                                                          const float* lse, const float* grad, const int32_t* idx,
                                                          const int32_t* count, int64_t n, uint16_t* hidden_c, int64_t* targets_c,
-                                                         float* lse_c, float* grad_c, float* resid_c) {
+                                                         float* lse_c, float* grad_c) {
     const int64_t i = blockIdx.x;
     const bool live = i < count[0];
     const int64_t src = live ? idx[i] : 0;
@@ -1388,7 +1353,6 @@ __global__ __launch_bounds__(256) void gather_live_kernel(const uint16_t* hidden
         targets_c[i] = live ? targets[src] : 0;
         lse_c[i] = live ? lse[src] : 0.f;
         grad_c[i] = live ? grad[src] : 0.f;
-        resid_c[i] = 0.f;
     }
 }
 
@@ -1664,7 +1628,7 @@ extern "C" int64_t nrl_lmhead_bwd_workspace_bytes(int64_t n_tokens, int64_t hidd
     const int64_t whole = n >= chunk ? dh_parts_bytes(chunk, hidden_size, vp) : 0, rest = dh_parts_bytes(n % chunk, hidden_size, vp);
     b += whole > rest ? whole : rest;
     b += n_pad * hidden_size * 2;     // hidden rows of the tokens that carry a gradient
-    b += n_pad * (8 + 4 + 4 + 4 + 4); // their targets, log-sum-exps, gradients, one-hot roundings and token indices
+    b += n_pad * (8 + 4 + 4 + 4);     // their targets, log-sum-exps, gradients and token indices
     return b + 4096;
 }
 
@@ -1705,7 +1669,6 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     int64_t* tgt_c = reinterpret_cast<int64_t*>(take(n_pad * 8));
     float* lse_c = reinterpret_cast<float*>(take(n_pad * 4));
     float* grad_c = reinterpret_cast<float*>(take(n_pad * 4));
-    float* resid_c = reinterpret_cast<float*>(take(n_pad * 4));
     int32_t* idx = reinterpret_cast<int32_t*>(take(n_pad * 4 + 256));
     int32_t* count = idx + n_pad;
     const uint16_t* hid = static_cast<const uint16_t*>(hidden);
@@ -1722,7 +1685,7 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
         // device; the launches are sized for all tokens and the workgroups beyond the live ones leave at once.
         live_tokens_kernel<<<dim3(1), dim3(1024), 0, s>>>(grad, n_tokens, idx, count);
         gather_live_kernel<<<dim3((unsigned)n_pad), dim3(256), 0, s>>>(hid, ldh, h, targets, lse, grad, idx, count, n_tokens, hid_c, tgt_c,
-                                                                        lse_c, grad_c, resid_c);
+                                                                        lse_c, grad_c);
         for (int64_t r = 0; r < n_tokens; r += 65535)  // dH rows of the other tokens are zero
             fill_zero_rows_kernel<<<dim3((unsigned)(n_tokens - r < 65535 ? n_tokens - r : 65535)), dim3(256), 0, s>>>(
                 dhidden_out + r * ld_dh, ld_dh, h);
@@ -1735,17 +1698,17 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
     for (int64_t t0 = 0; t0 < n_tokens; t0 += chunk) {
         const int64_t rows = n_tokens - t0 < chunk ? n_tokens - t0 : chunk;   // upper bound: the live rows of this chunk
         const int64_t rows_pad = round_up(rows, 64);
-        // G for this chunk of live tokens
+        // G for this chunk of live tokens (its one-hot term comes in behind the dH product)
         LmGradArgs ga;
         ga.op.a = hid_c + t0 * h; ga.op.b = w; ga.op.lda = h; ga.op.ldb = ldw; ga.op.m = rows; ga.op.n = vocab; ga.op.k = h;
         ga.op.live = count; ga.op.live_from = t0; ga.op.live_dim = 1;
-        ga.targets = tgt_c + t0; ga.vocab_start = vocab_start; ga.lse = lse_c + t0; ga.grad = grad_c + t0;
-        ga.g = g; ga.ldg = vp; ga.resid = resid_c + t0;
+        ga.lse = lse_c + t0; ga.grad = grad_c + t0;
+        ga.g = g; ga.ldg = vp;
         if (logits_kept) {
             LmGradKeptArgs ka;
             ka.logits = static_cast<const unsigned char*>(logits_kept); ka.n_vb = (vocab + 31) / 32; ka.row_map = idx + t0; ka.live = count;
-            ka.live_from = t0; ka.rows = rows; ka.vocab = vocab; ka.targets = ga.targets; ka.vocab_start = vocab_start;
-            ka.lse = ga.lse; ka.grad = ga.grad; ka.g = g; ka.ldg = vp; ka.resid = ga.resid;
+            ka.live_from = t0; ka.rows = rows; ka.vocab = vocab;
+            ka.lse = ga.lse; ka.grad = ga.grad; ka.g = g; ka.ldg = vp;
             lmhead_grad_kept_kernel<<<dim3((unsigned)((vp / 16 + 4 * kKeptBlocks - 1) / (4 * kKeptBlocks)), (unsigned)(rows_pad / 32)), dim3(256), 0, s>>>(ka);
         } else if (h % CoreB::BK == 0) launch_grad<CoreB>(ga, s);
         else launch_grad<CoreA>(ga, s);
@@ -1757,11 +1720,13 @@ extern "C" int nrl_lmhead_logprob_bwd(const void* hidden, int64_t n_tokens, int6
         if (dh_strips.splits > 1) {
             launch_gemm<false, 0>(dh, dh_strips, dh_parts, h, s);
             lmhead_finish_dh_kernel<true><<<dim3((unsigned)rows), dim3(256), 0, s>>>(
-                dhidden_out, ld_dh, dh_parts, dh_strips.splits, rows * h, idx + t0, count, t0, ga.resid, ga.targets, vocab_start, vocab, w, ldw, h);
+                dhidden_out, ld_dh, dh_parts, dh_strips.splits, rows * h, idx + t0, count, t0, ga.grad, tgt_c + t0, vocab_start, vocab, w, ldw, h,
+                g, vp);
         } else {
             launch_gemm<false, 0>(dh, dh_strips, dhidden_out, ld_dh, s, idx + t0);
             lmhead_finish_dh_kernel<false><<<dim3((unsigned)rows), dim3(256), 0, s>>>(
-                dhidden_out, ld_dh, nullptr, 1, 0, idx + t0, count, t0, ga.resid, ga.targets, vocab_start, vocab, w, ldw, h);
+                dhidden_out, ld_dh, nullptr, 1, 0, idx + t0, count, t0, ga.grad, tgt_c + t0, vocab_start, vocab, w, ldw, h,
+                g, vp);
         }
         // dW += G^T [V, rows] hidden [rows, H] (rows of both past the live ones, up to a multiple of 64, are zero)
         transpose_to_frag_kernel<<<dim3((unsigned)(h_pad / 256), (unsigned)(rows_pad / 64)), dim3(256), 0, s>>>(

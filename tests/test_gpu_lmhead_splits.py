@@ -58,7 +58,7 @@ def test_products_at_the_edges_of_tiles(n, h, v, keep):
 
 
 def test_products_of_a_shard_leave_other_ranks_targets_out():
-    """A rank that holds ids 100 .. 399: targets elsewhere have a softmax part but no one-hot element and no residual."""
+    """A rank that holds ids 100 .. 399: targets elsewhere have a softmax part but no one-hot term."""
     g = torch.Generator().manual_seed(9)
     n, h, v, first = 90, 64, 300, 100
     hid = torch.randn(n, h, generator=g).to(torch.bfloat16)
@@ -87,3 +87,26 @@ def test_no_live_token_gives_zero_gradients(n, h, v):
     _, lse, _ = _ops().lmhead_logprob_fwd(hid, w, tgt, 0, v)
     dh, dw = _ops().lmhead_logprob_bwd(hid, w, tgt, lse, torch.zeros(n, device=DEV), 0, v)
     assert bool((dh == 0).all()) and bool((dw == 0).all())
+
+
+@pytest.mark.parametrize("h", [64, 72])            # both gradient kernels that recompute logits
+@pytest.mark.parametrize("v", [4096, 65536])       # dH in one k range and in several
+def test_the_one_hot_term_of_dh_is_added_once(h, v):
+    """All logits are 0, so G is -g / V exactly (the bf16 nearest to exp(-log V) is the power of two), and dH = g (W[target] -
+    mean(W)).  The mean is below 1/2 next to a W[target] of 256 to 384: added to it once, the result is one rounding of 2^-16
+    away, besides the short sum's own, 2^-24 of the mean in each of its V / 16 steps.  Inside the running sum every step would
+    round at 256."""
+    g = torch.Generator().manual_seed(h + v)
+    n = 5
+    hid = torch.zeros(n, h, dtype=torch.bfloat16)
+    w = (torch.rand(v, h, generator=g) * 0.125).to(torch.bfloat16)
+    tgt = torch.arange(n) * 17
+    w[tgt] = 256 + 2 * torch.randint(0, 64, (n, h), generator=g).to(torch.bfloat16)
+    up = torch.tensor([1.0, -1.0, 1.0, 0.0, -1.0])
+    _, lse, kept = _ops().lmhead_logprob_fwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), 0, v, True)
+    mean = w.double().mean(0)
+    want = up.double().unsqueeze(-1) * (w[tgt].double() - mean)
+    bound = 2.0 ** -16 + v / 16 * 2.0 ** -24 * mean.max().item()
+    for k in (kept, None):
+        dh, _ = _ops().lmhead_logprob_bwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), lse, up.to(DEV), 0, v, k)
+        assert (dh.double().cpu() - want).abs().max().item() <= bound
