@@ -457,7 +457,8 @@ Tensor logsoftmax_rows(const Tensor& logits, int64_t n_inner) {
 }
 
 // Top-k distillation loss of fp32 logprobs [B, n, K], d loss / d student [B, n, K] and d loss / d h_all [B, n] (empty without
-// the correction).  The two gradients lie in one buffer, so that an upstream factor is one product.
+// the correction).  The two gradients lie in one buffer, so that an upstream factor is one product; one follows the other
+// directly, as what lay between them would take part in that product's own derivative.
 struct DistillOut {
     Tensor loss, both, d_s, d_h;
 };
@@ -468,8 +469,8 @@ struct DistillArgs {
     double log_inf;
 };
 DistillOut distill_views(const Tensor& both, at::IntArrayRef shape, bool correct) {
-    const int64_t b = shape[0], n = shape[1], ns = b * n * shape[2], h0 = (ns + 3) / 4 * 4;
-    return {Tensor(), both, both.narrow(0, 0, ns).view(shape), correct ? both.narrow(0, h0, b * n).view({b, n}) : both.narrow(0, 0, 0)};
+    const int64_t b = shape[0], n = shape[1], ns = b * n * shape[2];
+    return {Tensor(), both, both.narrow(0, 0, ns).view(shape), correct ? both.narrow(0, ns, b * n).view({b, n}) : both.narrow(0, 0, 0)};
 }
 DistillOut distill_topk_loss(const Tensor& student_in, const Tensor& teacher_in, const Tensor& h_in, const Tensor& token_mask_in, const Tensor& sample_mask_in,
                              const Tensor& toks_in, const DistillArgs& a) {
@@ -500,8 +501,7 @@ DistillOut distill_topk_loss(const Tensor& student_in, const Tensor& teacher_in,
     TORCH_CHECK_VALUE(!token_mask.defined() || (sample_mask.defined() && toks_in.defined()), "token_mask needs sample_mask and global_valid_toks");
     if (toks_in.defined()) toks = toks_in.reshape({-1}).slice(0, 0, 1).to(at::kFloat).contiguous();
     const c10::OptionalDeviceGuard guard(student.device());
-    const int64_t ns = b * n * k, h0 = (ns + 3) / 4 * 4;
-    DistillOut o = distill_views(f32({correct ? h0 + b * n : ns}, student), student.sizes(), correct);
+    DistillOut o = distill_views(f32({b * n * (correct ? k + 1 : k)}, student), student.sizes(), correct);
     o.loss = f32({}, student);
     const Tensor ws = workspace(nrl_distill_topk_loss_workspace_bytes(b, n), student);
     check(nrl_distill_topk_loss_fwd_bwd(ptr(student), ptr(teacher), ptr(h), ptr(token_mask), token_mask.defined() && b > 1 ? token_mask.stride(0) : n,

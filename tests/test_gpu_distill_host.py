@@ -48,6 +48,27 @@ def test_masks_counts_and_factors(kl, zero):
     torch.testing.assert_close(e, d * 0.25, rtol=2.0 ** -22, atol=0)   # one rounding of the factor's product each way
 
 
+@pytest.mark.parametrize("kl", ["reverse", "mixed"])
+@pytest.mark.parametrize("b,n,k", [(1, 5, 3), (1, 1, 1), (2, 3, 1), (3, 7, 5)])   # B * n * K off the multiples of four
+def test_nothing_but_the_two_gradients_takes_part_in_the_derivative_by_the_factor(kl, b, n, k):
+    from rl_amd.algorithms.loss import DistillationLossConfig, DistillationLossFn
+
+    g = torch.Generator(device=DEV).manual_seed(b * n * k)
+    student = torch.randn(b, n, k, generator=g, device=DEV).log_softmax(-1).requires_grad_(True)
+    h = -torch.rand(b, n, generator=g, device=DEV).requires_grad_(True)
+    teacher = torch.randn(b, n, k, generator=g, device=DEV).log_softmax(-1)
+    fn = DistillationLossFn(DistillationLossConfig(kl_type=kl, zero_outside_topk=True))
+    c = torch.tensor(3.0, device=DEV, requires_grad=True)
+    torch.cuda.synchronize()
+    stale = [torch.full((128,), float("nan"), device=DEV) for _ in range(64)]   # what the caching allocator hands out next
+    del stale
+    loss, _ = fn(student, teacher, h, {"input_ids": torch.zeros(b, n + 1)}, None, None)
+    d_s, d_h = torch.autograd.grad(loss * c, (student, h), create_graph=True)
+    (dc,) = torch.autograd.grad(d_s.sum() + d_h.sum(), c)
+    want = ((d_s.double().sum() + d_h.double().sum()) / 3.0).detach()
+    assert abs(dc.item() - want.item()) <= 2.0 ** -20 * (d_s.abs().sum() + d_h.abs().sum()).item()
+
+
 def test_the_gradient_follows_its_factor_under_create_graph():
     from rl_amd.algorithms.loss import DistillationLossConfig, DistillationLossFn
 
