@@ -457,8 +457,8 @@ Tensor logsoftmax_rows(const Tensor& logits, int64_t n_inner) {
 }
 
 // Top-k distillation loss of fp32 logprobs [B, n, K], d loss / d student [B, n, K] and d loss / d h_all [B, n] (empty without
-// the correction).  The two gradients lie in one buffer, so that an upstream factor is one product; one follows the other
-// directly, as what lay between them would take part in that product's own derivative.
+// the correction), in buffers of their own or, with `both`, in one, so that an upstream factor is one product; there one follows
+// the other directly, as what lay between them would take part in that product's own derivative.
 struct DistillOut {
     Tensor loss, both, d_s, d_h;
 };
@@ -473,7 +473,7 @@ DistillOut distill_views(const Tensor& both, at::IntArrayRef shape, bool correct
     return {Tensor(), both, both.narrow(0, 0, ns).view(shape), correct ? both.narrow(0, ns, b * n).view({b, n}) : both.narrow(0, 0, 0)};
 }
 DistillOut distill_topk_loss(const Tensor& student_in, const Tensor& teacher_in, const Tensor& h_in, const Tensor& token_mask_in, const Tensor& sample_mask_in,
-                             const Tensor& toks_in, const DistillArgs& a) {
+                             const Tensor& toks_in, const DistillArgs& a, bool both) {
     need_gpu(student_in, teacher_in, h_in, token_mask_in, sample_mask_in, toks_in);
     TORCH_CHECK_VALUE(student_in.dim() == 3 && student_in.sizes() == teacher_in.sizes(), "student / teacher logprobs must both be [B, n, K], got ",
                       student_in.sizes(), " and ", teacher_in.sizes());
@@ -501,7 +501,8 @@ DistillOut distill_topk_loss(const Tensor& student_in, const Tensor& teacher_in,
     TORCH_CHECK_VALUE(!token_mask.defined() || (sample_mask.defined() && toks_in.defined()), "token_mask needs sample_mask and global_valid_toks");
     if (toks_in.defined()) toks = toks_in.reshape({-1}).slice(0, 0, 1).to(at::kFloat).contiguous();
     const c10::OptionalDeviceGuard guard(student.device());
-    DistillOut o = distill_views(f32({b * n * (correct ? k + 1 : k)}, student), student.sizes(), correct);
+    DistillOut o = both ? distill_views(f32({b * n * (correct ? k + 1 : k)}, student), student.sizes(), correct)
+                        : DistillOut{Tensor(), Tensor(), f32({b, n, k}, student), correct ? f32({b, n}, student) : f32({0}, student)};
     o.loss = f32({}, student);
     const Tensor ws = workspace(nrl_distill_topk_loss_workspace_bytes(b, n), student);
     check(nrl_distill_topk_loss_fwd_bwd(ptr(student), ptr(teacher), ptr(h), ptr(token_mask), token_mask.defined() && b > 1 ? token_mask.stride(0) : n,
@@ -782,7 +783,7 @@ struct DistillLoss : torch::autograd::Function<DistillLoss> {
     static Tensor forward(AutogradContext* ctx, const Tensor& student, const Tensor& teacher, const OptTensor& h, const OptTensor& token_mask,
                           const OptTensor& sample_mask, const OptTensor& toks, const DistillArgs& a) {
         const auto plain = [](const OptTensor& t) { return t.has_value() ? t->detach() : Tensor(); };
-        const DistillOut o = distill_topk_loss(student.detach(), teacher.detach(), plain(h), plain(token_mask), plain(sample_mask), plain(toks), a);
+        const DistillOut o = distill_topk_loss(student.detach(), teacher.detach(), plain(h), plain(token_mask), plain(sample_mask), plain(toks), a, true);
         ctx->save_for_backward({o.both});
         ctx->saved_data["shape"] = student.sizes().vec();
         ctx->saved_data["h"] = h.has_value() && o.d_h.numel() > 0;
@@ -933,8 +934,8 @@ PYBIND11_MODULE(_host, m) {
     m.def("logsoftmax_rows", &logsoftmax_rows);
     m.def("distill_topk_loss", [](const Tensor& student, const Tensor& teacher, const OptTensor& h, const OptTensor& token_mask, const OptTensor& sample_mask,
                                   const OptTensor& toks, int64_t kl, double weight, bool zero_outside, double log_inf) {
-        const DistillOut o = distill_topk_loss(student, teacher, opt(h), opt(token_mask), opt(sample_mask), opt(toks), {kl, weight, zero_outside, log_inf});
-        return std::make_tuple(o.loss, o.d_s.clone(), o.d_h.clone());
+        const DistillOut o = distill_topk_loss(student, teacher, opt(h), opt(token_mask), opt(sample_mask), opt(toks), {kl, weight, zero_outside, log_inf}, false);
+        return std::make_tuple(o.loss, o.d_s, o.d_h);
     });
     // of logprobs on the GPU; masks and count in any dtype, anywhere: token_mask [B, >= n + 1], of which the columns 1 .. n count
     m.def("distill_loss", [](const Tensor& student_in, const Tensor& teacher, const OptTensor& h, const OptTensor& token_mask, const OptTensor& sample_mask,

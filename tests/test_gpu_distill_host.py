@@ -83,6 +83,20 @@ def test_the_gradient_follows_its_factor_under_create_graph():
     torch.testing.assert_close(dc, (d / 3.0).sum().detach())
 
 
+def test_the_operators_gradients_are_written_where_they_are_returned():
+    from rl_amd import ops  # noqa: F401
+
+    lp = torch.randn(2, 5, 4, device=DEV).log_softmax(-1)
+    h = -torch.rand(2, 5, device=DEV)
+    op = torch.ops.rl_amd.distill_topk_loss
+    op(lp, lp, h, None, None, None, 1, 0.5, True, -100.0)
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    loss, d_s, d_h = op(lp, lp, h, None, None, None, 1, 0.5, True, -100.0)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 4   # the loss, its two gradients, a workspace
+    assert d_s.shape == (2, 5, 4) and d_h.shape == (2, 5) and d_s.untyped_storage().data_ptr() != d_h.untyped_storage().data_ptr()
+    assert op(lp, lp, h, None, None, None, 0, 0.5, True, -100.0)[2].shape == (0,)
+
+
 def test_what_is_refused():
     logits, data = _case(2)
     with pytest.raises(RuntimeError):
