@@ -944,7 +944,9 @@ PYBIND11_MODULE(_host, m) {
         const Tensor student = to_f32(student_in, student_in);
         TORCH_CHECK(!toks.has_value() || toks->numel() == 1, "global_valid_toks must hold one value");
         const OptTensor mask = token_mask.has_value() ? OptTensor(token_mask->slice(1, 1).slice(1, 0, student.size(1))) : OptTensor();
-        return DistillLoss::apply(student, to_f32(teacher, student), on(h), on(mask), on(sample_mask), on(toks), DistillArgs{kl, weight, zero_outside, log_inf});
+        // (a count that asks for a gradient gets none and does not make the loss ask for one)
+        const OptTensor valid = toks.has_value() ? OptTensor(toks->detach()) : OptTensor();
+        return DistillLoss::apply(student, to_f32(teacher, student), on(h), on(mask), on(sample_mask), on(valid), DistillArgs{kl, weight, zero_outside, log_inf});
     });
     m.def("gather_entropy", [](const Tensor& logits, const Tensor& indices, int64_t n, bool entropy) {
         const variable_list o = GatherEntropy::apply(logits, indices, n, entropy);

@@ -83,6 +83,17 @@ def test_the_gradient_follows_its_factor_under_create_graph():
     torch.testing.assert_close(dc, (d / 3.0).sum().detach())
 
 
+@pytest.mark.parametrize("dev", ["cpu", DEV])
+def test_a_count_that_asks_for_a_gradient_does_not_make_the_loss_ask_for_one(dev):
+    from rl_amd.algorithms.loss import DistillationLossConfig, DistillationLossFn
+
+    lp = torch.randn(2, 5, 4, device=DEV).log_softmax(-1)
+    data = {"input_ids": torch.zeros(2, 6), "token_mask": torch.ones(2, 6, device=DEV), "sample_mask": torch.ones(2, device=DEV)}
+    fn = DistillationLossFn(DistillationLossConfig(kl_type="forward"))
+    loss, _ = fn(lp, lp, None, data, None, torch.tensor(10.0, device=dev, requires_grad=True))
+    assert not loss.requires_grad
+
+
 def test_the_operators_gradients_are_written_where_they_are_returned():
     from rl_amd import ops  # noqa: F401
 
