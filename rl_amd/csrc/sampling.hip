@@ -44,6 +44,7 @@ constexpr int kLooseHits = 768;  // top-p alone: more hit chunks than this under
 constexpr int kMassCopies = 8;  // copies of the histogram, by lane: most elements fall into the few lowest bins
 constexpr int kWideGrid = 2048;  // workgroups of the kernel that finishes the marked rows
 constexpr int32_t kTieUnresolved = -1;  // tie[] marker: the row's kept set did not fit the candidate list
+constexpr int32_t kTieNoCut = 0x7fffffff;  // tie[] marker: a bf16 row with +inf under top-p alone, of which nothing falls (its masses are NaN)
 constexpr int kSub = 8;                      // chunk maxima per thread
 constexpr int kChunks = kSelBlock * kSub;    // 2048
 constexpr int kCap = 4096;                   // candidate capacity (LDS); rows under a small top-k use kCapSmall
@@ -761,7 +762,7 @@ template <typename F> __device__ __forceinline__ int wave_fold_int(int v, F f) {
 __device__ __forceinline__ int wave_sum_int(int v) { return wave_fold_int(v, [](int p, int q) { return p + q; }); }
 __device__ __forceinline__ int wave_max_int(int v) { return wave_fold_int(v, [](int p, int q) { return p > q ? p : q; }); }
 
-constexpr int kOddNan = 1, kOddLarge = 2;  // a NaN or +inf; a finite value above the bins
+constexpr int kOddNan = 1, kOddLarge = 2, kOddInf = 4;  // a NaN; a finite value above the bins; +inf
 
 template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_count_kernel(SelArgs a) {
     using R = Row<NRL_BF16>;
@@ -826,7 +827,8 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
     auto count_one = [&](uint32_t t) {
         if (!(t & 0x6000u)) { atomicAdd(&sh.bin[(t & 0x1fffu) | ((t >> 2) & 0x2000u)], 1u); return; }
         const uint32_t bits = (t + kNucLow) & 0xffffu, mag = bits & 0x7fffu;
-        if (mag > 0x7f80u || bits == 0x7f80u) odd |= kOddNan;
+        if (mag > 0x7f80u) odd |= kOddNan;
+        else if (bits == 0x7f80u) odd |= kOddInf;
         else if (mag < static_cast<uint32_t>(kNucLow)) ++n_small;
         else if (!(bits & 0x8000u)) odd |= kOddLarge;
     };
@@ -955,17 +957,17 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
         }
     }
     if (pick < 0) {
-        // NaN and +inf make every result NaN, and so does a row of -inf; the wide kernel finishes the other rows, and finds
-        // the row's largest (scaled) logit in thr
+        // NaN and +inf make every result NaN, and so does a row of -inf; the gradient is NaN for +inf alone, 0 for the other two.
+        // The wide kernel finishes the other rows, and finds the row's largest (scaled) logit in thr
         const float row_max = bf16_bits_to_f32(max_bits);
-        const bool wide = !(odd & kOddNan) && row_max > -INFINITY;
+        const bool wide = !(odd & (kOddNan | kOddInf)) && row_max > -INFINITY;
         if (tid == 0) {
             const float nan = __builtin_nanf("");
             a.thr[r] = wide ? row_max : nan;
-            a.tie[r] = wide ? kTieUnresolved : 0;
+            a.tie[r] = wide ? kTieUnresolved : (odd & kOddNan) || !odd ? 0 : kTieNoCut;
             a.lse_kept[r] = nan;
             if (a.logprob) a.logprob[r] = nan;
-            if (a.lse_full) a.lse_full[r] = (odd & kOddNan) ? nan : -INFINITY;
+            if (a.lse_full) a.lse_full[r] = (odd & (kOddNan | kOddInf)) ? nan : -INFINITY;
             if (a.logprob_full) a.logprob_full[r] = nan;
             if (a.kept_n) a.kept_n[r] = -1;
         }
@@ -1606,7 +1608,7 @@ __device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_
 
     auto elem = [&](float x_raw, int64_t idx, bool& keep) -> float {
         const float x = scale_logit<DT, TEMP>(x_raw, a.tparam);
-        keep = x > thr || (x == thr && idx >= tie);
+        keep = x > thr || (x == thr && idx >= tie) || tie == kTieNoCut;
         if (MODE == 1) return keep ? x : -INFINITY;
         if (!keep) return 0.f;
         float d = ((idx == tg ? 1.f : 0.f) - fast_exp2((x - lse) * kLog2e)) * g;

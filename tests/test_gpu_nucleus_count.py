@@ -198,3 +198,31 @@ def test_lists_around_the_workgroup_size(dtype, top_k):
     assert torch.equal(keep[clear], want[clear])
     full = z.masked_fill(~keep, -math.inf).logsumexp(-1)
     assert bool(((lse[0].double() - full).abs() <= 2.0 ** -23 * (2 + full.abs() + z.amax(-1).abs())).all())
+
+
+def test_a_row_with_plus_inf_has_a_nan_gradient_and_is_not_filtered():
+    """Softmax makes such a row NaN, no NaN mass is under the cut, so nothing falls: the gradient says that the row has diverged.
+    The rows beside it are those of a batch without it."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(2)
+    for vocab in (9, 4099, 70000):
+        x = (torch.randn(1, 6, vocab, generator=g, device=DEV) * 3).to(torch.bfloat16)
+        plain = x.clone()
+        x[0, 1, 5] = math.inf
+        x[0, 3, vocab - 1] = math.inf
+        x[0, 3, 2] = -math.inf
+        x[0, 4, :] = -math.inf
+        t = torch.full((1, 5), 7, device=DEV)
+        up = torch.tensor([[1.0, 0.5, -1.0, math.nan, 1.0]], device=DEV)
+        op, back = torch.ops.rl_amd.topk_topp_logprob_fwd_rec, torch.ops.rl_amd.topk_topp_logprob_bwd
+        lp, thr, tie, lse, _, cnt, idx, val = op(x, t, 5, 0, 0.9, 1.0, NRL_TEMP_RCP, False, 64)
+        assert lp.isnan().tolist() == [[False, True, False, True, True]] and lse.isnan().tolist() == lp.isnan().tolist()
+        for rec in ((), (cnt, idx, val)):
+            d = back(x, t, thr, tie, lse, up, 5, 1.0, NRL_TEMP_RCP, *rec)
+            assert bool(d[0, (1, 3)].isnan().all()) and not bool(d[0, (0, 2, 4, 5)].isnan().any()) and not bool(d[0, 4].any())
+        _, thr0, tie0, lse0, _ = torch.ops.rl_amd.topk_topp_logprob_fwd(plain, t, 5, 0, 0.9, 1.0, NRL_TEMP_RCP, False)
+        assert torch.equal(d[0, ::2][:2], back(plain, t, thr0, tie0, lse0, up, 5, 1.0, NRL_TEMP_RCP)[0, ::2][:2])
+        f, keep = torch.ops.rl_amd.topk_topp_filter(x[:, :5], thr, tie, 1.0, NRL_TEMP_RCP)
+        assert torch.equal(f[0, (1, 3)], x[0, (1, 3)]) and bool(keep[0, (1, 3)].all())
