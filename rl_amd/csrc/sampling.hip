@@ -1550,10 +1550,10 @@ struct SelBwdArgs {
 // The number of kept entries on record for gradient row (o, i), or -1: the row is streamed from the logits.  `g` becomes its
 // upstream gradient, 0 for rows that have none (those are zero whatever the record says).
 __device__ __forceinline__ int topk_topp_on_record(const SelBwdArgs& a, int64_t o, int64_t i, float& g) {
-    g = i < a.n_inner ? a.grad[o * a.gs_outer + i * a.gs_inner] : 0.f;
-    if (g == 0.f) return 0;
-    const int n = a.kept_n[o * a.n_inner + i];
-    return n > a.kept_cap ? -1 : n;  // (above the capacity: not a count the forward writes)
+    const bool real = i < a.n_inner;
+    const int n = real ? a.kept_n[o * a.n_inner + i] : 0;  // (on its way together with the gradient)
+    g = real ? a.grad[o * a.gs_outer + i * a.gs_inner] : 0.f;
+    return g == 0.f ? 0 : n > a.kept_cap ? -1 : n;  // (above the capacity: not a count the forward writes)
 }
 
 // MODE 0: gradient, MODE 1: filtered logits (-inf outside the kept set) + keep mask
@@ -1671,35 +1671,79 @@ __device__ __forceinline__ void topk_topp_stream_row(const SelBwdArgs& a, int64_
     }
 }
 
-// Zero fill of the rows of a contiguous gradient that are not streamed from the logits, by one workgroup per compute unit in
-// 256 KiB spans: 6.0 TB/s where nothing is streamed, as a memset, where one workgroup per row reaches 5.5.  A 16-byte unit that a
-// streamed row shares with its neighbour is cleared too; the row is written later.  (1500 rows of V = 151 936, half of them
-// streamed: 57 us when every row was cleared, 29 now.)
+// Zero fill of a contiguous gradient by one workgroup per compute unit in 256 KiB spans, 6.0 TB/s, as a memset, where one
+// workgroup per row reaches 5.5.  Rows that are streamed from the logits are left out where that pays: a workgroup reads which
+// they are for all its spans at once, then clears what lies between them, neighbouring rows as one run (the two loads
+// a row waited for in turn before its stores cost more than the stores of a short row: 4096 rows of V = 1024 bf16, all on record,
+// 12 -> 70 us for the whole backward).  A 16-byte unit that a streamed row shares with its neighbour is cleared too; the row is
+// written later.  1500 rows of V = 151 936, half of them streamed: 57 us when every row is cleared, 17 so.
+// Everything is cleared where the flags take longer than what they can save: rows under 8 KiB, buffers of about one span per
+// workgroup (4096 rows of V = 8192 on record: 10.4 and 13.0), and records of less than kMixedRecord entries.
 constexpr int kFillGrid = 256;
-constexpr int64_t kFillSpan = 256 * 1024;
-template <int DT> __global__ __launch_bounds__(256) void fill_zero_rows_kernel(SelBwdArgs a, int64_t total_bytes) {
+constexpr int64_t kFillSpan = 256 * 1024, kFillShortRow = 8 * 1024, kFillSmall = kFillGrid * kFillSpan * 3 / 2;
+// A forward under top-k leaves a record with room for the k: its rows are on record but for those with ties, and flags for the
+// fill (4096 rows of V = 32 000: 32.7 us without, 34.5 with them) or several workgroups per row are for nothing.  Top-p alone
+// leaves room for this many; nearly flat rows do not fit.
+constexpr int kMixedRecord = 128;
+constexpr int kFillFlags = 1024, kFillRound = kFillFlags / 3;
+template <int DT> __global__ __launch_bounds__(256) void fill_zero_rows_kernel(SelBwdArgs a, int64_t total_bytes, double row_inverse) {
+    __shared__ uint8_t clear[kFillFlags];
+    __shared__ uint32_t first_row[kFillRound];  // of a span
     const u32x4 z = {0u, 0u, 0u, 0u};
     char* out = static_cast<char*>(a.out);
+    auto clear_run = [&](int64_t b0, int64_t b1) {
+        const int64_t v0 = b0 / 16, v1 = b1 / 16;  // whole units, from the one that holds the run's first byte
+        const int n = static_cast<int>(v1 - v0);
+        u32x4* zv = reinterpret_cast<u32x4*>(out) + v0;
+        for (int v = threadIdx.x; v < n; v += 256) zv[v] = z;
+        // the run's last bytes: the unit's other bytes are the next row's, or past the buffer's end
+        const int64_t b = (v1 * 16 > b0 ? v1 * 16 : b0) + static_cast<int64_t>(threadIdx.x) * Row<DT>::BYTES;
+        if (b < b1) Row<DT>::store1(out, b / Row<DT>::BYTES, 0.f);
+    };
     const int64_t row_bytes = a.vocab * Row<DT>::BYTES;
-    for (int64_t s0 = static_cast<int64_t>(blockIdx.x) * kFillSpan; s0 < total_bytes; s0 += static_cast<int64_t>(gridDim.x) * kFillSpan) {
-        const int64_t s1 = s0 + kFillSpan < total_bytes ? s0 + kFillSpan : total_bytes;
-        for (int64_t r = s0 / row_bytes; r * row_bytes < s1; ++r) {
-            const int64_t o = r / a.d_n_inner;
+    const auto span_end = [&](int64_t s0) { return s0 + kFillSpan < total_bytes ? s0 + kFillSpan : total_bytes; };
+    if (row_bytes < kFillShortRow || total_bytes <= kFillSmall || a.kept_cap < kMixedRecord) {
+        for (int64_t s0 = blockIdx.x * kFillSpan; s0 < total_bytes; s0 += gridDim.x * kFillSpan) clear_run(s0, span_end(s0));
+        return;
+    }
+    const uint32_t per = static_cast<uint32_t>(kFillSpan) / static_cast<uint32_t>(row_bytes < kFillSpan ? row_bytes : kFillSpan + 1) + 2;  // most rows that a span touches
+    const uint32_t round = kFillFlags / per;                                                                                         // spans at a time
+    for (int64_t base = blockIdx.x * kFillSpan; base < total_bytes; base += round * gridDim.x * kFillSpan) {
+        for (uint32_t i = threadIdx.x; i < round * per; i += 256) {
+            const uint32_t k = i / per, j = i - k * per;
+            const int64_t s0 = base + k * gridDim.x * kFillSpan;
+            if (s0 >= total_bytes) break;
+            int64_t r = static_cast<int64_t>(static_cast<double>(s0) * row_inverse);  // s0 / row_bytes, or one off
+            const int64_t rest = s0 - r * row_bytes;
+            r += rest < 0 ? -1 : rest >= row_bytes ? 1 : 0;
+            if (j == 0) first_row[k] = static_cast<uint32_t>(r);
+            r += j;
+            if (r * row_bytes >= span_end(s0)) continue;
+            const uint32_t o = static_cast<uint32_t>(r) / static_cast<uint32_t>(a.d_n_inner);  // (fewer than 2^31 rows)
             float g;
-            if (topk_topp_on_record(a, o, r - o * a.d_n_inner, g) < 0) continue;
-            const int64_t b0 = r * row_bytes > s0 ? r * row_bytes : s0, b1 = (r + 1) * row_bytes < s1 ? (r + 1) * row_bytes : s1;
-            const int64_t v1 = b1 / 16;  // whole units, from the one that holds the row's first byte
-            for (int64_t v = b0 / 16 + threadIdx.x; v < v1; v += 256) reinterpret_cast<u32x4*>(out)[v] = z;
-            // the row's last bytes: the unit's other bytes are the next row's, or past the buffer's end
-            const int64_t b = (v1 * 16 > b0 ? v1 * 16 : b0) + static_cast<int64_t>(threadIdx.x) * Row<DT>::BYTES;
-            if (b < b1) Row<DT>::store1(out, b / Row<DT>::BYTES, 0.f);
+            clear[i] = topk_topp_on_record(a, o, r - o * a.d_n_inner, g) >= 0;
         }
+        __syncthreads();
+        for (uint32_t k = 0; k < round; ++k) {
+            const int64_t s0 = base + k * gridDim.x * kFillSpan, s1 = span_end(s0);
+            if (s0 >= total_bytes) break;
+            const uint8_t* flag = clear + k * per;
+            int64_t b0 = -1, b = __builtin_amdgcn_readfirstlane(first_row[k]) * row_bytes;  // a run's first byte; row by row
+            for (; b < s1; b += row_bytes, ++flag) {
+                const bool yes = __builtin_amdgcn_readfirstlane(*flag);
+                if (yes && b0 < 0) b0 = b > s0 ? b : s0;
+                if (!yes && b0 >= 0) { clear_run(b0, b); b0 = -1; }
+            }
+            if (b0 >= 0) clear_run(b0, s1);
+        }
+        __syncthreads();
     }
 }
 
 // One workgroup per row, or several for few rows (a fixed set of 512 workgroups walking the rows, which fills memory
 // 10 % faster when it does nothing else, measured no gain here: with few workgroups per compute unit the record staging of a
-// row is exposed).
+// row is exposed; workgroups that take a part of each of three rows made an uneven round: 1500 rows of V = 151 936, half of them
+// streamed, 157 -> 193 us).
 template <int DT, int TEMP, int MODE>
 __global__ __launch_bounds__(kSelBlock) void topk_topp_stream_kernel(SelBwdArgs a) {
     const uint32_t r = blockIdx.x / static_cast<uint32_t>(a.parts);
@@ -1836,12 +1880,14 @@ extern "C" int nrl_topk_topp_logprob_bwd(const nrl_rows* rows, const float* thr,
     }
     if (a.prefilled) {
         const int64_t total = n * rows->vocab * elt;
-        if (rows->dtype == NRL_F32) fill_zero_rows_kernel<NRL_F32><<<dim3(kFillGrid), dim3(256), 0, s>>>(a, total);
-        else fill_zero_rows_kernel<NRL_BF16><<<dim3(kFillGrid), dim3(256), 0, s>>>(a, total);  // (zeros of two bytes, either type)
+        const double inverse = 1.0 / static_cast<double>(rows->vocab * elt);
+        if (rows->dtype == NRL_F32) fill_zero_rows_kernel<NRL_F32><<<dim3(kFillGrid), dim3(256), 0, s>>>(a, total, inverse);
+        else fill_zero_rows_kernel<NRL_BF16><<<dim3(kFillGrid), dim3(256), 0, s>>>(a, total, inverse);  // (zeros of two bytes, either type)
     }
-    // Parts of at least 32 KiB, as long as the rows alone are too few to keep the chip busy to the end: 1500 rows of V = 151 936,
-    // half of them streamed, 126 -> 110 us; 4096 rows that are all on record only pay for the workgroups (two a row: 11 -> 14).
-    const int64_t most = rows->vocab * elt / 32768;
+    // Parts of at least 32 KiB, as long as the rows alone are too few to keep the chip busy to the end.  1500 rows of V = 151 936 in
+    // 1, 2, 3 and 4 parts: half of them streamed 154, 154, 149 and 146 us (medians 176, 164, 172, 157); all on record 5.6, 7.0, 8.0
+    // and 10.1, so one part where that is to be expected.
+    const int64_t most = a.prefilled && a.kept_cap < kMixedRecord ? 1 : rows->vocab * elt / 32768;
     a.parts = static_cast<int>(6144 / n < most ? 6144 / n : most);
     if (a.parts < 1) a.parts = 1;
     NRL_SEL_DISPATCH(rows->dtype, tc, topk_topp_stream_kernel<DT, TEMP, 0><<<dim3((unsigned)(n * a.parts)), dim3(kSelBlock), 0, s>>>(a));

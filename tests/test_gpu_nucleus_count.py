@@ -226,3 +226,62 @@ def test_a_row_with_plus_inf_has_a_nan_gradient_and_is_not_filtered():
         assert torch.equal(d[0, ::2][:2], back(plain, t, thr0, tie0, lse0, up, 5, 1.0, NRL_TEMP_RCP)[0, ::2][:2])
         f, keep = torch.ops.rl_amd.topk_topp_filter(x[:, :5], thr, tie, 1.0, NRL_TEMP_RCP)
         assert torch.equal(f[0, (1, 3)], x[0, (1, 3)]) and bool(keep[0, (1, 3)].all())
+
+
+# (rows, vocabulary): rows of 8 KiB, of several to a 256 KiB span and of several spans, ends off the 16-byte grid; buffers of more
+# than a span and a half for each of 256 workgroups, so that rows to be streamed are left out of the fill
+@pytest.mark.parametrize("dtype,rows,vocab", [(torch.bfloat16, 13000, 4096), (torch.float32, 9001, 3001), (torch.bfloat16, 2600, 20003),
+                                              (torch.float32, 1300, 32000), (torch.bfloat16, 300, 200001), (torch.float32, 150, 262144)])
+@pytest.mark.parametrize("capacity", [64, 128])
+def test_large_gradients_cleared_around_streamed_rows(dtype, rows, vocab, capacity):
+    """The same bits as streaming every row, with runs of rows on record, streamed rows and rows without a gradient of random lengths."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    n = rows - 1
+    flat = torch.rand(rows, generator=g, device=DEV).view(-1, 1).expand(rows, 1)
+    flat = torch.where(torch.arange(rows, device=DEV).view(-1, 1) % 97 < 40, flat.round(), (flat > 0.9).float())   # singles, and long runs
+    x = torch.empty((1, rows, vocab), dtype=dtype, device=DEV).normal_(0, 1, generator=g)
+    x.mul_(torch.where(flat > 0.5, 0.3, 7.0).view(1, rows, 1).to(dtype))
+    t = torch.randint(0, vocab, (1, n), generator=g, device=DEV)
+    up = torch.randn(1, n, generator=g, device=DEV)
+    up[torch.rand(1, n, generator=g, device=DEV) < 0.1] = 0.0
+    _, thr, tie, lse, _, cnt, idx, val = torch.ops.rl_amd.topk_topp_logprob_fwd_rec(x, t, n, 0, 0.9, 1.0, NRL_TEMP_RCP, False, capacity)
+    assert int((cnt < 0).sum()) > n // 8 and int((cnt >= 0).sum()) > n // 8
+    back = torch.ops.rl_amd.topk_topp_logprob_bwd
+    bits = torch.int32 if dtype == torch.float32 else torch.int16
+    want = back(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP)
+    assert torch.equal(back(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP, cnt, idx, val).view(bits), want.view(bits))
+
+
+def test_short_rows_on_record_cost_a_fill_and_their_entries():
+    """4096 rows of 1024 ids: clearing 8 MiB takes a few microseconds and the entries about as much again; a fill that waits for
+    every row's flags takes fifteen times the clearing."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n, vocab = 4096, 1024
+    x = torch.empty((1, n + 1, vocab), dtype=torch.bfloat16, device=DEV).normal_(0, 3, generator=g)
+    t = torch.randint(0, vocab, (1, n), generator=g, device=DEV)
+    up = torch.randn(1, n, generator=g, device=DEV)
+    lp, thr, tie, lse, _, *rec = torch.ops.rl_amd.topk_topp_logprob_fwd_rec(x, t, n, 50, 0.95, 1.0, NRL_TEMP_RCP, False, 128)
+    assert bool((rec[0] >= 0).all())
+    out = torch.empty_like(x)
+
+    def shortest(f):
+        times = []
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                f()
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    shortest(lambda: out.zero_())
+    backward = shortest(lambda: torch.ops.rl_amd.topk_topp_logprob_bwd(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP, *rec))
+    assert backward < 8 * shortest(lambda: out.zero_())
