@@ -709,12 +709,14 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
 // larger value, is left to the wide kernel.  Larger negative values weigh nothing next to any value of the bins.
 // Counts are integers and every sum runs in a fixed order, so a row comes out the same every time.
 //
-// What bounds it: the LDS atomics of the first pass, about 15 cycles per 64 elements and compute unit, where the row
-// itself would arrive in 11; then the latency of the steps between two passes, which two workgroups of 1024 threads per
+// What bounds it: the LDS atomics of the first pass, about 15 cycles per 64 elements and compute unit where these differ (lanes
+// that add to one word take turns: see the common value), where the row itself would arrive in 11; then the latency of the steps between two passes, which two workgroups of 1024 threads per
 // compute unit cover for each other (workgroups of 512, of which the bins admit two as well: 195 us).  With a kept-set
 // record, top_p 0.95, standard deviations 2 - 6, against candidate lists, a sort and the radix descent of the wide kernel:
 // 1499 rows of V = 151 936 145 us (62 to read the rows) and 726; 180 rows of V = 205 350 47 and 470; 4000 rows of 32 000
-// with a temperature 158 and 408; 800 rows of 9001 37 and 185.
+// with a temperature 158 and 408; 800 rows of 9001 37 and 185.  Rows with a common value, 1499 of V = 151 936, against the same
+// two and against counting every element in LDS: 99 % of the ids masked with -1e9 148, 216 and 795; 80 % 245, 713 and 650; one
+// value 139, 774 and 961; two values of a half each 440, 603 and 688; ordinary rows take 1 - 2 % longer for the look at a sample.
 // ---------------------------------------------------------------------------------------------
 constexpr int kNucThreads = 1024, kNucWaves = kNucThreads / kWave;
 constexpr int kNucLow = 0x3000;                     // bf16 bits of 2^-31, the smallest magnitude with a bin of its own
@@ -723,6 +725,7 @@ constexpr int kNucBins = 2 * kNucSide;
 constexpr int kNucChunks = kNucBins / kWave;        // the bins in ascending order of the value, a wave's lanes at a time
 constexpr int kNucList = 4096;                      // entries of the list a small kept set is collected in (over the bins)
 constexpr int kNucLoads = 4;                        // 16-byte loads in flight per thread
+constexpr int kNucCommon = 16;                      // of 64 elements: a value that is counted in registers
 
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 typedef short i16x2 __attribute__((ext_vector_type(2)));
@@ -812,11 +815,23 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
         if (tg >= 0 && tg < vocab) x_tg = R::load1(row, tg);
     }
 
+    // and 64 elements from all over the row: lanes that see one value add to one word of LDS, one after the other, so a value of
+    // kNucCommon of these elements (of three elements' values the most frequent one) is counted in registers
+    const uint32_t sample = f32_to_bf16_bits(load_scaled((static_cast<uint64_t>(lane) * static_cast<uint64_t>(vocab)) >> 6));
+
     // ---- count the elements of every value ----
 #pragma unroll
     for (int i = tid; i < kNucBins / 4; i += kNucThreads) reinterpret_cast<u32x4*>(sh.bin)[i] = u32x4{0u, 0u, 0u, 0u};
     if (tid == 0) { sh.n_small = 0; sh.odd = 0; sh.n_list = 0; sh.n_hit = 0; }
     __syncthreads();
+    uint32_t common = 0u;
+    int most = 0;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+        const uint32_t v = __builtin_amdgcn_readlane(sample, 21 * l);
+        const int n = __popcll(__ballot(sample == v));
+        if (n > most) { most = n; common = v; }
+    }
     int n_small = 0, odd = 0;
     // the largest of this thread's bits as signed numbers, which is its largest value if that is not negative, and the
     // smallest as unsigned ones, which is its largest value if all are negative; by halves of the words
@@ -824,15 +839,16 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
     u16x2 least = {65535, 65535};
     // t: bits - kNucLow.  Its top four bits tell the ranges apart: 0, 1 and 8, 9 the bins of either sign, 2 - 4 larger
     // (also NaN), 5 - 7 and 13 - 15 smaller magnitudes, 10 - 12 larger negative ones (also NaN).
-    auto count_one = [&](uint32_t t) {
-        if (!(t & 0x6000u)) { atomicAdd(&sh.bin[(t & 0x1fffu) | ((t >> 2) & 0x2000u)], 1u); return; }
+    auto count_many = [&](uint32_t t, int n) {
+        if (!(t & 0x6000u)) { atomicAdd(&sh.bin[(t & 0x1fffu) | ((t >> 2) & 0x2000u)], static_cast<uint32_t>(n)); return; }
         const uint32_t bits = (t + kNucLow) & 0xffffu, mag = bits & 0x7fffu;
         if (mag > 0x7f80u) odd |= kOddNan;
         else if (bits == 0x7f80u) odd |= kOddInf;
-        else if (mag < static_cast<uint32_t>(kNucLow)) ++n_small;
+        else if (mag < static_cast<uint32_t>(kNucLow)) n_small += n;
         else if (!(bits & 0x8000u)) odd |= kOddLarge;
     };
-    for_vectors([&](const u32x4& q, int) {
+    auto count_one = [&](uint32_t t) { count_many(t, 1); };
+    auto count_vector = [&](const u32x4& q) {
         uint32_t t[4], outside = 0u;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
@@ -854,7 +870,34 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
 #pragma unroll
             for (int w = 0; w < 4; ++w) { count_one(t[w] & 0xffffu); count_one(t[w] >> 16); }
         }
-    });
+    };
+    if (most < kNucCommon) {
+        for_vectors([&](const u32x4& q, int) { count_vector(q); });
+    } else {
+        // (an element at a time, in little code: unrolled like the ordinary loop, this one's code made ordinary rows 2 - 7 % slower)
+        int n_common = 0;
+        for (int vi = tid; vi < n_vec; vi += kNucThreads) {
+            u32x4 q = scaled_bits(xv[vi]);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint32_t pair = q[w];
+                largest = __builtin_elementwise_max(largest, __builtin_bit_cast(i16x2, pair));
+                least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, pair));
+            }
+#pragma unroll 1
+            for (int k = 0; k < R::EPV; ++k) {
+                const uint32_t bits = q.x & 0xffffu;
+                q.x = (q.x >> 16) | (q.y << 16);
+                q.y = (q.y >> 16) | (q.z << 16);
+                q.z = (q.z >> 16) | (q.w << 16);
+                q.w >>= 16;
+                if (bits == common) ++n_common;
+                else count_one((bits - kNucLow) & 0xffffu);
+            }
+        }
+        n_common = wave_sum_int(n_common);
+        if (lane == 0 && n_common) count_many((common - kNucLow) & 0xffffu, n_common);
+    }
     auto count_scalar = [&](int64_t e) {
         const uint32_t bits = f32_to_bf16_bits(load_scaled(e));
         count_one((bits - kNucLow) & 0xffffu);
@@ -1065,6 +1108,7 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
         while ((static_cast<int64_t>(kNucThreads) << shift) < vocab) ++shift;
         const uint32_t bits = f32_to_bf16_bits(thr), both = bits | (bits << 16);
         uint32_t seen_n = 0u;
+        const bool many = n_eq >= vocab / 8;  // several to a vector, which are added together
         // (steps take turns at three counters: the one cleared in a step was last read two barriers ago)
         for (int base = 0, step = 0; base == 0 || base < n_vec; base += kNucStep, step = step == 2 ? 0 : step + 1) {
             int mine = 0;
@@ -1082,6 +1126,15 @@ template <int TEMP> __global__ __launch_bounds__(kNucThreads, 8) void nucleus_co
                     differ += __builtin_bit_cast(uint32_t, one);
                 }
                 if (differ != 0x00040004u) {
+                    if (many) {
+                        const int64_t index0 = head + static_cast<int64_t>(vi) * R::EPV;
+                        if (index0 >> shift == (index0 + R::EPV - 1) >> shift) {
+                            const uint32_t equal = R::EPV - (differ & 0xffffu) - (differ >> 16);
+                            atomicAdd(&sh.block[index0 >> shift], equal);
+                            mine += static_cast<int>(equal);
+                            return;
+                        }
+                    }
 #pragma unroll
                     for (int k = 0; k < R::EPV; ++k)
                         if (((q[k >> 1] >> (16 * (k & 1))) & 0xffffu) == bits) count(head + static_cast<int64_t>(vi) * R::EPV + k);

@@ -285,3 +285,49 @@ def test_short_rows_on_record_cost_a_fill_and_their_entries():
     shortest(lambda: out.zero_())
     backward = shortest(lambda: torch.ops.rl_amd.topk_topp_logprob_bwd(x, t, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP, *rec))
     assert backward < 8 * shortest(lambda: out.zero_())
+
+
+@pytest.mark.parametrize("value", [1.5, -1e9, -1e4, 0.0, -0.0, -math.inf, 7.0, 1e-20, math.nan, 2.0 ** 40])
+@pytest.mark.parametrize("vocab", [9, 64, 9001, 40008])
+def test_a_common_value(value, vocab):
+    """One value in none to all of a row's places, at random, at the front, at the end and every other place: whether it is counted
+    apart or with the others, and ties that are added up by the vector or one by one, the row comes out the same."""
+    g = torch.Generator(device=DEV).manual_seed(vocab)
+    x = torch.randn(1, 12, vocab, generator=g, device=DEV) * 3
+    at = torch.arange(vocab, device=DEV)
+    for i, share in enumerate((0.0, 0.1, 0.24, 0.26, 0.5, 0.8, 0.99, 1.0)):
+        x[0, i] = x[0, i].masked_fill(torch.rand(vocab, generator=g, device=DEV) < share, value)
+    x[0, 8] = x[0, 8].masked_fill(at < vocab * 3 // 4, value)
+    x[0, 9] = x[0, 9].masked_fill(at >= vocab // 3, value)
+    x[0, 10] = x[0, 10].masked_fill(at % 2 == 0, value)
+    for top_p in (0.3, 0.95):
+        _check(x.to(torch.bfloat16), top_p)
+    _check((x * 2).clamp(min=-3e38).to(torch.bfloat16), 0.9, temperature=2.0)
+
+
+def test_a_common_value_costs_no_more_than_others():
+    """Rows of which most places hold one value: counted in LDS one lane after the other they took 5 to 6 times what others take."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n, vocab = 512, 151936
+    x = torch.empty((1, n + 1, vocab), dtype=torch.bfloat16, device=DEV).normal_(0, 3, generator=g)
+    t = torch.randint(0, vocab, (1, n), generator=g, device=DEV)
+
+    def shortest(x):
+        times = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(4):
+                torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, n, 0, 0.95, 1.0, NRL_TEMP_RCP, False)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    shortest(x)
+    plain = shortest(x)
+    assert shortest(x.masked_fill(torch.rand(x.shape, generator=g, device=DEV) < 0.99, -1e9)) < 2.5 * plain
+    assert shortest(torch.full_like(x, 1.5)) < 2.5 * plain
