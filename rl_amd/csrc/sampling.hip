@@ -100,15 +100,19 @@ template <int CAP> struct SelShared {
 
 // k-th largest (1-based) of the workgroup's kChunks keys (kSub per thread, in registers), or a little less; every thread
 // returns it.  Two bits at a time from the top: the answer is the largest v with at least k keys >= v, v a multiple of
-// 2^LOW.  Below LOW the keys of a 16-bit type are constant, and for fp32 the bound needs no more than 20 bits (eight, ten and
-// ten rounds for bf16, fp16 and fp32, where all 32 bits take sixteen).  A round costs 3 * kSub ballots per wave, three LDS words per wave and one barrier (the buffers alternate), with
-// no atomics -- chunk maxima share their high bits, so a histogram would serialise on one bin.
-template <int DT> constexpr int kSelectLow = DT == NRL_BF16 ? 16 : 12;
+// 2^LOW, below which the keys of a 16-bit type are constant (eight and ten rounds for bf16 and fp16).  The 32 bits of fp32 end
+// where going on would leave out k / 32 + 2 keys at most: about ten rounds for logits of ordinary size, up to sixteen where
+// they share their leading bits (a fixed 20 bits let a whole row pass the bound at logits around 1e4: 1000 rows of V = 151 936,
+// top-k 50 110 us, 564 by way of the wide kernel).  A round costs 3 * kSub ballots per wave, three LDS words per wave and one
+// barrier (the buffers alternate), with no atomics -- chunk maxima share their high bits, so a histogram would serialise on
+// one bin.
+template <int DT> constexpr int kSelectLow = DT == NRL_BF16 ? 16 : DT == NRL_F16 ? 12 : 0;
 template <int LOW, int CAP>
 __device__ __forceinline__ uint32_t select_kth_largest(SelShared<CAP>& sh, const uint32_t (&keys)[kSub], int k) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     uint32_t v = 0u;
-    for (int bit = 30; bit >= LOW; bit -= 2) {  // two bits per round: three trial values, one barrier
+    int at_or_above = 0x7fffffff;  // (v = 0 is no answer: it would let -inf through; every key, chunks without elements too, is above that)
+    for (int bit = 30; bit >= LOW && (LOW > 0 || at_or_above > k + k / 32 + 2); bit -= 2) {  // two bits per round: three trial values, one barrier
         int cnt[3] = {0, 0, 0};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -127,6 +131,7 @@ __device__ __forceinline__ uint32_t select_kth_largest(SelShared<CAP>& sh, const
         // counts fall as the trial value rises: take the largest trial that still has k keys at or above it
         const uint32_t step = tot[2] >= k ? 3u : tot[1] >= k ? 2u : tot[0] >= k ? 1u : 0u;
         v |= step << bit;
+        at_or_above = step == 3u ? tot[2] : step == 2u ? tot[1] : step == 1u ? tot[0] : at_or_above;
     }
     return v;
 }

@@ -499,3 +499,58 @@ def test_nuclei_around_the_length_that_is_summed_in_double(nucleus):
     lp = rows_logprob_sampled(x, ids[None], rows, None, top_p, inference_only=True)[0]
     want = x64.gather(-1, ids[:, None])[:, 0] - x64.masked_fill(~keep, float("-inf")).logsumexp(-1)
     torch.testing.assert_close(lp.double(), want, rtol=0, atol=3e-6)  # fp32 logarithm and difference of values up to 9
+
+
+@pytest.mark.parametrize("vocab", [900, 2048, 9001, 40000])
+@pytest.mark.parametrize("top_k", [1, 50, 400, 2000])
+def test_fp32_rows_that_share_their_leading_bits(vocab, top_k):
+    """Logits around +-1e4 and 1e6 differ in their last bits only, logits of one value in none, logits at 1e-30 in all but their
+    first: the k-th largest and its ties come out as a sort gives them."""
+    g = torch.Generator().manual_seed(vocab + top_k)
+    n = 9
+    x = torch.randn(1, n + 1, vocab, generator=g) * 3
+    for i, off in enumerate((0.0, 1e4, -1e4, 1e6, 30.0)):
+        x[0, i] += off
+    x[0, 5] = 2.5
+    x[0, 6] *= 1e-30
+    x[0, 7] = (x[0, 7] * 4).round() / 4 + 1e4
+    x[0, 8, ::2] = float("-inf")
+    x = x.to(DEV)
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    t = x[:, :n].argmax(-1)
+    lp, thr, tie, lse, _ = torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, n, top_k, 1.0, 1.0, NRL_TEMP_RCP, False)
+    want = x[0, :n].topk(min(top_k, vocab), -1).values[:, -1]
+    if top_k > vocab // 2:
+        want[8] = x[0, 8][x[0, 8].isfinite()].min()   # -inf is never kept
+    assert torch.equal(thr[0], want) and not bool(tie.any())
+    z = x[0, :n].double()
+    full = z.masked_fill(z < want[:, None], float("-inf")).logsumexp(-1)
+    assert bool(((lse[0].double() - full).abs() <= 2.0 ** -23 * (2 + full.abs() + z.amax(-1).abs())).all())
+
+
+def test_fp32_rows_around_1e4_take_no_longer():
+    """A bound too coarse for such logits lets a whole row pass and sends it to the kernel for wide rows: 5 times as long."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n, vocab = 256, 151936
+    x = torch.empty((1, n + 1, vocab), device=DEV).normal_(0, 3, generator=g)
+    t = torch.randint(0, vocab, (1, n), generator=g, device=DEV)
+
+    def shortest(x):
+        times = []
+        for _ in range(8):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(8):
+                torch.ops.rl_amd.topk_topp_logprob_fwd(x, t, n, 50, 0.95, 1.0, NRL_TEMP_RCP, False)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    shortest(x)
+    assert shortest(x + 1e4) < 2 * shortest(x)
