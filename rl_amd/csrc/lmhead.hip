@@ -74,7 +74,7 @@ __device__ __forceinline__ int acc_row(int e, int lane) { return 8 * (e >> 2) + 
 // registers while slab k is consumed from one padded LDS buffer (row stride 72 elements).
 // ---------------------------------------------------------------------------------------------
 struct CoreA {
-    static constexpr int BM = 256, BN = 128, NI = 4, NJ = 2, BK = 64, LD = BK + 8, WAVES_N = 2;
+    static constexpr int BM = 256, BN = 128, NI = 4, NJ = 2, BK = 64, LD = BK + 8;
     static constexpr int LDS_BYTES = (BM + BN) * LD * 2;
     static constexpr int A_LOADS = BM * BK / 8 / GB_THREADS, B_LOADS = BN * BK / 8 / GB_THREADS;
     struct Regs {
@@ -169,7 +169,7 @@ struct CoreA {
 // against 12.6 with the key r & 7 and 32 without swizzling.  Per 16-wide k step a wave issues 8 fragment reads for 16 MFMAs.
 // ---------------------------------------------------------------------------------------------
 struct CoreB {
-    static constexpr int BM = 256, BN = 256, NI = 4, NJ = 4, BK = 64, WAVES_N = 2;
+    static constexpr int BM = 256, BN = 256, NI = 4, NJ = 4, BK = 64;
     static constexpr int TILE_BYTES = 256 * BK * 2;  // one operand, one buffer
     static constexpr int LDS_BYTES = 4 * TILE_BYTES;  // A0 A1 B0 B1
     static constexpr int ROUNDS = 256 * BK / 8 / GB_THREADS;  // direct loads per lane, operand and slab: 8
@@ -612,37 +612,31 @@ __device__ __forceinline__ float round_bf16(float v) { return bf16_bits_to_f32(f
 
 // How a launch covers its tile grid.  Workgroups go to the 8 XCDs (each with its own L2) round-robin by index, so index
 // w runs on XCD w % 8 as that XCD's (w / 8)-th workgroup; an XCD's 32 compute units hold one patch of px x py tiles at a
-// time (px * py <= 32), which share px A panels and py B panels through that L2.  A launch may carry several k ranges
-// (splits) of the same tile grid: their patches follow each other.
+// time (px * py <= 32), which share px A panels and py B panels through that L2.
 struct Patches {
     uint32_t px = 4, py = 8;
-    int splits = 1;
     __host__ __device__ int64_t along_x(int64_t nbx) const { return (nbx + px - 1) / px; }
     __host__ __device__ int64_t along_y(int64_t nby) const { return (nby + py - 1) / py; }
-    int64_t grid(int64_t nbx, int64_t nby) const { return (along_x(nbx) * along_y(nby) * splits + 7) / 8 * 8 * 32; }
+    int64_t grid(int64_t nbx, int64_t nby) const { return (along_x(nbx) * along_y(nby) + 7) / 8 * 8 * 32; }
     // How many times the busiest XCD fills its 32 compute units.  Patches at the edge of the grid are counted by the tiles
     // they really hold, on average: a compute unit takes the next workgroup when it is free, whatever its patch.
     double rounds(int64_t nbx, int64_t nby) const {
-        const int64_t patches = along_x(nbx) * along_y(nby) * splits, per_xcd = (patches + 7) / 8;
-        const double held = static_cast<double>(nbx) * nby * splits / patches;
+        const int64_t patches = along_x(nbx) * along_y(nby), per_xcd = (patches + 7) / 8;
+        const double held = static_cast<double>(nbx) * nby / patches;
         return static_cast<double>(static_cast<int64_t>(per_xcd * held / 32.0 + 0.999));
     }
 };
 
-// Tile coordinates (and k range) of workgroup w; slots and patches past the grid yield false.
-__device__ __forceinline__ bool patch_tile(const Patches& p, uint32_t w, int64_t nbx, int64_t nby, int64_t& bx, int64_t& by, int& split) {
+// Tile coordinates of workgroup w; slots and patches past the grid yield false.
+__device__ __forceinline__ bool patch_tile(const Patches& p, uint32_t w, int64_t nbx, int64_t nby, int64_t& bx, int64_t& by) {
     const uint32_t xcd = w & 7, s = w >> 3;
-    const uint32_t t = s & 31;
-    uint32_t patch = (s >> 5) * 8 + xcd;
-    const uint32_t npx = static_cast<uint32_t>(p.along_x(nbx)), npy = static_cast<uint32_t>(p.along_y(nby));
-    const uint32_t sp = patch / (npx * npy);
-    patch -= sp * npx * npy;
+    const uint32_t t = s & 31, patch = (s >> 5) * 8 + xcd;
+    const uint32_t npy = static_cast<uint32_t>(p.along_y(nby));
     const uint32_t ix = patch / npy, iy = patch - ix * npy, tx = t / p.py;
     // the divisions run on the vector unit; hand the (uniform) results back to scalar registers
     bx = __builtin_amdgcn_readfirstlane(static_cast<int>(ix * p.px + tx));
     by = __builtin_amdgcn_readfirstlane(static_cast<int>(iy * p.py + (t - tx * p.py)));
-    split = __builtin_amdgcn_readfirstlane(static_cast<int>(sp));
-    return tx < p.px && split < p.splits && bx < nbx && by < nby;
+    return tx < p.px && bx < nbx && by < nby;  // (past the last patch ix * px is past nbx)
 }
 
 // How a product of the backward covers its tiles.  The tiles (of every k range, one range after the other) are numbered along
@@ -745,8 +739,7 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_fwd_kernel(LmFwdArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     int64_t bx, by;
-    int one;
-    if (!patch_tile(a.patches, blockIdx.x, (a.op.n + BT - 1) / BT, a.n_splits, bx, by, one)) return;
+    if (!patch_tile(a.patches, blockIdx.x, (a.op.n + BT - 1) / BT, a.n_splits, bx, by)) return;
     const int64_t tok0 = bx * BT;
     const int split = static_cast<int>(by);
     const int64_t n_tiles = (a.op.m + BV - 1) / BV;
@@ -931,7 +924,7 @@ struct LmGradArgs {
 };
 
 // XCD patch of the recomputing gradient kernel, 8 token tiles x 4 vocabulary tiles: 1.7 % faster than 4 x 8
-constexpr Patches kGradPatches{8, 4, 1};
+constexpr Patches kGradPatches{8, 4};
 
 template <class Core>
 __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
@@ -942,8 +935,7 @@ __global__ __launch_bounds__(GB_THREADS) void lmhead_grad_kernel(LmGradArgs a) {
     const int wm = wave >> 1, wn = wave & 1;
     if (!resolve_live(a.op)) return;
     int64_t bx, by;
-    int one;
-    if (!patch_tile(kGradPatches, blockIdx.x, (a.op.m + BM - 1) / BM, (a.op.n + BN - 1) / BN, bx, by, one)) return;
+    if (!patch_tile(kGradPatches, blockIdx.x, (a.op.m + BM - 1) / BM, (a.op.n + BN - 1) / BN, bx, by)) return;
     const int64_t row0 = bx * BM, col0 = by * BN;
     {
         const int64_t grow = row0 + tid;
@@ -1161,7 +1153,7 @@ __global__ __launch_bounds__(GB_THREADS) void gemm_f32_kernel(GemmOperands op, S
     int split;
     if (!strip_tile(strips, blockIdx.x, (op.m + BM - 1) / BM, (op.n + BN - 1) / BN, bx, by, split)) return;
     if (!ACCUM && strips.splits > 1) {
-        // (as in patch_tile: the result of the division goes back to a scalar register, and with it all that follows)
+        // (as in strip_tile: the result of the division goes back to a scalar register, and with it all that follows)
         const int64_t per = __builtin_amdgcn_readfirstlane(static_cast<int>(((op.k + strips.splits - 1) / strips.splits + 63) / 64 * 64));
         const int64_t k0 = per * split;
         op.a += k0 * op.lda;  // (fragment-major, k a multiple of 32: the groups of 32 tokens are 32 lda apart)
@@ -1449,7 +1441,7 @@ struct FwdPlan {
 template <class Core> static FwdPlan fwd_plan(int64_t n, int64_t v, bool save) {
     const int64_t blocks = (n + Core::BN - 1) / Core::BN, tiles = (v + Core::BM - 1) / Core::BM;  // token blocks, vocabulary tiles
     const uint32_t want_px = save ? 4u : 8u;
-    FwdPlan best{Patches{want_px, 32u / want_px, 1}, 1};
+    FwdPlan best{Patches{want_px, 32u / want_px}, 1};
     double best_cost = 1e300;
     for (uint32_t px = 1; px <= 8; ++px) {
         if (px > 1 && static_cast<int64_t>(px) >= 2 * blocks) break;
@@ -1457,7 +1449,7 @@ template <class Core> static FwdPlan fwd_plan(int64_t n, int64_t v, bool save) {
         const int64_t nx = (blocks + px - 1) / px;
         for (int64_t ny = 1; ny <= 64; ++ny) {
             const int64_t splits = ny * py < tiles ? ny * py : tiles;
-            const Patches p{px, py, 1};
+            const Patches p{px, py};
             // (+ 1: what a workgroup spends before its first tile and after its last one, about half a tile each)
             double cost = p.rounds(blocks, splits) * static_cast<double>((tiles + splits - 1) / splits + 1);
             cost *= 1.0 + 0.002 * (32.0 * (px + py) / (px * py) - 12.0);  // operand panels an XCD reads per tile, against 4 x 8
