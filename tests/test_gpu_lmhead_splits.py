@@ -110,3 +110,22 @@ def test_the_one_hot_term_of_dh_is_added_once(h, v):
     for k in (kept, None):
         dh, _ = _ops().lmhead_logprob_bwd(hid.to(DEV), w.to(DEV), tgt.to(DEV), lse, up.to(DEV), 0, v, k)
         assert (dh.double().cpu() - want).abs().max().item() <= bound
+
+
+@pytest.mark.parametrize("n,h,v,pad", [(300, 256, 2000, 8), (70, 264, 700, 248), (512, 64, 9001, 64), (5, 8, 65, 1016)])
+@pytest.mark.parametrize("keep", [False, True])
+def test_weights_and_hidden_states_with_rows_further_apart(n, h, v, pad, keep):
+    """A weight that is a column slice of a wider one: dH's product reads it with its own row stride.  The same bits as of a copy."""
+    g = torch.Generator().manual_seed(n + pad)
+    hid = torch.randn(n, h + pad, generator=g).to(torch.bfloat16).to(DEV)[:, pad:]
+    w = (torch.randn(v, h + pad, generator=g) * 0.05).to(torch.bfloat16).to(DEV)[:, pad:]
+    assert w.stride(0) == h + pad and w.data_ptr() % 16 == 0
+    tgt = torch.randint(0, v, (n,), generator=g).to(DEV)
+    up = torch.randn(n, generator=g).to(DEV)
+    up[1::4] = 0
+    out = []
+    for a, b in ((hid, w), (hid.contiguous(), w.contiguous())):
+        lp, lse, kept = _ops().lmhead_logprob_fwd(a, b, tgt, 0, v, keep)
+        out.append((lp, lse) + tuple(_ops().lmhead_logprob_bwd(a, b, tgt, lse, up, 0, v, kept if keep else None)))
+    for x, y in zip(*out):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
