@@ -116,8 +116,9 @@ __global__ void group_stats_kernel(const int32_t* group, int64_t batch, const fl
 // The three launches in one workgroup, for batches small enough: a wave hashes, then compares, a row at a time; hashes and
 // what the statistics read stay in LDS.  The same comparisons and the same sums in the same order.  Bound by latency, the
 // launches' and that of a wave's rows one after the other.  us, back to back in a graph, groups of 8, against three launches:
-// 8 rows of 64 tokens 4.0 and 6.6, 16 of 256 5.3 and 7.1, 32 of 256 7.9 and 8.0 (and the host launches once).  The limits are
-// where one workgroup stops winning: 32 rows of 512 10.9 and 8.3, 64 of 64 11.9 and 9.0, 8 of 1024 6.5 and 7.4, 16 9.7 and 7.8.
+// 8 rows of 64 tokens 4.0 and 6.6, 16 of 256 5.3 and 7.1, 32 of 256 7.9 and 8.0 (and the host launches once).  Beyond
+// the limits one workgroup loses, 32 rows of 512 10.9 and 8.3, 64 of 64 11.9 and 9.0, 16 of 1024 9.7 and 7.8, but for a few long
+// rows (8 of 1024: 6.5 and 7.4), which two plain limits leave to the three launches.
 constexpr int kSmallThreads = 1024, kSmallWaves = kSmallThreads / kWave;
 constexpr int64_t kSmallBatch = 32, kSmallLen = 256;
 
