@@ -349,7 +349,9 @@ struct CoreB {
 //       dH (GA false): A = W [K, M], a slab is 64 rows of 512 bytes; the 16-byte chunk c of row r sits at c ^ ((r & 3) << 1).
 //       dW (GA true): A = G, K the tokens: a slab is 2 x 16 blocks, each copied as it is but for the order of its 16-byte
 //         units: unit (token t, ids 8 h ..) of the block of ids 16 b .. sits at t ^ 4 h ^ 8 (b & 1) of half h.
-//     Either way the 16 lanes of a read fall on different banks (4.1 cycles per read and wave; 8.1 unswizzled; full rate 4).
+//     Either way the 16 lanes that share a block fall on different banks.  The counters see no conflict in dW; in dH lanes of two
+//     blocks read at the same time meet, half of its LDS cycles (1.25e9 of 2.49e9 for 16384 tokens): the LDS is at work in 44 %
+//     of the kernel's cycles then, the matrix cores in 88 %.
 // Bound by the matrix cores under the power limit, for short batches by the stores of dW.  H 4096, V 151936, us for (dH, dW, the
 // gradient and the layout kernels), against products from W^T and G^T laid out in memory (a [M, K] operand A through LDS):
 // 6912 tokens 6615 + 6290 + 830 and 6863 + 6040 + 1985; 2048: 1830 + 2035 + 240 and 1800 + 2098 + 810; 448: 490 + 773 + 65 and 483
