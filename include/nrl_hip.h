@@ -161,7 +161,8 @@ int nrl_logprob_packed_bwd(const void* logits, int32_t dtype, int64_t total_toke
  * sorting the vocabulary.  rows->vocab_start must be 0 and vocab_end == vocab.
  * top_k <= 0 and top_p >= 1 switch the respective filter off (at least one must be on).
  * Per row the forward emits the keep predicate (thr_out, tie_out): element v is kept iff
- * x_v > thr, or x_v == thr and v >= tie; and lse_kept_out, the log-sum-exp over the kept set.
+ * x_v > thr, or x_v == thr and v >= tie; and lse_kept_out, the log-sum-exp over the kept set.  (tie 0x7fffffff
+ * means every v: a bf16 row with +inf under top-p alone, whose log-sum-exp and gradient are NaN.)
  * logprob_out (may be NULL, then rows->targets may be NULL): x_t - lse_kept, or -inf when the target
  * was filtered out.  logprob_unfiltered_out / lse_full_out (may be NULL): the same row's unfiltered
  * logprob (what the KL penalty needs, loss/utils.py:104-118) from the same pass.

@@ -1743,7 +1743,7 @@ constexpr int64_t kFillSpan = 256 * 1024, kFillShortRow = 8 * 1024, kFillSmall =
 // fill (4096 rows of V = 32 000: 32.7 us without, 34.5 with them) or several workgroups per row are for nothing.  Top-p alone
 // leaves room for this many; nearly flat rows do not fit.
 constexpr int kMixedRecord = 128;
-constexpr int kFillFlags = 1024, kFillRound = kFillFlags / 3;
+constexpr int kFillFlags = 1024, kFillRound = kFillFlags / 2;  // flags, and spans, of a round: a span touches two rows or more
 template <int DT> __global__ __launch_bounds__(256) void fill_zero_rows_kernel(SelBwdArgs a, int64_t total_bytes, double row_inverse) {
     __shared__ uint8_t clear[kFillFlags];
     __shared__ uint32_t first_row[kFillRound];  // of a span

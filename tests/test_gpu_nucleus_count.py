@@ -331,3 +331,28 @@ def test_a_common_value_costs_no_more_than_others():
     plain = shortest(x)
     assert shortest(x.masked_fill(torch.rand(x.shape, generator=g, device=DEV) < 0.99, -1e9)) < 2.5 * plain
     assert shortest(torch.full_like(x, 1.5)) < 2.5 * plain
+
+
+def test_a_gradient_of_more_spans_than_a_round_of_flags_holds():
+    """88 000 rows just over a 256 KiB span, 23 GB: every workgroup reads flags for more spans than fit one round of two rows each.
+    What is not cleared or written keeps the NaN that the buffer's memory held before."""
+    from rl_amd import ops  # noqa: F401
+    from rl_amd._lib import NRL_TEMP_RCP
+
+    n, vocab = 88000, 131080
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 64 GB of free GPU memory")
+    x = torch.zeros(1, n, vocab, dtype=torch.bfloat16, device=DEV)
+    row = torch.arange(n, device=DEV).view(1, n)
+    at = (row * 7919) % vocab
+    up = torch.where(row % 5 == 3, 0.0, 2.0)
+    cnt = torch.where(row % 7 == 2, -1, 1).to(torch.int32)                 # every seventh row streams: none of it is kept
+    thr, tie = torch.full((1, n), 0.5, device=DEV), torch.zeros(1, n, dtype=torch.int32, device=DEV)
+    lse = torch.full((1, n), math.log(2.0), device=DEV)
+    idx = at.unsqueeze(-1).to(torch.int32).expand(1, n, 128).contiguous()
+    val = torch.zeros(1, n, 128, device=DEV)
+    torch.full((x.numel() + (1 << 21),), math.nan, dtype=torch.bfloat16, device=DEV)
+    d = torch.ops.rl_amd.topk_topp_logprob_bwd(x, at, thr, tie, lse, up, n, 1.0, NRL_TEMP_RCP, cnt, idx, val)
+    want = torch.where((cnt > 0) & (up != 0), 1.0, 0.0)                   # (1 - exp(0 - log 2)) * 2
+    assert torch.equal(d.gather(-1, at.unsqueeze(-1))[..., 0].float(), want)
+    assert sum(int(torch.count_nonzero(part)) for part in d[0].split(4000)) == int(want.sum())
