@@ -111,8 +111,10 @@ template <int LOW, int CAP>
 __device__ __forceinline__ uint32_t select_kth_largest(SelShared<CAP>& sh, const uint32_t (&keys)[kSub], int k) {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     uint32_t v = 0u;
-    int at_or_above = 0x7fffffff;  // (v = 0 is no answer: it would let -inf through; every key, chunks without elements too, is above that)
-    for (int bit = 30; bit >= LOW && (LOW > 0 || at_or_above > k + k / 32 + 2); bit -= 2) {  // two bits per round: three trial values, one barrier
+    // (v = 0 is no answer: it would let -inf through; every key, of chunks without elements too, is above that)
+    int at_or_above = 0x7fffffff;
+    // two bits per round: three trial values, one barrier
+    for (int bit = 30; bit >= LOW && (LOW > 0 || at_or_above > k + k / 32 + 2); bit -= 2) {
         int cnt[3] = {0, 0, 0};
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -714,9 +716,10 @@ __global__ __launch_bounds__(kSelBlock) void topk_topp_fwd_kernel(SelArgs a) {
 // larger value, is left to the wide kernel.  Larger negative values weigh nothing next to any value of the bins.
 // Counts are integers and every sum runs in a fixed order, so a row comes out the same every time.
 //
-// What bounds it: the LDS atomics of the first pass, about 15 cycles per 64 elements and compute unit where these differ (lanes
-// that add to one word take turns: see the common value), where the row itself would arrive in 11; then the latency of the steps between two passes, which two workgroups of 1024 threads per
-// compute unit cover for each other (workgroups of 512, of which the bins admit two as well: 195 us).  With a kept-set
+// What bounds it: the LDS atomics of the first pass, about 15 cycles per 64 elements and compute unit where these differ
+// (lanes that add to one word take turns: see the common value), where the row itself would arrive in 11, and next to them the
+// vector unit; then the latency of the steps between two passes, which two workgroups of 1024 threads per compute unit cover
+// for each other (workgroups of 512, of which the bins admit two as well: 195 us).  With a kept-set
 // record, top_p 0.95, standard deviations 2 - 6, against candidate lists, a sort and the radix descent of the wide kernel:
 // 1499 rows of V = 151 936 145 us (62 to read the rows) and 726; 180 rows of V = 205 350 47 and 470; 4000 rows of 32 000
 // with a temperature 158 and 408; 800 rows of 9001 37 and 185.  Rows with a common value, 1499 of V = 151 936, against the same
@@ -1764,8 +1767,9 @@ template <int DT> __global__ __launch_bounds__(256) void fill_zero_rows_kernel(S
         for (int64_t s0 = blockIdx.x * kFillSpan; s0 < total_bytes; s0 += gridDim.x * kFillSpan) clear_run(s0, span_end(s0));
         return;
     }
-    const uint32_t per = static_cast<uint32_t>(kFillSpan) / static_cast<uint32_t>(row_bytes < kFillSpan ? row_bytes : kFillSpan + 1) + 2;  // most rows that a span touches
-    const uint32_t round = kFillFlags / per;                                                                                         // spans at a time
+    // most rows that a span touches, and spans whose flags are held at a time
+    const uint32_t per = static_cast<uint32_t>(kFillSpan) / static_cast<uint32_t>(row_bytes < kFillSpan ? row_bytes : kFillSpan + 1) + 2;
+    const uint32_t round = kFillFlags / per;
     for (int64_t base = blockIdx.x * kFillSpan; base < total_bytes; base += round * gridDim.x * kFillSpan) {
         for (uint32_t i = threadIdx.x; i < round * per; i += 256) {
             const uint32_t k = i / per, j = i - k * per;
